@@ -190,7 +190,7 @@ typedef struct pat_flat_bucket {
   int32_t first;       /* launch buckets: position of the first box in the parent's
                           launch order; plan buckets: 0                                   */
   int32_t flags;       /* PAT_BUCKET_* hints that hold for the bucket                    */
-  int32_t pad_;
+  int32_t num_items;   /* launch buckets: rows of the item table behind kv (see PAT_BUCKET_ITEMS), 0 = none */
   int64_t q_table, q_slot, block_table, num_seqs, rank, kv;
 } pat_flat_bucket;
 
@@ -239,7 +239,7 @@ typedef struct pat_fwd_bucket {
   const int32_t* block_table; /* [num_boxes, block_table_stride]              */
   const int32_t* num_seqs;    /* [num_boxes]                                  */
   const int32_t* rank;        /* [num_boxes]                                  */
-  const int32_t* kv;          /* [num_boxes]                                  */
+  const int32_t* kv;          /* [num_boxes] (and see PAT_BUCKET_ITEMS)       */
   const int32_t* q_slot;      /* optional [num_boxes, q_table_stride] (see     */
                               /* pat_bucket_view.q_slot); NULL: use CTA_rank   */
   /* Filing by CTA_rank (q_slot NULL) is what the reference does and is right only where every
@@ -254,6 +254,7 @@ typedef struct pat_fwd_bucket {
   int32_t max_blocks;         /* valid columns of block_table                 */
   int32_t mnw[3];
   int32_t flags;              /* PAT_BUCKET_* hints, 0 when nothing is known  */
+  int32_t num_items;          /* read only with PAT_BUCKET_ITEMS              */
 } pat_fwd_bucket;
 
 /* Hint: no box of the bucket is shorter than 3/4 of its widest box (the launcher cannot see
@@ -261,13 +262,17 @@ typedef struct pat_fwd_bucket {
  * (contiguous reads across heads; safe only when no workgroup outlasts the others by much).
  * A wrong hint costs time, never correctness. */
 #define PAT_BUCKET_EVEN 1
+/* kv[num_boxes] is followed in memory by an item table, int32 [num_items, 2]: boxes of the bucket (by row) that
+ * attend to the same blocks with different sequences (boxes of one tree node) in twos, -1 = no second box; every box
+ * stands in exactly one item. A launch may serve the two boxes of an item with one workgroup, or ignore the table. */
+#define PAT_BUCKET_ITEMS 2
 
 /* Overrides of the launch geometry. pat_fwd_set_tuning sets them process-wide (a tuning and test
  * aid, not meant to change while launches are in flight on other threads); pat_fwd_args.tuning sets
  * them for one launch (what pat_fwd_autotune's result is for). 0 / -1 = automatic, as noted per field. The
  * initial values come from the environment variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS,
  * PAT_HEAD_PER_WAVE_TOKENS, PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS,
- * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, read once; pat_fwd_set_tuning(NULL) reads them again. */
+ * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, PAT_TALL_ROWS, PAT_PAIRS, read once; pat_fwd_set_tuning(NULL) reads them again. */
 typedef struct pat_fwd_tuning {
   int32_t chunk_tokens;              /* KV tokens per workgroup, boxes <= 16 rows (0: automatic)   */
   int32_t tall_chunk_tokens;         /* same for boxes of 17..64 rows (0: automatic)                */
@@ -281,7 +286,8 @@ typedef struct pat_fwd_tuning {
   int32_t tall_rows;                 /* rows per wave on boxes of 17..64 rows: 32 (32x32x16 MFMA    */
                                      /* tiles, 2 workgroups per CU at head_dim 128), 16 (16x16x32,  */
                                      /* 3 per CU), 0: chosen per launch from its sizes              */
-  int32_t reserved;                  /* 0                                                           */
+  int32_t pairs;                     /* two boxes of an item served by one workgroup (32-row form): */
+                                     /* 0 chosen per launch from its sizes, 1 always, 2 never       */
 } pat_fwd_tuning;
 int pat_fwd_set_tuning(const pat_fwd_tuning* tuning);
 int pat_fwd_get_tuning(pat_fwd_tuning* out);

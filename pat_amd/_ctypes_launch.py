@@ -34,7 +34,7 @@ class _Launch:
 
 def prepare(q, k, v, num_split, q_tables, block_tables, num_seqs, ranks, kvs, MNW, max_split,
             max_seqs, max_blocks, scale, out, lse, slot_tables=None, bucket_flags=None, autotune=False, tuning=None,
-            build_records=True) -> _Launch:
+            build_records=True, items=None) -> _Launch:
     lib = _lib.load()
     # --- checks that need tensor metadata (csrc/api.h:131-181, :256-277) -----------------
     _check(q.dtype in (torch.float16, torch.bfloat16), "only support fp16 and bf16 data type")
@@ -87,6 +87,9 @@ def prepare(q, k, v, num_split, q_tables, block_tables, num_seqs, ranks, kvs, MN
         fb.num_boxes, fb.max_seqs, fb.max_blocks = ctas, qt.shape[1], bt.shape[1]
         fb.mnw[0], fb.mnw[1], fb.mnw[2] = int(MNW[i][0]), int(MNW[i][1]), int(MNW[i][2])
         fb.flags = int(bucket_flags[i]) if bucket_flags else 0
+        if items is not None and items[i].numel():
+            _check(items[i].data_ptr() == kv.data_ptr() + 4 * ctas, "an item table stands right behind its bucket's kv table")
+            fb.flags, fb.num_items = fb.flags | _lib.PAT_BUCKET_ITEMS, items[i].shape[0]
 
     a = _lib.FwdArgs()
     a.dtype = _lib.PAT_DTYPE_BF16 if q.dtype == torch.bfloat16 else _lib.PAT_DTYPE_F16
@@ -152,7 +155,7 @@ def prepare(q, k, v, num_split, q_tables, block_tables, num_seqs, ranks, kvs, MN
     # plan tensors stay referenced as long as the prepared launch does; q/k/v/out are the
     # caller's for the duration of the call only
     L.keep = (num_split, list(q_tables), list(block_tables), list(num_seqs), list(ranks), list(kvs),
-              None if slot_tables is None else list(slot_tables), derived, records)
+              None if slot_tables is None else list(slot_tables), derived, records, None if items is None else list(items))
     L.workspace = None
     return L
 

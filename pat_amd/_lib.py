@@ -58,7 +58,7 @@ class PlanView(C.Structure):
 class FlatBucket(C.Structure):
     _fields_ = [("mnw", C.c_int32 * 3), ("num_boxes", C.c_int32), ("max_seqs", C.c_int32),
                 ("max_blocks", C.c_int32), ("parent", C.c_int32), ("first", C.c_int32),
-                ("flags", C.c_int32), ("pad_", C.c_int32), ("q_table", C.c_int64), ("q_slot", C.c_int64), ("block_table", C.c_int64),
+                ("flags", C.c_int32), ("num_items", C.c_int32), ("q_table", C.c_int64), ("q_slot", C.c_int64), ("block_table", C.c_int64),
                 ("num_seqs", C.c_int64), ("rank", C.c_int64), ("kv", C.c_int64)]
 
 
@@ -79,10 +79,11 @@ class FwdBucket(C.Structure):
                 ("rank", C.c_void_p), ("kv", C.c_void_p), ("q_slot", C.c_void_p),
                 ("q_table_stride", C.c_int64), ("block_table_stride", C.c_int64),
                 ("num_boxes", C.c_int32), ("max_seqs", C.c_int32), ("max_blocks", C.c_int32),
-                ("mnw", C.c_int32 * 3), ("flags", C.c_int32)]
+                ("mnw", C.c_int32 * 3), ("flags", C.c_int32), ("num_items", C.c_int32)]
 
 
 PAT_BUCKET_EVEN = 1
+PAT_BUCKET_ITEMS = 2
 
 
 class BaselineArgs(C.Structure):
@@ -100,7 +101,7 @@ class FwdTuning(C.Structure):
     _fields_ = [("chunk_tokens", C.c_int32), ("tall_chunk_tokens", C.c_int32),
                 ("head_per_wave_tokens", C.c_int32), ("head_per_wave_long_tokens", C.c_int32),
                 ("head_per_wave_long_wgs", C.c_int64), ("equalize_chunks", C.c_int32),
-                ("direct_out", C.c_int32), ("tall_rows", C.c_int32), ("reserved", C.c_int32)]
+                ("direct_out", C.c_int32), ("tall_rows", C.c_int32), ("pairs", C.c_int32)]
 
     @classmethod
     def automatic(cls) -> "FwdTuning":

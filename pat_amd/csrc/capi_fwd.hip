@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -27,6 +28,7 @@ constexpr int kTargetWgsPerCU = 2;  // what fits at once: 2 workgroups of 4 wave
 constexpr int kMinChunk = 128;      // tokens
 constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
+constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
 constexpr int kLongHeadPerWaveChunk = 1024;   // tokens a wave walks alone (long boxes, a kv head per wave)
 // workgroups of the split kernel a CU holds at once: 3, or 2 at head_dim 128 with 32-row tiles on tall boxes
@@ -44,13 +46,14 @@ inline int row_tiles(int m_label) { return m_label <= 16 ? 1 : (m_label <= 32 ? 
 
 // Overrides of the launch geometry (pat_fwd_set_tuning). The defaults come from the environment
 // variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS, PAT_HEAD_PER_WAVE_TOKENS,
-// PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS, PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT and
-// PAT_TALL_ROWS, read once per process: no launch reads the environment.
+// PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS, PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT,
+// PAT_TALL_ROWS and PAT_PAIRS, read once per process: no launch reads the environment.
 pat_fwd_tuning env_tuning() {
   pat_fwd_tuning t;
   t.chunk_tokens = 0; t.tall_chunk_tokens = 0; t.head_per_wave_tokens = -1;
   t.head_per_wave_long_wgs = -1; t.head_per_wave_long_tokens = 0; t.equalize_chunks = -1; t.direct_out = -1;
-  t.tall_rows = 0; t.reserved = 0;
+  t.tall_rows = 0; t.pairs = 0;
+  if (const char* e = std::getenv("PAT_PAIRS")) t.pairs = std::atoi(e);
   if (const char* e = std::getenv("PAT_TALL_ROWS")) t.tall_rows = std::atoi(e);
   if (const char* e = std::getenv("PAT_CHUNK_TOKENS")) t.chunk_tokens = std::atoi(e);
   if (const char* e = std::getenv("PAT_TALL_CHUNK_TOKENS")) t.tall_chunk_tokens = std::atoi(e);
@@ -86,10 +89,17 @@ struct Geometry {
   int bucket_heads_per_wg[kMaxBuckets] = {0};   // 1, or kWaves: one kv head per wave
   int64_t total_wgs = 0;
   int tall_rows = 32;        // rows per wave on boxes of 17..64 rows: 32 or 16 (the split kernel's instance)
+  bool tall_apart = false;   // 32-row form: K and V tiles handed over apart
+  bool pairs = false;        // the two boxes of an item (pat_fwd_bucket.items) are served by one workgroup
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
   // launch records (one per workgroup): entries per record and bytes between records
   int record_max_seqs = 0, record_max_pages = 0, record_stride = 0;
 };
+
+// Work items of a bucket along the box axis.
+inline int64_t items_of(const pat_fwd_bucket& b, bool pairs) {
+  return pairs && (b.flags & PAT_BUCKET_ITEMS) && row_tiles(b.mnw[0]) > 1 ? b.num_items : b.num_boxes;
+}
 
 int check_args(const pat_fwd_args* a) {
   if (a == nullptr) return fail(PAT_ERR_INVALID, "args is NULL");
@@ -151,6 +161,8 @@ int check_args(const pat_fwd_args* a) {
       return fail(PAT_ERR_INVALID, "plan tables must be device int32 tensors" + at);
     if (b.q_table_stride < b.max_seqs || b.block_table_stride < b.max_blocks)
       return fail(PAT_ERR_INVALID, "plan table row stride smaller than its width" + at);
+    if ((b.flags & PAT_BUCKET_ITEMS) && (b.num_items > b.num_boxes || b.num_items < (b.num_boxes + 1) / 2))
+      return fail(PAT_ERR_INVALID, "a bucket's items hold one or two of its boxes each" + at);
     if (b.q_table_stride > INT32_MAX || b.block_table_stride > INT32_MAX)
       return fail(PAT_ERR_INVALID, "plan table row stride too large" + at);
     if ((int64_t)b.max_seqs * ratio > 64)
@@ -160,6 +172,30 @@ int check_args(const pat_fwd_args* a) {
       return fail(PAT_ERR_INVALID, "a box packs more rows (sequences x heads per kv head) than its bucket's tile_q" + at);
   }
   return PAT_OK;
+}
+
+// Times of a launch estimated from sizes alone (us): what its <= 16-row boxes take to stream (~5.8 TB/s; ragged
+// buckets, without the PAT_BUCKET_EVEN hint, hold ~0.6 of their widest box on average), what its tall boxes take
+// spread over all CUs, and the longest tall box walked by one workgroup. A super-step of 64 tokens takes ~1.25 us for
+// one box and ~1.5 us for two (32-row form); in the 16-row form 1.7 us alone, ~3 us beside two others on the CU.
+struct LaunchEstimate { double short_us = 0., tall_us = 0., chain_us = 0.; };
+constexpr double kShortestLaunchUs = 5.5;
+LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs) {
+  LaunchEstimate e;
+  for (int i = 0; i < a->num_buckets; ++i) {
+    const pat_fwd_bucket& b = a->buckets[i];
+    if (b.num_boxes <= 0) continue;
+    const double tokens = (double)b.max_blocks * a->page_size;
+    if (row_tiles(b.mnw[0]) > 1) {
+      const int64_t items = items_of(b, pairs);
+      const double step_us = tall_rows == 16 ? 1.7 : (items < b.num_boxes ? 1.5 : 1.25);
+      e.tall_us += tokens * (double)(items * a->kv_heads) / 64. * step_us / kNumCUs;
+      e.chain_us = std::max(e.chain_us, tokens / 64. * (tall_rows == 16 ? 3.0 : step_us));
+    } else {
+      e.short_us += tokens * (double)b.num_boxes * a->kv_heads * ((b.flags & PAT_BUCKET_EVEN) ? 1.0 : 0.6) * a->head_dim * 4. / 5.8e6;
+    }
+  }
+  return e;
 }
 
 // Launch geometry. A workgroup streams one chunk of one box's KV for one kv head; a bucket
@@ -172,8 +208,8 @@ int check_args(const pat_fwd_args* a) {
 //    write 16..32 KB of partial output per workgroup: their chunk is at least 256 tokens, and
 //    longer when they alone would still fill the device.
 // pat_fwd_tuning.chunk_tokens / tall_chunk_tokens override the two sizes (tuning aid).
-// (tall_rows: the form of the tall path the geometry is made for, 16 or 32)
-int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
+// (tall_rows: the form of the tall path the geometry is made for, 16 or 32; pairs: items of two boxes as one workgroup)
+int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pairs) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
   const int page = a->page_size;
   const int64_t unit = (int64_t)page * kStepTokens / gcd64(page, kStepTokens);  // lcm(page, 32)
@@ -186,6 +222,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     if (row_tiles(a->buckets[i].mnw[0]) == 1) work += w;
   }
   g->tall_rows = tall_rows;
+  g->pairs = pairs;
   const int64_t resident = (int64_t)resident_wgs_per_cu(a->head_dim, tall_rows) * kNumCUs;
   int64_t chunk = tune.chunk_tokens, tall = tune.tall_chunk_tokens;
   const bool env_tall = tall > 0, env_chunk = chunk > 0;
@@ -196,21 +233,19 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     chunk = std::max<int64_t>(kMinChunk, std::min<int64_t>(kMaxChunk, chunk));
   }
   if (tall <= 0) {
-    // Tall boxes are cut only as far as it takes to have about three workgroups per eight CUs (with
-    // fewer, a tall workgroup's chain of 64-token super-steps is the launch's critical path:
-    // 2048 tokens of a lone box run ~45 us); beyond that every further piece only adds 16-32 KB of
-    // partial rows and a merge slot per row. Measured on the benchmark workloads: the shared
-    // 2048-token prefix of 64 requests (4 boxes x 8 kv heads) is fastest in 3-4 pieces, 16 boxes
-    // and more uncut.
-    int64_t tall_box_heads = 0, widest_tall = 0;
+    // Tall boxes are cut only as far as it takes for a tall workgroup's chain of 64-token super-steps not to
+    // outlast the launch: the estimated time of the whole launch (and never less than kShortestLaunchUs: that
+    // much is launch, prologue and tail whatever the work), over the chain of an uncut box. Beyond that every further
+    // piece only adds 16-32 KB of partial rows and a merge slot per row. Measured (us per call by piece): a
+    // 2048-token prefix of 64 requests, 8 kv heads: 512 tokens 25.2, 768 22.2, 1536 25.5; 16 boxes of 1408 tokens:
+    // 512 35.4, 768-1024 32.4, uncut 36; 8 boxes of 1536 tokens, 8 kv heads, 16-row form: 768 71.7, uncut 75.5; 24 rows over 784 tokens, 32 kv heads: 512 18.4, uncut 19.2; 17 boxes of
+    // 864-1728 tokens, 2 kv heads: 256 18.1, 384 18.4, 768 19.5, uncut 23.4; one box of 288 tokens, 8 kv heads: 256 12.5, uncut 13.8.
+    int64_t widest_tall = 0;
     for (int i = 0; i < a->num_buckets; ++i)
-      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0) {
-        tall_box_heads += (int64_t)a->buckets[i].num_boxes * a->kv_heads;
+      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0)
         widest_tall = std::max<int64_t>(widest_tall, (int64_t)a->buckets[i].max_blocks * page);
-      }
-    // (the 16-row form's steps are slower: it wants a tall workgroup per two CUs)
-    const int64_t want_tall_wgs = tall_rows == 32 ? 3 * kNumCUs / 8 : kNumCUs / 2;
-    const int64_t pieces = tall_box_heads > 0 ? std::max<int64_t>(1, ceil_div64(want_tall_wgs, tall_box_heads)) : 1;
+    const LaunchEstimate est = estimate_launch(a, tall_rows, pairs);
+    const int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil(est.chain_us / std::max(est.tall_us + est.short_us, kShortestLaunchUs)));
     tall = ceil_div64(ceil_div64(widest_tall, pieces), 128) * 128;
     tall = std::max<int64_t>(kTallChunk, std::min<int64_t>(kMaxChunk, tall));
   }
@@ -222,7 +257,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     int64_t n_tall = 0;
     for (int i = 0; i < a->num_buckets; ++i)
       if (row_tiles(a->buckets[i].mnw[0]) > 1)
-        n_tall += (int64_t)a->buckets[i].num_boxes *
+        n_tall += items_of(a->buckets[i], pairs) *
                   std::max<int64_t>(1, ceil_div64((int64_t)a->buckets[i].max_blocks * page, round_unit(tall))) * a->kv_heads;
     if (n_tall > kNumCUs) {
       const int64_t slots = std::max<int64_t>(kNumCUs, resident - n_tall);
@@ -261,7 +296,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
   for (int i = 0; i < a->num_buckets; ++i) {
     const bool is_tall = row_tiles(a->buckets[i].mnw[0]) > 1;
     const int64_t tok = (int64_t)a->buckets[i].max_blocks * page;
-    const int64_t wgs = (int64_t)a->buckets[i].num_boxes * std::max<int64_t>(1, ceil_div64(tok, is_tall ? g->tall_chunk : g->chunk)) * a->kv_heads;
+    const int64_t wgs = items_of(a->buckets[i], pairs) * std::max<int64_t>(1, ceil_div64(tok, is_tall ? g->tall_chunk : g->chunk)) * a->kv_heads;
     (is_tall ? kind_tall_wgs : kind_short_wgs) += wgs;
   }
   const int equalize = tune.equalize_chunks;   // 0/1 override the rule below (tuning aid)
@@ -269,6 +304,10 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     const int64_t tok = (int64_t)a->buckets[i].max_blocks * page;
     int64_t c = row_tiles(a->buckets[i].mnw[0]) > 1 ? g->tall_chunk : g->chunk;
     while (ceil_div64(tok, c) > kMaxChunksPerRank && c + unit <= cap) c += unit;   // bounded slots per box
+    if (row_tiles(a->buckets[i].mnw[0]) > 1 && tall_rows == 32 && std::min(c, tok) > kMaxTall32Tokens) {
+      g->tall_rows = 0;   // a piece longer than this form takes (see plan_geometry)
+      return PAT_OK;
+    }
     if (ceil_div64(tok, c) > kMaxChunksPerRank)
       return fail(PAT_ERR_INVALID, "a box spans more KV blocks than one launch supports");
     const int n = (int)std::max<int64_t>(1, ceil_div64(tok, c));
@@ -283,7 +322,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     g->bucket_chunks[i] = n;
     g->bucket_heads_per_wg[i] = 1;
     g->chunks_per_rank = std::max(g->chunks_per_rank, n);
-    g->total_wgs += (int64_t)a->buckets[i].num_boxes * n * (a->kv_heads / g->bucket_heads_per_wg[i]);
+    g->total_wgs += items_of(a->buckets[i], pairs) * n * (a->kv_heads / g->bucket_heads_per_wg[i]);
   }
   // Buckets whose widest box is a few steps long leave most waves of a workgroup idle and pay the
   // workgroup's fixed cost once per kv head: there each wave takes a kv head of its own and walks
@@ -315,7 +354,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     bool changed = false;
     int64_t tall_wgs = 0;
     for (int i = 0; i < a->num_buckets; ++i)
-      if (row_tiles(a->buckets[i].mnw[0]) > 1) tall_wgs += (int64_t)a->buckets[i].num_boxes * g->bucket_chunks[i] * a->kv_heads;
+      if (row_tiles(a->buckets[i].mnw[0]) > 1) tall_wgs += items_of(a->buckets[i], pairs) * g->bucket_chunks[i] * a->kv_heads;
     for (int i = 0; i < a->num_buckets; ++i) {
       const int64_t tok = (int64_t)a->buckets[i].max_blocks * page;
       if (row_tiles(a->buckets[i].mnw[0]) != 1 || g->bucket_heads_per_wg[i] != 1 || tok <= 256) continue;
@@ -348,9 +387,23 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
       g->total_wgs = 0;
       for (int i = 0; i < a->num_buckets; ++i) {
         g->chunks_per_rank = std::max(g->chunks_per_rank, g->bucket_chunks[i]);
-        g->total_wgs += (int64_t)a->buckets[i].num_boxes * g->bucket_chunks[i] * (a->kv_heads / g->bucket_heads_per_wg[i]);
+        g->total_wgs += items_of(a->buckets[i], pairs) * g->bucket_chunks[i] * (a->kv_heads / g->bucket_heads_per_wg[i]);
       }
     }
+  }
+  // Where the tall workgroups do not fill the CUs twice, nothing covers a super-step's wait for memory but requests made
+  // earlier: K and V tiles are handed over apart there, in flight for a step and a half instead of one (us per call,
+  // together / apart: 192 tall workgroups of 21 super-steps 59.9 / 58.2, 32 layers of 96 workgroups of 12 871 / 857). With
+  // two tall workgroups per CU, or chains too short to run ahead in, the second barrier per step costs more (512
+  // workgroups of 32 super-steps 118.0 / 123.7; 114 of 6 17.3 / 18.4; 64 of 7 18.5 / 18.9).
+  {
+    int64_t n_tall = 0, longest = 0;
+    for (int i = 0; i < a->num_buckets; ++i)
+      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0) {
+        n_tall += items_of(a->buckets[i], pairs) * g->bucket_chunks[i] * a->kv_heads;
+        longest = std::max<int64_t>(longest, std::min<int64_t>(g->bucket_chunk[i], (int64_t)a->buckets[i].max_blocks * page));
+      }
+    g->tall_apart = n_tall <= kNumCUs && longest >= kApartTokens;
   }
   g->num_slots = g->chunks_per_rank * a->max_split_per_seq;
   // One slot per row (no sequence in two boxes, no box in two chunks): nothing to merge, the
@@ -362,10 +415,10 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
     return fail(PAT_ERR_INVALID, "too many workgroups for one launch");
   for (int i = 0; i < a->num_buckets; ++i) {
     if (a->buckets[i].num_boxes == 0) continue;
-    g->record_max_seqs = std::max(g->record_max_seqs, (int)a->buckets[i].max_seqs);
+    g->record_max_seqs = std::max(g->record_max_seqs, (int)a->buckets[i].max_seqs * (items_of(a->buckets[i], pairs) < a->buckets[i].num_boxes ? 2 : 1));
     g->record_max_pages = std::max(g->record_max_pages, (int)ceil_div64(g->bucket_chunk[i], page));
   }
-  g->record_max_seqs = std::min(std::max(g->record_max_seqs, 1), 64);
+  g->record_max_seqs = std::min(std::max(g->record_max_seqs, 1), 128);
   g->record_max_pages = std::min(std::max(g->record_max_pages, 1), kMaxChunkPages);
   g->record_stride = (int)((sizeof(RecordHead) + (2 * g->record_max_seqs + g->record_max_pages) * sizeof(int32_t) + 63) / 64 * 64);
   // the kernels index partial rows with 32-bit integers
@@ -378,32 +431,42 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows) {
 // resident workgroup per CU at head_dim 128. They are taken when that costs nothing - the whole launch
 // is resident at two workgroups per CU anyway - or when the launch waits for its tall boxes: those are
 // long (1024 tokens or more: short ones are mostly prologue and epilogue in either form) and, estimated
-// from sizes, take at least as long as the <= 16-row boxes (a tall workgroup ~1.25 us per 64 tokens;
-// the others stream at ~5.8 TB/s; ragged buckets, without the PAT_BUCKET_EVEN hint, hold ~0.6 of their
-// widest box on average). Measured (us per call, 16 / 32 rows): c2 26.1 / 25.7, c3 70.9 / 72.7,
-// c5a 70.6 / 67.4; sweep trees with 512-1024 short leaves 5-14 % faster on 16, `1,1024_2048,32` 3 % on 32.
+// from sizes, take at least as long as the <= 16-row boxes. Measured (us per call, 16 / 32 rows): c2 26.1 / 25.7,
+// c3 70.9 / 72.7, c5a 70.6 / 67.4; sweep trees with 512-1024 short leaves 5-14 % faster on 16, `1,1024_2048,32` 3 % on 32.
+// Two boxes of a node are served by one workgroup (32-row form, pat_fwd_bucket items) where the tall boxes fill the
+// device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
+// part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
+// boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice
+// as often to be as many, only add partial rows (4 boxes x 8 of 2048 tokens: 22.4 / 23.5).
 int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
-  if (tune.tall_rows == 16 || tune.tall_rows == 32) return plan_geometry_for(a, g, tune.tall_rows);
-  double tall_us = 0., short_us = 0.;
-  int64_t widest_tall = 0;
+  int64_t widest_tall = 0, tall_box_heads = 0;
+  bool pairs = false;
   for (int i = 0; i < a->num_buckets; ++i) {
     const pat_fwd_bucket& b = a->buckets[i];
-    if (b.num_boxes <= 0) continue;
-    const double token_heads = (double)b.max_blocks * a->page_size * b.num_boxes * a->kv_heads;
-    if (row_tiles(b.mnw[0]) > 1) {
-      tall_us += token_heads / 64. * 1.25 / kNumCUs;
-      widest_tall = std::max<int64_t>(widest_tall, (int64_t)b.max_blocks * a->page_size);
-    } else {
-      short_us += token_heads * ((b.flags & PAT_BUCKET_EVEN) ? 1.0 : 0.6) * a->head_dim * 4. / 5.8e6;
-    }
+    if (b.num_boxes <= 0 || row_tiles(b.mnw[0]) == 1) continue;
+    widest_tall = std::max<int64_t>(widest_tall, (int64_t)b.max_blocks * a->page_size);
+    tall_box_heads += (int64_t)b.num_boxes * a->kv_heads;
+    pairs = pairs || items_of(b, true) < b.num_boxes;
   }
-  if (widest_tall == 0) return plan_geometry_for(a, g, 16);   // no tall box: the form with more resident workgroups
-  if (int rc = plan_geometry_for(a, g, 32)) return rc;
+  pairs = pairs && tune.pairs != 2 && (tune.pairs == 1 || tall_box_heads >= 3 * kNumCUs / 8);
+  // (boxes of more than 64 x kMaxTall32Tokens tokens, which the bound on pieces per box makes longer pieces of, take the 16-row form)
+  auto in_32 = [&]() -> int {
+    if (int rc = plan_geometry_for(a, g, 32, pairs)) return rc;
+    if (g->tall_rows == 32) return PAT_OK;
+    *g = Geometry();
+    return plan_geometry_for(a, g, 16, false);
+  };
+  if (tune.tall_rows == 32) return in_32();
+  if (tune.tall_rows == 16) return plan_geometry_for(a, g, 16, false);
+  if (widest_tall == 0) return plan_geometry_for(a, g, 16, false);   // no tall box: the form with more resident workgroups
+  if (int rc = in_32()) return rc;
+  if (g->tall_rows == 16) return PAT_OK;
   if (g->total_wgs <= (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs) return PAT_OK;
-  if (widest_tall >= 1024 && tall_us >= short_us) return PAT_OK;
+  const LaunchEstimate est = estimate_launch(a, 32, false);
+  if (widest_tall >= 1024 && est.tall_us >= est.short_us) return PAT_OK;
   *g = Geometry();
-  return plan_geometry_for(a, g, 16);
+  return plan_geometry_for(a, g, 16, false);
 }
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -430,13 +493,14 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
   mix((uint64_t)g.tall_rows); mix((uint64_t)g.total_wgs); mix((uint64_t)g.record_stride); mix((uint64_t)g.record_max_seqs); mix((uint64_t)g.record_max_pages);
   mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0);
   mix((uint64_t)a->batch); mix((uint64_t)a->heads); mix((uint64_t)a->kv_heads); mix((uint64_t)a->page_size);
-  mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq);
+  mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq); mix(g.pairs ? 1 : 0);
   for (int i = 0; i < a->num_buckets; ++i) {
     const pat_fwd_bucket& b = a->buckets[i];
     mix((uint64_t)g.bucket_chunk[i]); mix((uint64_t)g.bucket_chunks[i]); mix((uint64_t)g.bucket_heads_per_wg[i]);
     mix((uint64_t)b.num_boxes); mix((uint64_t)b.max_seqs); mix((uint64_t)b.max_blocks); mix((uint64_t)b.mnw[0]);
     mix((uint64_t)reinterpret_cast<uintptr_t>(b.q_table)); mix((uint64_t)reinterpret_cast<uintptr_t>(b.block_table));
     mix((uint64_t)reinterpret_cast<uintptr_t>(b.kv)); mix((uint64_t)reinterpret_cast<uintptr_t>(b.q_slot));
+    if (g.pairs) mix((uint64_t)items_of(b, true));
   }
   return h ? h : 1;
 }
@@ -508,27 +572,37 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
   // the engine whose turn it is is full, so work must not correlate with the launch index: in
   // box-major order the filled chunks of short boxes recur with the period of the reserved
   // chunks, land on the same engines every time and leave the others idle.
-  const int chunk = local / bk.num_boxes;
-  const int box = local - chunk * bk.num_boxes;
+  const int chunk = local / bk.num_items;
+  const int item = local - chunk * bk.num_items;
+  // the item's boxes (indices clamped: a malformed table gives wrong numbers, not a fault)
+  int box = item, box2 = -1;
+  if (bk.items != nullptr) {
+    box = bk.items[2 * item];
+    box2 = bk.items[2 * item + 1];
+    box = box < 0 ? 0 : (box >= bk.num_boxes ? bk.num_boxes - 1 : box);
+    box2 = box2 >= bk.num_boxes ? -1 : box2;
+  }
   const int page = p.page_size;
-  int nseq = bk.num_seqs[box];
-  nseq = nseq < 0 ? 0 : (nseq > bk.max_seqs ? bk.max_seqs : nseq);
-  int rows = nseq * p.group;
-  if (rows > 16 * bk.row_tiles) rows = 16 * bk.row_tiles;
+  auto seqs_of = [&](int b) {
+    const int n = bk.num_seqs[b], most = min(bk.max_seqs, 16 * bk.row_tiles / p.group);
+    return n < 0 ? 0 : (n > most ? most : n);
+  };
+  const int nseq0 = seqs_of(box);
+  const int nseq = nseq0 + (box2 >= 0 ? seqs_of(box2) : 0);
+  const int rows = nseq * p.group;
   int kv = bk.kv[box];
   const int kv_cap = bk.max_blocks * page;
   kv = kv < 0 ? 0 : (kv > kv_cap ? kv_cap : kv);
   const int t_begin = chunk * bk.chunk_tokens;
   int tokens = kv - t_begin;
   tokens = tokens < 0 ? 0 : (tokens > bk.chunk_tokens ? bk.chunk_tokens : tokens);
-  const int rank = bk.rank[box];
 
   char* rec = p.records + (size_t)wg * (size_t)p.record_stride;
   if (lane == 0) {
     RecordHead h;
     h.tokens = rows > 0 ? tokens : 0;
     h.rows = rows;
-    h.mode = bk.row_tiles | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0);
+    h.mode = (box2 >= 0 ? 2 * bk.row_tiles : bk.row_tiles) | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0);
     h.head = hgroup * bk.heads_per_wg;
     // slots of this box that no workgroup fills: this one's own when it has no tokens, and the
     // ones past the bucket's last chunk (the launch reserves chunks_per_rank per box ordinal)
@@ -542,10 +616,12 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
   // them, the box's ordinal among the boxes of that sequence)
   for (int j = lane; j < p.record_max_seqs; j += 64) {
     int seq = -1, slot = -1;
-    if (j < nseq && j * p.group < rows) {
-      const int q = bk.q_table[(int64_t)box * bk.q_stride + j];
+    if (j < nseq) {
+      const int b = j < nseq0 ? box : box2;
+      const int64_t at = (int64_t)b * bk.q_stride + (j < nseq0 ? j : j - nseq0);
+      const int q = bk.q_table[at];
       if ((unsigned)q < (unsigned)p.batch) seq = q;
-      const int ord = bk.q_slot ? bk.q_slot[(int64_t)box * bk.q_stride + j] : rank;
+      const int ord = bk.q_slot ? bk.q_slot[at] : bk.rank[b];
       if ((unsigned)ord < (unsigned)p.max_split) slot = ord * p.chunks_per_rank + chunk;
     }
     tab[j] = seq;
@@ -584,8 +660,10 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
     d.row_tiles = row_tiles(b.mnw[0]);
     d.heads_per_wg = g.bucket_heads_per_wg[i];
     d.item_begin = (int32_t)items;
+    d.num_items = (int32_t)items_of(b, g.pairs);
+    d.items = d.num_items < b.num_boxes ? b.kv + b.num_boxes : nullptr;
     ++nb;
-    items += (int64_t)b.num_boxes * d.chunks * (args->kv_heads / d.heads_per_wg);
+    items += (int64_t)d.num_items * d.chunks * (args->kv_heads / d.heads_per_wg);
   }
   if (items != g.total_wgs) return fail(PAT_ERR_INVALID, "internal: workgroup count of the records differs from the geometry");
   rp.num_buckets = nb;
@@ -625,6 +703,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   sp.o_part = o_part; sp.lse_part = lse_part;
   sp.direct = g.direct ? 1 : 0;
   sp.tall_rows = g.tall_rows;
+  sp.tall_apart = g.tall_apart ? 1 : 0;
   if (g.direct) {
     sp.out = args->out; sp.lse_out = args->lse_out;
     sp.o_stride_b = args->o_stride[0]; sp.o_stride_h = args->o_stride[2];
@@ -870,7 +949,7 @@ pat_fwd_tuning automatic_tuning() {
   pat_fwd_tuning t;
   t.chunk_tokens = 0; t.tall_chunk_tokens = 0; t.head_per_wave_tokens = -1; t.head_per_wave_long_tokens = 0;
   t.head_per_wave_long_wgs = -1; t.equalize_chunks = -1; t.direct_out = -1;
-  t.tall_rows = 0; t.reserved = 0;
+  t.tall_rows = 0; t.pairs = 0;
   return t;
 }
 // Candidates beside the automatic geometry: a kv head per wave on <= 16-row boxes in chunks of 256

@@ -1,8 +1,10 @@
 // extern "C" surface of the scheduler (declared in include/pat_amd.h).
 #include <algorithm>
+#include <array>
 #include <climits>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <new>
 #include <string>
@@ -200,6 +202,42 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   }
   layout->num_launch_buckets = (int32_t)parts.size();
 
+  // Boxes of one node (same blocks, different sequences) in twos, for launches that serve two of them with one
+  // workgroup. Only buckets of more than 16 rows, and only boxes of several sequences: a box of one sequence may be
+  // grown in place between decode steps.
+  std::vector<std::vector<int32_t>> items(parts.size());
+  for (size_t i = 0; i < parts.size(); ++i) {
+    const Part& pt = parts[i];
+    const pat::Bucket& bk = p.buckets[(size_t)pt.parent];
+    if (bk.mnw[0] <= 16) continue;
+    const auto& ord = order[(size_t)pt.parent];
+    std::map<std::array<int32_t, 3>, int32_t> open;   // (first block, last block, tokens) -> item that waits for its second box
+    bool any = false;
+    for (int at = pt.lo; at < pt.hi; ++at) {
+      const size_t box = (size_t)ord[(size_t)at];
+      const int32_t len = bk.block_len[box];
+      const int32_t* blocks = bk.block_table.data() + box * (size_t)bk.max_blocks;
+      if (bk.num_seqs[box] > 1 && len > 0) {
+        const std::array<int32_t, 3> key{blocks[0], blocks[len - 1], bk.kv[box]};
+        const auto it = open.find(key);
+        if (it != open.end()) {
+          const size_t first = (size_t)ord[(size_t)(pt.lo + items[i][(size_t)it->second * 2])];
+          if (bk.block_len[first] == len &&
+              std::memcmp(bk.block_table.data() + first * (size_t)bk.max_blocks, blocks, (size_t)len * sizeof(int32_t)) == 0) {
+            items[i][(size_t)it->second * 2 + 1] = at - pt.lo;
+            open.erase(it);
+            any = true;
+            continue;
+          }
+        }
+        open[key] = (int32_t)(items[i].size() / 2);
+      }
+      items[i].push_back(at - pt.lo);
+      items[i].push_back(-1);
+    }
+    if (!any) items[i].clear();
+  }
+
   // offsets
   int64_t at = 0;
   auto take = [&](int64_t n) { const int64_t o = at; at += n; return o; };
@@ -222,6 +260,8 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   for (size_t i = 0; i < parts.size(); ++i) {
     const Part& pt = parts[i];
     place(layout->launch[i], p.buckets[(size_t)pt.parent], pt.hi - pt.lo, pt.width, pt.parent, pt.lo);
+    layout->launch[i].num_items = (int32_t)(items[i].size() / 2);
+    take((int64_t)items[i].size());   // (right behind kv, the last table of the bucket)
   }
   // hints: a bucket is even when no box is shorter than 3/4 of its widest one
   auto even = [&](const pat::Bucket& bk, const int32_t* ord, int lo, int hi) {
@@ -269,6 +309,7 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   for (size_t i = 0; i < parts.size(); ++i) {
     const Part& pt = parts[i];
     fill(layout->launch[i], p.buckets[(size_t)pt.parent], order[(size_t)pt.parent].data(), pt.lo, pt.hi);
+    std::copy(items[i].begin(), items[i].end(), dst + layout->launch[i].kv + layout->launch[i].num_boxes);
   }
   return PAT_OK;
 }

@@ -9,6 +9,7 @@ constexpr int kWaves = 4;          // waves per split-kernel workgroup
 constexpr int kThreads = kWaves * 64;
 constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop iteration
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
+constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
 
 // One workgroup's work: a launch record, written once per plan by the record kernel
@@ -19,9 +20,9 @@ constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wa
 // already clamped to the cache. Records are record_stride bytes apart (a multiple of 64).
 struct RecordHead {
   int32_t tokens;      // KV tokens of this piece; 0: nothing to compute (the workgroup only marks slots empty)
-  int32_t rows;        // rows of the box (sequences x heads per kv head), <= 16 x tiles
+  int32_t rows;        // rows of the box, or of the two boxes of an item (sequences x heads per kv head), <= 16 x tiles
   int32_t mode;        // bits 0-7: 16-row tiles (1 = KV steps split over waves on wave-private tiles,
-                       // 2/4 = one wave per tile on tiles shared through LDS); bit 8: a kv head per wave
+                       // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave
   int32_t head;        // first kv head this workgroup serves
   int32_t fill_begin;  // slots slot[j] + fill_begin .. slot[j] + fill_end - 1 of every row stay empty:
   int32_t fill_end;    // this workgroup marks them (-inf)
@@ -54,6 +55,7 @@ struct SplitParams {
   float* lse_out;    // optional [batch, heads] fp32
   int64_t o_stride_b, o_stride_h;              // elements
   int32_t direct;    // 1: such a launch
+  int32_t tall_apart;  // 32-row form: K and V tiles of a super-step handed over apart (see the kernel)
   int32_t tall_rows; // rows per wave on boxes of 17..64 rows: 32 (32x32x16 tiles) or 16 (host side: picks the kernel instance)
 };
 
@@ -74,6 +76,8 @@ struct RecordBucket {
   int32_t chunks;        // workgroups along the KV axis reserved per box
   int32_t item_begin;    // first workgroup of this bucket in the launch
   int32_t row_tiles;     // 16-row tiles per box: 1, 2 or 4
+  const int32_t* items;  // [num_items, 2]: boxes served together (-1: no second one), or null: every box by itself
+  int32_t num_items;     // work items along the box axis: rows of `items`, or num_boxes
   int32_t heads_per_wg;  // 1, or kWaves: wave w serves kv head h0 + w alone
 };
 

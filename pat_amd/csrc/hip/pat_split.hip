@@ -20,13 +20,10 @@
 //    the chunk on wave-private tiles and runs an independent online softmax; the 4 states are
 //    combined through LDS at the end. K rows are the MFMA A operand of S^T = K.Q^T, so a lane
 //    loads 16 contiguous bytes of one token straight from HBM into operand layout (no LDS).
-//  * boxes of 17..64 rows: 32-row tiles on v_mfma_f32_32x32x16. All waves walk the chunk in
-//    super-steps of 64 tokens whose K and V tiles are fetched once per workgroup (coalesced
-//    256-byte rows, two super-steps ahead in registers) into a two-stage LDS buffer; wave w works on
-//    rows 32(w&1).. and on tokens 32(w>>1).. of every super-step, so the two wave pairs run
-//    independent online softmaxes over alternate 32-token steps and are combined through LDS at the
-//    end. Per row and token that is half the MFMA, operand-read and softmax instructions of
-//    16-row tiles.
+//  * boxes of 17..64 rows, and two boxes of one node together (up to 128 rows): 32-row tiles on
+//    v_mfma_f32_32x32x16. All waves walk the chunk in super-steps of 64 tokens whose K and V tiles are
+//    fetched once per workgroup, straight from memory into a two-stage LDS buffer. Per row and token that is
+//    half the MFMA, operand-read and softmax instructions of 16-row tiles.
 //  * S^T on v_mfma_f32_16x16x32 (32x32x16 for tall boxes); its accumulator layout is the B-operand
 //    layout of O^T = V^T.P^T, so P never moves between lanes.
 //  * V must be contracted along tokens but is contiguous along head_dim: V tiles sit row-major
@@ -86,8 +83,8 @@ __device__ __forceinline__ float neg_inf() { return -__builtin_inff(); }
 
 // Two forms of the tall path (boxes of 17..64 rows), one kernel instance each:
 //  TALLK 32: 32-row tiles on 32x32x16 MFMAs, 64-token super-steps; the faster walk of a tall box
-//            (a lone workgroup: 1.1-1.3 us per 64 tokens), at the price of 64 accumulator registers
-//            and 75 KB of LDS: 2 workgroups per CU at head_dim 128;
+//            (a lone workgroup: 1.1-1.3 us per 64 tokens of one box, ~1.5 of two), at the price of 64
+//            accumulator registers and 64 KB of LDS: 2 workgroups per CU at head_dim 128;
 //  TALLK 16: a 16-row tile per wave on 16x16x32 MFMAs, 32-token steps, three steps ahead in registers
 //            (1.7 us per 64 tokens), in the register and LDS budget of the <= 16-row path: 3 per CU.
 // The host picks per launch: 32 where the tall boxes are what the launch waits for, 16 where the
@@ -100,10 +97,19 @@ __host__ __device__ constexpr int split_occupancy(int head_dim, int tallk) {
 __host__ __device__ constexpr int split_smem_bytes(int D, int tallk) {
   const int wave_private = kWaves * kStepTokens * (D * 2 + 32);     // 4 private V tiles
   const int combine = kWaves * 16 * (D + 4) * 4;                     // short boxes: the waves' states
-  const int tall = tallk == 32 ? 2 * (2 * kStepTokens) * ((D * 2 + 16) + (D * 2 + 64))   // two stages of 64 K rows + 64 V rows
+  const int tall = tallk == 32 ? 2 * (2 * kStepTokens) * 2 * (D * 2)                     // two stages of 64 K rows + 64 V rows
                                : 2 * kStepTokens * ((D * 2 + 16) + (D * 2 + 32));        // two stages of 32 K rows + 32 V rows
   int m = wave_private > combine ? wave_private : combine;
   return m > tall ? m : tall;
+}
+
+// 16 bytes per lane from memory into LDS: lane i's go to lds + 16 i (`lds` uniform: an offset in the workgroup's
+// LDS). The compiler does not see the loads: the caller waits for them (vmcnt) ahead of the barrier that hands the tile over.
+__device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offset, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void load_to_lds(const char* lane_address, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(lane_address), "s"(lds) : "memory");
 }
 
 // DIRECT instances serve launches in which every row has one partial slot: they store `out`.
@@ -160,12 +166,13 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   const bool head_per_wave = (mode & kRecordModeHeadPerWave) != 0;
   // Boxes of up to 16 rows: the 4 waves split the piece's steps, each on wave-private tiles (or,
   // with a kv head per wave, each wave walks all steps of its own head).
-  // Taller boxes: wave w owns rows 32(w&1).. and tokens 32(w>>1).. of every 64-token super-step,
-  // on tiles shared through LDS.
+  // Taller boxes: tiles shared through LDS; the 32-row form gives a wave rows 32w.. and every token, or, up to
+  // 64 rows, rows 32(w&1).. and tokens 32(w>>1).. of every 64-token super-step.
   const bool tall = (mode & 0xff) > 1;
   // (both uniform, and known to be: branches on them are scalar branches)
-  const int rt = __builtin_amdgcn_readfirstlane(wave & 1);   // tall boxes: this wave's 32-row tile
-  const int ph = __builtin_amdgcn_readfirstlane(wave >> 1);  //             and which half of a super-step it works on
+  const bool one_tile_per_wave = R > 64;   // tall boxes, 32-row tiles: four row tiles, a wave each
+  const int rt = __builtin_amdgcn_readfirstlane(one_tile_per_wave ? wave : wave & 1);   // this wave's 32-row tile
+  const int ph = __builtin_amdgcn_readfirstlane(one_tile_per_wave ? 0 : wave >> 1);     // and which half of a super-step it works on
   // (uniform over the wave: kept in a scalar register so that address arithmetic stays scalar)
   const int head = __builtin_amdgcn_readfirstlane(rh0.w + (head_per_wave ? (int)(threadIdx.x >> 6) : 0));
   const int fill_begin = __builtin_amdgcn_readfirstlane(rh1.x);
@@ -447,10 +454,18 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     }
     } else {
     // ====================== tall box: 32-row tiles, K/V shared through LDS ======================
-    // The chunk is walked in super-steps of 64 tokens. Thread t loads pieces t, t + 256 .. of a
-    // super-step's K and V tiles (16 lanes cover one 256-byte row), PF2 super-steps ahead in
-    // registers, and drops them into one of two LDS stages; after a barrier the wave pair ph = 0
-    // runs tokens 0..31 of the stage and the pair ph = 1 tokens 32..63, each wave on its 32 rows.
+    // The piece is walked in super-steps of 64 tokens, whose K and V rows go from memory straight into one of
+    // two LDS stages (global_load_lds, 16 bytes per lane): the next super-step is in flight while the waves work
+    // on the current one, and no register holds a tile on its way. Wave w fetches the 16-token half w of every
+    // super-step: one page id, one address.
+    // What bounds it: two of these workgroups on a CU take ~2 us per super-step of two boxes, i.e. ~1050 TFLOP/s in the
+    // steady state (65536 rows x 16384 tokens, 8 kv heads; a library matrix product reaches 1200): MFMA 37 %, VALU 32 %,
+    // LDS 37 % busy, the rest is the chain score - softmax - weighted sum of each wave. With the tiles staged through
+    // registers and one box per workgroup (four workgroups reading what one does now) 65536 rows x 2048 tokens took
+    // 105 us, now ~80.
+    //  * more than 64 rows (two boxes of one node): wave w owns row tile w (rows 32w..) and all 64 tokens;
+    //  * up to 64 rows: the wave pair ph = w >> 1 takes tokens 32ph.. of every super-step, wave w row tile
+    //    w & 1; the pairs' states are combined through LDS at the end.
     //   S^T = K.Q^T on 32x32x16 tiles: A = K (lane: token n32, dims 16kk + 8h2 ..+7, a 16-byte
     //   LDS read), B = Q^T in registers; the accumulator holds, in lane (n32, h2), row n32's scores
     //   for tokens 8b + 4h2 + r (register 4b + r).
@@ -458,23 +473,28 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     //   for token 16t + 8(j>>2) + 4h2 + (j&3), any order does as long as V^T uses the same - and
     //   A = V^T read transposed from LDS (two 4-token groups per lane and MFMA). The row's softmax
     //   state lives in the two lanes n32 and n32 + 32.
+    // A load into LDS writes 64 consecutive 16-byte pieces, so rows cannot be padded: bank conflicts are kept
+    // away by permuting the pieces inside a row instead (each lane fetches the piece that belongs where it
+    // writes). K: piece p of row r stands at p ^ (r & 15) (head_dim 128; 64: p ^ ((r >> 1) & 7)), so the 16 rows
+    // of a read step over all banks; V: 64-byte block b of row r at b ^ (r & 3) (64: b ^ ((r >> 1) & 1)), so the
+    // four rows of a transposed read do.
     constexpr int KK2 = D / 16;            // MFMA k-steps across head_dim in S^T
     constexpr int DB2 = D / 32;            // 32-wide head_dim blocks of O^T
-    constexpr int NP2 = D / 32;            // 16-byte K (and V) loads per thread and super-step
-    constexpr int PF2 = 1;                 // super-steps in flight in registers beside the one in LDS (2: no faster, 34 more registers)
     constexpr int SST = 2 * kStepTokens;   // tokens per super-step
-    constexpr int RSK2 = D * 2 + 16;       // LDS row stride of a K tile (conflict-free 16-byte row reads)
-    constexpr int RSV2 = D * 2 + 64;       // LDS row stride of a V tile (conflict-free transposed reads)
-    constexpr int STAGE2 = SST * (RSK2 + RSV2);
-    constexpr int TPR = kThreads / CPR;    // tokens one load round of the workgroup covers: 16 (D 128) or 32 (D 64)
+    constexpr int ROWB = D * 2;            // bytes of a K or V row
+    constexpr int KTILE = SST * ROWB;      // one operand's tile of a super-step
+    constexpr int STAGE2 = 2 * KTILE;      // K rows, then V rows
+    constexpr int RPI = 64 / CPR;          // rows one load instruction covers
+    constexpr int NI = 16 / RPI;           // load instructions per wave, operand and super-step
     static_assert(2 * STAGE2 <= split_smem_bytes(D, 32), "LDS size");
     static_assert(2 * (D / 8) * 64 * 16 <= 2 * STAGE2, "the exchange buffer of the epilogue fits the stages");
     const int nss_u = (ntok_u + SST - 1) / SST;
-    const float sc_abs = __builtin_fabsf(p.scale_log2);
+    const int last_rel_u = ntok_u - 1;
+    const float sc_abs = fmaxf(__builtin_fabsf(p.scale_log2), 1e-30f);   // (a scale of 0 keeps masked scores at -inf)
 
     // Q^T operand (lane (n32, h2): row n32, dims 16kk + 8h2 ..+7). A negative softmax scale is
     // folded into Q's sign (exact), so that the row maximum can be taken over the raw scores.
-    vec8 q2[KK2];
+    u32x4 q2[KK2];
     {
       const bool ok = my_seq >= 0;
       const T* qrow = (const T*)p.q + (ok ? ((int64_t)my_seq * p.q_stride_b + (int64_t)my_hq * p.q_stride_h) : 0);
@@ -483,8 +503,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       for (int kk = 0; kk < KK2; ++kk) {
         u32x4 raw = u32x4{0u, 0u, 0u, 0u};
         if (ok) raw = *(const u32x4*)(qrow + kk * 16 + h2 * 8);
-        raw = raw ^ u32x4{flip, flip, flip, flip};
-        q2[kk] = __builtin_bit_cast(vec8, raw);
+        q2[kk] = raw ^ u32x4{flip, flip, flip, flip};
       }
     }
     f32x16 acc2[DB2];
@@ -493,122 +512,112 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc2[db][i] = 0.f;
 
-    u32x4 kst[PF2][NP2], vst[PF2][NP2];
-    const int tok_r = tid / CPR;                        // this thread's token within a load round
-    const unsigned col16 = (unsigned)(tid % CPR) * 16u;
-    const unsigned koff = (unsigned)((tok_r & 15) * kss) + col16;
-    const unsigned voff = (unsigned)((tok_r & 15) * vss) + col16;
-    // Where the next half (16 tokens) of the chunk lies. Fast route (pages of 16 tokens, K and V
-    // laid out alike - two tensors of one shape or the two halves of one; the usual case): half h is
-    // page h, its id comes out of the page registers with one v_readlane, the page's byte offset is
-    // one 32 x 32 -> 64 bit scalar multiply (page strides are below 4 GiB, checked on the host), V's
-    // address is K's plus the distance between the two caches, and the loads take the scalar address
-    // plus a 32-bit lane offset that never changes. General route: the half is tracked on the scalar
-    // unit (page of the chunk, slot in the page, byte offset of the slot), K and V apart.
-    int f_page = 0, f_slot = 0;
-    unsigned f_koff = 0, f_voff = 0;
-    const unsigned ksp32 = (unsigned)ksp, vsp32 = (unsigned)vsp, k16 = (unsigned)(16 * kss), v16 = (unsigned)(16 * vss);
-    // (pages of 32, 64 or 128 tokens take the same route with the half's place inside its page added)
-    const int fast_route = (ksp == vsp && kss == vss) ? (hpp == 1 ? 1 : (hshift > 0 ? 2 : 0)) : 0;
-    const int64_t kv_delta = vbase - kbase;
-    auto next_half = [&]() {
-      ++f_slot; f_koff += k16; f_voff += v16;
-      if (f_slot == hpp) { f_slot = 0; f_koff = 0; f_voff = 0; ++f_page; }
+    // this lane's place in its wave's half: row RPI*i + r_in of load i, and the piece it fetches there
+    const int r_in = lane / CPR, c_in = lane % CPR;
+    auto k_piece = [&](int i) { return (unsigned)(D == 128 ? c_in ^ ((RPI * i + r_in) & 15) : c_in ^ (((RPI * i + r_in) >> 1) & 7)) * 16u; };
+    const unsigned v_piece = (unsigned)(D == 128 ? c_in ^ ((r_in & 3) << 2) : c_in ^ (((r_in >> 1) & 1) << 2)) * 16u;
+    unsigned koff[NI], voff[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      koff[i] = (unsigned)((RPI * i + r_in) * kss) + k_piece(i);
+      voff[i] = (unsigned)((RPI * i + r_in) * vss) + v_piece;
+    }
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const unsigned lds_base = (unsigned)(size_t)(PAT_LDS char*)smem + (unsigned)wave_u * 16u * ROWB;
+    // Addresses of this wave's halves, worked out once: lane i holds those of super-step i (the host plans no piece of
+    // more than kMaxTall32Tokens = 64 super-steps for this form). Halves past the end stand in for the last one. Two
+    // v_readlane per operand and super-step are all that is left of the addressing inside the loop.
+    uint64_t k_at, v_at;
+    {
+      int h = lane * (SST / 16) + wave_u;
+      h = h > (last_rel >> 4) ? last_rel >> 4 : h;
+      int pidx, s16;
+      if (hshift >= 0) { pidx = h >> hshift; s16 = h & (hpp - 1); }
+      else { pidx = (int)__umulhi((unsigned)h, p.hpp_magic); s16 = h - pidx * hpp; }
+      const int a0 = __shfl(pg0, pidx & 63), a1 = __shfl(pg1, pidx & 63);
+      const int64_t pg = pidx < 64 ? a0 : a1;
+      k_at = (uint64_t)(kbase + pg * ksp + (int64_t)(s16 * 16) * kss);
+      v_at = (uint64_t)(vbase + pg * vsp + (int64_t)(s16 * 16) * vss);
+    }
+    auto at_step = [&](uint64_t v, int ss) -> const char* {
+      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, ss), hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), ss);
+      return (const char*)(((uint64_t)hi << 32) | lo);
     };
-    // D = 64: a load round covers two halves, waves 2 and 3 read the second one
-    const int wave_half = TPR == 32 ? __builtin_amdgcn_readfirstlane(wave >> 1) : 0;
-    if (wave_half) next_half();
-    auto fetch = [&](auto fast, int ss, u32x4 (&kd)[NP2], u32x4 (&vd)[NP2]) {
-      if ((ss + 1) * SST <= ntok_u) {
-        if (decltype(fast)::value == 1) {
-          const int h0 = ss * (SST / 16) + wave_half;         // this wave's first half (= page) of the super-step
-          const int pgsel = h0 < 64 ? pg0 : pg1;              // (a super-step's 4 pages lie in one register)
-          // (kept out of loop-invariant hoisting: next to the scalar base the 32-bit offset becomes the
-          // load's own offset operand instead of a 64-bit vector add per load)
-          unsigned ko = koff, vo = voff;
-          asm volatile("" : "+v"(ko), "+v"(vo));
+    auto fetch_k = [&](int ss) {
+      const char* base = at_step(k_at, ss);
+      const unsigned dst = lds_base + (unsigned)(ss & 1) * STAGE2;
+      // (rows past the end of the piece re-read its last token: their scores are masked)
+      const int left = last_rel_u - ss * SST - wave_u * 16;
+      if (left >= 15) {
 #pragma unroll
-          for (int i = 0; i < NP2; ++i) {
-            const unsigned pg = (unsigned)__builtin_amdgcn_readlane(pgsel, (h0 + i * (TPR / 16)) & 63);
-            const char* ka = kbase + (uint64_t)pg * ksp32;
-            kd[i] = *(const u32x4*)(ka + ko);
-            vd[i] = *(const u32x4*)(ka + kv_delta + vo);
-          }
-        } else if (decltype(fast)::value == 2) {
-          const int h0 = ss * (SST / 16) + wave_half;         // this wave's first half of the super-step
-          const int pgsel = (h0 >> hshift) < 64 ? pg0 : pg1;  // (a super-step's pages lie in one register)
-          unsigned ko = koff, vo = voff;
-          asm volatile("" : "+v"(ko), "+v"(vo));
-#pragma unroll
-          for (int i = 0; i < NP2; ++i) {
-            const int hh = h0 + i * (TPR / 16);
-            const unsigned pg = (unsigned)__builtin_amdgcn_readlane(pgsel, (hh >> hshift) & 63);
-            const char* ka = kbase + ((uint64_t)pg * ksp32 + (unsigned)(hh & (hpp - 1)) * k16);
-            kd[i] = *(const u32x4*)(ka + ko);
-            vd[i] = *(const u32x4*)(ka + kv_delta + vo);
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < NP2; ++i) {
-            const unsigned pg = (unsigned)__builtin_amdgcn_readlane(f_page < 64 ? pg0 : pg1, f_page & 63);
-            kd[i] = *(const u32x4*)(kbase + ((uint64_t)pg * ksp32 + f_koff) + koff);
-            vd[i] = *(const u32x4*)(vbase + ((uint64_t)pg * vsp32 + f_voff) + voff);
-            next_half();
-            if (TPR == 32) next_half();
-          }
-        }
+        for (int i = 0; i < NI; ++i) load_to_lds(base, koff[i], dst + i * 1024);
       } else {
-        // the chunk's last, partial super-step: per-lane addresses, clamped to the last token
+        const int lim = left < 0 ? last_rel_u & 15 : left;
 #pragma unroll
-        for (int i = 0; i < NP2; ++i) {
-          kd[i] = *(const u32x4*)(lane_row(kbase, ksp, kss, ss * SST + i * TPR + tok_r) + col16);
-          vd[i] = *(const u32x4*)(lane_row(vbase, vsp, vss, ss * SST + i * TPR + tok_r) + col16);
-        }
+        for (int i = 0; i < NI; ++i) load_to_lds(base, RPI * i + r_in > lim ? (unsigned)(lim * kss) + k_piece(i) : koff[i], dst + i * 1024);
+      }
+    };
+    auto fetch_v = [&](int ss) {
+      const char* base = at_step(v_at, ss);
+      const unsigned dst = lds_base + (unsigned)(ss & 1) * STAGE2 + KTILE;
+      const int left = last_rel_u - ss * SST - wave_u * 16;
+      if (left >= 15) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) load_to_lds(base, voff[i], dst + i * 1024);
+      } else {
+        const int lim = left < 0 ? last_rel_u & 15 : left;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) load_to_lds(base, RPI * i + r_in > lim ? (unsigned)(lim * vss) + v_piece : voff[i], dst + i * 1024);
       }
     };
 
-    // LDS offsets of this lane's operand reads inside a stage
-    const unsigned k_rd = (unsigned)((ph * 32 + n32) * RSK2 + h2 * 16);
-    const unsigned v_rd = (unsigned)(SST * RSK2 + (ph * 32 + h2 * 4 + (n >> 2)) * RSV2 + (g & 1) * 32 + (n & 3) * 8);
+    // LDS offsets of this lane's operand reads inside a stage (token 0 of the stage; + 32 ROWB for tokens 32..)
+    unsigned k_rd[KK2], v_rd[DB2];
+#pragma unroll
+    for (int kk = 0; kk < KK2; ++kk)
+      k_rd[kk] = (unsigned)(n32 * ROWB + ((2 * kk + h2) ^ (D == 128 ? n32 & 15 : (n32 >> 1) & 7)) * 16);
+#pragma unroll
+    for (int db = 0; db < DB2; ++db)
+      v_rd[db] = (unsigned)(KTILE + (h2 * 4 + (n >> 2)) * ROWB + (db ^ (D == 128 ? n >> 2 : (n >> 3) & 1)) * 64 + (g & 1) * 32 + (n & 3) * 8);
 
-    // One 32-token step of online-softmax attention for this wave's 32 rows against a stage.
-    auto attend32 = [&](const PAT_LDS char* stage, int t0) {
-      // every K operand of the step is requested before the first MFMA waits for one (left alone, the
+    // HALVES x 32 tokens of online-softmax attention for this wave's 32 rows; `stage` points at the first of them
+    // (its K rows; the V rows KTILE further), t0 is that token's place in the piece. First the scores and probabilities ...
+    auto score32 = [&](auto halves_c, vec8 (&pv)[2 * decltype(halves_c)::value], const PAT_LDS char* stage, int t0) {
+      constexpr int HALVES = decltype(halves_c)::value;
+      f32x16 s[HALVES];
+      // every K operand of a half is requested before the first MFMA waits for one (left alone, the
       // compiler reads each operand right ahead of its use and exposes the LDS latency KK2 times)
-      vec8 kop[KK2];
 #pragma unroll
-      for (int kk = 0; kk < KK2; ++kk) kop[kk] = *(const PAT_LDS vec8*)(stage + k_rd + kk * 32);
-      __builtin_amdgcn_sched_barrier(0);
-      f32x16 s;
+      for (int a = 0; a < HALVES; ++a) {
+        vec8 kop[KK2];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = 0.f;
+        for (int kk = 0; kk < KK2; ++kk) kop[kk] = *(const PAT_LDS vec8*)(stage + k_rd[kk] + a * 32 * ROWB);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < KK2; ++kk) s = E::mfma32(kop[kk], q2[kk], s);
+        for (int i = 0; i < 16; ++i) s[a][i] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < KK2; ++kk) s[a] = E::mfma32(kop[kk], __builtin_bit_cast(vec8, q2[kk]), s[a]);
+      }
       // The rows' reference maxima move only when some row's maximum has left a window of kLazy
       // (base-2 exponent units) above its reference: probabilities then reach 2^kLazy at most, which
       // fp32 sums and 16-bit P hold as well as values below 1, and the accumulator is rescaled a few
-      // times per chunk instead of at nearly every step (with 32 rows per wave some row's maximum
+      // times per piece instead of at nearly every step (with 32 rows per wave some row's maximum
       // moves at almost every step).
       constexpr float kLazy = 8.f;
-      float e[16];
-      float mx;
-      const bool full = t0 + kStepTokens <= ntok_u;
-      if (full) {
-        mx = s[0];
+      if (t0 + HALVES * kStepTokens > ntok_u) {
+        // the piece's last step: tokens past its end are masked
 #pragma unroll
-        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = max_xor32(mx) * sc_abs;
-      } else {
-        // the chunk's last step: tokens past its end are masked
-        mx = neg_inf();
+        for (int a = 0; a < HALVES; ++a)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int tok = t0 + (i >> 2) * 8 + h2 * 4 + (i & 3);
-          e[i] = tok < ntok_u ? s[i] * sc_abs : neg_inf();
-          mx = fmaxf(mx, e[i]);
-        }
-        mx = max_xor32(mx);
+          for (int i = 0; i < 16; ++i)
+            if (t0 + a * kStepTokens + (i >> 2) * 8 + h2 * 4 + (i & 3) >= ntok_u) s[a][i] = neg_inf();
       }
+      float mx = s[0][0];
+#pragma unroll
+      for (int a = 0; a < HALVES; ++a)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[a][i]);
+      mx = max_xor32(mx) * sc_abs;
       if (__builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0) {
         asm volatile("" ::: "memory");   // a real branch: if-converted, the skipped multiplies come back as selects
         const float m_new = fmaxf(m_run, mx);
@@ -618,64 +627,110 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
 #pragma unroll
         for (int db = 0; db < DB2; ++db) acc2[db] = acc2[db] * alpha;
       }
-      if (full) {
+      float psum[2] = {0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) e[i] = fast_exp2(__builtin_fmaf(s[i], sc_abs, -m_run));
-      } else {
+      for (int a = 0; a < HALVES; ++a)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) e[i] = fast_exp2(e[i] - m_run);
-      }
-      float psum = 0.f;
-      vec8 pv[2];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        psum += e[i];
-        pv[i >> 3][i & 7] = (T)e[i];
-      }
-      l_run += psum;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int i = 0; i < 16; ++i) {
+          const float e = fast_exp2(__builtin_fmaf(s[a][i], sc_abs, -m_run));
+          psum[i & 1] += e;
+          pv[2 * a + (i >> 3)][i & 7] = (T)e;
+        }
+      l_run += psum[0] + psum[1];
+    };
+    // ... then the weighted sum of the V rows.
+    auto gather32 = [&](auto halves_c, const vec8 (&pv)[2 * decltype(halves_c)::value], const PAT_LDS char* stage) {
+      constexpr int HALVES = decltype(halves_c)::value;
+      auto read_v = [&](int t, s16x8 (&v)[DB2]) {
 #pragma unroll
         for (int db = 0; db < DB2; ++db) {
-          const PAT_LDS char* src = stage + v_rd + t * 16 * RSV2 + db * 64;
+          const PAT_LDS char* src = stage + v_rd[db] + t * 16 * ROWB;
           s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)src);
-          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)(src + 8 * RSV2));
-          s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-          acc2[db] = E::mfma32(__builtin_bit_cast(vec8, both), pv[t], acc2[db]);
+          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)(src + 8 * ROWB));
+          v[db] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         }
+      };
+      s16x8 vop[2][DB2];
+      read_v(0, vop[0]);
+      read_v(1, vop[1]);
+#pragma unroll
+      for (int t = 0; t < 2 * HALVES; ++t) {
+#pragma unroll
+        for (int db = 0; db < DB2; ++db) acc2[db] = E::mfma32(__builtin_bit_cast(vec8, vop[t & 1][db]), pv[t], acc2[db]);
+        if (t + 2 < 2 * HALVES) read_v(t + 2, vop[t & 1]);
+      }
     };
 
-    // LDS offsets of this thread's tile writes inside a stage (round i: + i * TPR rows)
-    const unsigned k_wr = (unsigned)(tok_r * RSK2) + col16;
-    const unsigned v_wr = (unsigned)(SST * RSK2 + tok_r * RSV2) + col16;
-    auto walk = [&](auto same) {
+    // Q has to be there before the first load into LDS is issued: a wait for it inside the loop would, loads
+    // returning in order, wait for the super-step in flight as well.
 #pragma unroll
-      for (int s = 0; s < PF2; ++s)
-        if (s < nss_u) fetch(same, s, kst[s], vst[s]);
-      for (int ss0 = 0; ss0 < nss_u; ss0 += PF2) {
-#pragma unroll
-        for (int s = 0; s < PF2; ++s) {
-          const int ss = ss0 + s;
-          if (ss >= nss_u) break;
-          PAT_LDS char* stage = (PAT_LDS char*)smem + (ss & 1) * STAGE2;
-          PAT_LDS char* kw = stage + k_wr;
-          PAT_LDS char* vw = stage + v_wr;
-#pragma unroll
-          for (int i = 0; i < NP2; ++i) {
-            *(PAT_LDS u32x4*)(kw + i * TPR * RSK2) = kst[s][i];
-            *(PAT_LDS u32x4*)(vw + i * TPR * RSV2) = vst[s][i];
-          }
-          if (ss + PF2 < nss_u) fetch(same, ss + PF2, kst[s], vst[s]);
-          __syncthreads();
-          if (has_rows && ss * SST + ph * kStepTokens < ntok_u) attend32(stage, ss * SST + ph * kStepTokens);
+    for (int kk = 0; kk < KK2; ++kk) asm volatile("" : "+v"(q2[kk]));
+    // A stage's K and V tiles are handed over together or apart (p.tall_apart, the host's choice). Together: one barrier
+    // per super-step, the next super-step's tiles are in flight for one step. Apart, half a step from each other: the K
+    // tile of step ss + 2 is requested as soon as every wave has read its K operands of step ss, the V tile of step ss + 1
+    // as soon as everybody has left step ss - 1; either is then in flight for a step and a half, at the price of a
+    // second barrier per step.
+    const bool apart = p.tall_apart != 0;
+    fetch_k(0);
+    fetch_v(0);
+    if (apart && nss_u > 1) fetch_k(1);
+    // (loops of their own: in one loop the operands of both splits of the waves take 60 more registers, and a second
+    // barrier that is only sometimes there keeps the V reads from being issued ahead of the softmax)
+    auto walk = [&](auto halves_c, auto apart_c) {
+      constexpr bool kApart = decltype(apart_c)::value;
+      vec8 pv[2 * decltype(halves_c)::value];
+      for (int ss = 0; ss < nss_u; ++ss) {
+        const bool more = ss + 1 < nss_u;
+        // this wave's part of the tiles has arrived (apart: of the K tile; the V tile and the next K tile were requested after it), ...
+        if (!kApart) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
+        __syncthreads();   // ... everybody's has, and nobody reads the other stage (apart: its V rows) any more
+        if (more) {
+          if (!kApart) fetch_k(ss + 1);
+          fetch_v(ss + 1);
+        }
+        const int t0 = ss * SST + ph * kStepTokens;
+        const PAT_LDS char* stage = (const PAT_LDS char*)smem + (ss & 1) * STAGE2 + ph * 32 * ROWB;
+        const bool mine = has_rows && t0 < ntok_u;
+        if constexpr (kApart) {
+          if (mine) score32(halves_c, pv, stage, t0);
+          if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");
+          else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();   // the V tile is there, and nobody reads this stage's K rows any more
+          if (ss + 2 < nss_u) fetch_k(ss + 2);
+          if (mine) gather32(halves_c, pv, stage);
+        } else if (mine) {
+          score32(halves_c, pv, stage, t0);
+          gather32(halves_c, pv, stage);
         }
       }
     };
-    if (fast_route == 1) walk(std::integral_constant<int, 1>{});
-    else if (fast_route == 2) walk(std::integral_constant<int, 2>{});
-    else walk(std::integral_constant<int, 0>{});
-    // ---- the two wave pairs' states of the same rows are combined through LDS ----------------
+    if (one_tile_per_wave) {
+      if (apart) walk(std::integral_constant<int, 2>{}, std::true_type{});
+      else walk(std::integral_constant<int, 2>{}, std::false_type{});
+    } else {
+      if (apart) walk(std::integral_constant<int, 1>{}, std::true_type{});
+      else walk(std::integral_constant<int, 1>{}, std::false_type{});
+    }
     l_run = sum_xor32(l_run);
+    if (one_tile_per_wave) {
+      if (my_slot0 >= 0) {
+        const int64_t prow = (int64_t)my_slot0;
+        const float inv = 1.f / l_run;
+        float* dst = p.o_part + prow * D + h2 * 4;
+        T* o = direct ? row_out(my_slot0) + h2 * 4 : nullptr;
+#pragma unroll
+        for (int db = 0; db < DB2; ++db)
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            put4(dst + db * 32 + b * 8, o + db * 32 + b * 8,
+                 f32x4{acc2[db][4 * b], acc2[db][4 * b + 1], acc2[db][4 * b + 2], acc2[db][4 * b + 3]} * inv);
+        if (h2 == 0) put_lse(prow, (m_run + __builtin_amdgcn_logf(l_run)) * 0.6931471805599453f);
+      }
+      return;
+    }
+    // ---- the two wave pairs' states of the same rows are combined through LDS ----------------
     float* xbuf = (float*)smem;                 // [rt][DB2 * 4 pieces][64 lanes] x 16 bytes
     __syncthreads();                            // every wave is done with the stages
     if (ph == 1 && has_rows) {

@@ -245,6 +245,7 @@ struct PlanTables {
   const TensorList* slots;                       // may be null
   const std::vector<std::vector<int>>* mnw;
   const std::vector<int>* flags;                 // may be null
+  const TensorList* items = nullptr;             // per bucket [items, 2] (pat_fwd_bucket.items) or empty; may be null
 };
 
 // Checks that need tensor metadata follow csrc/api.h:131-181, :256-277 of the reference.
@@ -314,6 +315,11 @@ std::shared_ptr<Prepared> prepare(const at::Tensor& q, const at::Tensor& k, cons
     for (int j = 0; j < 3; ++j) fb.mnw[j] = (*pt.mnw)[i][(size_t)j];
     fb.flags = (pt.flags != nullptr && !pt.flags->empty()) ? (*pt.flags)[i] : 0;
     for (const auto& nt : named) L->keep.push_back(*nt.second);
+    if (pt.items != nullptr && (*pt.items)[i].numel() > 0) {
+      require((*pt.items)[i].data_ptr<int32_t>() == fb.kv + ctas, "an item table stands right behind its bucket's kv table");
+      fb.flags |= PAT_BUCKET_ITEMS; fb.num_items = (int32_t)(*pt.items)[i].size(0);
+      L->keep.push_back((*pt.items)[i]);
+    }
   }
   L->keep.push_back(num_split);
 
@@ -425,7 +431,7 @@ struct KernelInfo {
   int max_split = 0, max_boxes = 0, max_seqs = 0, max_blocks = 0;
   // launch copies: every bucket's boxes longest first, a bucket with a wide head split in two
   bool has_launch = false;
-  TensorList l_q_tables, l_block_tables, l_num_seqs, l_ranks, l_kvs, l_slot_tables;
+  TensorList l_q_tables, l_block_tables, l_num_seqs, l_ranks, l_kvs, l_slot_tables, l_items;
   std::vector<std::vector<int>> l_mnws;
   std::vector<int> l_flags;
   TensorList launch_order;                          // per bucket: launch position -> scheduler row
@@ -467,7 +473,7 @@ struct KernelInfo {
 
   void clear_tables() {
     for (TensorList* l : {&q_tables, &block_tables, &num_seqs, &ranks, &kvs, &slot_tables, &l_q_tables,
-                          &l_block_tables, &l_num_seqs, &l_ranks, &l_kvs, &l_slot_tables, &launch_order,
+                          &l_block_tables, &l_num_seqs, &l_ranks, &l_kvs, &l_slot_tables, &l_items, &launch_order,
                           &ws_q_table, &ws_block_table, &ws_num_seqs, &ws_rank, &ws_kv})
       l->clear();
     ws_mnw.clear();
@@ -506,6 +512,7 @@ struct KernelInfo {
       l_num_seqs.push_back(vec(f.num_seqs, f.num_boxes));
       l_ranks.push_back(vec(f.rank, f.num_boxes));
       l_kvs.push_back(vec(f.kv, f.num_boxes));
+      l_items.push_back(mat(f.kv + f.num_boxes, f.num_items, 2));
       launch_parts[(size_t)f.parent].push_back({i, f.first, f.first + f.num_boxes});
     }
     has_launch = true;
@@ -551,6 +558,7 @@ struct KernelInfo {
     d["kv_in_CTAs"] = l ? l_kvs : kvs;
     d["MNWs"] = l ? l_mnws : mnws;
     d["flags"] = l ? l_flags : std::vector<int>(mnws.size(), 0);
+    d["items"] = l ? py::cast(l_items) : py::none();
     return d;
   }
 
@@ -992,7 +1000,7 @@ void fwd_tree(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, Pre
     PlanTables pt{l ? &info.l_q_tables : &info.q_tables, l ? &info.l_block_tables : &info.block_tables,
                   l ? &info.l_num_seqs : &info.num_seqs, l ? &info.l_ranks : &info.ranks, l ? &info.l_kvs : &info.kvs,
                   l ? &info.l_slot_tables : &info.slot_tables, l ? &info.l_mnws : &info.mnws,
-                  l ? &info.l_flags : &no_flags};
+                  l ? &info.l_flags : &no_flags, l ? &info.l_items : nullptr};
     require(!pt.mnw->empty(), "the tree has no plan: call pack_schedule and kernel_info.to_gpu first");
     if (info.whole_seqs && !info.ws_q_table.empty()) {
       // a small batch of short requests: one work item per request, one kernel (see KernelInfo::whole_seqs)

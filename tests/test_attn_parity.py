@@ -1232,3 +1232,44 @@ def test_little_sharing_is_launched_as_whole_sequences(spec, heads, kernels):
     assert (info._launch_workspace_bytes == [0]) == (kernels == 1)
     ref_out, ref_lse = _oracle(w, q, k, v)
     _assert_close("whole sequences " + spec, out, lse, ref_out, ref_lse, w.dtype)
+
+
+@pytest.mark.parametrize("seqs,prefix,heads,d,dtype,page,chunk,scale", [
+    (32, 16, (32, 8), 128, torch.float16, 16, 0, 0.09),      # one pair of full boxes, a piece of a quarter super-step
+    (40, 48, (32, 8), 128, torch.bfloat16, 48, 0, 0.09),     # pair + a box of another label; pages of 48
+    (24, 80, (64, 8), 64, torch.float16, 16, 0, -0.1),       # pair + single, negative scale, one token past a super-step
+    (130, 1040, (8, 8), 64, torch.bfloat16, 16, 256, 0.1),   # no query-head groups: 64 sequences a box; cut into pieces
+    (64, 2112, (16, 4), 128, torch.float16, 32, 0, 0.09),    # pieces long enough for K and V tiles handed over apart
+    (22, 1152, (32, 8), 128, torch.bfloat16, 64, 640, 0.0),  # 64 + 24 rows; scale 0
+])
+def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, page, chunk, scale, tuning, monkeypatch):
+    print(f"[case] pairs of boxes: {seqs} x ({prefix} + tails), heads {heads}, d {d}, page {page}", flush=True)
+    import random
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    r = random.Random(seqs)
+    shared = -(-prefix // page)
+    tails = [r.randint(1, 40) for _ in range(seqs)]
+    rows, nxt = [], shared
+    for n in tails:
+        need = -(-n // page)
+        rows.append(list(range(shared)) + list(range(nxt, nxt + need)))
+        nxt += need
+    w = workloads.Workload("pairs", heads[0], heads[1], d, dtype, page, [shared * page + n for n in tails], rows, nxt, 0, seqs)
+    q, k, v = w.tensors(dev)
+    tree = PrefixTreeCPP(page)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+    info = tree.kernel_info
+    info.to_gpu(dev)
+    items = [t for t in info.launch_tables()["items"] if t.numel()]
+    assert seqs == 22 or any((t[:, 1] >= 0).any() for t in items), "the case has no two boxes of one node"
+    ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, w.seq_lens, scale)
+    for pairs in (1, 2):
+        tuning(tall_rows=32, tall_chunk_tokens=chunk, pairs=pairs)
+        tree.kernel_info.invalidate()
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((seqs, heads[0]), float("nan"), dtype=torch.float32, device=dev)
+        prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
+        torch.cuda.synchronize()
+        _assert_close(f"pairs {pairs}", out, lse, ref_out, ref_lse, dtype)

@@ -257,3 +257,26 @@ def test_repeated_pack_keeps_slots_and_box_counts_consistent():
     assert torch.equal(seen[0][0], seen[0][1])            # first pack: the two counts agree
     assert torch.equal(seen[1][0], 2 * seen[0][0])        # second pack: the reference's counter doubled
     assert torch.equal(seen[1][1], seen[0][1])            # ... the plan's own count did not
+
+
+@pytest.mark.parametrize("name", ["c2", "c3", "c5a"])
+def test_item_tables_pair_boxes_of_one_node(name):
+    # every box of a tall launch bucket stands in one item; the two boxes of an item attend to the same blocks
+    from pat_amd import PrefixTreeCPP, workloads
+    w = workloads.make(name, seed=0)
+    t = PrefixTreeCPP(w.page_size)
+    t.build_radix_tree(w.seq_lens, w.padded_table())
+    t.pack_schedule(None, w.heads // w.kv_heads, w.kv_heads)
+    lt = t.kernel_info.launch_tables()
+    pairs = 0
+    for mnw, items, kv, bt in zip(lt["MNWs"], lt["items"], lt["kv_in_CTAs"], lt["block_tables"]):
+        if items.numel() == 0:
+            continue
+        assert mnw[0] > 16
+        boxes = [b for row in items.tolist() for b in row if b >= 0]
+        assert sorted(boxes) == list(range(len(kv)))
+        for a, b in items.tolist():
+            if b >= 0:
+                pairs += 1
+                assert kv[a] == kv[b] and torch.equal(bt[a], bt[b])
+    assert pairs == {"c2": 2, "c3": 0, "c5a": 12}[name]
