@@ -698,7 +698,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   SplitParams sp;
   std::memset(&sp, 0, sizeof(sp));
   sp.records = static_cast<const char*>(records);
-  sp.record_stride = g.record_stride; sp.record_max_seqs = g.record_max_seqs;
+  sp.record_stride = g.record_stride; sp.record_max_seqs = g.record_max_seqs; sp.record_max_pages = g.record_max_pages;
   sp.q = args->q; sp.k = args->k; sp.v = args->v;
   sp.o_part = o_part; sp.lse_part = lse_part;
   sp.direct = g.direct ? 1 : 0;

@@ -35,6 +35,7 @@ struct SplitParams {
   const char* records;      // one per workgroup, in launch order
   int32_t record_stride;    // bytes
   int32_t record_max_seqs;  // seq[] / slot[] entries per record
+  int32_t record_max_pages; // page[] entries per record
   const void* q;
   const void* k;
   const void* v;

@@ -30,8 +30,8 @@
 //    in padded LDS rows and are read back transposed with ds_read_b64_tr_b16.
 //  * all softmax state of a row lives in the 4 lanes {n, n+16, n+32, n+48}.
 //  * the chunk's page ids live in two VGPRs per wave (lane i holds page i) and are
-//    broadcast with v_readlane; with the launch record the prologue is two dependent memory
-//    round trips: {record: header, sequence ids, slots, page ids} -> {K, V, Q}.
+//    broadcast with v_readlane; with the launch record the prologue is three dependent memory
+//    round trips: {record: header, page ids} -> {sequence ids, slots: the record's lines again} -> {K, V, Q}.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -115,7 +115,7 @@ __device__ __forceinline__ void load_to_lds(const char* lane_address, unsigned l
 // DIRECT instances serve launches in which every row has one partial slot: they store `out`.
 template <typename T, int D, bool DIRECT, int TALLK>
 __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
-                                                                             const int record_max_seqs, const SplitParams p) {
+                                                                             const int record_max_seqs, const int record_max_pages, const SplitParams p) {
   using E = Elem<T>;
   using vec8 = typename E::vec8;
   constexpr int KK = D / 32;             // MFMA k-steps across head_dim in S^T = K.Q^T (16x16x32 tiles)
@@ -153,6 +153,18 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   const char* __restrict__ rec = records + (size_t)wg_id * (unsigned)record_stride;
   const int4 rh0 = *(const int4*)rec;
   const int4 rh1 = *(const int4*)(rec + 16);
+  const int* __restrict__ rows_tab = (const int*)(rec + sizeof(RecordHead));
+  const int* __restrict__ pages_tab = rows_tab + 2 * record_max_seqs;
+  // Page ids of the piece: lane i of every wave holds pages i and 64 + i. The first 64 are requested with the header,
+  // not behind it (the record kernel filled all record_max_pages entries with pages of the cache, so which of them the
+  // piece has does not matter); the others, which few pieces have, wait for it. So do the rows' entries: requested with
+  // the header as well, by all lanes and picked by shuffles, they made single launches of one long request 1 % faster
+  // and launches that queue workgroups 1-2 % slower (369 boxes at head_dim 64 90.7 -> 92.5 us, 64 requests behind one
+  // prefix 22.1 -> 22.5).
+  const int pg0 = pages_tab[min(lane, record_max_pages - 1)];
+  // the rest of the kernel's arguments, requested here as well (left alone, a round trip of their own ahead of K and V)
+  asm volatile("" ::"s"(p.k), "s"(p.v), "s"(p.q), "s"(p.q_stride_b), "s"(p.k_stride_page), "s"(p.k_stride_slot), "s"(p.k_stride_h),
+               "s"(p.v_stride_page), "s"(p.v_stride_slot), "s"(p.v_stride_h), "s"(p.page_size), "s"(p.scale_log2));
   // The piece's length, twice: as a scalar for the loops of the tall path, and laundered
   // into a vector register for the wave-private path. With loop bounds it can prove uniform the
   // compiler schedules the wave-private loops for 50 more registers; with vector bounds in the
@@ -180,19 +192,13 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   const int G = p.group;                       // 1, 2, 4 or 8 (checked on the host)
   const int gshift = 31 - __builtin_clz(G);
   const int page = p.page_size;
+  const int pg1 = ntok_u > 64 * page ? pages_tab[min(64 + lane, record_max_pages - 1)] : 0;
   // this lane's row: sequence id and partial-result slot (-1: no such row)
   const int my_row = tall ? (TALLK == 32 ? rt * 32 + n32 : wave * 16 + n) : n;
   const int my_j = my_row >> gshift;
   const bool j_ok = (my_row < R) && my_j < record_max_seqs;
-  const int* __restrict__ rows_tab = (const int*)(rec + sizeof(RecordHead));
   const int my_seq = j_ok ? rows_tab[my_j] : -1;
   const int my_sl = j_ok ? rows_tab[record_max_seqs + my_j] : -1;
-  // page ids of the piece: lane i of every wave holds pages i and 64 + i (the record kernel
-  // filled all kMaxChunkPages-or-fewer entries it reserved, so no bound is checked here)
-  const int* __restrict__ pages_tab = rows_tab + 2 * record_max_seqs;
-  const int npages = (ntok + page - 1) / page;
-  const int pg0 = (lane < npages) ? pages_tab[lane] : 0;
-  const int pg1 = (64 + lane < npages) ? pages_tab[64 + lane] : 0;
 
   const bool has_rows = !tall || (TALLK == 32 ? rt * 32 : wave * 16) < R;   // false: a wave that only helps loading shared tiles
   const bool row_ok = my_seq >= 0 && my_sl >= 0;
@@ -661,10 +667,6 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       }
     };
 
-    // Q has to be there before the first load into LDS is issued: a wait for it inside the loop would, loads
-    // returning in order, wait for the super-step in flight as well.
-#pragma unroll
-    for (int kk = 0; kk < KK2; ++kk) asm volatile("" : "+v"(q2[kk]));
     // A stage's K and V tiles are handed over together or apart (p.tall_apart, the host's choice). Together: one barrier
     // per super-step, the next super-step's tiles are in flight for one step. Apart, half a step from each other: the K
     // tile of step ss + 2 is requested as soon as every wave has read its K operands of step ss, the V tile of step ss + 1
@@ -673,6 +675,10 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     const bool apart = p.tall_apart != 0;
     fetch_k(0);
     fetch_v(0);
+    // Q has to be there before the next load into LDS is issued (the first ones follow it right away): a wait for it
+    // inside the loop would, loads returning in order, wait for the super-step in flight as well.
+#pragma unroll
+    for (int kk = 0; kk < KK2; ++kk) asm volatile("" : "+v"(q2[kk]));
     if (apart && nss_u > 1) fetch_k(1);
     // (loops of their own: in one loop the operands of both splits of the waves take 60 more registers, and a second
     // barrier that is only sometimes there keeps the V reads from being issued ahead of the softmax)
@@ -887,7 +893,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
 }
 
 // Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path).
-typedef void (*SplitFn)(const char*, int, int, const SplitParams);
+typedef void (*SplitFn)(const char*, int, int, int, const SplitParams);
 template <bool DIRECT, int TALLK>
 static SplitFn split_instance(bool bf16, int head_dim) {
   if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK> : pat_split_kernel<__bf16, 128, DIRECT, TALLK>;
@@ -916,7 +922,8 @@ hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const Split
   }
   const unsigned wgs = (unsigned)params.total_items;
   const dim3 grid(wgs < (unsigned)kGridX ? wgs : (unsigned)kGridX, (wgs + kGridX - 1) / kGridX);
-  hipLaunchKernelGGL(fn, grid, dim3(kThreads), lds, stream, params.records, params.record_stride, params.record_max_seqs, params);
+  hipLaunchKernelGGL(fn, grid, dim3(kThreads), lds, stream, params.records, params.record_stride, params.record_max_seqs,
+                     params.record_max_pages, params);
   return hipGetLastError();
 }
 
