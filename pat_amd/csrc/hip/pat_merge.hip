@@ -23,44 +23,62 @@ namespace pat {
 #ifndef PAT_MERGE_PAIRS_MIN
 #define PAT_MERGE_PAIRS_MIN 16384   // rows from which a half-wave takes a row (launches of up to 8 slots per row)
 #endif
+// Launches of 9..32 slots per row where a workgroup takes a row: up to so many slots over all rows. It requests every slot,
+// empty ones too, which has to cost less than the two round trips it saves (us per merge, general / workgroup per row: 32 rows
+// x 27 slots 5.7 / 2.5, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
+constexpr int kMergeWideSlots = 32;
+constexpr int64_t kMergeWideMost = 32768;
 
-// (the leading scalar arguments repeat the fields of `p` that the first two memory reads need:
-// they are preloaded into SGPRs with the wave, the rest of `p` arrives by load meanwhile)
+// u / d with m = ceil(2^32 / d) (0 for d = 1), any 32-bit u: the product is the quotient or one more.
+__device__ __forceinline__ unsigned divide(unsigned u, unsigned d, unsigned m) {
+  if (m == 0) return u;
+  const unsigned q = __umulhi(u, m);
+  return q * d > u ? q - 1 : q;
+}
+
+// Which (sequence, head) is row u of workgroup list `xcd`? Workgroups are dealt to the 8 XCDs round-robin, and the
+// split kernel's launch order put every partial row of kv head h through the L2 of XCD h mod 8
+// (where most of it still sits): with a multiple of 8 kv heads, workgroup b serves heads of the kv
+// heads = b mod 8, so the rows are found in its own L2. A matter of speed only. Otherwise there is one list.
+// (32-bit arithmetic with a multiplier from the host: batch x heads x slots is below 2^31, and a 64-bit division
+// by an argument is 150 instructions ahead of the first load)
+__device__ __forceinline__ void row_of(unsigned u, unsigned xcd, int per_list, unsigned per_list_magic, int mapping, int& s, int& hq) {
+  s = (int)divide(u, (unsigned)per_list, per_list_magic);
+  const int local = (int)u - s * per_list;
+  const int group = mapping & 255;
+  if (mapping & 256) {
+    const int gshift = 31 - __builtin_clz(group);            // group: 1, 2, 4 or 8
+    hq = (((int)xcd + 8 * (local >> gshift)) << gshift) + (local & (group - 1));   // kv head (xcd + 8 i), head g of its group
+  } else {
+    hq = local;
+  }
+}
+
+// The leading arguments of the kernels, all that stands ahead of their first memory reads: 14 dwords, preloaded into
+// SGPRs with the wave; the rest of `p` arrives by load meanwhile.
+//   rows_per_list   rows a list holds; per_list: those of one sequence, with its multiplier (0 for 1)
+//   mapping         query heads per kv head, + 256 where there are eight lists, one per XCD
+#define MERGE_ROWS                                                                                                      \
+  const int32_t* __restrict__ num_split_per_seq, const float* __restrict__ lse_part, const float* __restrict__ o_part, \
+      const int num_slots, const int chunks_per_rank, const int max_split, const int heads, const int rows_per_list,   \
+      const int per_list, const unsigned per_list_magic, const int mapping
 template <typename T, int D>
-__global__ void __launch_bounds__(256) pat_merge_kernel(const int32_t* __restrict__ num_split_per_seq,
-                                                        const float* __restrict__ lse_part, const int num_slots,
-                                                        const int chunks_per_rank, const int max_split, const int batch,
-                                                        const int heads, const int kv_heads, const MergeParams p) {
+__global__ void __launch_bounds__(256) pat_merge_kernel(MERGE_ROWS, const MergeParams p) {
   constexpr int CPL = D / 64;   // columns per lane
   constexpr int kRegs = 4;      // LSE registers per lane: up to 256 slots stay in registers
   constexpr int kBatch = 16;    // partial rows fetched together
   constexpr int kSpec = 8;      // launches with up to this many slots per row fetch every slot's row at once
   const int lane = threadIdx.x & 63;
-  // Which (sequence, head) is this wave's? Workgroups are dealt to the 8 XCDs round-robin, and the
-  // split kernel's launch order put every partial row of kv head h through the L2 of XCD h mod 8
-  // (where most of it still sits): with a multiple of 8 kv heads, workgroup b serves heads of the kv
-  // heads = b mod 8, so the rows are found in its own L2. A matter of speed only.
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned u = (mapping & 256 ? blockIdx.x >> 3 : blockIdx.x) * 4 + wave;
+  if (u >= (unsigned)rows_per_list) return;
   int s, hq;
-  if (kv_heads % 8 == 0) {
-    const int xcd = blockIdx.x & 7;
-    const int per_seq = heads >> 3;                       // heads of one sequence served by one XCD
-    const int64_t u = (int64_t)(blockIdx.x >> 3) * 4 + (threadIdx.x >> 6);
-    if (u >= (int64_t)batch * per_seq) return;
-    s = (int)(u / per_seq);
-    const int local = (int)(u - (int64_t)s * per_seq);      // kv head (xcd + 8 i), head g of its group
-    const int group = heads / kv_heads;
-    hq = (xcd + 8 * (local / group)) * group + local % group;
-  } else {
-    const int64_t u = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (u >= (int64_t)batch * heads) return;
-    s = (int)(u / heads);
-    hq = (int)(u % heads);
-  }
+  row_of(u, blockIdx.x & 7, per_list, per_list_magic, mapping, s, hq);
   const int64_t pair = (int64_t)s * heads + hq;
   const float ninf = -__builtin_inff();
 
   const float* __restrict__ lse = lse_part + pair * num_slots;
-  const float* __restrict__ op = p.o_part + pair * (int64_t)num_slots * D;
+  const float* __restrict__ op = o_part + pair * (int64_t)num_slots * D;
   if (num_slots <= kSpec) {
     // Few slots: nothing here depends on the split count but which slots count, so the count, the
     // slot LSEs and every slot's row are requested together (one round trip instead of three);
@@ -199,40 +217,21 @@ __global__ void __launch_bounds__(256) pat_merge_kernel(const int32_t* __restric
 // half-wave takes a (sequence, head), 16 bytes of a partial row per lane, which halves the waves and
 // the load instructions per byte. Same arithmetic in the same order as the kernel above.
 template <typename T, int D>
-__global__ void __launch_bounds__(256) pat_merge_pairs_kernel(const int32_t* __restrict__ num_split_per_seq,
-                                                              const float* __restrict__ lse_part, const int num_slots,
-                                                              const int chunks_per_rank, const int max_split, const int batch,
-                                                              const int heads, const int kv_heads, const MergeParams p) {
+__global__ void __launch_bounds__(256) pat_merge_pairs_kernel(MERGE_ROWS, const MergeParams p) {
   constexpr int CPL = D / 32;   // columns per lane
   constexpr int kSpec = 8;
   const int lane = threadIdx.x & 63;
   const int half = lane >> 5, l32 = lane & 31;
   const int slot_in_wg = (int)(threadIdx.x >> 6) * 2 + half;   // 8 rows per workgroup
+  unsigned u = (mapping & 256 ? blockIdx.x >> 3 : blockIdx.x) * 8 + slot_in_wg;
+  const bool live = u < (unsigned)rows_per_list;
+  if (!live) u = (unsigned)rows_per_list - 1;   // (an idle half repeats the last row's reads and stores nothing)
   int s, hq;
-  bool live;
-  if (kv_heads % 8 == 0) {
-    const int xcd = blockIdx.x & 7;
-    const int per_seq = heads >> 3;
-    int64_t u = (int64_t)(blockIdx.x >> 3) * 8 + slot_in_wg;
-    const int64_t n = (int64_t)batch * per_seq;
-    live = u < n;
-    if (!live) u = n - 1;          // (an idle half repeats the last row's reads and stores nothing)
-    s = (int)(u / per_seq);
-    const int local = (int)(u - (int64_t)s * per_seq);
-    const int group = heads / kv_heads;
-    hq = (xcd + 8 * (local / group)) * group + local % group;
-  } else {
-    int64_t u = (int64_t)blockIdx.x * 8 + slot_in_wg;
-    const int64_t n = (int64_t)batch * heads;
-    live = u < n;
-    if (!live) u = n - 1;
-    s = (int)(u / heads);
-    hq = (int)(u % heads);
-  }
+  row_of(u, blockIdx.x & 7, per_list, per_list_magic, mapping, s, hq);
   const int64_t pair = (int64_t)s * heads + hq;
   const float ninf = -__builtin_inff();
   const float* __restrict__ lse = lse_part + pair * num_slots;
-  const float* __restrict__ op = p.o_part + pair * (int64_t)num_slots * D;
+  const float* __restrict__ op = o_part + pair * (int64_t)num_slots * D;
   int ns = num_split_per_seq[s];
   float l = (l32 < num_slots) ? lse[l32] : ninf;
   float v[kSpec][CPL];
@@ -281,25 +280,113 @@ __global__ void __launch_bounds__(256) pat_merge_pairs_kernel(const int32_t* __r
   if (p.lse_out != nullptr && l32 == 0) p.lse_out[pair] = total;
 }
 
+// Launches of 9..32 slots per row and few rows (a long request cut over the whole chip, a deep tree of a few dozen
+// requests): a workgroup takes a (sequence, head), each of its four waves the next num_slots / 4 slots, whose LSEs and
+// rows it requests at once like the kernels above; the four sums are combined through LDS. One round trip where the
+// general kernel's chain is split count -> LSEs -> rows by sixteens, and four times the waves where rows are few.
+template <typename T, int D>
+__global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const MergeParams p) {
+  constexpr int CPL = D / 64;
+  constexpr int kSpec = kMergeWideSlots / 4;   // slots per wave
+  __shared__ float s_acc[4][D];
+  __shared__ float s_max[4], s_sum[4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned u = mapping & 256 ? blockIdx.x >> 3 : blockIdx.x;
+  if (u >= (unsigned)rows_per_list) return;
+  int s, hq;
+  row_of(u, blockIdx.x & 7, per_list, per_list_magic, mapping, s, hq);
+  const int64_t pair = (int64_t)s * heads + hq;
+  const float ninf = -__builtin_inff();
+  const int mine = (num_slots + 3) >> 2, first = wave * mine;   // this wave's slots
+  const float* __restrict__ lse = lse_part + pair * num_slots;
+  const float* __restrict__ op = o_part + pair * (int64_t)num_slots * D;
+  int ns = num_split_per_seq[s];
+  float l = (lane < mine && first + lane < num_slots) ? lse[first + lane] : ninf;
+  float v[kSpec][CPL];
+#pragma unroll
+  for (int b = 0; b < kSpec; ++b)
+    if (b < mine && first + b < num_slots) {
+      const float* row = op + (int64_t)(first + b) * D + lane * CPL;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) v[b][c] = row[c];
+    }
+  ns = ns < 0 ? 0 : (ns > max_split ? max_split : ns);
+  if (first + lane >= ns * chunks_per_rank) l = ninf;
+  float mx = l;
+#pragma unroll
+  for (int off = kSpec / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+  mx = __shfl(mx, 0);
+  const float w_mine = (l > ninf) ? __expf(l - mx) : 0.f;
+  float sum = w_mine;
+#pragma unroll
+  for (int off = kSpec / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  float acc[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) acc[c] = 0.f;
+#pragma unroll
+  for (int b = 0; b < kSpec; ++b) {
+    const float w = __shfl(w_mine, b);
+    // (rows of slots that are empty or beyond the count hold anything: dropped, not multiplied)
+    if (b < mine && first + b < num_slots && w > 0.f) {
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) s_acc[wave][lane * CPL + c] = acc[c];
+  if (lane == 0) { s_max[wave] = mx; s_sum[wave] = sum; }
+  __syncthreads();
+  if (wave != 0) return;
+  float most = s_max[0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) most = fmaxf(most, s_max[w]);
+  float weight[4], all = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    weight[w] = s_max[w] > ninf ? __expf(s_max[w] - most) : 0.f;
+    all += weight[w] * s_sum[w];
+  }
+  const float inv = all > 0.f ? 1.f / all : 0.f;
+  T* dst = (T*)p.out + (int64_t)s * p.o_stride_b + (int64_t)hq * p.o_stride_h + lane * CPL;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) x += weight[w] * s_acc[w][lane * CPL + c];
+    dst[c] = (T)(x * inv);
+  }
+  if (p.lse_out != nullptr && lane == 0) p.lse_out[pair] = all > 0.f ? most + logf(all) : ninf;
+}
+
 // Host launcher: one wave per (sequence, query head), four per workgroup; a half-wave each in large launches
-// of few slots.
+// of few slots, a workgroup each in small launches of many.
 hipError_t launch_merge(bool bf16, int head_dim, hipStream_t stream, const MergeParams& params) {
   const int64_t pairs = (int64_t)params.batch * params.heads;
-  void (*fn)(const int32_t*, const float*, int, int, int, int, int, int, const MergeParams);
+  void (*fn)(const int32_t*, const float*, const float*, int, int, int, int, int, int, unsigned, int, const MergeParams);
   int per_wg = 4;
   if (params.num_slots <= 8 && pairs >= PAT_MERGE_PAIRS_MIN) {
     per_wg = 8;
     if (bf16) fn = head_dim == 64 ? pat_merge_pairs_kernel<__bf16, 64> : pat_merge_pairs_kernel<__bf16, 128>;
     else fn = head_dim == 64 ? pat_merge_pairs_kernel<_Float16, 64> : pat_merge_pairs_kernel<_Float16, 128>;
+  } else if (params.num_slots > 8 && params.num_slots <= kMergeWideSlots && pairs * params.num_slots <= kMergeWideMost) {
+    per_wg = 1;
+    if (bf16) fn = head_dim == 64 ? pat_merge_wide_kernel<__bf16, 64> : pat_merge_wide_kernel<__bf16, 128>;
+    else fn = head_dim == 64 ? pat_merge_wide_kernel<_Float16, 64> : pat_merge_wide_kernel<_Float16, 128>;
   } else {
     if (bf16) fn = head_dim == 64 ? pat_merge_kernel<__bf16, 64> : pat_merge_kernel<__bf16, 128>;
     else fn = head_dim == 64 ? pat_merge_kernel<_Float16, 64> : pat_merge_kernel<_Float16, 128>;
   }
   // (a multiple of 8 kv heads: 8 interleaved lists of pairs, one per XCD, each rounded up to whole workgroups)
-  const int64_t wgs = params.kv_heads % 8 == 0 ? 8 * ((pairs / 8 + per_wg - 1) / per_wg) : (pairs + per_wg - 1) / per_wg;
+  const bool xcd_lists = params.kv_heads % 8 == 0;
+  const int lists = xcd_lists ? 8 : 1, per_list = params.heads / lists, group = params.heads / params.kv_heads;
+  const uint32_t magic = per_list > 1 ? (uint32_t)((((uint64_t)1 << 32) + per_list - 1) / per_list) : 0u;
+  const int64_t rows_per_list = pairs / lists;   // (below 2^31: checked with the launch)
+  const int64_t wgs = lists * ((rows_per_list + per_wg - 1) / per_wg);
   const dim3 grid((unsigned)wgs), block(256);
-  hipLaunchKernelGGL(fn, grid, block, 0, stream, params.num_split_per_seq, params.lse_part, params.num_slots,
-                     params.chunks_per_rank, params.max_split, params.batch, params.heads, params.kv_heads, params);
+  hipLaunchKernelGGL(fn, grid, block, 0, stream, params.num_split_per_seq, params.lse_part, params.o_part, params.num_slots,
+                     params.chunks_per_rank, params.max_split, params.heads, (int)rows_per_list, per_list, magic,
+                     group + (xcd_lists ? 256 : 0), params);
   return hipGetLastError();
 }
 

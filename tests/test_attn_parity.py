@@ -1273,3 +1273,42 @@ def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, pag
         prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
         torch.cuda.synchronize()
         _assert_close(f"pairs {pairs}", out, lse, ref_out, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("slots,batch,heads,d,dtype", [
+    (9, 3, (8, 8), 64, torch.float16),         # first size of the workgroup-per-row merge
+    (13, 5, (24, 3), 128, torch.bfloat16),     # one list of rows, 24 a sequence
+    (14, 3, (48, 24), 64, torch.bfloat16),     # eight lists, 6 rows a sequence in each
+    (32, 2, (32, 8), 128, torch.float16),      # the last slot count of it
+    (33, 2, (32, 8), 128, torch.float16),      # past it: a wave per row
+    (10, 409, (8, 1), 64, torch.float16),      # 32720 slots: a workgroup per row ...
+    (10, 410, (8, 1), 64, torch.float16),      # ... 32800: a wave per row
+])
+def test_merge_of_many_slots(slots, batch, heads, d, dtype, tuning):
+    print(f"[case] merge of {slots} slots, {batch} requests, heads {heads}, d {d}", flush=True)
+    import ctypes as C
+    import random
+    from pat_amd import _ctypes_launch, _lib
+    dev = _device()
+    r = random.Random(slots)
+    # one item per request in pieces of 32 tokens; all but the first leave slots empty
+    lens = [slots * 32 - 5] + [r.choice([1, r.randint(1, slots * 32), slots * 32]) for _ in range(batch - 1)]
+    rows, nxt = [], 0
+    for n in lens:
+        rows.append(list(range(nxt, nxt + -(-n // 16))))
+        nxt += -(-n // 16)
+    w = workloads.Workload("slots", heads[0], heads[1], d, dtype, 16, lens, rows, nxt, 0, batch)
+    q, k, v = w.tensors(dev)
+    tuning(chunk_tokens=32, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    ob = workloads.oblivious_plan(w, dev)
+    plan = [ob[x] for x in ("num_split_per_seq", "query_tables", "block_tables", "num_seqs_per_CTAs", "CTA_ranks", "kv_in_CTAs",
+                            "MNW", "max_split_per_seq", "max_seqs_in_CTA", "max_blocks_in_CTA")]
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((batch, heads[0]), float("nan"), dtype=torch.float32, device=dev)
+    L = _ctypes_launch.prepare(q, k, v, *plan, 1.0 / math.sqrt(d), out, lse)
+    geo = _lib.FwdGeometry()
+    assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(geo)) == 0 and geo.num_slots == slots
+    prefix_attn_with_kvcache(q, k, v, *plan, 1.0 / math.sqrt(d), out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    ref_out, ref_lse = _oracle(w, q, k, v)
+    _assert_close(f"{slots} slots", out, lse, ref_out, ref_lse, dtype)
