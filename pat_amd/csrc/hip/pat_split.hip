@@ -106,10 +106,7 @@ __host__ __device__ constexpr int split_smem_bytes(int D, int tallk) {
 // 16 bytes per lane from memory into LDS: lane i's go to lds + 16 i (`lds` uniform: an offset in the workgroup's
 // LDS). The compiler does not see the loads: the caller waits for them (vmcnt) ahead of the barrier that hands the tile over.
 __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offset, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds) : "memory");
-}
-__device__ __forceinline__ void load_to_lds(const char* lane_address, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(lane_address), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds) : "memory", "m0");
 }
 
 // DIRECT instances serve launches in which every row has one partial slot: they store `out`.
