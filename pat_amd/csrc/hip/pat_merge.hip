@@ -14,6 +14,8 @@
 // slots per row make it one: slot addresses do not depend on the split count, so everything is
 // requested at once and what turns out unused is dropped (measured: 0.3-0.8 us less per launch;
 // with 16 rows requested blindly the extra registers and reads cost what the round trips save).
+// Two more forms stand below: a half-wave per row where rows are many and slots few, a workgroup per row where
+// slots are many (9..32) and rows few.
 #include <hip/hip_runtime.h>
 
 #include "fwd_params.hpp"

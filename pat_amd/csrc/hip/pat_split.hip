@@ -27,7 +27,8 @@
 //  * S^T on v_mfma_f32_16x16x32 (32x32x16 for tall boxes); its accumulator layout is the B-operand
 //    layout of O^T = V^T.P^T, so P never moves between lanes.
 //  * V must be contracted along tokens but is contiguous along head_dim: V tiles sit row-major
-//    in padded LDS rows and are read back transposed with ds_read_b64_tr_b16.
+//    in LDS (padded rows, or permuted ones where memory is loaded straight into LDS) and are read back
+//    transposed with ds_read_b64_tr_b16.
 //  * all softmax state of a row lives in the 4 lanes {n, n+16, n+32, n+48}.
 //  * the chunk's page ids live in two VGPRs per wave (lane i holds page i) and are
 //    broadcast with v_readlane; with the launch record the prologue is three dependent memory
