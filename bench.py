@@ -165,7 +165,8 @@ def measure(a, workload: str, steps: int, warmup: int, headline: bool) -> dict:
                                        plan_kw["block_tables"], plan_kw["num_seqs_per_CTAs"], plan_kw["CTA_ranks"],
                                        plan_kw["kv_in_CTAs"], plan_kw["MNW"], plan_kw["max_split_per_seq"],
                                        plan_kw["max_seqs_in_CTA"], plan_kw["max_blocks_in_CTA"], scale, out, None, slots,
-                                       plan_kw.get("bucket_flags"), autotune=autotune and i == 0, tuning=tuning)
+                                       plan_kw.get("bucket_flags"), autotune=autotune and i == 0, tuning=tuning,
+                                       items=plan_kw.get("items"))
             tuning = L.tuning
             launches.append(L)
         ws = torch.empty(max(max(L.need for L in launches), 256), dtype=torch.uint8, device=dev)
@@ -178,7 +179,7 @@ def measure(a, workload: str, steps: int, warmup: int, headline: bool) -> dict:
                   block_tables=lt["block_tables"], num_seqs_per_CTAs=lt["num_seqs_per_CTAs"],
                   CTA_ranks=lt["CTA_ranks"], kv_in_CTAs=lt["kv_in_CTAs"], MNW=lt["MNWs"],
                   max_split_per_seq=info.max_split_per_seq, max_seqs_in_CTA=info.max_seqs_in_CTA,
-                  max_blocks_in_CTA=info.max_blocks_in_CTA, bucket_flags=lt.get("flags"))
+                  max_blocks_in_CTA=info.max_blocks_in_CTA, bucket_flags=lt.get("flags"), items=lt.get("items"))
     pat_slots = lt["slot_tables"]
     whole = info.whole_sequence_tables()
     if whole is not None:
@@ -187,7 +188,7 @@ def measure(a, workload: str, steps: int, warmup: int, headline: bool) -> dict:
                       block_tables=whole["block_tables"], num_seqs_per_CTAs=whole["num_seqs_per_CTAs"],
                       CTA_ranks=whole["CTA_ranks"], kv_in_CTAs=whole["kv_in_CTAs"], MNW=whole["MNWs"],
                       max_split_per_seq=whole["max_split_per_seq"], max_seqs_in_CTA=whole["max_seqs_in_CTA"],
-                      max_blocks_in_CTA=whole["max_blocks_in_CTA"], bucket_flags=None)
+                      max_blocks_in_CTA=whole["max_blocks_in_CTA"], bucket_flags=None, items=None)
         pat_slots = None
     pat_launches, pat_ws = prepare(pat_kw, pat_slots, False)
 
@@ -348,7 +349,7 @@ def measure(a, workload: str, steps: int, warmup: int, headline: bool) -> dict:
 
     if not a.no_oblivious:
         ob = workloads.oblivious_plan(w, dev)
-        ob_kw = {k: ob[k] for k in pat_kw}
+        ob_kw = {k: ob.get(k) for k in pat_kw}   # (no items: the comparator packs one sequence per box)
         ob_launches, ob_ws = prepare(ob_kw, None, False)
         ob_ms, _, _ = timed_median(ob_launches, steps, warmup, reps=3)
         result["oblivious_us_per_call"] = round(ob_ms * 1e3, 3)
