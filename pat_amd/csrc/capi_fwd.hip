@@ -28,6 +28,7 @@ constexpr int kTargetWgsPerCU = 2;  // what fits at once: 2 workgroups of 4 wave
 constexpr int kMinChunk = 128;      // tokens
 constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
+constexpr double kTall32Share = 0.6;          // see plan_geometry
 constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
 constexpr int kLongHeadPerWaveChunk = 1024;   // tokens a wave walks alone (long boxes, a kv head per wave)
@@ -429,10 +430,13 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 
 // Which form of the tall path (boxes of 17..64 rows)? 32-row tiles walk a tall box faster and cost a
 // resident workgroup per CU at head_dim 128. They are taken when that costs nothing - the whole launch
-// is resident at two workgroups per CU anyway - or when the launch waits for its tall boxes: those are
-// long (1024 tokens or more: short ones are mostly prologue and epilogue in either form) and, estimated
-// from sizes, take at least as long as the <= 16-row boxes. Measured (us per call, 16 / 32 rows): c2 26.1 / 25.7,
-// c3 70.9 / 72.7, c5a 70.6 / 67.4; sweep trees with 512-1024 short leaves 5-14 % faster on 16, `1,1024_2048,32` 3 % on 32.
+// is resident at two workgroups per CU anyway - or when, estimated from sizes, its tall boxes take at least
+// kTall32Share of what its <= 16-row boxes do and are longer than the shortest piece (those are mostly prologue and
+// epilogue in either form). Measured (us per call, 16 / 32 rows; tall over short estimate in brackets), trees of the
+// reference's sweep at 64/8 or 16/8 heads: `1,1024_2048,32` 185.5 / 136.5 [6.9], `1,4,256_32,256,32` 28.4 / 22.7 [0.97],
+// `4,16,256,512_512,32,128,32` 69.9 / 68.4 [0.61], `8,16,32,256_512,512,256,32` 36.1 / 33.0 [0.65], but 48.0 / 50.2 [0.15],
+// `1,16,32,64,256,1024_...` 56.0 / 60.8 [0.35] at 16/8; between 0.23 and 0.55 within 2 % either way where neither is resident.
+// At 256 tokens `1,256_256,32` 21.1 / 21.7 [0.86]. Benchmark: c2 29.2 / 25.0, c3 70.2 / 70.3, c5a 68.7 / 57.4.
 // Two boxes of a node are served by one workgroup (32-row form, pat_fwd_bucket items) where the tall boxes fill the
 // device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
 // part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
@@ -464,7 +468,7 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   if (g->tall_rows == 16) return PAT_OK;
   if (g->total_wgs <= (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs) return PAT_OK;
   const LaunchEstimate est = estimate_launch(a, 32, false);
-  if (widest_tall >= 1024 && est.tall_us >= est.short_us) return PAT_OK;
+  if (widest_tall > kTallChunk && est.tall_us >= kTall32Share * est.short_us) return PAT_OK;
   *g = Geometry();
   return plan_geometry_for(a, g, 16, false);
 }
