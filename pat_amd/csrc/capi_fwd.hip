@@ -30,6 +30,7 @@ constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
 constexpr double kTall32Share = 0.6;          // see plan_geometry
 constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
+constexpr int kMaxBesideTall = 1024;         // tokens of a short boxes' chunk sized for the slots that tall workgroups leave
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
 constexpr int kLongHeadPerWaveChunk = 1024;   // tokens a wave walks alone (long boxes, a kv head per wave)
 // workgroups of the split kernel a CU holds at once: 3, or 2 at head_dim 128 with 32-row tiles on tall boxes
@@ -255,6 +256,8 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     // third of the resident slots, the short boxes' chunk is sized for the slots that are left
     // (at least one per CU) instead of for two per CU: short workgroups that have to queue behind
     // the tall ones start late and make the tail.
+    // (up to 1024 tokens: beyond, one workgroup's walk of a long box is the tail. us per call, up to 2048 / up to 1024:
+    // 32 x (16384 + 256..2048) at 64/8 heads, boxes not in twos, 82.6 / 72.0; seven other batches within 1 %)
     int64_t n_tall = 0;
     for (int i = 0; i < a->num_buckets; ++i)
       if (row_tiles(a->buckets[i].mnw[0]) > 1)
@@ -262,7 +265,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
                   std::max<int64_t>(1, ceil_div64((int64_t)a->buckets[i].max_blocks * page, round_unit(tall))) * a->kv_heads;
     if (n_tall > kNumCUs) {
       const int64_t slots = std::max<int64_t>(kNumCUs, resident - n_tall);
-      const int64_t c = std::min<int64_t>(kMaxChunk, ceil_div64(ceil_div64(work, slots), 128) * 128);
+      const int64_t c = std::min<int64_t>(kMaxBesideTall, ceil_div64(ceil_div64(work, slots), 128) * 128);
       chunk = std::max(chunk, c);
     }
   }
@@ -436,6 +439,8 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 // reference's sweep at 64/8 or 16/8 heads: `1,1024_2048,32` 185.5 / 136.5 [6.9], `1,4,256_32,256,32` 28.4 / 22.7 [0.97],
 // `4,16,256,512_512,32,128,32` 69.9 / 68.4 [0.61], `8,16,32,256_512,512,256,32` 36.1 / 33.0 [0.65], but 48.0 / 50.2 [0.15],
 // `1,16,32,64,256,1024_...` 56.0 / 60.8 [0.35] at 16/8; between 0.23 and 0.55 within 2 % either way where neither is resident.
+// That holds for launches with items of two boxes; without, the 32-row form has to take them from 1024 tokens and
+// an equal share (128 x (4096 + 64..512) at 32/8 heads, boxes not in twos: 52.5 / 57.3).
 // At 256 tokens `1,256_256,32` 21.1 / 21.7 [0.86]. Benchmark: c2 29.2 / 25.0, c3 70.2 / 70.3, c5a 68.7 / 57.4.
 // Two boxes of a node are served by one workgroup (32-row form, pat_fwd_bucket items) where the tall boxes fill the
 // device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
@@ -468,7 +473,8 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   if (g->tall_rows == 16) return PAT_OK;
   if (g->total_wgs <= (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs) return PAT_OK;
   const LaunchEstimate est = estimate_launch(a, 32, false);
-  if (widest_tall > kTallChunk && est.tall_us >= kTall32Share * est.short_us) return PAT_OK;
+  if (pairs ? widest_tall > kTallChunk && est.tall_us >= kTall32Share * est.short_us
+            : widest_tall >= 1024 && est.tall_us >= est.short_us) return PAT_OK;
   *g = Geometry();
   return plan_geometry_for(a, g, 16, false);
 }
