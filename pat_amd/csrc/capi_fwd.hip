@@ -437,7 +437,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 // kTall32Share of what its <= 16-row boxes do and are longer than the shortest piece (those are mostly prologue and
 // epilogue in either form). Measured (us per call, 16 / 32 rows; tall over short estimate in brackets), trees of the
 // reference's sweep at 64/8 or 16/8 heads: `1,1024_2048,32` 185.5 / 136.5 [6.9], `1,4,256_32,256,32` 28.4 / 22.7 [0.97],
-// `4,16,256,512_512,32,128,32` 69.9 / 68.4 [0.61], `8,16,32,256_512,512,256,32` 36.1 / 33.0 [0.65], but 48.0 / 50.2 [0.15],
+// `4,16,256,512_512,32,128,32` 69.9 / 68.4 [0.61], but 48.0 / 50.2 [0.15] and
 // `1,16,32,64,256,1024_...` 56.0 / 60.8 [0.35] at 16/8; between 0.23 and 0.55 within 2 % either way where neither is resident.
 // That holds for launches with items of two boxes; without, the 32-row form has to take them from 1024 tokens and
 // an equal share (128 x (4096 + 64..512) at 32/8 heads, boxes not in twos: 52.5 / 57.3).
