@@ -264,7 +264,9 @@ typedef struct pat_fwd_bucket {
 #define PAT_BUCKET_EVEN 1
 /* kv[num_boxes] is followed in memory by an item table, int32 [num_items, 2]: boxes of the bucket (by row) that
  * attend to the same blocks with different sequences (boxes of one tree node) in twos, -1 = no second box; every box
- * stands in exactly one item. A launch may serve the two boxes of an item with one workgroup, or ignore the table. */
+ * stands in exactly one item. A launch may serve the two boxes of an item with one workgroup, which then reads kv and
+ * the block_table row of the first box only, or ignore the table. The caller vouches for the items: after a write to
+ * kv or block_table that may have parted two boxes of an item, launch (and build records) without this flag. */
 #define PAT_BUCKET_ITEMS 2
 
 /* Overrides of the launch geometry. pat_fwd_set_tuning sets them process-wide (a tuning and test
@@ -441,8 +443,10 @@ typedef struct pat_fwd_geometry {
   int32_t num_slots;         /* max_split_per_seq * chunks_per_rank                */
   int64_t num_workgroups;    /* split-kernel workgroups                            */
   int32_t tall_rows;         /* form of the tall path: 32 or 16 rows per wave      */
-  int32_t reserved;
+  int32_t flags;             /* PAT_GEOMETRY_*                                     */
 } pat_fwd_geometry;
+#define PAT_GEOMETRY_PAIRS 1 /* the two boxes of an item are served by one workgroup */
+#define PAT_GEOMETRY_APART 2 /* 32-row form: K and V tiles handed over apart         */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);
 
 /* ------------------------------------------------------------------------ *

@@ -84,6 +84,8 @@ class FwdBucket(C.Structure):
 
 PAT_BUCKET_EVEN = 1
 PAT_BUCKET_ITEMS = 2
+PAT_GEOMETRY_PAIRS = 1
+PAT_GEOMETRY_APART = 2
 
 
 class BaselineArgs(C.Structure):
@@ -128,7 +130,7 @@ class FwdArgs(C.Structure):
 class FwdGeometry(C.Structure):
     _fields_ = [("chunk_tokens", C.c_int32), ("tall_chunk_tokens", C.c_int32),
                 ("chunks_per_rank", C.c_int32), ("num_slots", C.c_int32),
-                ("num_workgroups", C.c_int64), ("tall_rows", C.c_int32), ("reserved", C.c_int32)]
+                ("num_workgroups", C.c_int64), ("tall_rows", C.c_int32), ("flags", C.c_int32)]
 
 
 # Every symbol include/pat_amd.h declares: name -> (restype, argtypes)

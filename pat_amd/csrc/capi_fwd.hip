@@ -537,7 +537,7 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   out->num_slots = g.num_slots;
   out->num_workgroups = g.total_wgs;
   out->tall_rows = g.tall_rows;
-  out->reserved = 0;
+  out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0);
   return PAT_OK;
 }
 

@@ -81,9 +81,22 @@ struct Prepared {
   size_t need = 0;          // workspace bytes with prebuilt records
   size_t need_inline = 0;   // workspace bytes when the launch builds its records itself (args.records NULL)
   bool derive_slots = false;   // the plan came without slot tables: ordinals derived on the device
+  std::vector<size_t> item_buckets;   // buckets with an item table (see use_items)
+  bool items_on = false;    // ... and whether `buckets` hands them to the launch
+  bool records_items = false;   // the same when `records` were built
   pat_fwd_tuning tuning;    // the measured geometry of this plan shape (args.tuning points here when set)
   Prepared() { std::memset(&args, 0, sizeof(args)); std::memset(&tuning, 0, sizeof(tuning)); }
 };
+
+// Hands the plan's item tables (boxes that one workgroup may serve together) to the launch, or keeps them back. An item
+// is a statement about the tables' contents - its boxes have the same length and blocks, and the launch reads those of the
+// first box only - so it goes with a snapshot of tables nobody has written to since the planner made them
+// (KernelInfo::items_hold); wherever the tables are read as they are at the time, every box stands alone.
+void use_items(Prepared& L, bool on) {
+  if (L.items_on == on) return;
+  for (size_t i : L.item_buckets) L.buckets[i].flags ^= PAT_BUCKET_ITEMS;
+  L.items_on = on;
+}
 
 // ---- measured launch geometry, remembered per plan shape ---------------------------------------
 // pat_fwd_autotune times a launch under a few candidate geometries. One measurement serves every
@@ -228,6 +241,7 @@ void attach_records(Prepared& L, RecordStore& store, int64_t version, const c10:
   }
   L.records = it->second;
   L.plan_version = version;
+  L.records_items = L.items_on;
   a.records = L.records->tensor.data_ptr(); a.records_bytes = (size_t)L.records->tensor.numel(); a.records_tag = tag;
   check(pat_fwd_workspace_bytes(&a, &L.need));
 }
@@ -252,7 +266,8 @@ struct PlanTables {
 std::shared_ptr<Prepared> prepare(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                   const at::Tensor& num_split, const PlanTables& pt, int max_split, int max_seqs,
                                   int max_blocks, double scale, const at::Tensor& out,
-                                  const std::optional<at::Tensor>& lse, RecordStore& store, int64_t plan_version) {
+                                  const std::optional<at::Tensor>& lse, RecordStore& store, int64_t plan_version,
+                                  bool items_hold = false) {
   require(q.scalar_type() == at::kHalf || q.scalar_type() == at::kBFloat16, "only support fp16 and bf16 data type");
   require(k.scalar_type() == q.scalar_type(), "query and key must have the same dtype");
   require(v.scalar_type() == q.scalar_type(), "query and value must have the same dtype");
@@ -317,7 +332,8 @@ std::shared_ptr<Prepared> prepare(const at::Tensor& q, const at::Tensor& k, cons
     for (const auto& nt : named) L->keep.push_back(*nt.second);
     if (pt.items != nullptr && (*pt.items)[i].numel() > 0) {
       require((*pt.items)[i].data_ptr<int32_t>() == fb.kv + ctas, "an item table stands right behind its bucket's kv table");
-      fb.flags |= PAT_BUCKET_ITEMS; fb.num_items = (int32_t)(*pt.items)[i].size(0);
+      fb.num_items = (int32_t)(*pt.items)[i].size(0);
+      L->item_buckets.push_back(i);
       L->keep.push_back((*pt.items)[i]);
     }
   }
@@ -364,16 +380,19 @@ std::shared_ptr<Prepared> prepare(const at::Tensor& q, const at::Tensor& k, cons
     a.num_split_per_seq = base;
     L->keep.push_back(store.derived_slots);
   }
+  use_items(*L, items_hold);
   tune(*L, q.device());
+  use_items(*L, false);   // (a launch that builds its records itself reads the tables as they are)
   a.records = nullptr; a.records_bytes = 0;
   check(pat_fwd_workspace_bytes(&a, &L->need_inline));
   return L;
 }
 
-void run(Prepared& L, RecordStore& store, int64_t version, const c10::Device& dev) {
+void run(Prepared& L, RecordStore& store, int64_t version, const c10::Device& dev, bool items_hold = false) {
   void* stream = raw_stream(dev);
   const bool snapshot = version != kUntracked && !capturing(stream);
   pat_fwd_args& a = L.args;
+  use_items(L, snapshot && items_hold);
   if (L.derive_slots && (!snapshot || store.derived_version != version)) {
     std::vector<int64_t> offsets(store.derived_offsets.size(), 0);
     a.records = nullptr;
@@ -382,7 +401,7 @@ void run(Prepared& L, RecordStore& store, int64_t version, const c10::Device& de
   }
   size_t need;
   if (snapshot) {
-    if (!L.records || L.plan_version != version) attach_records(L, store, version, dev);
+    if (!L.records || L.plan_version != version || L.records_items != L.items_on) attach_records(L, store, version, dev);
     a.records = L.records->tensor.data_ptr(); a.records_bytes = (size_t)L.records->tensor.numel();
     need = L.need;
     if (!L.records->seen_ready && stream != L.records->stream) {
@@ -470,6 +489,12 @@ struct KernelInfo {
     return v;
   }
   void invalidate() { ++generation; }
+  // Do the item tables still describe the plan tables? Only as long as nobody has written to the plan since the planner
+  // made it: items_version is the plan's version then. A writer that knows the items stay right - an edit of boxes that
+  // stand in none, DecodePlan.advance_step's - calls hold_items() after it, if they held before it.
+  int64_t items_version = kUntracked;
+  bool items_hold() const { const int64_t v = plan_version(); return has_launch && v != kUntracked && v == items_version; }
+  void hold_items() { items_version = plan_version(); }
 
   void clear_tables() {
     for (TensorList* l : {&q_tables, &block_tables, &num_seqs, &ranks, &kvs, &slot_tables, &l_q_tables,
@@ -535,8 +560,10 @@ struct KernelInfo {
     // counters are what tells a launch that DecodePlan.advance_step edited them)
     c10::InferenceMode plain(false);
     if (flat.has_value()) {
+      const bool held = items_hold();
       flat = flat->to(device, /*non_blocking=*/true);
       bind(*flat);
+      items_version = held ? plan_version() : kUntracked;
       return;
     }
     auto move = [&](TensorList& l) { for (auto& t : l) t = t.to(device, true); };
@@ -861,6 +888,7 @@ struct PrefixTreeCPP {
       fresh->max_seqs = fresh->layout.max_seqs_in_box;
       fresh->max_blocks = fresh->layout.max_blocks_in_box;
       fresh->bind(host);
+      fresh->hold_items();
     } else {
       // more buckets than one launch takes: the plan can still be read, table by table
       pat_plan_view view;
@@ -1009,12 +1037,12 @@ void fwd_tree(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, Pre
       L = prepare(q, k, v, info.ws_num_split, ws, 1, 1, info.ws_width, scale, out, lse, info.records, version);
     } else {
       L = prepare(q, k, v, info.num_boxes_per_seq, pt, info.max_boxes, info.max_seqs, info.max_blocks, scale, out, lse,
-                  info.records, version);
+                  info.records, version, info.items_hold());
     }
     if (info.cache.size() >= 256) info.cache.clear();
     info.cache[key.bytes] = L;
   }
-  run(*L, info.records, version, q.device());
+  run(*L, info.records, version, q.device(), info.items_hold());
 }
 
 void paged_decode_baseline(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& block_table,
@@ -1086,6 +1114,8 @@ PYBIND11_MODULE(_prefix_attn, m) {
       .def("invalidate", &KernelInfo::invalidate,
            "Drops what launches remember about the plan tables' contents (launch records, derived slots): call it "
            "after writing to the tables by means torch's version counters do not see.")
+      .def("_items_hold", &KernelInfo::items_hold)
+      .def("_hold_items", &KernelInfo::hold_items)
       .def("launch_tables", &KernelInfo::launch_tables,
            "The per-bucket tables as the kernels get them (boxes longest first, a bucket with a wide head split "
            "in two) with their tile labels under \"MNWs\" and hints under \"flags\".")
@@ -1114,6 +1144,19 @@ PYBIND11_MODULE(_prefix_attn, m) {
           if (kv.second->args.tuning == nullptr) out.emplace_back();
           else out.push_back({t.chunk_tokens, t.tall_chunk_tokens, t.head_per_wave_tokens, t.head_per_wave_long_tokens,
                               t.head_per_wave_long_wgs, t.equalize_chunks, t.direct_out, t.tall_rows});
+        }
+        return out;
+      })
+      .def_property_readonly("_launch_geometries", [](const KernelInfo& ki) {
+        py::list out;   // per cached launch: what pat_fwd_geometry_of says of its last call
+        for (const auto& kv : ki.cache) {
+          pat_fwd_geometry g;
+          check(pat_fwd_geometry_of(&kv.second->args, &g));
+          py::dict d;
+          d["chunk_tokens"] = g.chunk_tokens; d["tall_chunk_tokens"] = g.tall_chunk_tokens; d["num_slots"] = g.num_slots;
+          d["num_workgroups"] = g.num_workgroups; d["tall_rows"] = g.tall_rows;
+          d["pairs"] = (g.flags & PAT_GEOMETRY_PAIRS) != 0; d["apart"] = (g.flags & PAT_GEOMETRY_APART) != 0;
+          out.append(d);
         }
         return out;
       })

@@ -189,6 +189,7 @@ class DecodePlan:
                 return False
         self._tail_kv += 1
         device = info.num_split_per_seq.device
+        hold = info._items_hold()             # the edits below are of boxes of one request, which no item holds
         if whole is not None:
             whole["kv_in_CTAs"][0].add_(1)
             crossed = [s for s, n_old in enumerate(old) if n_old % bs == 0]
@@ -209,6 +210,8 @@ class DecodePlan:
                         flat = rows * tables[t].shape[1] + cols[which]
                         tables[t].view(-1).index_copy_(0, torch.as_tensor(flat, device=device),
                                                        torch.as_tensor(ids[which], dtype=torch.int32, device=device))
+        if hold:
+            info._hold_items()
         return True
 
 

@@ -1259,20 +1259,87 @@ def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, pag
     q, k, v = w.tensors(dev)
     tree = PrefixTreeCPP(page)
     tree.build_radix_tree(w.seq_lens, w.padded_table())
-    tree.pack_schedule(None, heads[0] // heads[1], heads[1])
-    info = tree.kernel_info
-    info.to_gpu(dev)
-    items = [t for t in info.launch_tables()["items"] if t.numel()]
-    assert seqs == 22 or any((t[:, 1] >= 0).any() for t in items), "the case has no two boxes of one node"
     ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, w.seq_lens, scale)
     for pairs in (1, 2):
         tuning(tall_rows=32, tall_chunk_tokens=chunk, pairs=pairs)
-        tree.kernel_info.invalidate()
+        tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+        info = tree.kernel_info
+        info.to_gpu(dev)
+        assert seqs == 22 or any((t[:, 1] >= 0).any() for t in info.launch_tables()["items"]), "the case has no two boxes of one node"
         out = torch.full_like(q, float("nan"))
         lse = torch.full((seqs, heads[0]), float("nan"), dtype=torch.float32, device=dev)
         prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
         torch.cuda.synchronize()
+        assert [g["pairs"] for g in info._launch_geometries] == [pairs == 1 and seqs != 22]
         _assert_close(f"pairs {pairs}", out, lse, ref_out, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_edit_of_one_box_of_a_pair(captured, tuning):
+    # two boxes of a node share a workgroup, which reads the first one's length and blocks: a write to the plan tables that
+    # parts them - the second loses its last blocks, then gets another block, then the first loses some - is seen for the box
+    # it was made to and no other, by the next call and by every replay of a graph that holds the write
+    print(f"[case] edits of one box of a pair, captured {captured}", flush=True)
+    dev = _device()
+    w = workloads.shared_prefix("pair-edit", 64, 40 * 16, 20, 60, 32, 8, 128, torch.float16, 3)
+    q, k, v = w.tensors(dev)
+    scale = 1.0 / math.sqrt(w.head_dim)
+    tuning(tall_rows=32, pairs=1)
+    tree = PrefixTreeCPP(w.page_size)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, w.heads // w.kv_heads, w.kv_heads)
+    info = tree.kernel_info
+    info.to_gpu(dev)
+    lt = info.launch_tables()
+    bucket, a, b = next((i, *row) for i, t in enumerate(lt["items"]) for row in t.tolist() if row[1] >= 0)
+    kv, table = lt["kv_in_CTAs"][bucket], lt["block_tables"][bucket]
+    kv0, table0 = kv.clone(), table.clone()
+    used = [set(lt["q_tables"][bucket][box][:int(lt["num_seqs_per_CTAs"][bucket][box])].tolist()) for box in (a, b)]
+    assert kv0[a] == kv0[b] == 640 and torch.equal(table0[a], table0[b]) and not used[0] & used[1]
+    lse = torch.empty(w.batch, w.heads, dtype=torch.float32, device=dev)
+    out = torch.empty_like(q)
+
+    def call():
+        prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
+
+    call()
+    torch.cuda.synchronize()
+    ref = _oracle(w, q, k, v)
+    _assert_close("before any edit", out, lse, *ref, w.dtype)
+    assert info._launch_geometries[0]["pairs"]
+    other = w.num_blocks - 1                         # a block of some request's tail
+    # (box, blocks it loses, (column, block) it gets)
+    edits = [(b, 3, None), (b, 0, (5, other)), (a, 7, None), (b, 0, None)]
+    staged_kv, staged_table = kv0.clone(), table0.clone()
+    if captured:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            kv.copy_(staged_kv)
+            table.copy_(staged_table)
+            call()
+    for box, lost, swap in edits:
+        staged_kv.copy_(kv0)
+        staged_table.copy_(table0)
+        staged_kv[box] -= 16 * lost
+        if swap:
+            staged_table[box, swap[0]] = swap[1]
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        if captured:
+            graph.replay()
+        else:
+            kv.copy_(staged_kv)
+            table.copy_(staged_table)
+            call()
+        torch.cuda.synchronize()
+        rows, lens = [list(r) for r in w.rows], list(w.seq_lens)
+        for s in used[0] if box == a else used[1]:
+            if swap:
+                rows[s][swap[0]] = swap[1]
+            del rows[s][40 - lost:40]
+            lens[s] -= 16 * lost
+        ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, lens, scale)
+        _assert_close(f"{'second' if box == b else 'first'} box, {lost} blocks lost, {swap} set", out, lse, ref_out, ref_lse, w.dtype)
 
 
 @pytest.mark.parametrize("slots,batch,heads,d,dtype", [

@@ -145,6 +145,27 @@ def _little_sharing():
     return workloads.Workload("little-sharing", 8, 8, 64, torch.float16, 16, lens, rows, nxt, 512 + sum(n - 512 for n in lens), 0)
 
 
+def test_item_tables_hold_until_somebody_else_writes_to_the_plan():
+    # boxes are served in twos only while their tables are as the planner made them: advance_step's own edits (boxes of
+    # one request, which stand in no item) leave that alone, any other write and invalidate() end it
+    w = workloads.shared_prefix("items", 64, 640, 33, 46, 32, 8, 128, torch.float16, 5)   # (no tail crosses a page)
+    meta = fake_metadata(w, torch.device("cpu"))
+    plan = DecodePlan.from_metadata(meta)
+    info = plan._ready_tree().kernel_info
+    assert any((t[:, 1] >= 0).any() for t in info.launch_tables()["items"]) and info._items_hold()
+    rows, _ = _grown(w, 1, range(w.num_blocks, w.num_blocks + 64))
+    version = info._flat._version
+    assert plan.advance_step(_table(rows, w.padded_table().shape[1])) and info._flat._version > version
+    assert info._items_hold()
+    info.invalidate()
+    assert not info._items_hold()
+    info._hold_items()
+    info.launch_tables()["kv_in_CTAs"][0][0] -= 1
+    assert not info._items_hold()
+    info.to_gpu("cpu")
+    assert not info._items_hold()
+
+
 @pytest.mark.parametrize("case", ["c1", "wide-head", "little-sharing"])
 def test_advance_step_keeps_the_plan_right_on_cpu(case):
     """After every in-place advance the plan, executed item by item by the oracle, gives dense
