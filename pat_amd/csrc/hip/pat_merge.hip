@@ -15,7 +15,8 @@
 // requested at once and what turns out unused is dropped (measured: 0.3-0.8 us less per launch;
 // with 16 rows requested blindly the extra registers and reads cost what the round trips save).
 // Two more forms stand below: a half-wave per row where rows are many and slots few, a workgroup per row where
-// slots are many (9..32) and rows few.
+// slots are many (9..32) and rows few. In all of them a slot is empty where its LSE is -inf, and nowhere else: a NaN (from
+// a NaN in Q or K, or an infinite score) is a filled slot, and makes the row NaN as it makes one that is not cut up.
 #include <hip/hip_runtime.h>
 
 #include "fwd_params.hpp"
@@ -108,20 +109,20 @@ __global__ void __launch_bounds__(256) pat_merge_kernel(MERGE_ROWS, const MergeP
 #pragma unroll
     for (int off = kSpec / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     mx = __shfl(mx, 0);
-    float e = (l > ninf) ? __expf(l - mx) : 0.f;
+    float e = (l != ninf) ? __expf(l - mx) : 0.f;
     float sum = e;
 #pragma unroll
     for (int off = kSpec / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     sum = __shfl(sum, 0);
-    const float total = (sum > 0.f) ? mx + logf(sum) : ninf;
-    const float w_mine = (l > ninf) ? __expf(l - total) : 0.f;
+    const float total = (sum != 0.f) ? mx + logf(sum) : ninf;
+    const float w_mine = (l != ninf) ? __expf(l - total) : 0.f;
     float acc[CPL];
 #pragma unroll
     for (int c = 0; c < CPL; ++c) acc[c] = 0.f;
 #pragma unroll
     for (int b = 0; b < kSpec; ++b) {
       const float w = __shfl(w_mine, b);
-      if (b < num_slots && w > 0.f) {
+      if (b < num_slots && w != 0.f) {
 #pragma unroll
         for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
       }
@@ -150,14 +151,12 @@ __global__ void __launch_bounds__(256) pat_merge_kernel(MERGE_ROWS, const MergeP
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
   float sum = 0.f;
-  if (mx > ninf) {
 #pragma unroll
-    for (int r = 0; r < kRegs; ++r) sum += __expf(mine[r] - mx);   // exp(-inf) = 0
-    for (int i = kRegs * 64 + lane; i < nslots; i += 64) sum += __expf(lse[i] - mx);
-  }
+  for (int r = 0; r < kRegs; ++r) sum += (mine[r] != ninf) ? __expf(mine[r] - mx) : 0.f;
+  for (int i = kRegs * 64 + lane; i < nslots; i += 64) { const float l = lse[i]; sum += (l != ninf) ? __expf(l - mx) : 0.f; }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  const float total = (sum > 0.f) ? mx + logf(sum) : ninf;
+  const float total = (sum != 0.f) ? mx + logf(sum) : ninf;
 
   float acc[CPL];
 #pragma unroll
@@ -165,7 +164,7 @@ __global__ void __launch_bounds__(256) pat_merge_kernel(MERGE_ROWS, const MergeP
 
   // weighted sum of the filled slots of one 64-slot group
   auto accumulate = [&](int base, float w_mine) {
-    unsigned long long live = __ballot(w_mine > 0.f);
+    unsigned long long live = __ballot(w_mine != 0.f);
     while (live) {
       int js[kBatch];
       float v[kBatch][CPL];
@@ -200,12 +199,12 @@ __global__ void __launch_bounds__(256) pat_merge_kernel(MERGE_ROWS, const MergeP
 #pragma unroll
   for (int r = 0; r < kRegs; ++r) {
     if (r * 64 >= nslots) break;
-    accumulate(r * 64, (mine[r] > ninf) ? __expf(mine[r] - total) : 0.f);
+    accumulate(r * 64, (mine[r] != ninf) ? __expf(mine[r] - total) : 0.f);
   }
   for (int base = kRegs * 64; base < nslots; base += 64) {
     const int i = base + lane;
     const float l = (i < nslots) ? lse[i] : ninf;
-    accumulate(base, (l > ninf) ? __expf(l - total) : 0.f);
+    accumulate(base, (l != ninf) ? __expf(l - total) : 0.f);
   }
 
   T* dst = (T*)p.out + (int64_t)s * p.o_stride_b + (int64_t)hq * p.o_stride_h + lane * CPL;
@@ -257,20 +256,20 @@ __global__ void __launch_bounds__(256) pat_merge_pairs_kernel(MERGE_ROWS, const 
 #pragma unroll
   for (int off = kSpec / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
   mx = __shfl(mx, half * 32);
-  float e = (l > ninf) ? __expf(l - mx) : 0.f;
+  float e = (l != ninf) ? __expf(l - mx) : 0.f;
   float sum = e;
 #pragma unroll
   for (int off = kSpec / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
   sum = __shfl(sum, half * 32);
-  const float total = (sum > 0.f) ? mx + logf(sum) : ninf;
-  const float w_mine = (l > ninf) ? __expf(l - total) : 0.f;
+  const float total = (sum != 0.f) ? mx + logf(sum) : ninf;
+  const float w_mine = (l != ninf) ? __expf(l - total) : 0.f;
   float acc[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) acc[c] = 0.f;
 #pragma unroll
   for (int b = 0; b < kSpec; ++b) {
     const float w = __shfl(w_mine, half * 32 + b);
-    if (b < num_slots && w > 0.f) {
+    if (b < num_slots && w != 0.f) {
 #pragma unroll
       for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
     }
@@ -319,7 +318,7 @@ __global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const M
 #pragma unroll
   for (int off = kSpec / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
   mx = __shfl(mx, 0);
-  const float w_mine = (l > ninf) ? __expf(l - mx) : 0.f;
+  const float w_mine = (l != ninf) ? __expf(l - mx) : 0.f;
   float sum = w_mine;
 #pragma unroll
   for (int off = kSpec / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
@@ -330,7 +329,7 @@ __global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const M
   for (int b = 0; b < kSpec; ++b) {
     const float w = __shfl(w_mine, b);
     // (rows of slots that are empty or beyond the count hold anything: dropped, not multiplied)
-    if (b < mine && first + b < num_slots && w > 0.f) {
+    if (b < mine && first + b < num_slots && w != 0.f) {
 #pragma unroll
       for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
     }
@@ -346,10 +345,10 @@ __global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const M
   float weight[4], all = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    weight[w] = s_max[w] > ninf ? __expf(s_max[w] - most) : 0.f;
+    weight[w] = s_sum[w] != 0.f ? __expf(s_max[w] - most) : 0.f;
     all += weight[w] * s_sum[w];
   }
-  const float inv = all > 0.f ? 1.f / all : 0.f;
+  const float inv = all != 0.f ? 1.f / all : 0.f;
   T* dst = (T*)p.out + (int64_t)s * p.o_stride_b + (int64_t)hq * p.o_stride_h + lane * CPL;
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
@@ -358,7 +357,7 @@ __global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const M
     for (int w = 0; w < 4; ++w) x += weight[w] * s_acc[w][lane * CPL + c];
     dst[c] = (T)(x * inv);
   }
-  if (p.lse_out != nullptr && lane == 0) p.lse_out[pair] = all > 0.f ? most + logf(all) : ninf;
+  if (p.lse_out != nullptr && lane == 0) p.lse_out[pair] = all != 0.f ? most + logf(all) : ninf;
 }
 
 // Host launcher: one wave per (sequence, query head), four per workgroup; a half-wave each in large launches

@@ -1379,3 +1379,28 @@ def test_merge_of_many_slots(slots, batch, heads, d, dtype, tuning):
     torch.cuda.synchronize()
     ref_out, ref_lse = _oracle(w, q, k, v)
     _assert_close(f"{slots} slots", out, lse, ref_out, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("slots,batch,heads,d,dtype", [
+    (4, 3, (8, 8), 64, torch.float16),           # a wave per row, every slot requested at once
+    (3, 600, (32, 8), 128, torch.bfloat16),      # a half-wave per row
+    (16, 3, (32, 8), 128, torch.float16),        # a workgroup per row
+    (40, 2, (8, 8), 64, torch.bfloat16),         # a wave per row, slots by sixteens
+])
+def test_a_nan_in_one_piece_shows_in_the_row(slots, batch, heads, d, dtype, tuning, monkeypatch):
+    # one NaN in K: the rows of its request and kv head are NaN, LSE too, however many pieces the request is cut in
+    print(f"[case] NaN in one of {slots} pieces, {batch} requests, heads {heads}, d {d}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    w = workloads.independent("nan", batch, slots * 32, heads[0], heads[1], d, dtype, 1)
+    q, k, v = w.tensors(dev)
+    group = heads[0] // heads[1]
+    bad = torch.zeros(batch, heads[0], dtype=torch.bool)
+    k[w.rows[1][2 * (slots - 1)], 3, 2, 5] = float("nan")    # request 1, its last piece, kv head 2
+    bad[1, 2 * group:3 * group] = True
+    tuning(chunk_tokens=32, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    out, lse = _run_tree(w, q, k, v)
+    assert torch.isnan(out.float().cpu()[:, 0][bad]).all() and torch.isnan(lse.cpu()[bad]).all()
+    ref_out, ref_lse = _oracle(w, q, k, v)
+    good = ~bad
+    _assert_close("the other rows", out.cpu()[:, 0][good], lse.cpu()[good], ref_out[:, 0][good], ref_lse[good], dtype)
