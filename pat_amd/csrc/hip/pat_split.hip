@@ -494,7 +494,8 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     static_assert(2 * (D / 8) * 64 * 16 <= 2 * STAGE2, "the exchange buffer of the epilogue fits the stages");
     const int nss_u = (ntok_u + SST - 1) / SST;
     const int last_rel_u = ntok_u - 1;
-    const float sc_abs = fmaxf(__builtin_fabsf(p.scale_log2), 1e-30f);   // (a scale of 0 keeps masked scores at -inf)
+    // (a scale of 0 stands as the smallest normal number, which keeps masked scores at -inf; a NaN stays one)
+    const float sc_abs = p.scale_log2 == 0.f ? 1.17549435e-38f : __builtin_fabsf(p.scale_log2);
 
     // Q^T operand (lane (n32, h2): row n32, dims 16kk + 8h2 ..+7). A negative softmax scale is
     // folded into Q's sign (exact), so that the row maximum can be taken over the raw scores.

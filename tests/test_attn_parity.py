@@ -1404,3 +1404,28 @@ def test_a_nan_in_one_piece_shows_in_the_row(slots, batch, heads, d, dtype, tuni
     ref_out, ref_lse = _oracle(w, q, k, v)
     good = ~bad
     _assert_close("the other rows", out.cpu()[:, 0][good], lse.cpu()[good], ref_out[:, 0][good], ref_lse[good], dtype)
+
+
+@pytest.mark.parametrize("tall_rows", [16, 32])
+@pytest.mark.parametrize("scale", [float("nan"), 1e-33])
+def test_scale_at_the_ends_of_its_range(scale, tall_rows, tuning):
+    # a NaN scale gives NaN rows in both forms of the tall path; a tiny one is not rounded up (scores of about 1e33 here)
+    print(f"[case] softmax scale {scale}, {tall_rows}-row tiles", flush=True)
+    dev = _device()
+    w = workloads.shared_prefix("scale", 32, 640, 20, 60, 32, 8, 128, torch.bfloat16, 3)
+    q, k, v = w.tensors(dev)
+    q, k = q * 1e16, k * 1e16
+    tuning(tall_rows=tall_rows)
+    tree = PrefixTreeCPP(w.page_size)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, w.heads // w.kv_heads, w.kv_heads)
+    tree.kernel_info.to_gpu(dev)
+    out = torch.zeros_like(q)
+    lse = torch.zeros(w.batch, w.heads, dtype=torch.float32, device=dev)
+    prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    if math.isnan(scale):
+        assert torch.isnan(out).all() and torch.isnan(lse).all()
+    else:
+        ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), w.rows, w.seq_lens, scale)
+        _assert_close(f"scale {scale}", out, lse, ref_out, ref_lse, w.dtype)
