@@ -546,7 +546,11 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     }
     auto at_step = [&](uint64_t v, int ss) -> const char* {
       const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, ss), hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), ss);
-      return (const char*)(((uint64_t)hi << 32) | lo);
+      uint64_t at = ((uint64_t)hi << 32) | lo;
+      // A vector memory instruction may read a scalar register 5 wait states after a vector instruction wrote it. The
+      // compiler keeps that distance for loads it sees; load_to_lds it does not see.
+      asm volatile("s_nop 4" : "+s"(at));
+      return (const char*)at;
     };
     auto fetch_k = [&](int ss) {
       const char* base = at_step(k_at, ss);
