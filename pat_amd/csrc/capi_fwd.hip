@@ -28,7 +28,6 @@ constexpr int kTargetWgsPerCU = 2;  // what fits at once: 2 workgroups of 4 wave
 constexpr int kMinChunk = 128;      // tokens
 constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
-constexpr double kTall32Share = 0.6;          // see plan_geometry
 constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
 constexpr int kMaxBesideTall = 1024;         // tokens of a short boxes' chunk sized for the slots that tall workgroups leave
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
@@ -177,10 +176,11 @@ int check_args(const pat_fwd_args* a) {
 }
 
 // Times of a launch estimated from sizes alone (us): what its <= 16-row boxes take to stream (~5.8 TB/s; ragged
-// buckets, without the PAT_BUCKET_EVEN hint, hold ~0.6 of their widest box on average), what its tall boxes take
-// spread over all CUs, and the longest tall box walked by one workgroup. A super-step of 64 tokens takes ~1.25 us for
-// one box and ~1.5 us for two (32-row form); in the 16-row form 1.7 us alone, ~3 us beside two others on the CU.
-struct LaunchEstimate { double short_us = 0., tall_us = 0., chain_us = 0.; };
+// buckets, without the PAT_BUCKET_EVEN hint, hold ~0.6 of their widest box on average) and how many rounds of three
+// workgroups per CU they are, what its tall boxes take spread over all CUs, and the longest tall box walked by one
+// workgroup. A super-step of 64 tokens takes ~1.25 us for one box and ~1.5 us for two (32-row form); in the 16-row form
+// 1.7 us alone, ~3 us beside two others on the CU.
+struct LaunchEstimate { double short_us = 0., short_rounds = 0., tall_us = 0., chain_us = 0.; };
 constexpr double kShortestLaunchUs = 5.5;
 LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs) {
   LaunchEstimate e;
@@ -194,7 +194,9 @@ LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs)
       e.tall_us += tokens * (double)(items * a->kv_heads) / 64. * step_us / kNumCUs;
       e.chain_us = std::max(e.chain_us, tokens / 64. * (tall_rows == 16 ? 3.0 : step_us));
     } else {
-      e.short_us += tokens * (double)b.num_boxes * a->kv_heads * ((b.flags & PAT_BUCKET_EVEN) ? 1.0 : 0.6) * a->head_dim * 4. / 5.8e6;
+      const double box_heads = (double)b.num_boxes * a->kv_heads;
+      e.short_us += tokens * box_heads * ((b.flags & PAT_BUCKET_EVEN) ? 1.0 : 0.6) * a->head_dim * 4. / 5.8e6;
+      e.short_rounds += box_heads / (tokens <= 128. && a->kv_heads % kWaves == 0 ? kWaves : 1) / (3. * kNumCUs);
     }
   }
   return e;
@@ -433,15 +435,18 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 
 // Which form of the tall path (boxes of 17..64 rows)? 32-row tiles walk a tall box faster and cost a
 // resident workgroup per CU at head_dim 128. They are taken when that costs nothing - the whole launch
-// is resident at two workgroups per CU anyway - or when, estimated from sizes, its tall boxes take at least
-// kTall32Share of what its <= 16-row boxes do and are longer than the shortest piece (those are mostly prologue and
-// epilogue in either form). Measured (us per call, 16 / 32 rows; tall over short estimate in brackets), trees of the
-// reference's sweep at 64/8 or 16/8 heads: `1,1024_2048,32` 185.5 / 136.5 [6.9], `1,4,256_32,256,32` 28.4 / 22.7 [0.97],
-// `4,16,256,512_512,32,128,32` 69.9 / 68.4 [0.61], but 48.0 / 50.2 [0.15] and
-// `1,16,32,64,256,1024_...` 56.0 / 60.8 [0.35] at 16/8; between 0.23 and 0.55 within 2 % either way where neither is resident.
-// That holds for launches with items of two boxes; without, the 32-row form has to take them from 1024 tokens and
-// an equal share (128 x (4096 + 64..512) at 32/8 heads, boxes not in twos: 52.5 / 57.3).
-// At 256 tokens `1,256_256,32` 21.1 / 21.7 [0.86]. Benchmark: c2 29.2 / 25.0, c3 70.2 / 70.3, c5a 68.7 / 57.4.
+// is resident anyway - or when its tall boxes outweigh that, estimated from sizes (tall_us against short_us and
+// short_rounds of estimate_launch). The lines were checked on 420 batches drawn over 1..1024 requests, 2..32 kv heads and both
+// head sizes whose launch is not resident in the 32-row form, both forms timed in their own cuts:
+//  * with items of two boxes (119 at head_dim 128): tall boxes longer than the shortest piece (shorter ones are mostly
+//    prologue and epilogue in either form) that take 0.6 of the others' streaming time and 3 us for every round of their
+//    workgroups, each of which waits longer for a place (us per call, 16 / 32 rows: 691 x (368 + 6..48) tokens at 16/2 heads
+//    23.7 / 25.2, 777 x (400 + 9..72) 26.1 / 27.6, but 198 x (512 + 1..2) at 64/8 21.8 / 19.8, `1,1024_2048,32` 153 / 117,
+//    `1,4,256_32,256,32` 25.8 / 21.4). More than 3 % behind the other form: 8.
+//  * without items (213 at head_dim 128): from 1024 tokens and an equal share (128 x (4096 + 64..512) at 32/8 heads,
+//    boxes not in twos: 52.5 / 57.3). More than 3 % behind: 54, nearly all left to the 16-row form.
+//  * at head_dim 64 (88) the 32-row form costs no place: from 640 tokens, 0.3 of the streaming time and 2 us a round
+//    (102 x (4848 + 580..1160) at 32/8 heads, six nodes: 69.6 / 62.3). More than 3 % behind: 7; the lines above: 11.
 // Two boxes of a node are served by one workgroup (32-row form, pat_fwd_bucket items) where the tall boxes fill the
 // device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
 // part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
@@ -473,8 +478,10 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   if (g->tall_rows == 16) return PAT_OK;
   if (g->total_wgs <= (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs) return PAT_OK;
   const LaunchEstimate est = estimate_launch(a, 32, false);
-  if (pairs ? widest_tall > kTallChunk && est.tall_us >= kTall32Share * est.short_us
-            : widest_tall >= 1024 && est.tall_us >= est.short_us) return PAT_OK;
+  const bool outweigh = a->head_dim == 64 ? widest_tall >= 640 && est.tall_us >= 0.3 * est.short_us + 2. * est.short_rounds
+                        : pairs           ? widest_tall > kTallChunk && est.tall_us >= std::max(0.6 * est.short_us, 3. * est.short_rounds)
+                                          : widest_tall >= 1024 && est.tall_us >= est.short_us;
+  if (outweigh) return PAT_OK;
   *g = Geometry();
   return plan_geometry_for(a, g, 16, false);
 }

@@ -293,3 +293,25 @@ def test_form_of_the_tall_path_follows_the_launch():
     assert form(24, 171, 32, 128, 32)[0] == 32          # a 16k prefix in 2736-token tall boxes over 2048-token suffixes
     assert form(128, 8, 1024, 2, 1024)[0] == 16         # many short tall boxes over a thousand 32-token leaves
     assert form(0, 128, 512, 64, 512)[0] == 16          # no tall box at all
+
+    # items of two boxes: hundreds of two- to five-page boxes at 2 kv heads wait for places (32-row form 6-9 % slower), a few
+    # workgroups of four heads each do not (9 % faster); head_dim 64, where the 32-row form costs no place, without items
+    def form_of(buckets, heads, kv_heads, d, batch):
+        a = _args(batch=batch, heads=heads, kv_heads=kv_heads, head_dim=d)
+        a.q_stride = a.o_stride = (C.c_int64 * 3)(heads * d, heads * d, d)
+        a.k_stride = a.v_stride = (C.c_int64 * 3)(16 * kv_heads * d, kv_heads * d, d)
+        bs = (_lib.FwdBucket * len(buckets))()
+        for b, (tile, boxes, seqs, tokens, flags, items) in zip(bs, buckets):
+            b.q_table = b.block_table = b.num_seqs = b.rank = b.kv = 0x10000
+            b.mnw[0], b.mnw[1], b.mnw[2] = tile, 64, 4
+            b.num_boxes, b.max_seqs, b.max_blocks, b.flags, b.num_items = boxes, seqs, tokens // 16, flags, items
+            b.q_table_stride, b.block_table_stride = seqs, tokens // 16
+        a.num_buckets, a.buckets, a.max_blocks_in_box = len(bs), C.cast(bs, C.POINTER(_lib.FwdBucket)), 400
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        return g.tall_rows, bool(g.flags & _lib.PAT_GEOMETRY_PAIRS), g.num_slots
+
+    both = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS
+    assert form_of([(64, 97, 8, 400, both, 49), (16, 1, 1, 448, 1, 0), (16, 108, 1, 80, 1, 0), (16, 387, 1, 64, 0, 0),
+                    (16, 281, 1, 32, 0, 0)], 16, 2, 128, 777)[:2] == (16, False)
+    assert form_of([(64, 25, 8, 512, both, 13), (16, 198, 1, 32, 1, 0)], 64, 8, 128, 198)[:2] == (32, True)
+    assert form_of([(64, 12, 16, 3968, 0, 0), (32, 1, 6, 3968, 0, 0), (16, 102, 1, 1776, 0, 0)], 32, 8, 64, 102)[:2] == (32, False)
