@@ -258,18 +258,35 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     // third of the resident slots, the short boxes' chunk is sized for the slots that are left
     // (at least one per CU) instead of for two per CU: short workgroups that have to queue behind
     // the tall ones start late and make the tail.
-    // (up to 1024 tokens: beyond, one workgroup's walk of a long box is the tail. us per call, up to 2048 / up to 1024:
-    // 32 x (16384 + 256..2048) at 64/8 heads, boxes not in twos, 82.6 / 72.0; seven other batches within 1 %)
-    int64_t n_tall = 0;
+    // Up to 1024 tokens, and for the slots that boxes served in twos leave: beyond, one workgroup's walk of a long box is the
+    // tail (us per call, up to 2048 / up to 1024: 32 x (16384 + 256..2048) at 64/8 heads, boxes not in twos, 82.6 / 72.0;
+    // seven other batches within 1 %). But only where that does not cut some box into more pieces than any box is cut into
+    // anyway: every row of the launch has a slot per piece, so one long box - the few requests that a node's tall boxes leave
+    // over - doubles the partial rows of all requests (666 requests over 1152 tokens at
+    // 64/8 heads, two of them left over: 1056-token pieces 74.2 us and 84 MiB of partial rows, whole 67.3 and 42; 777 over 1536
+    // 98.3 / 90.7; 489 over 2176 115.3 / 109.7).
+    int64_t n_tall = 0, n_tall_boxes = 0, tall_pieces = 1;
     for (int i = 0; i < a->num_buckets; ++i)
-      if (row_tiles(a->buckets[i].mnw[0]) > 1)
-        n_tall += items_of(a->buckets[i], pairs) *
-                  std::max<int64_t>(1, ceil_div64((int64_t)a->buckets[i].max_blocks * page, round_unit(tall))) * a->kv_heads;
-    if (n_tall > kNumCUs) {
-      const int64_t slots = std::max<int64_t>(kNumCUs, resident - n_tall);
-      const int64_t c = std::min<int64_t>(kMaxBesideTall, ceil_div64(ceil_div64(work, slots), 128) * 128);
-      chunk = std::max(chunk, c);
-    }
+      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0) {
+        const int64_t n = std::max<int64_t>(1, ceil_div64((int64_t)a->buckets[i].max_blocks * page, round_unit(tall)));
+        n_tall += items_of(a->buckets[i], pairs) * n * a->kv_heads;
+        n_tall_boxes += (int64_t)a->buckets[i].num_boxes * n * a->kv_heads;
+        tall_pieces = std::max(tall_pieces, n);
+      }
+    auto beside = [&](int64_t tall_wgs, int64_t most) {   // the chunk beside so many tall workgroups
+      if (tall_wgs <= kNumCUs) return chunk;
+      const int64_t slots = std::max<int64_t>(kNumCUs, resident - tall_wgs);
+      return std::max(chunk, std::min(most, ceil_div64(ceil_div64(work, slots), 128) * 128));
+    };
+    auto pieces_of = [&](int64_t c) {                     // pieces of the longest <= 16-row box
+      int64_t n = 1;
+      for (int i = 0; i < a->num_buckets; ++i)
+        if (row_tiles(a->buckets[i].mnw[0]) == 1 && a->buckets[i].num_boxes > 0)
+          n = std::max(n, ceil_div64((int64_t)a->buckets[i].max_blocks * page, std::min(round_unit(c), cap)));
+      return n;
+    };
+    const int64_t fine = beside(n_tall, kMaxBesideTall), coarse = beside(n_tall_boxes, kMaxChunk);
+    chunk = pieces_of(fine) <= std::max(tall_pieces, pieces_of(coarse)) ? fine : coarse;
   }
   // No sequence sits in two boxes (max_split_per_seq 1: a batch without shared prefixes, 27 boxes
   // or more): with one chunk per box every row has a single partial slot and the split kernel

@@ -315,3 +315,40 @@ def test_form_of_the_tall_path_follows_the_launch():
                     (16, 281, 1, 32, 0, 0)], 16, 2, 128, 777)[:2] == (16, False)
     assert form_of([(64, 25, 8, 512, both, 13), (16, 198, 1, 32, 1, 0)], 64, 8, 128, 198)[:2] == (32, True)
     assert form_of([(64, 12, 16, 3968, 0, 0), (32, 1, 6, 3968, 0, 0), (16, 102, 1, 1776, 0, 0)], 32, 8, 64, 102)[:2] == (32, False)
+
+
+def _bucket_args(buckets, heads, kv_heads, d, batch, page):
+    """Args of a launch of (tile, boxes, sequences, tokens, flags, items) buckets, fake addresses."""
+    a = _args(batch=batch, heads=heads, kv_heads=kv_heads, head_dim=d, page_size=page)
+    a.q_stride = a.o_stride = (C.c_int64 * 3)(heads * d, heads * d, d)
+    a.k_stride = a.v_stride = (C.c_int64 * 3)(page * kv_heads * d, kv_heads * d, d)
+    bs = (_lib.FwdBucket * len(buckets))()
+    for b, (tile, boxes, seqs, tokens, flags, items) in zip(bs, buckets):
+        b.q_table = b.block_table = b.num_seqs = b.rank = b.kv = 0x10000
+        b.mnw[0], b.mnw[1], b.mnw[2] = tile, 64, 4
+        b.num_boxes, b.max_seqs, b.max_blocks, b.flags, b.num_items = boxes, seqs, tokens // page, flags, items
+        b.q_table_stride, b.block_table_stride = seqs, tokens // page
+    a.num_buckets, a.buckets, a.max_blocks_in_box, a._keep = len(bs), C.cast(bs, C.POINTER(_lib.FwdBucket)), 400, bs
+    return a
+
+
+def test_one_long_short_box_does_not_multiply_every_rows_slots():
+    """The few requests that a node's tall boxes leave over keep the whole shared length in a box of <= 16 rows; how it is
+    cut sets the partial slots of all rows. Pairs and the 1024-token bound on its pieces cut such boxes finer only where
+    no row gets more slots for it."""
+    lib, g, need = _lib.load(), _lib.FwdGeometry(), C.c_size_t()
+    even, both = _lib.PAT_BUCKET_EVEN, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS
+    cases = [  # (args, slots of a row)
+        (_bucket_args([(64, 83, 8, 1152, both, 42), (16, 1, 2, 1152, even, 0), (16, 596, 1, 96, 0, 0), (16, 70, 1, 48, 0, 0)], 64, 8, 128, 666, 48), 2),
+        (_bucket_args([(64, 27, 16, 3888, both, 14), (16, 1, 1, 3984, even, 0), (16, 32, 1, 96, 0, 0), (16, 269, 1, 96, 0, 0),
+                       (16, 131, 1, 48, 0, 0)], 32, 8, 128, 433, 48), 6),
+        (_bucket_args([(64, 6, 64, 6880, both, 3), (16, 1, 6, 6880, even, 0), (16, 390, 1, 32, 0, 0)], 16, 16, 128, 390, 16), 12),
+        (_bucket_args([(64, 61, 8, 2176, even, 0), (16, 1, 1, 2304, even, 0), (16, 488, 1, 128, even, 0)], 64, 8, 128, 489, 16), 4),
+    ]
+    for a, slots in cases:
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        assert g.num_slots == slots
+        assert lib.pat_fwd_workspace_bytes(C.byref(a), C.byref(need)) == 0 and need.value <= lib.pat_fwd_static_scratch_bytes()
+    # pieces of 1024 tokens where the tall boxes have as many anyway
+    a = _bucket_args([(64, 24, 8, 2736, even, 0), (16, 32, 1, 2048, 0, 0)], 64, 8, 128, 32, 16)
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0 and (g.chunk_tokens, g.chunks_per_rank) == (1024, 2)
