@@ -894,7 +894,20 @@ int pat_fwd_launch_static(const pat_fwd_args* args, void* hip_stream) {
   if (int rc = check_args(args)) return rc;
   Geometry g;
   if (int rc = plan_geometry(args, &g)) return rc;
-  const size_t need = workspace_need(args, g);
+  size_t need = workspace_need(args, g);
+  // The records of boxes served in twos are longer: a launch that only fits box by box is made box by box.
+  pat_fwd_args box_by_box;
+  pat_fwd_tuning tune;
+  if (need > kStaticScratchBytes && g.pairs && args->records == nullptr) {
+    box_by_box = *args;
+    tune = args->tuning != nullptr ? *args->tuning : tuning();
+    tune.pairs = 2;
+    box_by_box.tuning = &tune;
+    args = &box_by_box;
+    g = Geometry();
+    if (int rc = plan_geometry(args, &g)) return rc;
+    need = workspace_need(args, g);
+  }
   if (need > kStaticScratchBytes)
     return fail(PAT_ERR_WORKSPACE, "pat_fwd_launch_static: this launch needs " + std::to_string(need) +
                                        " bytes of partial results, the built-in scratch holds " +

@@ -5,6 +5,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from pat_amd import _lib
 
@@ -352,3 +353,12 @@ def test_one_long_short_box_does_not_multiply_every_rows_slots():
     # pieces of 1024 tokens where the tall boxes have as many anyway
     a = _bucket_args([(64, 24, 8, 2736, even, 0), (16, 32, 1, 2048, 0, 0)], 64, 8, 128, 32, 16)
     assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0 and (g.chunk_tokens, g.chunks_per_rank) == (1024, 2)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on fake addresses")
+def test_static_launch_that_only_fits_box_by_box_is_not_refused():
+    # records of items hold twice the sequences: 65.8 MiB with the boxes in twos, 64.0 one by one
+    lib, need = _lib.load(), C.c_size_t()
+    a = _bucket_args([(64, 8, 64, 7744, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS, 4), (16, 482, 1, 64, 0, 0)], 32, 32, 128, 482, 64)
+    assert lib.pat_fwd_workspace_bytes(C.byref(a), C.byref(need)) == 0 and need.value > lib.pat_fwd_static_scratch_bytes()
+    assert lib.pat_fwd_launch_static(C.byref(a), None) == _lib.PAT_ERR_HIP      # (got past the check: there is no GPU here)
