@@ -28,6 +28,7 @@ constexpr int kTargetWgsPerCU = 2;  // what fits at once: 2 workgroups of 4 wave
 constexpr int kMinChunk = 128;      // tokens
 constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
+constexpr int64_t kMostPartialBytes = (int64_t)48 << 20;   // partial rows up to which tall boxes are cut (kStaticScratchBytes less room for records)
 constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
 constexpr int kMaxBesideTall = 1024;         // tokens of a short boxes' chunk sized for the slots that tall workgroups leave
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
@@ -182,6 +183,7 @@ int check_args(const pat_fwd_args* a) {
 // 1.7 us alone, ~3 us beside two others on the CU.
 struct LaunchEstimate { double short_us = 0., short_rounds = 0., tall_us = 0., chain_us = 0.; };
 constexpr double kShortestLaunchUs = 5.5;
+constexpr double kTallEndsUs = 1.;   // a tall workgroup's record, Q and first tile, and its stores
 LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs) {
   LaunchEstimate e;
   for (int i = 0; i < a->num_buckets; ++i) {
@@ -208,9 +210,9 @@ LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs)
 //  * boxes of <= 16 rows split the chunk's 32-token steps over the 4 waves: the chunk is sized
 //    so that this work fills the device with about kTargetWgsPerCU workgroups per CU - few
 //    enough that all are resident at once, so every CU has loads in flight from start to end;
-//  * boxes of 17..64 rows walk the chunk step by step with all 4 waves (one row tile each) and
-//    write 16..32 KB of partial output per workgroup: their chunk is at least 256 tokens, and
-//    longer when they alone would still fill the device.
+//  * boxes of 17..64 rows, or two boxes of a node together, walk the chunk super-step by super-step with all 4 waves and
+//    write 16..64 KB of partial output per workgroup: their chunk is at least 256 tokens, and as much longer as the
+//    estimated time of the launch allows (see below).
 // pat_fwd_tuning.chunk_tokens / tall_chunk_tokens override the two sizes (tuning aid).
 // (tall_rows: the form of the tall path the geometry is made for, 16 or 32; pairs: items of two boxes as one workgroup)
 int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pairs) {
@@ -236,20 +238,39 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     chunk = ceil_div64(work / (kTargetWgsPerCU * kNumCUs), 128) * 128;
     chunk = std::max<int64_t>(kMinChunk, std::min<int64_t>(kMaxChunk, chunk));
   }
-  if (tall <= 0) {
-    // Tall boxes are cut only as far as it takes for a tall workgroup's chain of 64-token super-steps not to
-    // outlast the launch: the estimated time of the whole launch (and never less than kShortestLaunchUs: that
-    // much is launch, prologue and tail whatever the work), over the chain of an uncut box. Beyond that every further
-    // piece only adds 16-32 KB of partial rows and a merge slot per row. Measured (us per call by piece): a
-    // 2048-token prefix of 64 requests, 8 kv heads: 512 tokens 25.2, 768 22.2, 1536 25.5; 16 boxes of 1408 tokens:
-    // 512 35.4, 768-1024 32.4, uncut 36; 8 boxes of 1536 tokens, 8 kv heads, 16-row form: 768 71.7, uncut 75.5; 24 rows over 784 tokens, 32 kv heads: 512 18.4, uncut 19.2; 17 boxes of
-    // 864-1728 tokens, 2 kv heads: 256 18.1, 384 18.4, 768 19.5, uncut 23.4; one box of 288 tokens, 8 kv heads: 256 12.5, uncut 13.8.
-    int64_t widest_tall = 0;
+  auto pieces_of = [&](int64_t c) {   // pieces of the longest <= 16-row box
+    int64_t n = 1;
     for (int i = 0; i < a->num_buckets; ++i)
-      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0)
+      if (row_tiles(a->buckets[i].mnw[0]) == 1 && a->buckets[i].num_boxes > 0)
+        n = std::max(n, ceil_div64((int64_t)a->buckets[i].max_blocks * page, std::min(round_unit(c), cap)));
+    return n;
+  };
+  if (tall <= 0) {
+    // Tall boxes are cut only as far as it takes for a tall workgroup not to outlast the launch: what the workgroup spends on
+    // an uncut box, the chain of its 64-token super-steps and kTallEndsUs ahead of the first and after the last of them, over
+    // the estimated time of the whole launch (never less than kShortestLaunchUs: that much is launch, prologue and tail
+    // whatever the work). Beyond that every further piece only adds 16-64 KB of partial rows and a merge slot per row.
+    // Measured on 155 batches, every cut of both forms (us per call by piece): without the ends 3.0 % behind the best cut and
+    // form on average, with them 2.5 % (24 requests over 352 tokens, three nodes of 992, 8 kv heads: uncut 15.4, 256 tokens
+    // 14.0; 425 over 1440 at 64/8 heads, head_dim 64: uncut 39.2, 768 30.1; 2048-token prefix of 64 requests, 8 kv heads:
+    // 512 25.2, 768 22.2, 1536 25.5; 24 rows over 784 tokens, 32 kv heads: 512 18.4, uncut 19.2).
+    int64_t widest_tall = 0, tall_box_heads = 0;
+    for (int i = 0; i < a->num_buckets; ++i)
+      if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0) {
         widest_tall = std::max<int64_t>(widest_tall, (int64_t)a->buckets[i].max_blocks * page);
+        tall_box_heads += (int64_t)a->buckets[i].num_boxes * a->kv_heads;
+      }
     const LaunchEstimate est = estimate_launch(a, tall_rows, pairs);
-    const int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil(est.chain_us / std::max(est.tall_us + est.short_us, kShortestLaunchUs)));
+    int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil((est.chain_us + kTallEndsUs) / std::max(est.tall_us + est.short_us, kShortestLaunchUs)));
+    // (not past the slots up to which the merge of few rows gives each a workgroup, where the <= 16-row boxes leave it those: 10
+    // requests over 4944 tokens in 17 boxes each, 336-token tall boxes in one piece 12.0, in two 13.7)
+    if ((int64_t)a->batch * a->heads * kMergeWideSlots <= kMergeWideMost && pieces_of(chunk) * a->max_split_per_seq <= kMergeWideSlots)
+      pieces = std::min(pieces, std::max<int64_t>(1, kMergeWideSlots / a->max_split_per_seq));
+    // (and not past kMostPartialBytes of partial rows, which deep trees of many boxes per request would reach, but for what it
+    // takes to have a tall workgroup on three of eight CUs, in the 16-row form on half of them)
+    const int64_t slot_bytes = (int64_t)a->batch * a->heads * a->max_split_per_seq * (a->head_dim + 1) * (int64_t)sizeof(float);
+    const int64_t spread = tall_box_heads > 0 ? ceil_div64(tall_rows == 32 ? 3 * kNumCUs / 8 : kNumCUs / 2, tall_box_heads) : 1;
+    pieces = std::min(pieces, std::max<int64_t>(spread, kMostPartialBytes / slot_bytes));
     tall = ceil_div64(ceil_div64(widest_tall, pieces), 128) * 128;
     tall = std::max<int64_t>(kTallChunk, std::min<int64_t>(kMaxChunk, tall));
   }
@@ -262,9 +283,8 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     // tail (us per call, up to 2048 / up to 1024: 32 x (16384 + 256..2048) at 64/8 heads, boxes not in twos, 82.6 / 72.0;
     // seven other batches within 1 %). But only where that does not cut some box into more pieces than any box is cut into
     // anyway: every row of the launch has a slot per piece, so one long box - the few requests that a node's tall boxes leave
-    // over - doubles the partial rows of all requests (666 requests over 1152 tokens at
-    // 64/8 heads, two of them left over: 1056-token pieces 74.2 us and 84 MiB of partial rows, whole 67.3 and 42; 777 over 1536
-    // 98.3 / 90.7; 489 over 2176 115.3 / 109.7).
+    // over - doubles the partial rows of all requests (666 requests over 1152 tokens at 64/8 heads, two of them left over: 1056-token
+    // pieces 74.2 us and 84 MiB of partial rows, whole 67.3 and 42; 777 over 1536 98.3 / 90.7; 489 over 2176 115.3 / 109.7).
     int64_t n_tall = 0, n_tall_boxes = 0, tall_pieces = 1;
     for (int i = 0; i < a->num_buckets; ++i)
       if (row_tiles(a->buckets[i].mnw[0]) > 1 && a->buckets[i].num_boxes > 0) {
@@ -277,13 +297,6 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
       if (tall_wgs <= kNumCUs) return chunk;
       const int64_t slots = std::max<int64_t>(kNumCUs, resident - tall_wgs);
       return std::max(chunk, std::min(most, ceil_div64(ceil_div64(work, slots), 128) * 128));
-    };
-    auto pieces_of = [&](int64_t c) {                     // pieces of the longest <= 16-row box
-      int64_t n = 1;
-      for (int i = 0; i < a->num_buckets; ++i)
-        if (row_tiles(a->buckets[i].mnw[0]) == 1 && a->buckets[i].num_boxes > 0)
-          n = std::max(n, ceil_div64((int64_t)a->buckets[i].max_blocks * page, std::min(round_unit(c), cap)));
-      return n;
     };
     const int64_t fine = beside(n_tall, kMaxBesideTall), coarse = beside(n_tall_boxes, kMaxChunk);
     chunk = pieces_of(fine) <= std::max(tall_pieces, pieces_of(coarse)) ? fine : coarse;

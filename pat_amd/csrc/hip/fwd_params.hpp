@@ -11,6 +11,11 @@ constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop itera
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
 constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
+// Launches of 9..32 slots per row where a workgroup takes a row: up to so many slots over all rows. It requests every slot,
+// empty ones too, which has to cost less than the two round trips it saves (us per merge, general / workgroup per row: 32 rows
+// x 27 slots 5.7 / 2.5, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
+constexpr int kMergeWideSlots = 32;
+constexpr int64_t kMergeWideMost = 32768;
 
 // One workgroup's work: a launch record, written once per plan by the record kernel
 // (capi_fwd.hip) and read by the split kernel in a single round trip. In memory:

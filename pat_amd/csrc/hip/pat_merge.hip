@@ -26,11 +26,6 @@ namespace pat {
 #ifndef PAT_MERGE_PAIRS_MIN
 #define PAT_MERGE_PAIRS_MIN 16384   // rows from which a half-wave takes a row (launches of up to 8 slots per row)
 #endif
-// Launches of 9..32 slots per row where a workgroup takes a row: up to so many slots over all rows. It requests every slot,
-// empty ones too, which has to cost less than the two round trips it saves (us per merge, general / workgroup per row: 32 rows
-// x 27 slots 5.7 / 2.5, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
-constexpr int kMergeWideSlots = 32;
-constexpr int64_t kMergeWideMost = 32768;
 
 // u / d with m = ceil(2^32 / d) (0 for d = 1), any 32-bit u: the product is the quotient or one more.
 __device__ __forceinline__ unsigned divide(unsigned u, unsigned d, unsigned m) {

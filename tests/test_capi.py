@@ -355,6 +355,28 @@ def test_one_long_short_box_does_not_multiply_every_rows_slots():
     assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0 and (g.chunk_tokens, g.chunks_per_rank) == (1024, 2)
 
 
+def test_tall_boxes_are_cut_by_what_a_workgroup_takes_ends_included():
+    lib, g, need = _lib.load(), _lib.FwdGeometry(), C.c_size_t()
+    even, both = _lib.PAT_BUCKET_EVEN, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS
+
+    def plan(max_split, *args):
+        a = _bucket_args(*args)
+        a.max_split_per_seq = max_split
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        assert lib.pat_fwd_workspace_bytes(C.byref(a), C.byref(need)) == 0
+        return g
+
+    # in two: the chain of 352 tokens alone is shorter than the launch, with the workgroup's ends it is not
+    assert plan(3, [(64, 1, 24, 352, even, 0), (16, 3, 8, 992, even, 0), (16, 24, 8, 512, 0, 0)], 16, 8, 128, 24, 16).tall_chunk_tokens == 256
+    assert plan(2, [(64, 53, 8, 1440, both, 27), (16, 1, 1, 1472, even, 0), (16, 424, 1, 32, even, 0)], 64, 8, 64, 425, 32).tall_chunk_tokens == 768
+    # not in two: 34 slots a row are past what the merge gives a workgroup per row for
+    assert plan(17, [(32, 16, 10, 336, even, 0), (16, 10, 8, 48, 0, 0)], 16, 8, 128, 10, 48).num_slots == 17
+    # a forest of nine boxes per request: fewer pieces than its chains call for, so that the partial rows stay in bounds
+    plan(9, [(64, 2, 7, 3216, 0, 0), (64, 9, 7, 816, 0, 0), (32, 6, 4, 480, 0, 0), (16, 13, 2, 512, 0, 0), (16, 43, 2, 384, 0, 0),
+             (16, 24, 2, 128, 0, 0)], 64, 8, 128, 66, 16)
+    assert g.num_slots == 18 and need.value <= 48 << 20
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on fake addresses")
 def test_static_launch_that_only_fits_box_by_box_is_not_refused():
     # records of items hold twice the sequences: 65.8 MiB with the boxes in twos, 64.0 one by one
