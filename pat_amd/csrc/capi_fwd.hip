@@ -92,7 +92,7 @@ struct Geometry {
   int64_t total_wgs = 0;
   int tall_rows = 32;        // rows per wave on boxes of 17..64 rows: 32 or 16 (the split kernel's instance)
   bool tall_apart = false;   // 32-row form: K and V tiles handed over apart
-  bool pairs = false;        // the two boxes of an item (pat_fwd_bucket.items) are served by one workgroup
+  bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
   // launch records (one per workgroup): entries per record and bytes between records
   int record_max_seqs = 0, record_max_pages = 0, record_stride = 0;
@@ -183,6 +183,7 @@ int check_args(const pat_fwd_args* a) {
 // 1.7 us alone, ~3 us beside two others on the CU.
 struct LaunchEstimate { double short_us = 0., short_rounds = 0., tall_us = 0., chain_us = 0.; };
 constexpr double kShortestLaunchUs = 5.5;
+constexpr double kMergeWideUs = 3.;  // the workgroup-per-row merge against the general one (2.1 us at 32 rows x 32 slots), and the cut's own slots
 constexpr double kTallEndsUs = 1.;   // a tall workgroup's record, Q and first tile, and its stores
 LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs) {
   LaunchEstimate e;
@@ -261,11 +262,15 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
         tall_box_heads += (int64_t)a->buckets[i].num_boxes * a->kv_heads;
       }
     const LaunchEstimate est = estimate_launch(a, tall_rows, pairs);
-    int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil((est.chain_us + kTallEndsUs) / std::max(est.tall_us + est.short_us, kShortestLaunchUs)));
-    // (not past the slots up to which the merge of few rows gives each a workgroup, where the <= 16-row boxes leave it those: 10
-    // requests over 4944 tokens in 17 boxes each, 336-token tall boxes in one piece 12.0, in two 13.7)
-    if ((int64_t)a->batch * a->heads * kMergeWideSlots <= kMergeWideMost && pieces_of(chunk) * a->max_split_per_seq <= kMergeWideSlots)
-      pieces = std::min(pieces, std::max<int64_t>(1, kMergeWideSlots / a->max_split_per_seq));
+    const double launch_us = std::max(est.tall_us + est.short_us, kShortestLaunchUs);
+    int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil((est.chain_us + kTallEndsUs) / launch_us));
+    // (not past the slots up to which the merge of few rows gives each a workgroup, where the <= 16-row boxes leave it those and
+    // the longer pieces cost less than the kMergeWideUs that this form saves: 10 requests over 4944 tokens in 17 boxes each,
+    // 336-token tall boxes in one piece 12.0 us, in two 13.7, but 33 over 8096 in three boxes each, 384 tokens 12.7, 896 16.1)
+    if ((int64_t)a->batch * a->heads * kMergeWideSlots <= kMergeWideMost && pieces_of(chunk) * a->max_split_per_seq <= kMergeWideSlots) {
+      const int64_t most = std::max<int64_t>(1, kMergeWideSlots / a->max_split_per_seq);
+      if (est.chain_us / (double)most + kTallEndsUs <= launch_us + kMergeWideUs) pieces = std::min(pieces, most);
+    }
     // (and not past kMostPartialBytes of partial rows, which deep trees of many boxes per request would reach, but for what it
     // takes to have a tall workgroup on three of eight CUs, in the 16-row form on half of them)
     const int64_t slot_bytes = (int64_t)a->batch * a->heads * a->max_split_per_seq * (a->head_dim + 1) * (int64_t)sizeof(float);
@@ -477,7 +482,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 //    boxes not in twos: 52.5 / 57.3). More than 3 % behind: 54, nearly all left to the 16-row form.
 //  * at head_dim 64 (88) the 32-row form costs no place: from 640 tokens, 0.3 of the streaming time and 2 us a round
 //    (102 x (4848 + 580..1160) at 32/8 heads, six nodes: 69.6 / 62.3). More than 3 % behind: 7; the lines above: 11.
-// Two boxes of a node are served by one workgroup (32-row form, pat_fwd_bucket items) where the tall boxes fill the
+// Two boxes of a node are served by one workgroup (32-row form, PAT_BUCKET_ITEMS) where the tall boxes fill the
 // device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
 // part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
 // boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice

@@ -371,6 +371,8 @@ def test_tall_boxes_are_cut_by_what_a_workgroup_takes_ends_included():
     assert plan(2, [(64, 53, 8, 1440, both, 27), (16, 1, 1, 1472, even, 0), (16, 424, 1, 32, even, 0)], 64, 8, 64, 425, 32).tall_chunk_tokens == 768
     # not in two: 34 slots a row are past what the merge gives a workgroup per row for
     assert plan(17, [(32, 16, 10, 336, even, 0), (16, 10, 8, 48, 0, 0)], 16, 8, 128, 10, 48).num_slots == 17
+    # ... but in 384-token pieces where those of 32 slots would be more than twice as long
+    assert plan(3, [(64, 1, 33, 8096, even, 0), (32, 1, 17, 864, even, 0), (16, 1, 16, 864, even, 0), (16, 33, 1, 32, 0, 0)], 8, 8, 64, 33, 32).tall_chunk_tokens == 384
     # a forest of nine boxes per request: fewer pieces than its chains call for, so that the partial rows stay in bounds
     plan(9, [(64, 2, 7, 3216, 0, 0), (64, 9, 7, 816, 0, 0), (32, 6, 4, 480, 0, 0), (16, 13, 2, 512, 0, 0), (16, 43, 2, 384, 0, 0),
              (16, 24, 2, 128, 0, 0)], 64, 8, 128, 66, 16)
