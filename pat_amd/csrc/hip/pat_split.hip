@@ -76,12 +76,6 @@ template <> struct Elem<__bf16> {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float neg_inf() { return -__builtin_inff(); }
 
-// Tuning knob: steps a wave keeps in flight on wave-private tiles (measured on MI355X: deeper rings
-// lose more to registers and to late-arriving first tiles than they gain).
-#ifndef PAT_DEPTH
-#define PAT_DEPTH 1
-#endif
-
 // Two forms of the tall path (boxes of 17..64 rows), one kernel instance each:
 //  TALLK 32: 32-row tiles on 32x32x16 MFMAs, 64-token super-steps; the faster walk of a tall box
 //            (a lone workgroup: 1.1-1.3 us per 64 tokens of one box, ~1.5 of two), at the price of 64
@@ -119,7 +113,6 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   constexpr int KK = D / 32;             // MFMA k-steps across head_dim in S^T = K.Q^T (16x16x32 tiles)
   constexpr int DB = D / 16;             // 16-wide head_dim blocks of O^T (16x16x32 tiles)
   constexpr int NV = D / 16;             // 16-byte V loads per lane per step (wave-private tiles)
-  constexpr int DEPTH = PAT_DEPTH;       // wave-private tiles: steps kept in flight per wave
   constexpr int CPR = D / 8;             // 16-byte pieces per token row
   constexpr int TPL = 64 / CPR;          // tokens covered by one wave-wide load instruction
   constexpr int RSV = D * 2 + 32;        // LDS row stride of a wave-private V tile (conflict-free transposed reads)
@@ -462,11 +455,11 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     // two LDS stages (global_load_lds, 16 bytes per lane): the next super-step is in flight while the waves work
     // on the current one, and no register holds a tile on its way. Wave w fetches the 16-token half w of every
     // super-step: one page id, one address.
-    // What bounds it: two of these workgroups on a CU take ~2 us per super-step of two boxes, i.e. ~1050 TFLOP/s in the
-    // steady state (65536 rows x 16384 tokens, 8 kv heads; a library matrix product reaches 1200): MFMA 37 %, VALU 32 %,
-    // LDS 37 % busy, the rest is the chain score - softmax - weighted sum of each wave. With the tiles staged through
-    // registers and one box per workgroup (four workgroups reading what one does now) 65536 rows x 2048 tokens took
-    // 105 us, now ~80.
+    // What bounds it: the chain score - softmax - weighted sum of each wave. Two of these workgroups on a CU take ~2 us per
+    // super-step of two boxes, ~1050 TFLOP/s in the steady state (65536 rows x 16384 tokens, 8 kv heads; a library matrix
+    // product reaches 1200); over 65536 rows x 2048 tokens, prologue, stores and short boxes included, the MFMA pipe is
+    // busy 29 % of the launch and LDS 16 %. With the tiles staged through registers and one box per workgroup (four workgroups
+    // reading what one does now) that launch took 156 us, now 117.
     //  * more than 64 rows (two boxes of one node): wave w owns row tile w (rows 32w..) and all 64 tokens;
     //  * up to 64 rows: the wave pair ph = w >> 1 takes tokens 32ph.. of every super-step, wave w row tile
     //    w & 1; the pairs' states are combined through LDS at the end.
@@ -774,10 +767,8 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     }   // TALLK
   } else {
     // ====================== short box: KV steps split over the 4 waves ========================
-    // Each wave keeps DEPTH of its steps in flight in a ring of register buffers: when a step has
-    // been consumed its buffer is refilled with the step DEPTH rounds ahead. The chunk is short
-    // (a few steps per wave), so most of a workgroup's bytes are requested before the first
-    // arrives: the kernel's run time is then set by bandwidth, not by a chain of round trips.
+    // Each wave holds one step's K and V in registers and refills either as soon as it has been consumed: V when it has gone to
+    // LDS, K behind the score MFMAs. (Two steps in registers, 243 VGPRs: no faster where the memory system is full.)
     load_q();
     // K rows go straight into MFMA operand layout (16 rows x 64 bytes per load instruction); V rows
     // are fetched TPL whole rows per instruction and staged in this wave's LDS region. (Staging K
@@ -785,7 +776,6 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     PAT_LDS char* vstage = (PAT_LDS char*)smem + wave * WSTAGE;
     const unsigned koff = (unsigned)(n * kss) + g * 16;                          // K: row n of a half, dims g*8..
     const unsigned voff = (unsigned)((lane / CPR) * vss) + (lane % CPR) * 16;    // V: TPL rows per instruction
-    u32x4 kring[DEPTH][2][KK], vring[DEPTH][NV];
     auto fetch_v = [&](int st, u32x4 (&vd)[NV]) {
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -815,29 +805,38 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     // steps of this wave: every kWaves-th one of the chunk, or, with a kv head per wave, all of them
     const int step0 = head_per_wave ? 0 : wave;
     const int stride = head_per_wave ? 1 : kWaves;
+    if (step0 < nsteps) {
+      u32x4 kd[2][KK], vd[NV];
+      fetch_v(step0, vd);
+      fetch_k(step0, kd);
+      // Q is here before the loop starts, and the last step, which requests nothing, stands apart from it: every wait inside
+      // then counts exactly the loads behind the one it is for. In one loop with Q on its way and requests that may not be made,
+      // the score MFMAs of every step waited for the V tile requested just ahead of them (fp16, 8 kv heads: 123 requests over
+      // 240 + 224 tokens 17.0 us, now 15.6; head_dim 64, 48 over 768 11.7 / 10.2; 32 x 4096 at 64/8 heads 96.0 / 94.6).
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d)
-      if (step0 + d * stride < nsteps) {
-        fetch_v(step0 + d * stride, vring[d]);
-        fetch_k(step0 + d * stride, kring[d]);
-      }
-    for (int st0 = step0; st0 < nsteps; st0 += DEPTH * stride) {
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        const int st = st0 + d * stride;
-        if (st >= nsteps) break;
-        const int nxt = st + DEPTH * stride;
-        const bool more = nxt < nsteps;
-        // V tile -> this wave's LDS region, row-major with padded rows; its registers are free
-        // again at once and take the ring's next V tile
+      for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qreg[kk]));
+      auto step = [&](int st, auto more_c) {
+        constexpr bool more = decltype(more_c)::value;
+        // V tile -> this wave's LDS region, row-major with padded rows; its registers are free again at once and take the
+        // next V tile
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-          *(PAT_LDS u32x4*)(vstage + (j * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vring[d][j];
-        if (more) fetch_v(nxt, vring[d]);
+          *(PAT_LDS u32x4*)(vstage + (j * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vd[j];
+        if (more) fetch_v(st + stride, vd);
+        // Few tall workgroups with long chains (p.tall_apart): the launch ends on those, and these waves' requests, of two
+        // steps at once, hold theirs up (us per call without / with this wait: 64 requests over 2048 tokens, 32/8 heads, 22.8 /
+        // 22.0, 32 over 16384 at 64/8 57.6 / 56.3). Of 125 launches of this form measured both ways the 35 such are 1.4 %
+        // slower without it, the other 90 1.6 % faster, 37 x (848 + 239..478) at 32/8 heads 19 %.
+        if constexpr (more && TALLK == 32) {
+          if (p.tall_apart) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         // the K registers are refilled as soon as the score MFMAs have read them
-        attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kring[d][a][kk]); }, vstage,
-               t_begin + st * kStepTokens, [&]() { if (more) fetch_k(nxt, kring[d]); });
-      }
+        attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kd[a][kk]); }, vstage,
+               t_begin + st * kStepTokens, [&]() { if (more) fetch_k(st + stride, kd); });
+      };
+      int st = step0;
+      for (; st + stride < nsteps; st += stride) step(st, std::true_type{});
+      step(st, std::false_type{});
     }
     l_run = sum_xor32(sum_xor16(l_run));
 

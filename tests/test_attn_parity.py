@@ -1274,6 +1274,36 @@ def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, pag
         _assert_close(f"pairs {pairs}", out, lse, ref_out, ref_lse, dtype)
 
 
+@pytest.mark.parametrize("head_per_wave", [0, 256])
+@pytest.mark.parametrize("chunk", [256, 512])
+@pytest.mark.parametrize("heads,d,dtype", [((32, 8), 128, torch.bfloat16), ((8, 8), 64, torch.float16)])
+def test_short_boxes_beside_tall_ones(heads, d, dtype, chunk, head_per_wave, tuning, monkeypatch):
+    # the <= 16-row path of the 32-row form: waves of no step, one, two and more, full and partial last steps; pieces of 256
+    # tokens of the tall boxes leave its next step's V tile in flight during the scores, pieces of 512 make it wait for that
+    print(f"[case] short boxes beside tall ones, heads {heads}, d {d}, pieces of {chunk}, head per wave {head_per_wave}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    tails = [1, 15, 31, 32, 33, 64, 65, 96, 127, 128, 129, 160, 161, 224, 255, 256] * 5
+    shared, rows, nxt = 40, [], 40
+    for n in tails:
+        rows.append(list(range(shared)) + list(range(nxt, nxt + -(-n // 16))))
+        nxt += -(-n // 16)
+    w = workloads.Workload("beside", heads[0], heads[1], d, dtype, 16, [shared * 16 + n for n in tails], rows, nxt, 0, 6)
+    q, k, v = w.tensors(dev)
+    tuning(tall_rows=32, tall_chunk_tokens=chunk, equalize_chunks=0, head_per_wave_tokens=head_per_wave)
+    tree = PrefixTreeCPP(16)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+    tree.kernel_info.to_gpu(dev)
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((w.batch, w.heads), float("nan"), dtype=torch.float32, device=dev)
+    prefix_attn_with_kvcache(q, k, v, tree, 1.0 / math.sqrt(d), out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    geo = tree.kernel_info._launch_geometries[0]
+    assert geo["tall_rows"] == 32 and geo["apart"] == (chunk == 512)
+    _assert_close(f"pieces of {chunk}", out, lse, *_oracle(w, q, k, v), dtype)
+
+
 @pytest.mark.parametrize("captured", [False, True])
 def test_edit_of_one_box_of_a_pair(captured, tuning):
     # two boxes of a node share a workgroup, which reads the first one's length and blocks: a write to the plan tables that
