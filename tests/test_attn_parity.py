@@ -273,23 +273,25 @@ def test_table_overload_with_even_hint(name):
     _assert_close(f"{name}/even hint", out, lse, ref_out, ref_lse, w.dtype)
 
 
-@pytest.mark.parametrize("case", ["combine", "head_per_wave", "tall_identical"])
+@pytest.mark.parametrize("case", ["combine", "head_per_wave", "tall_identical", "tall_pairs", "tall_pairs_64"])
 def test_single_slot_launch_writes_out_directly(case, tuning):
     # every row has one partial slot (no sequence in two boxes, no box in two chunks): the split
     # kernel stores `out` itself, needs no workspace and no merge kernel follows
-    # (csrc/api.h:230-238 does the same for max_split_per_seq == 1). All three epilogues. (Batches
+    # (csrc/api.h:230-238 does the same for max_split_per_seq == 1). All epilogues. (Batches
     # of 27 boxes or more: below that the balancer halves boxes and every row has two slots.)
     print(f"[case] direct output, {case}", flush=True)
-    from pat_amd import _ctypes_launch
+    import ctypes as C
+    from pat_amd import _ctypes_launch, _lib
     dev = _device()
     if case == "combine":          # few boxes of a few steps: 4 waves share a box, states combined in LDS
         w = workloads.independent("direct-a", 32, 300, 32, 8, 128, torch.bfloat16, 5)
     elif case == "head_per_wave":  # many one-step boxes: a kv head per wave
         w = workloads.independent("direct-b", 256, 100, 16, 8, 64, torch.float16, 6)
-    else:                          # 32 groups of 8 requests with the same pages: boxes of 32 rows
-        base = workloads.independent("direct-c", 32, 200, 32, 8, 128, torch.float16, 7)
-        w = workloads.Workload("direct-c", 32, 8, 128, torch.float16, base.page_size, [200] * 256,
-                               [list(base.rows[i // 8]) for i in range(256)], base.num_blocks, 32 * 200, 7)
+    else:                          # groups of requests with the same pages: boxes of 32 rows, or two boxes of 64 a workgroup
+        groups, each, d = {"tall_identical": (32, 8, 128), "tall_pairs": (16, 32, 128), "tall_pairs_64": (16, 32, 64)}[case]
+        base = workloads.independent("direct-c", groups, 200, 32, 8, d, torch.float16, 7)
+        w = workloads.Workload("direct-c", 32, 8, d, torch.float16, base.page_size, [200] * (groups * each),
+                               [list(base.rows[i // each]) for i in range(groups * each)], base.num_blocks, groups * 200, 7)
     q, k, v = w.tensors(dev)
     tree = PrefixTreeCPP(w.page_size)
     tree.build_radix_tree(w.seq_lens, w.padded_table())
@@ -299,15 +301,18 @@ def test_single_slot_launch_writes_out_directly(case, tuning):
     assert info.max_split_per_seq == 1
     lt = info.launch_tables()
 
-    def run(direct):
-        tuning(direct_out=1 if direct else 0)
+    def run(direct, pairs=0):
+        tuning(direct_out=1 if direct else 0, pairs=pairs)
         out = torch.full_like(q, float("nan"))
         lse = torch.full((w.batch, w.heads), float("nan"), dtype=torch.float32, device=dev)
         L = _ctypes_launch.prepare(q, k, v, info.num_split_per_seq, lt["q_tables"], lt["block_tables"],
                                   lt["num_seqs_per_CTAs"], lt["CTA_ranks"], lt["kv_in_CTAs"], lt["MNWs"],
                                   info.max_split_per_seq, info.max_seqs_in_CTA, info.max_blocks_in_CTA,
-                                  1.0 / math.sqrt(w.head_dim), out, lse, lt.get("slot_tables"), lt.get("flags"))
+                                  1.0 / math.sqrt(w.head_dim), out, lse, lt.get("slot_tables"), lt.get("flags"), items=lt.get("items"))
         assert (L.need == 0) == direct, f"direct {direct}: workspace {L.need} bytes"
+        geo = _lib.FwdGeometry()
+        assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(geo)) == 0
+        assert bool(geo.flags & _lib.PAT_GEOMETRY_PAIRS) == (case.startswith("tall_pairs") and pairs != 2)
         _ctypes_launch.run(L, dev)
         torch.cuda.synchronize()
         return out, lse
@@ -318,6 +323,9 @@ def test_single_slot_launch_writes_out_directly(case, tuning):
     _assert_close(f"direct/{case}", out_d, lse_d, ref_out, ref_lse, w.dtype)
     assert torch.equal(out_d, out_m), "direct store and merge kernel must agree bit for bit"
     assert torch.equal(lse_d, lse_m)
+    if case.startswith("tall_pairs"):
+        out_1, lse_1 = run(True, pairs=2)
+        _assert_close(f"direct/{case}, box by box", out_1, lse_1, ref_out, ref_lse, w.dtype)
 
 
 @pytest.mark.parametrize("pad", [8, 2])
@@ -635,7 +643,7 @@ def test_both_forms_of_the_tall_path(name, tall_rows, tuning):
     L = _ctypes_launch.prepare(q, k, v, info.num_boxes_per_seq, lt["q_tables"], lt["block_tables"], lt["num_seqs_per_CTAs"],
                                lt["CTA_ranks"], lt["kv_in_CTAs"], lt["MNWs"], info.max_boxes_per_seq, info.max_seqs_in_CTA,
                                info.max_blocks_in_CTA, 1.0 / math.sqrt(w.head_dim), torch.empty_like(q), None,
-                               lt["slot_tables"], lt.get("flags"))
+                               lt["slot_tables"], lt.get("flags"), items=lt.get("items"))
     geo = _lib.FwdGeometry()
     assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(geo)) == 0 and geo.tall_rows == tall_rows
     assert any(m[0] > 16 for m in info.MNWs), "the case has no tall box"
@@ -1237,10 +1245,14 @@ def test_little_sharing_is_launched_as_whole_sequences(spec, heads, kernels):
 @pytest.mark.parametrize("seqs,prefix,heads,d,dtype,page,chunk,scale", [
     (32, 16, (32, 8), 128, torch.float16, 16, 0, 0.09),      # one pair of full boxes, a piece of a quarter super-step
     (40, 48, (32, 8), 128, torch.bfloat16, 48, 0, 0.09),     # pair + a box of another label; pages of 48
-    (24, 80, (64, 8), 64, torch.float16, 16, 0, -0.1),       # pair + single, negative scale, one token past a super-step
+    (24, 80, (64, 8), 64, torch.float16, 16, 0, -0.1),       # pair + single, negative scale, 16 tokens past a super-step
     (130, 1040, (8, 8), 64, torch.bfloat16, 16, 256, 0.1),   # no query-head groups: 64 sequences a box; cut into pieces
-    (64, 2112, (16, 4), 128, torch.float16, 32, 0, 0.09),    # pieces long enough for K and V tiles handed over apart
+    (64, 2112, (16, 4), 128, torch.float16, 32, 0, 0.09),    # pieces of 256 tokens (in twos) or 384
     (22, 1152, (32, 8), 128, torch.bfloat16, 64, 640, 0.0),  # 64 + 24 rows; scale 0
+    # K and V tiles handed over apart (from 512 tokens a piece): pieces of eight super-steps and a half, the last of one, partial
+    (64, 1680, (32, 8), 128, torch.bfloat16, 16, 544, 0.09),
+    (64, 1680, (64, 8), 64, torch.float16, 16, 544, -0.1),
+    (40, 1680, (32, 8), 64, torch.bfloat16, 48, 576, 0.1),   # pair + a box of another label
 ])
 def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, page, chunk, scale, tuning, monkeypatch):
     print(f"[case] pairs of boxes: {seqs} x ({prefix} + tails), heads {heads}, d {d}, page {page}", flush=True)
@@ -1261,7 +1273,7 @@ def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, pag
     tree.build_radix_tree(w.seq_lens, w.padded_table())
     ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, w.seq_lens, scale)
     for pairs in (1, 2):
-        tuning(tall_rows=32, tall_chunk_tokens=chunk, pairs=pairs)
+        tuning(tall_rows=32, tall_chunk_tokens=chunk, pairs=pairs, equalize_chunks=0 if prefix == 1680 else -1)
         tree.pack_schedule(None, heads[0] // heads[1], heads[1])
         info = tree.kernel_info
         info.to_gpu(dev)
@@ -1270,7 +1282,7 @@ def test_two_boxes_of_a_node_in_one_workgroup(seqs, prefix, heads, d, dtype, pag
         lse = torch.full((seqs, heads[0]), float("nan"), dtype=torch.float32, device=dev)
         prefix_attn_with_kvcache(q, k, v, tree, scale, out, softmax_lse=lse)
         torch.cuda.synchronize()
-        assert [g["pairs"] for g in info._launch_geometries] == [pairs == 1 and seqs != 22]
+        assert [(g["pairs"], g["apart"]) for g in info._launch_geometries] == [(pairs == 1 and seqs != 22, chunk >= 512)]
         _assert_close(f"pairs {pairs}", out, lse, ref_out, ref_lse, dtype)
 
 
@@ -1302,6 +1314,21 @@ def test_short_boxes_beside_tall_ones(heads, d, dtype, chunk, head_per_wave, tun
     geo = tree.kernel_info._launch_geometries[0]
     assert geo["tall_rows"] == 32 and geo["apart"] == (chunk == 512)
     _assert_close(f"pieces of {chunk}", out, lse, *_oracle(w, q, k, v), dtype)
+
+
+def test_pairs_with_k_and_v_laid_out_apart(tuning):
+    # V's pages, tokens and heads lie further apart than K's: neither's addresses can be told from the other's
+    print("[case] pairs of boxes, K and V of different strides", flush=True)
+    dev = _device()
+    w = workloads.shared_prefix("pair-strides", 64, 43 * 16, 20, 60, 32, 8, 128, torch.bfloat16, 4)
+    q, k, v = w.tensors(dev)
+    big = torch.full((v.shape[0] + 1, v.shape[1] + 1, v.shape[2] + 3, v.shape[3] + 8), float("nan"), dtype=v.dtype, device=dev)
+    view = big[1:, :v.shape[1], :v.shape[2], :v.shape[3]]
+    view.copy_(v)
+    ref = _oracle(w, q, k, v)
+    for chunk in (0, 512):
+        tuning(tall_rows=32, pairs=1, tall_chunk_tokens=chunk, equalize_chunks=0 if chunk else -1)   # (512: tiles handed over apart)
+        _assert_close(f"chunk {chunk}", *_run_tree(w, q, k, view), *ref, w.dtype)
 
 
 @pytest.mark.parametrize("captured", [False, True])

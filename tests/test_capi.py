@@ -379,6 +379,18 @@ def test_tall_boxes_are_cut_by_what_a_workgroup_takes_ends_included():
     assert g.num_slots == 18 and need.value <= 48 << 20
 
 
+@pytest.mark.parametrize("force", [0, 32])
+def test_pieces_too_long_for_the_32_row_form_take_the_other(force, tuning):
+    # 64 pieces a box at most, so a box of more than 64 x 4096 tokens is cut into pieces longer than that form takes
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    if force:
+        tuning(tall_rows=force)
+    for tokens, rows in ((64 * 4096, 32), (64 * 4096 + 64, 16)):
+        a = _bucket_args([(64, 2, 16, tokens, _lib.PAT_BUCKET_ITEMS, 1), (16, 32, 1, 64, 0, 0)], 32, 8, 128, 32, 64)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        assert g.tall_rows == rows and g.chunks_per_rank <= 64 and not (rows == 16 and g.flags & _lib.PAT_GEOMETRY_PAIRS)
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on fake addresses")
 def test_static_launch_that_only_fits_box_by_box_is_not_refused():
     # records of items hold twice the sequences: 65.8 MiB with the boxes in twos, 64.0 one by one
