@@ -13,7 +13,8 @@ constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-ro
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
 // Launches of 9..32 slots per row where a workgroup takes a row: up to so many slots over all rows. It requests every slot,
 // empty ones too, which has to cost less than the two round trips it saves (us per merge, general / workgroup per row: 32 rows
-// x 27 slots 5.7 / 2.5, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
+// x 32 slots 5.1 / 3.0, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2). 32 slots are eight for each of its
+// four waves, as many rows as a wave of the other forms requests at once.
 constexpr int kMergeWideSlots = 32;
 constexpr int64_t kMergeWideMost = 32768;
 

@@ -1,6 +1,6 @@
-// Split-KV forward kernel for gfx950 (MI355X): one workgroup streams one chunk of one
-// packed box's KV for one kv-head and one 16-row tile of the box, and writes a normalised
-// partial output + LSE per row.
+// Split-KV forward kernel for gfx950 (MI355X): one workgroup streams one chunk of a packed box's
+// KV for one kv head (short boxes: of four) and all rows of the box, or of two boxes of one tree
+// node, and writes a normalised partial output + LSE per row.
 //
 // Functional contract (what the reference's pat_fwd_splitkv_kernel computes,
 // csrc/pat_fwd_kernel.h:25-299): rows r = g + G*j of a box are (sequence

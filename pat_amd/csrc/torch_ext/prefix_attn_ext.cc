@@ -259,7 +259,7 @@ struct PlanTables {
   const TensorList* slots;                       // may be null
   const std::vector<std::vector<int>>* mnw;
   const std::vector<int>* flags;                 // may be null
-  const TensorList* items = nullptr;             // per bucket [items, 2] (pat_fwd_bucket.items) or empty; may be null
+  const TensorList* items = nullptr;             // per bucket [items, 2] (PAT_BUCKET_ITEMS) or empty; may be null
 };
 
 // Checks that need tensor metadata follow csrc/api.h:131-181, :256-277 of the reference.
