@@ -274,7 +274,7 @@ typedef struct pat_fwd_bucket {
  * them for one launch (what pat_fwd_autotune's result is for). 0 / -1 = automatic, as noted per field. The
  * initial values come from the environment variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS,
  * PAT_HEAD_PER_WAVE_TOKENS, PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS,
- * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, PAT_TALL_ROWS, PAT_PAIRS, read once; pat_fwd_set_tuning(NULL) reads them again. */
+ * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, PAT_TALL_ROWS, PAT_PAIRS, PAT_STREAM_V, read once; pat_fwd_set_tuning(NULL) reads them again. */
 typedef struct pat_fwd_tuning {
   int32_t chunk_tokens;              /* KV tokens per workgroup, boxes <= 16 rows (0: automatic)   */
   int32_t tall_chunk_tokens;         /* same for boxes of 17..64 rows (0: automatic)                */
@@ -289,8 +289,12 @@ typedef struct pat_fwd_tuning {
                                      /* tiles, 2 workgroups per CU at head_dim 128), 16 (16x16x32,  */
                                      /* 3 per CU), 0: chosen per launch from its sizes              */
   int32_t pairs;                     /* two boxes of an item served by one workgroup (32-row form): */
-                                     /* 0 chosen per launch from its sizes, 1 always, 2 never       */
+                                     /* 0 chosen per launch from its sizes, 1 always, 2 never;      */
+                                     /* + PAT_STREAM_V_ALWAYS / _NEVER: V of boxes <= 16 rows read  */
+                                     /* past the caches where no other box reads it                 */
 } pat_fwd_tuning;
+#define PAT_STREAM_V_ALWAYS 4 /* (neither: chosen per launch from its sizes) */
+#define PAT_STREAM_V_NEVER 8
 int pat_fwd_set_tuning(const pat_fwd_tuning* tuning);
 int pat_fwd_get_tuning(pat_fwd_tuning* out);
 
@@ -447,6 +451,7 @@ typedef struct pat_fwd_geometry {
 } pat_fwd_geometry;
 #define PAT_GEOMETRY_PAIRS 1 /* the two boxes of an item are served by one workgroup */
 #define PAT_GEOMETRY_APART 2 /* 32-row form: K and V tiles handed over apart         */
+#define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows read past the caches (pieces of one reader) */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);
 
 /* ------------------------------------------------------------------------ *

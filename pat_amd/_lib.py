@@ -84,8 +84,11 @@ class FwdBucket(C.Structure):
 
 PAT_BUCKET_EVEN = 1
 PAT_BUCKET_ITEMS = 2
+PAT_STREAM_V_ALWAYS = 4
+PAT_STREAM_V_NEVER = 8
 PAT_GEOMETRY_PAIRS = 1
 PAT_GEOMETRY_APART = 2
+PAT_GEOMETRY_STREAM_V = 4
 
 
 class BaselineArgs(C.Structure):

@@ -29,6 +29,7 @@ constexpr int kMinChunk = 128;      // tokens
 constexpr int kMaxChunk = 2048;
 constexpr int kTallChunk = 256;
 constexpr int64_t kMostPartialBytes = (int64_t)48 << 20;   // partial rows up to which tall boxes are cut (kStaticScratchBytes less room for records)
+constexpr double kStreamBytes = 92e6;        // K and V of the boxes of <= 16 rows from which V is read past the caches (below)
 constexpr int kApartTokens = 512;            // pieces of tall boxes from which their K and V tiles are handed over apart
 constexpr int kMaxBesideTall = 1024;         // tokens of a short boxes' chunk sized for the slots that tall workgroups leave
 constexpr int kSmallLaunchTokens = 512;      // boxes up to this length stay whole in launches of less than a workgroup per CU
@@ -49,13 +50,14 @@ inline int row_tiles(int m_label) { return m_label <= 16 ? 1 : (m_label <= 32 ? 
 // Overrides of the launch geometry (pat_fwd_set_tuning). The defaults come from the environment
 // variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS, PAT_HEAD_PER_WAVE_TOKENS,
 // PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS, PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT,
-// PAT_TALL_ROWS and PAT_PAIRS, read once per process: no launch reads the environment.
+// PAT_TALL_ROWS, PAT_PAIRS and PAT_STREAM_V, read once per process: no launch reads the environment.
 pat_fwd_tuning env_tuning() {
   pat_fwd_tuning t;
   t.chunk_tokens = 0; t.tall_chunk_tokens = 0; t.head_per_wave_tokens = -1;
   t.head_per_wave_long_wgs = -1; t.head_per_wave_long_tokens = 0; t.equalize_chunks = -1; t.direct_out = -1;
   t.tall_rows = 0; t.pairs = 0;
   if (const char* e = std::getenv("PAT_PAIRS")) t.pairs = std::atoi(e);
+  if (const char* e = std::getenv("PAT_STREAM_V")) t.pairs |= std::atoi(e) == 1 ? PAT_STREAM_V_ALWAYS : std::atoi(e) == 2 ? PAT_STREAM_V_NEVER : 0;
   if (const char* e = std::getenv("PAT_TALL_ROWS")) t.tall_rows = std::atoi(e);
   if (const char* e = std::getenv("PAT_CHUNK_TOKENS")) t.chunk_tokens = std::atoi(e);
   if (const char* e = std::getenv("PAT_TALL_CHUNK_TOKENS")) t.tall_chunk_tokens = std::atoi(e);
@@ -93,6 +95,7 @@ struct Geometry {
   int tall_rows = 32;        // rows per wave on boxes of 17..64 rows: 32 or 16 (the split kernel's instance)
   bool tall_apart = false;   // 32-row form: K and V tiles handed over apart
   bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
+  bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
   // launch records (one per workgroup): entries per record and bytes between records
   int record_max_seqs = 0, record_max_pages = 0, record_stride = 0;
@@ -174,6 +177,18 @@ int check_args(const pat_fwd_args* a) {
       return fail(PAT_ERR_INVALID, "a box packs more rows (sequences x heads per kv head) than its bucket's tile_q" + at);
   }
   return PAT_OK;
+}
+
+// K and V bytes that a launch's boxes of <= 16 rows stream, from sizes: ragged buckets, without the PAT_BUCKET_EVEN hint, hold
+// ~0.6 of their widest box on average.
+double short_bytes(const pat_fwd_args* a) {
+  double bytes = 0.;
+  for (int i = 0; i < a->num_buckets; ++i) {
+    const pat_fwd_bucket& b = a->buckets[i];
+    if (b.num_boxes > 0 && row_tiles(b.mnw[0]) == 1)
+      bytes += (double)b.max_blocks * a->page_size * b.num_boxes * a->kv_heads * ((b.flags & PAT_BUCKET_EVEN) ? 1.0 : 0.6) * a->head_dim * 4.;
+  }
+  return bytes;
 }
 
 // Times of a launch estimated from sizes alone (us): what its <= 16-row boxes take to stream (~5.8 TB/s; ragged
@@ -446,6 +461,15 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
       }
     g->tall_apart = n_tall <= kNumCUs && longest >= kApartTokens;
   }
+  // Reading V past the caches (non-temporal loads, the pieces that one box alone reads: the record kernel looks). A launch
+  // whose K and V exceed a third of the 256 MB memory-side cache finds little of them there at its next call, and V's lines,
+  // kept like K's, only push out K's, the shared pages and the partial rows. us per call, kept / past the caches: 32 requests
+  // of 4096 tokens at 64/8 heads (537 MB) 94.5 / 85.0, three levels of 128 (336 MB) 71.0 / 66.7, 1024 over 512 + 100..200 at
+  // 16/2 46.1 / 40.0, 32 of 1024 at 32/8 (134 MB) 26.0 / 22.6, 24 (101 MB) 24.4 / 23.5; below the line the same calls, repeated
+  // on the same caches, find V there: 22 of 1024 (93 MB) 23.0 / 23.1, 20 18.1 / 18.8, 12 13.7 / 14.5 (but 16 layers of 16 of
+  // 1024, each with its own, 412 / 394). K stays as it is: a load of its operand layout takes 64 bytes of a row, half a line,
+  // and the other half would be fetched again (16 rows' halves per load; with it 837 -> 915 for 32 layers of 89 MB).
+  g->stream_v = !(tune.pairs & PAT_STREAM_V_NEVER) && ((tune.pairs & PAT_STREAM_V_ALWAYS) || short_bytes(a) >= kStreamBytes);
   g->num_slots = g->chunks_per_rank * a->max_split_per_seq;
   // One slot per row (no sequence in two boxes, no box in two chunks): nothing to merge, the
   // split kernel stores the rows in `out` itself (8-byte stores: needs `out` laid out for them).
@@ -498,7 +522,7 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
     tall_box_heads += (int64_t)b.num_boxes * a->kv_heads;
     pairs = pairs || items_of(b, true) < b.num_boxes;
   }
-  pairs = pairs && tune.pairs != 2 && (tune.pairs == 1 || tall_box_heads >= 3 * kNumCUs / 8);
+  pairs = pairs && (tune.pairs & 3) != 2 && ((tune.pairs & 3) == 1 || tall_box_heads >= 3 * kNumCUs / 8);
   // (boxes of more than 64 x kMaxTall32Tokens tokens, which the bound on pieces per box makes longer pieces of, take the 16-row form)
   auto in_32 = [&]() -> int {
     if (int rc = plan_geometry_for(a, g, 32, pairs)) return rc;
@@ -543,7 +567,7 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
   uint64_t h = 0x9e3779b97f4a7c15ull;
   auto mix = [&](uint64_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); };
   mix((uint64_t)g.tall_rows); mix((uint64_t)g.total_wgs); mix((uint64_t)g.record_stride); mix((uint64_t)g.record_max_seqs); mix((uint64_t)g.record_max_pages);
-  mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0);
+  mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0); mix(g.stream_v ? 1 : 0);
   mix((uint64_t)a->batch); mix((uint64_t)a->heads); mix((uint64_t)a->kv_heads); mix((uint64_t)a->page_size);
   mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq); mix(g.pairs ? 1 : 0);
   for (int i = 0; i < a->num_buckets; ++i) {
@@ -579,7 +603,7 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   out->num_slots = g.num_slots;
   out->num_workgroups = g.total_wgs;
   out->tall_rows = g.tall_rows;
-  out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0);
+  out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0);
   return PAT_OK;
 }
 
@@ -648,13 +672,28 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
   const int t_begin = chunk * bk.chunk_tokens;
   int tokens = kv - t_begin;
   tokens = tokens < 0 ? 0 : (tokens > bk.chunk_tokens ? bk.chunk_tokens : tokens);
+  const int first_page = t_begin / page;
+
+  // Is this box the only reader of its piece? The piece's first page against that page of up to 64 other boxes of the
+  // bucket, the next ones behind it (boxes over the same blocks lie next to each other in a plan, and all of a small
+  // one's are looked at).
+  bool stream = false;
+  if (p.stream_v && bk.row_tiles == 1 && tokens > 0) {
+    const int id = bk.block_table[(int64_t)box * bk.bt_stride + first_page];
+    int other = box + 1 + lane;
+    other = other >= bk.num_boxes ? other - bk.num_boxes : other;
+    const bool same = lane < bk.num_boxes - 1 && other < bk.num_boxes && bk.kv[other] > t_begin &&
+                      bk.block_table[(int64_t)other * bk.bt_stride + first_page] == id;
+    stream = __ballot(same) == 0;
+  }
 
   char* rec = p.records + (size_t)wg * (size_t)p.record_stride;
   if (lane == 0) {
     RecordHead h;
     h.tokens = rows > 0 ? tokens : 0;
     h.rows = rows;
-    h.mode = (box2 >= 0 ? 2 * bk.row_tiles : bk.row_tiles) | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0);
+    h.mode = (box2 >= 0 ? 2 * bk.row_tiles : bk.row_tiles) | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0) |
+             (stream ? kRecordModeStreamV : 0);
     h.head = hgroup * bk.heads_per_wg;
     // slots of this box that no workgroup fills: this one's own when it has no tokens, and the
     // ones past the bucket's last chunk (the launch reserves chunks_per_rank per box ordinal)
@@ -680,7 +719,6 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
     tab[p.record_max_seqs + j] = slot;
   }
   // pages of the piece
-  const int first_page = t_begin / page;
   for (int i = lane; i < p.record_max_pages; i += 64) {
     int pg = (first_page + i < bk.max_blocks) ? bk.block_table[(int64_t)box * bk.bt_stride + first_page + i] : 0;
     pg = pg < 0 ? 0 : (pg >= p.num_pages ? p.num_pages - 1 : pg);
@@ -695,7 +733,7 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   rp.record_stride = g.record_stride; rp.record_max_seqs = g.record_max_seqs; rp.record_max_pages = g.record_max_pages;
   rp.batch = args->batch; rp.kv_heads = args->kv_heads; rp.group = args->heads / args->kv_heads;
   rp.page_size = args->page_size; rp.num_pages = args->num_pages;
-  rp.chunks_per_rank = g.chunks_per_rank; rp.max_split = args->max_split_per_seq;
+  rp.chunks_per_rank = g.chunks_per_rank; rp.max_split = args->max_split_per_seq; rp.stream_v = g.stream_v ? 1 : 0;
   // buckets in plan order (tall, long boxes come first in the default order)
   int nb = 0;
   int64_t items = 0;
@@ -755,6 +793,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   sp.o_part = o_part; sp.lse_part = lse_part;
   sp.direct = g.direct ? 1 : 0;
   sp.tall_rows = g.tall_rows;
+  sp.stream_v = g.stream_v ? 1 : 0;
   sp.tall_apart = g.tall_apart ? 1 : 0;
   if (g.direct) {
     sp.out = args->out; sp.lse_out = args->lse_out;
@@ -919,7 +958,7 @@ int pat_fwd_launch_static(const pat_fwd_args* args, void* hip_stream) {
   if (need > kStaticScratchBytes && g.pairs && args->records == nullptr) {
     box_by_box = *args;
     tune = args->tuning != nullptr ? *args->tuning : tuning();
-    tune.pairs = 2;
+    tune.pairs = (tune.pairs & ~3) | 2;
     box_by_box.tuning = &tune;
     args = &box_by_box;
     g = Geometry();

@@ -28,7 +28,7 @@ struct RecordHead {
   int32_t tokens;      // KV tokens of this piece; 0: nothing to compute (the workgroup only marks slots empty)
   int32_t rows;        // rows of the box, or of the two boxes of an item (sequences x heads per kv head), <= 16 x tiles
   int32_t mode;        // bits 0-7: 16-row tiles (1 = KV steps split over waves on wave-private tiles,
-                       // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave
+                       // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave; bit 9: V read past the caches
   int32_t head;        // first kv head this workgroup serves
   int32_t fill_begin;  // slots slot[j] + fill_begin .. slot[j] + fill_end - 1 of every row stay empty:
   int32_t fill_end;    // this workgroup marks them (-inf)
@@ -36,6 +36,7 @@ struct RecordHead {
 };
 static_assert(sizeof(RecordHead) == 32, "RecordHead is read as two 16-byte pieces");
 constexpr int kRecordModeHeadPerWave = 0x100;
+constexpr int kRecordModeStreamV = 0x200;
 
 struct SplitParams {
   const char* records;      // one per workgroup, in launch order
@@ -63,6 +64,7 @@ struct SplitParams {
   int64_t o_stride_b, o_stride_h;              // elements
   int32_t direct;    // 1: such a launch
   int32_t tall_apart;  // 32-row form: K and V tiles of a super-step handed over apart (see the kernel)
+  int32_t stream_v;  // records may ask for V past the caches (host side: picks the kernel instance)
   int32_t tall_rows; // rows per wave on boxes of 17..64 rows: 32 (32x32x16 tiles) or 16 (host side: picks the kernel instance)
 };
 
@@ -95,6 +97,7 @@ struct RecordParams {
   int32_t batch, kv_heads, group, page_size, num_pages;
   int32_t chunks_per_rank;  // slots reserved per box ordinal
   int32_t max_split;
+  int32_t stream_v;         // V tiles of pieces that no other box reads go past the caches (kRecordModeStreamV)
   RecordBucket bucket[kMaxBuckets];
 };
 

@@ -104,8 +104,10 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds) : "memory", "m0");
 }
 
-// DIRECT instances serve launches in which every row has one partial slot: they store `out`.
-template <typename T, int D, bool DIRECT, int TALLK>
+// DIRECT instances serve launches in which every row has one partial slot: they store `out`. STREAM instances serve launches
+// whose records may ask for V past the caches (kRecordModeStreamV): a second loop over short boxes, whose mere presence cost
+// the smallest launches 0.14 us of 5.5.
+template <typename T, int D, bool DIRECT, int TALLK, bool STREAM>
 __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
                                                                              const int record_max_seqs, const int record_max_pages, const SplitParams p) {
   using E = Elem<T>;
@@ -776,7 +778,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     PAT_LDS char* vstage = (PAT_LDS char*)smem + wave * WSTAGE;
     const unsigned koff = (unsigned)(n * kss) + g * 16;                          // K: row n of a half, dims g*8..
     const unsigned voff = (unsigned)((lane / CPR) * vss) + (lane % CPR) * 16;    // V: TPL rows per instruction
-    auto fetch_v = [&](int st, u32x4 (&vd)[NV]) {
+    auto fetch_v = [&](int st, u32x4 (&vd)[NV], auto stream_c) {
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
         int lim;
@@ -786,7 +788,8 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
         for (int j = 0; j < NV / 2; ++j) {
           unsigned vo = voff + (unsigned)(j * TPL) * (unsigned)vss;
           if (lim < 15 && j * TPL + lane / CPR > lim) vo = (unsigned)(lim * vss) + (lane % CPR) * 16;
-          vd[a * (NV / 2) + j] = *(const u32x4*)(vb + vo);
+          const u32x4* at = (const u32x4*)(vb + vo);
+          vd[a * (NV / 2) + j] = decltype(stream_c)::value ? __builtin_nontemporal_load(at) : *at;
         }
       }
     };
@@ -805,9 +808,9 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     // steps of this wave: every kWaves-th one of the chunk, or, with a kv head per wave, all of them
     const int step0 = head_per_wave ? 0 : wave;
     const int stride = head_per_wave ? 1 : kWaves;
-    if (step0 < nsteps) {
+    auto walk = [&](auto stream_c) {
       u32x4 kd[2][KK], vd[NV];
-      fetch_v(step0, vd);
+      fetch_v(step0, vd, stream_c);
       fetch_k(step0, kd);
       // Q is here before the loop starts, and the last step, which requests nothing, stands apart from it: every wait inside
       // then counts exactly the loads behind the one it is for. In one loop with Q on its way and requests that may not be made,
@@ -822,7 +825,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
 #pragma unroll
         for (int j = 0; j < NV; ++j)
           *(PAT_LDS u32x4*)(vstage + (j * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vd[j];
-        if (more) fetch_v(st + stride, vd);
+        if (more) fetch_v(st + stride, vd, stream_c);
         // Few tall workgroups with long chains (p.tall_apart): the launch ends on those, and these waves' requests, of two
         // steps at once, hold theirs up (us per call without / with this wait: 64 requests over 2048 tokens, 32/8 heads, 22.8 /
         // 22.0, 32 over 16384 at 64/8 57.6 / 56.3). Of 125 launches of this form measured both ways the 35 such are 1.4 %
@@ -837,6 +840,19 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       int st = step0;
       for (; st + stride < nsteps; st += stride) step(st, std::true_type{});
       step(st, std::false_type{});
+    };
+    // (V past the caches: the host's choice for launches of ~100 MB and more, there 4-20 % faster. A loop of its own: inside one
+    // loop the two kinds of load are either merged, without the hint, or cost 3 % as a branch; and a branch known to be uniform
+    // costs 28 spilled registers, like uniform loop bounds above)
+    if (step0 < nsteps) {
+      if constexpr (STREAM) {
+        int past = mode & kRecordModeStreamV;
+        asm volatile("" : "+v"(past));
+        if (past) walk(std::true_type{});
+        else walk(std::false_type{});
+      } else {
+        walk(std::false_type{});
+      }
     }
     l_run = sum_xor32(sum_xor16(l_run));
 
@@ -894,26 +910,31 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   }
 }
 
-// Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path).
+// Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path, V past the caches).
 typedef void (*SplitFn)(const char*, int, int, int, const SplitParams);
-template <bool DIRECT, int TALLK>
+template <bool DIRECT, int TALLK, bool STREAM>
 static SplitFn split_instance(bool bf16, int head_dim) {
-  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK> : pat_split_kernel<__bf16, 128, DIRECT, TALLK>;
-  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK> : pat_split_kernel<_Float16, 128, DIRECT, TALLK>;
+  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM>;
+  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM>;
+}
+template <bool STREAM>
+static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
+  if (direct) return t32 ? split_instance<true, 32, STREAM>(bf16, head_dim) : split_instance<true, 16, STREAM>(bf16, head_dim);
+  return t32 ? split_instance<false, 32, STREAM>(bf16, head_dim) : split_instance<false, 16, STREAM>(bf16, head_dim);
 }
 
 hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const SplitParams& params) {
   const bool t32 = params.tall_rows != 16;
-  SplitFn fn = params.direct ? (t32 ? split_instance<true, 32>(bf16, head_dim) : split_instance<true, 16>(bf16, head_dim))
-                             : (t32 ? split_instance<false, 32>(bf16, head_dim) : split_instance<false, 16>(bf16, head_dim));
+  const bool past = params.stream_v != 0;
+  SplitFn fn = past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
   const unsigned lds = (unsigned)split_smem_bytes(head_dim, t32 ? 32 : 16);
   // more dynamic LDS than the default limit of a kernel: raised once per instance and device
   {
     static std::mutex mutex;
-    static bool raised[64][16] = {{false}};
+    static bool raised[64][32] = {{false}};
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const int inst = (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
+    const int inst = (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
     std::lock_guard<std::mutex> lock(mutex);
     if (dev >= 0 && dev < 64 && !raised[dev][inst]) {
       if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -1156,6 +1156,7 @@ PYBIND11_MODULE(_prefix_attn, m) {
           d["chunk_tokens"] = g.chunk_tokens; d["tall_chunk_tokens"] = g.tall_chunk_tokens; d["num_slots"] = g.num_slots;
           d["num_workgroups"] = g.num_workgroups; d["tall_rows"] = g.tall_rows;
           d["pairs"] = (g.flags & PAT_GEOMETRY_PAIRS) != 0; d["apart"] = (g.flags & PAT_GEOMETRY_APART) != 0;
+          d["stream_v"] = (g.flags & PAT_GEOMETRY_STREAM_V) != 0;
           out.append(d);
         }
         return out;

@@ -1486,3 +1486,43 @@ def test_scale_at_the_ends_of_its_range(scale, tall_rows, tuning):
     else:
         ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), w.rows, w.seq_lens, scale)
         _assert_close(f"scale {scale}", out, lse, ref_out, ref_lse, w.dtype)
+
+
+@pytest.mark.parametrize("kind", ["tall", "long", "direct", "siblings"])
+@pytest.mark.parametrize("heads,d,dtype", [((32, 8), 128, torch.bfloat16), ((8, 8), 64, torch.float16), ((16, 2), 128, torch.float16)])
+def test_v_read_past_the_caches(kind, heads, d, dtype, tuning, monkeypatch):
+    # the same launch with V's loads as they are and past the caches gives the same bits, and the oracle's values: boxes beside
+    # tall ones, long ones in pieces, single-slot launches, and boxes whose pages other boxes read too (which keep their loads)
+    from pat_amd import _lib
+    print(f"[case] V past the caches, {kind}, heads {heads}, d {d}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "1" if kind == "direct" else "0")
+    dev = _device()
+    tails = [1, 31, 33, 64, 95, 128, 200, 257] * (40 if kind == "direct" else 4)
+    if kind == "long":
+        tails = [1, 700, 1500, 2049]
+    shared = {"tall": 512, "siblings": 48}.get(kind, 0)
+    per_node = 3 if kind == "siblings" else len(tails)
+    rows, nxt = [], 0
+    for i, n in enumerate(tails):
+        if i % per_node == 0:
+            node = list(range(nxt, nxt + shared // 16))
+            nxt += shared // 16
+        rows.append(node + list(range(nxt, nxt + -(-n // 16))))
+        nxt += -(-n // 16)
+    w = workloads.Workload("past", heads[0], heads[1], d, dtype, 16, [shared + n for n in tails], rows, nxt, 0, 6)
+    q, k, v = w.tensors(dev)
+    results = []
+    for stream in (_lib.PAT_STREAM_V_ALWAYS, _lib.PAT_STREAM_V_NEVER):
+        tuning(pairs=stream)
+        tree = PrefixTreeCPP(16)             # (a tree of its own: its split counters run on over plans)
+        tree.build_radix_tree(w.seq_lens, w.padded_table())
+        tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+        tree.kernel_info.to_gpu(dev)
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((w.batch, w.heads), float("nan"), dtype=torch.float32, device=dev)
+        prefix_attn_with_kvcache(q, k, v, tree, 1.0 / math.sqrt(d), out, softmax_lse=lse)
+        torch.cuda.synchronize()
+        assert tree.kernel_info._launch_geometries[0]["stream_v"] == (stream == _lib.PAT_STREAM_V_ALWAYS)
+        results.append((out, lse))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    _assert_close(kind, *results[0], *_oracle(w, q, k, v), dtype)
