@@ -11,12 +11,22 @@ constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop itera
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
 constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
-// Launches of 9..32 slots per row where a workgroup takes a row: up to so many slots over all rows. It requests every slot,
-// empty ones too, which has to cost less than the two round trips it saves (us per merge, general / workgroup per row: 32 rows
-// x 32 slots 5.1 / 3.0, 592 x 10 4.5 / 4.0, 2048 x 14 5.6 / 5.0, but 4096 x 18 5.2 / 7.2). 32 slots are eight for each of its
-// four waves, as many rows as a wave of the other forms requests at once.
-constexpr int kMergeWideSlots = 32;
+// Launches of 9 slots per row and more where a workgroup takes a row. A wave of it requests eight rows at once, as many as one of
+// the other forms. Whole calls, us (the split kernel is the same in all), a wave per row / the form taken:
+//  * 9..32 slots, four waves, every slot requested at once: up to so many slots over all rows. Empty slots are requested too,
+//    which has to cost less than the two round trips it saves (merges: 32 rows x 32 slots 5.1 / 3.0, 592 x 10 4.5 / 4.0, 2048 x 14
+//    5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
+//  * 33..64 slots, eight waves, the same: one request of 16384 tokens in 64 pieces 20.9 / 15.9, 96 rows x 41 slots 14.1 / 10.8,
+//    288 x 56 21.1 / 18.2, 768 x 64 (head_dim 64) 16.0 / 14.1; 1024 x 64 24.4 / 24.5, with the LSEs first 23.0.
+//  * more, and where that is too many: the LSEs first, then the filled slots only, with eight waves up to so many rows, with
+//    four up to so many (eight / four waves): 64 x 72 15.6 / 11.2, 528 x 138 21.1 / 14.3, 1024 x 128 36.2 / 33.3, 2048 x 64
+//    35.5 / 35.8 / 35.2, 2112 x 100 42.9 / 42.1 / 40.7, 4096 x 64 70.1 / 71.5 / 69.8.
+constexpr int kMergeWideBatch = 8;
+constexpr int kMergeWideSlots = 4 * kMergeWideBatch;
 constexpr int64_t kMergeWideMost = 32768;
+constexpr int64_t kMergeWide8Most = 49152;
+constexpr int64_t kMergeWide8Rows = 1536;
+constexpr int64_t kMergeWide4Rows = 8192;
 
 // One workgroup's work: a launch record, written once per plan by the record kernel
 // (capi_fwd.hip) and read by the split kernel in a single round trip. In memory:

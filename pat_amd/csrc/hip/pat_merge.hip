@@ -15,7 +15,7 @@
 // requested at once and what turns out unused is dropped (measured: 0.3-0.8 us less per launch;
 // with 16 rows requested blindly the extra registers and reads cost what the round trips save).
 // Two more forms stand below: a half-wave per row where rows are many and slots few, a workgroup per row where
-// slots are many (9..32) and rows few. In all of them a slot is empty where its LSE is -inf, and nowhere else: a NaN (from
+// slots are many (9 and more) and rows few. In all of them a slot is empty where its LSE is -inf, and nowhere else: a NaN (from
 // a NaN in Q or K, or an infinite score) is a filled slot, and makes the row NaN as it makes one that is not cut up.
 #include <hip/hip_runtime.h>
 
@@ -276,16 +276,20 @@ __global__ void __launch_bounds__(256) pat_merge_pairs_kernel(MERGE_ROWS, const 
   if (p.lse_out != nullptr && l32 == 0) p.lse_out[pair] = total;
 }
 
-// Launches of 9..32 slots per row and few rows (a long request cut over the whole chip, a deep tree of a few dozen
-// requests): a workgroup takes a (sequence, head), each of its four waves the next num_slots / 4 slots, whose LSEs and
-// rows it requests at once like the kernels above; the four sums are combined through LDS. One round trip where the
-// general kernel's chain is split count -> LSEs -> rows by sixteens, and four times the waves where rows are few.
-template <typename T, int D>
-__global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const MergeParams p) {
+// Launches of 9 slots per row and more and few rows (a long request cut over the whole chip, a deep tree of a few dozen
+// requests): a workgroup takes a (sequence, head), each of its WAVES waves every WAVES-th slot; the waves' sums are combined
+// through LDS.
+//  * SPEC: up to 8 slots per wave, whose LSEs and rows it requests at once like the kernels above: one round trip where the
+//    general kernel's chain is split count -> LSEs -> rows by sixteens, and WAVES times the waves where rows are few. Empty
+//    slots are requested too.
+//  * otherwise the LSEs first, then the rows of the filled slots, eight at a time: two round trips, and nothing read for
+//    empty slots, which most are where a launch reserves many (a slot per piece of the longest box for every box).
+template <typename T, int D, int WAVES, bool SPEC>
+__global__ void __launch_bounds__(WAVES * 64) pat_merge_wide_kernel(MERGE_ROWS, const MergeParams p) {
   constexpr int CPL = D / 64;
-  constexpr int kSpec = kMergeWideSlots / 4;   // slots per wave
-  __shared__ float s_acc[4][D];
-  __shared__ float s_max[4], s_sum[4];
+  constexpr int kBatch = kMergeWideBatch;   // rows a wave requests at once
+  __shared__ float s_acc[WAVES][D];
+  __shared__ float s_max[WAVES], s_sum[WAVES];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned u = mapping & 256 ? blockIdx.x >> 3 : blockIdx.x;
@@ -294,81 +298,137 @@ __global__ void __launch_bounds__(256) pat_merge_wide_kernel(MERGE_ROWS, const M
   row_of(u, blockIdx.x & 7, per_list, per_list_magic, mapping, s, hq);
   const int64_t pair = (int64_t)s * heads + hq;
   const float ninf = -__builtin_inff();
-  const int mine = (num_slots + 3) >> 2, first = wave * mine;   // this wave's slots
   const float* __restrict__ lse = lse_part + pair * num_slots;
   const float* __restrict__ op = o_part + pair * (int64_t)num_slots * D;
   int ns = num_split_per_seq[s];
-  float l = (lane < mine && first + lane < num_slots) ? lse[first + lane] : ninf;
-  float v[kSpec][CPL];
-#pragma unroll
-  for (int b = 0; b < kSpec; ++b)
-    if (b < mine && first + b < num_slots) {
-      const float* row = op + (int64_t)(first + b) * D + lane * CPL;
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) v[b][c] = row[c];
-    }
-  ns = ns < 0 ? 0 : (ns > max_split ? max_split : ns);
-  if (first + lane >= ns * chunks_per_rank) l = ninf;
-  float mx = l;
-#pragma unroll
-  for (int off = kSpec / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-  mx = __shfl(mx, 0);
-  const float w_mine = (l != ninf) ? __expf(l - mx) : 0.f;
-  float sum = w_mine;
-#pragma unroll
-  for (int off = kSpec / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  float acc[CPL];
+  float mx = ninf, sum = 0.f, acc[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) acc[c] = 0.f;
+  if (SPEC) {
+    const int mine = wave + lane * WAVES;   // this lane's slot
+    float l = (lane < kBatch && mine < num_slots) ? lse[mine] : ninf;
+    float v[kBatch][CPL];
 #pragma unroll
-  for (int b = 0; b < kSpec; ++b) {
-    const float w = __shfl(w_mine, b);
-    // (rows of slots that are empty or beyond the count hold anything: dropped, not multiplied)
-    if (b < mine && first + b < num_slots && w != 0.f) {
+    for (int b = 0; b < kBatch; ++b)
+      if (wave + b * WAVES < num_slots) {
+        const float* row = op + (int64_t)(wave + b * WAVES) * D + lane * CPL;
 #pragma unroll
-      for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
+        for (int c = 0; c < CPL; ++c) v[b][c] = row[c];
+      }
+    ns = ns < 0 ? 0 : (ns > max_split ? max_split : ns);
+    if (mine >= ns * chunks_per_rank) l = ninf;
+    mx = l;
+#pragma unroll
+    for (int off = kBatch / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    mx = __shfl(mx, 0);
+    const float w_mine = (l != ninf) ? __expf(l - mx) : 0.f;
+    sum = w_mine;
+#pragma unroll
+    for (int off = kBatch / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) {
+      const float w = __shfl(w_mine, b);
+      // (rows of slots that are empty or beyond the count hold anything: dropped, not multiplied)
+      if (wave + b * WAVES < num_slots && w != 0.f) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
+      }
+    }
+  } else {
+    // (WAVES x 64 slots at a time: one turn of the loop but for plans of caller's buckets)
+    for (int base = 0; base < num_slots; base += WAVES * 64) {
+      const int mine = base + wave + lane * WAVES;
+      float l = mine < num_slots ? lse[mine] : ninf;
+      int n = ns < 0 ? 0 : (ns > max_split ? max_split : ns);
+      if (mine >= n * chunks_per_rank) l = ninf;
+      float m_new = fmaxf(mx, l);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) m_new = fmaxf(m_new, __shfl_xor(m_new, off));
+      const float w_mine = (l != ninf) ? __expf(l - m_new) : 0.f;
+      const float scale = mx == m_new ? 1.f : __expf(mx - m_new);   // (equal: the first turn's -inf as well)
+      mx = m_new;
+      float part = w_mine;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off);
+      sum = sum * scale + part;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) acc[c] *= scale;
+      unsigned long long live = __ballot(w_mine != 0.f);
+      while (live) {
+        int js[kBatch];
+        float v[kBatch][CPL];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+          js[b] = live ? __builtin_ctzll(live) : -1;
+          live &= live - 1;   // 0 stays 0
+        }
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
+          if (js[b] >= 0) {
+            const float* row = op + (int64_t)(base + wave + js[b] * WAVES) * D + lane * CPL;
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) v[b][c] = row[c];
+          }
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
+          if (js[b] >= 0) {
+            const float w = __shfl(w_mine, js[b]);
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) acc[c] += w * v[b][c];
+          }
+      }
     }
   }
 #pragma unroll
   for (int c = 0; c < CPL; ++c) s_acc[wave][lane * CPL + c] = acc[c];
   if (lane == 0) { s_max[wave] = mx; s_sum[wave] = sum; }
   __syncthreads();
-  if (wave != 0) return;
+  if (threadIdx.x >= D) return;
   float most = s_max[0];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) most = fmaxf(most, s_max[w]);
-  float weight[4], all = 0.f;
+  for (int w = 1; w < WAVES; ++w) most = fmaxf(most, s_max[w]);
+  float all = 0.f, x = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    weight[w] = s_sum[w] != 0.f ? __expf(s_max[w] - most) : 0.f;
-    all += weight[w] * s_sum[w];
+  for (int w = 0; w < WAVES; ++w) {
+    const float weight = s_sum[w] != 0.f ? __expf(s_max[w] - most) : 0.f;
+    all += weight * s_sum[w];
+    x += weight * s_acc[w][threadIdx.x];
   }
-  const float inv = all != 0.f ? 1.f / all : 0.f;
-  T* dst = (T*)p.out + (int64_t)s * p.o_stride_b + (int64_t)hq * p.o_stride_h + lane * CPL;
-#pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-    float x = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) x += weight[w] * s_acc[w][lane * CPL + c];
-    dst[c] = (T)(x * inv);
-  }
-  if (p.lse_out != nullptr && lane == 0) p.lse_out[pair] = all != 0.f ? most + logf(all) : ninf;
+  T* dst = (T*)p.out + (int64_t)s * p.o_stride_b + (int64_t)hq * p.o_stride_h + threadIdx.x;
+  *dst = (T)(all != 0.f ? x / all : 0.f);
+  if (p.lse_out != nullptr && threadIdx.x == 0) p.lse_out[pair] = all != 0.f ? most + logf(all) : ninf;
+}
+
+typedef void (*MergeFn)(const int32_t*, const float*, const float*, int, int, int, int, int, int, unsigned, int, const MergeParams);
+template <int WAVES, bool SPEC>
+static MergeFn wide_instance(bool bf16, int head_dim) {
+  if (bf16) return head_dim == 64 ? pat_merge_wide_kernel<__bf16, 64, WAVES, SPEC> : pat_merge_wide_kernel<__bf16, 128, WAVES, SPEC>;
+  return head_dim == 64 ? pat_merge_wide_kernel<_Float16, 64, WAVES, SPEC> : pat_merge_wide_kernel<_Float16, 128, WAVES, SPEC>;
 }
 
 // Host launcher: one wave per (sequence, query head), four per workgroup; a half-wave each in large launches
-// of few slots, a workgroup each in small launches of many.
+// of few slots, a workgroup each where slots are many (the lines: fwd_params.hpp).
 hipError_t launch_merge(bool bf16, int head_dim, hipStream_t stream, const MergeParams& params) {
   const int64_t pairs = (int64_t)params.batch * params.heads;
-  void (*fn)(const int32_t*, const float*, const float*, int, int, int, int, int, int, unsigned, int, const MergeParams);
-  int per_wg = 4;
+  MergeFn fn;
+  int per_wg = 4, threads = 256;
+  const int64_t slots = pairs * params.num_slots;
   if (params.num_slots <= 8 && pairs >= PAT_MERGE_PAIRS_MIN) {
     per_wg = 8;
     if (bf16) fn = head_dim == 64 ? pat_merge_pairs_kernel<__bf16, 64> : pat_merge_pairs_kernel<__bf16, 128>;
     else fn = head_dim == 64 ? pat_merge_pairs_kernel<_Float16, 64> : pat_merge_pairs_kernel<_Float16, 128>;
-  } else if (params.num_slots > 8 && params.num_slots <= kMergeWideSlots && pairs * params.num_slots <= kMergeWideMost) {
+  } else if (params.num_slots > 8 && params.num_slots <= kMergeWideSlots && slots <= kMergeWideMost) {
     per_wg = 1;
-    if (bf16) fn = head_dim == 64 ? pat_merge_wide_kernel<__bf16, 64> : pat_merge_wide_kernel<__bf16, 128>;
-    else fn = head_dim == 64 ? pat_merge_wide_kernel<_Float16, 64> : pat_merge_wide_kernel<_Float16, 128>;
+    fn = wide_instance<4, true>(bf16, head_dim);
+  } else if (params.num_slots > kMergeWideSlots && params.num_slots <= 2 * kMergeWideSlots && slots <= kMergeWide8Most) {
+    per_wg = 1; threads = 512;
+    fn = wide_instance<8, true>(bf16, head_dim);
+  } else if (params.num_slots > kMergeWideSlots && pairs <= kMergeWide8Rows) {
+    per_wg = 1; threads = 512;
+    fn = wide_instance<8, false>(bf16, head_dim);
+  } else if (params.num_slots > kMergeWideSlots && pairs <= kMergeWide4Rows) {
+    per_wg = 1;
+    fn = wide_instance<4, false>(bf16, head_dim);
   } else {
     if (bf16) fn = head_dim == 64 ? pat_merge_kernel<__bf16, 64> : pat_merge_kernel<__bf16, 128>;
     else fn = head_dim == 64 ? pat_merge_kernel<_Float16, 64> : pat_merge_kernel<_Float16, 128>;
@@ -379,7 +439,7 @@ hipError_t launch_merge(bool bf16, int head_dim, hipStream_t stream, const Merge
   const uint32_t magic = per_list > 1 ? (uint32_t)((((uint64_t)1 << 32) + per_list - 1) / per_list) : 0u;
   const int64_t rows_per_list = pairs / lists;   // (below 2^31: checked with the launch)
   const int64_t wgs = lists * ((rows_per_list + per_wg - 1) / per_wg);
-  const dim3 grid((unsigned)wgs), block(256);
+  const dim3 grid((unsigned)wgs), block((unsigned)threads);
   hipLaunchKernelGGL(fn, grid, block, 0, stream, params.num_split_per_seq, params.lse_part, params.o_part, params.num_slots,
                      params.chunks_per_rank, params.max_split, params.heads, (int)rows_per_list, per_list, magic,
                      group + (xcd_lists ? 256 : 0), params);

@@ -1526,3 +1526,39 @@ def test_v_read_past_the_caches(kind, heads, d, dtype, tuning, monkeypatch):
         results.append((out, lse))
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
     _assert_close(kind, *results[0], *_oracle(w, q, k, v), dtype)
+
+
+@pytest.mark.parametrize("slots,batch,heads,d,dtype", [
+    (33, 2, (32, 8), 128, torch.float16),      # eight waves a row, first slot count ...
+    (64, 3, (8, 8), 64, torch.bfloat16),       # ... and the last
+    (48, 128, (8, 1), 64, torch.float16),      # 49152 slots: every slot requested at once ...
+    (49, 128, (8, 1), 64, torch.float16),      # ... 50176: the filled ones only
+    (60, 36, (24, 3), 128, torch.bfloat16),    # the same, 24 rows a sequence in one list
+    (64, 193, (8, 8), 64, torch.float16),      # 1544 rows: four waves a row
+    (64, 1025, (8, 1), 64, torch.bfloat16),    # 8200 rows: a wave per row
+])
+def test_merge_of_more_than_32_slots(slots, batch, heads, d, dtype, tuning):
+    # (requests of very different lengths: most slots of most rows are empty, some rows fill one, some all)
+    test_merge_of_many_slots(slots, batch, heads, d, dtype, tuning)
+
+
+def test_merge_of_more_slots_than_a_workgroup_looks_at_at_once(tuning, monkeypatch):
+    # two requests cut into 32-token pieces, the longer one's boxes into 40 and more each: over 512 slots a row
+    print("[case] merge of more than 512 slots per row", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    lens = [36000, 700]
+    rows = [list(range(2250)), list(range(2250, 2250 + 44))]
+    w = workloads.Workload("slots", 8, 8, 64, torch.float16, 16, lens, rows, 2294, 0, 3)
+    q, k, v = w.tensors(dev)
+    tuning(chunk_tokens=32, tall_chunk_tokens=32, head_per_wave_tokens=0, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    tree = PrefixTreeCPP(16)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, 1, 8)
+    tree.kernel_info.to_gpu(dev)
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((2, 8), float("nan"), dtype=torch.float32, device=dev)
+    prefix_attn_with_kvcache(q, k, v, tree, 0.125, out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    assert tree.kernel_info._launch_geometries[0]["num_slots"] > 512
+    _assert_close("over 512 slots", out, lse, *_oracle(w, q, k, v), w.dtype)
