@@ -398,3 +398,16 @@ def test_static_launch_that_only_fits_box_by_box_is_not_refused():
     a = _bucket_args([(64, 8, 64, 7744, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS, 4), (16, 482, 1, 64, 0, 0)], 32, 32, 128, 482, 64)
     assert lib.pat_fwd_workspace_bytes(C.byref(a), C.byref(need)) == 0 and need.value > lib.pat_fwd_static_scratch_bytes()
     assert lib.pat_fwd_launch_static(C.byref(a), None) == _lib.PAT_ERR_HIP      # (got past the check: there is no GPU here)
+
+
+@pytest.mark.parametrize("boxes,tokens,heads,kv_heads,d,whole", [
+    (24, 640, 32, 8, 128, True), (27, 768, 64, 8, 128, True), (26, 624, 8, 8, 64, True), (3, 736, 16, 8, 128, False),
+    (64, 2048, 32, 8, 128, True), (8, 1344, 16, 16, 128, False), (1, 4096, 32, 8, 128, False),
+])
+def test_boxes_of_one_request_each_walked_whole_or_cut(boxes, tokens, heads, kv_heads, d, whole):
+    # one slot a row, written by the split kernel, where that costs less than pieces and a second kernel
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    a = _bucket_args([(16, boxes, 1, tokens, 0, 0)], heads, kv_heads, d, boxes, 16)
+    a.max_split_per_seq = 1
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+    assert (g.num_slots == 1) == whole, g.num_slots
