@@ -16,16 +16,17 @@ constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wa
 //  * 9..32 slots, four waves, every slot requested at once: up to so many slots over all rows. Empty slots are requested too,
 //    which has to cost less than the two round trips it saves (merges: 32 rows x 32 slots 5.1 / 3.0, 592 x 10 4.5 / 4.0, 2048 x 14
 //    5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
-//  * 33..64 slots, eight waves, the same: one request of 16384 tokens in 64 pieces 20.9 / 15.9, 96 rows x 41 slots 14.1 / 10.8,
-//    288 x 56 21.1 / 18.2, 768 x 64 (head_dim 64) 16.0 / 14.1; 1024 x 64 24.4 / 24.5, with the LSEs first 23.0.
+//  * 33..64 slots, eight waves, the same, up to so many slots of 512 bytes (head_dim 64: 256): one request of 16384 tokens in 64
+//    pieces 20.9 / 15.9, 96 rows x 41 slots 14.1 / 10.8, 512 x 48 18.6 / 16.2, 768 x 64 (head_dim 64) 16.0 / 14.1; 832 x 45
+//    25.9 / 27.2, with the LSEs first 25.7, 1024 x 64 24.4 / 24.5, 23.0.
 //  * more, and where that is too many: the LSEs first, then the filled slots only, with eight waves up to so many rows, with
-//    four up to so many (eight / four waves): 64 x 72 15.6 / 11.2, 528 x 138 21.1 / 14.3, 1024 x 128 36.2 / 33.3, 2048 x 64
-//    35.5 / 35.8 / 35.2, 2112 x 100 42.9 / 42.1 / 40.7, 4096 x 64 70.1 / 71.5 / 69.8.
+//    four up to so many (eight / four waves): 64 x 72 15.6 / 11.2 / 11.5, 528 x 138 21.1 / 14.3 / 15.1, 832 x 45 25.9 / 26.3 /
+//    25.7, 1024 x 128 36.2 / 33.3 / 33.4, 2048 x 64 35.5 / 35.8 / 35.2, 2112 x 100 42.9 / 42.1 / 40.7, 4096 x 64 70.1 / 71.5 / 69.8.
 constexpr int kMergeWideBatch = 8;
 constexpr int kMergeWideSlots = 4 * kMergeWideBatch;
 constexpr int64_t kMergeWideMost = 32768;
-constexpr int64_t kMergeWide8Most = 49152;
-constexpr int64_t kMergeWide8Rows = 1536;
+constexpr int64_t kMergeWide8Most = 28672;
+constexpr int64_t kMergeWide8Rows = 768;
 constexpr int64_t kMergeWide4Rows = 8192;
 
 // One workgroup's work: a launch record, written once per plan by the record kernel

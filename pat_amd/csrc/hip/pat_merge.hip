@@ -420,7 +420,7 @@ hipError_t launch_merge(bool bf16, int head_dim, hipStream_t stream, const Merge
   } else if (params.num_slots > 8 && params.num_slots <= kMergeWideSlots && slots <= kMergeWideMost) {
     per_wg = 1;
     fn = wide_instance<4, true>(bf16, head_dim);
-  } else if (params.num_slots > kMergeWideSlots && params.num_slots <= 2 * kMergeWideSlots && slots <= kMergeWide8Most) {
+  } else if (params.num_slots > kMergeWideSlots && params.num_slots <= 2 * kMergeWideSlots && slots * head_dim <= kMergeWide8Most * 128) {
     per_wg = 1; threads = 512;
     fn = wide_instance<8, true>(bf16, head_dim);
   } else if (params.num_slots > kMergeWideSlots && pairs <= kMergeWide8Rows) {

@@ -1531,10 +1531,10 @@ def test_v_read_past_the_caches(kind, heads, d, dtype, tuning, monkeypatch):
 @pytest.mark.parametrize("slots,batch,heads,d,dtype", [
     (33, 2, (32, 8), 128, torch.float16),      # eight waves a row, first slot count ...
     (64, 3, (8, 8), 64, torch.bfloat16),       # ... and the last
-    (48, 128, (8, 1), 64, torch.float16),      # 49152 slots: every slot requested at once ...
-    (49, 128, (8, 1), 64, torch.float16),      # ... 50176: the filled ones only
-    (60, 36, (24, 3), 128, torch.bfloat16),    # the same, 24 rows a sequence in one list
-    (64, 193, (8, 8), 64, torch.float16),      # 1544 rows: four waves a row
+    (64, 112, (8, 1), 64, torch.float16),      # 57344 slots of 256 bytes: every slot requested at once ...
+    (64, 113, (8, 1), 64, torch.float16),      # ... 57856: four waves a row, the filled ones only
+    (56, 32, (24, 3), 128, torch.bfloat16),    # 768 rows, 43008 slots: eight waves a row, the filled ones only, 24 rows a sequence
+    (64, 97, (8, 8), 64, torch.float16),       # 776 rows
     (64, 1025, (8, 1), 64, torch.bfloat16),    # 8200 rows: a wave per row
 ])
 def test_merge_of_more_than_32_slots(slots, batch, heads, d, dtype, tuning):
