@@ -434,6 +434,12 @@ struct Key {
     for (int64_t s : t.sizes()) add(s);
     for (int64_t s : t.strides()) add(s);
   }
+  // ... as tensor() gives them for a 4-D view of t that is not made
+  void view(const void* ptr, const at::Tensor& t, const int64_t (&sizes)[4], const int64_t (&strides)[4]) {
+    add(ptr); add((int)t.scalar_type()); add((int64_t)4);
+    for (int64_t s : sizes) add(s);
+    for (int64_t s : strides) add(s);
+  }
   void plan_tensor(const at::Tensor& t) {   // ... and the version counter: in-place edits of a plan count
     tensor(t); add(t.is_inference() ? kUntracked : (int64_t)t._version());
   }
@@ -1006,43 +1012,76 @@ void fwd_tables(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   run(*L, *store, version, q.device());
 }
 
+// A new launch of the tree's plan on these tensors, remembered under their key.
+std::shared_ptr<Prepared> prepare_tree(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, PrefixTreeCPP& tree, double scale,
+                                       const at::Tensor& out, const std::optional<at::Tensor>& lse, const Key& key) {
+  KernelInfo& info = *tree.info;
+  const int64_t version = info.plan_version();
+  std::shared_ptr<Prepared> L;
+  const bool l = info.has_launch;
+  const std::vector<int> no_flags;
+  // partial results are filed by slot_tables: the launch merges each sequence's boxes of THIS plan
+  // (num_split_per_seq counts on over repeated pack_schedule calls)
+  PlanTables pt{l ? &info.l_q_tables : &info.q_tables, l ? &info.l_block_tables : &info.block_tables,
+                l ? &info.l_num_seqs : &info.num_seqs, l ? &info.l_ranks : &info.ranks, l ? &info.l_kvs : &info.kvs,
+                l ? &info.l_slot_tables : &info.slot_tables, l ? &info.l_mnws : &info.mnws,
+                l ? &info.l_flags : &no_flags, l ? &info.l_items : nullptr};
+  require(!pt.mnw->empty(), "the tree has no plan: call pack_schedule and kernel_info.to_gpu first");
+  if (info.whole_seqs && !info.ws_q_table.empty()) {
+    // a small batch of short requests: one work item per request, one kernel (see KernelInfo::whole_seqs)
+    PlanTables ws{&info.ws_q_table, &info.ws_block_table, &info.ws_num_seqs, &info.ws_rank, &info.ws_kv, nullptr,
+                  &info.ws_mnw, &no_flags};
+    L = prepare(q, k, v, info.ws_num_split, ws, 1, 1, info.ws_width, scale, out, lse, info.records, version);
+  } else {
+    L = prepare(q, k, v, info.num_boxes_per_seq, pt, info.max_boxes, info.max_seqs, info.max_blocks, scale, out, lse,
+                info.records, version, info.items_hold());
+  }
+  if (info.cache.size() >= 256) info.cache.clear();
+  info.cache[key.bytes] = L;
+  return L;
+}
+
 void fwd_tree(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, PrefixTreeCPP& tree, double scale,
               const at::Tensor& out, const std::optional<at::Tensor>& lse) {
   require(k.is_cuda(), "kcache must be on CUDA");
   require(v.is_cuda(), "vcache must be on CUDA");
   DeviceScope scope(q);
-  KernelInfo& info = *tree.info;
   Key key;
   key.tensor(q); key.tensor(k); key.tensor(v); key.tensor(out); key.add(scale);
   key.add(lse.has_value()); if (lse.has_value()) key.tensor(*lse);
-  std::shared_ptr<Prepared> L;
-  const int64_t version = info.plan_version();
+  KernelInfo& info = *tree.info;
   auto it = info.cache.find(key.bytes);
-  if (it != info.cache.end()) {
-    L = it->second;   // (run() takes a new snapshot when the plan tables were edited in place since)
-  } else {
-    const bool l = info.has_launch;
-    const std::vector<int> no_flags;
-    // partial results are filed by slot_tables: the launch merges each sequence's boxes of THIS plan
-    // (num_split_per_seq counts on over repeated pack_schedule calls)
-    PlanTables pt{l ? &info.l_q_tables : &info.q_tables, l ? &info.l_block_tables : &info.block_tables,
-                  l ? &info.l_num_seqs : &info.num_seqs, l ? &info.l_ranks : &info.ranks, l ? &info.l_kvs : &info.kvs,
-                  l ? &info.l_slot_tables : &info.slot_tables, l ? &info.l_mnws : &info.mnws,
-                  l ? &info.l_flags : &no_flags, l ? &info.l_items : nullptr};
-    require(!pt.mnw->empty(), "the tree has no plan: call pack_schedule and kernel_info.to_gpu first");
-    if (info.whole_seqs && !info.ws_q_table.empty()) {
-      // a small batch of short requests: one work item per request, one kernel (see KernelInfo::whole_seqs)
-      PlanTables ws{&info.ws_q_table, &info.ws_block_table, &info.ws_num_seqs, &info.ws_rank, &info.ws_kv, nullptr,
-                    &info.ws_mnw, &no_flags};
-      L = prepare(q, k, v, info.ws_num_split, ws, 1, 1, info.ws_width, scale, out, lse, info.records, version);
-    } else {
-      L = prepare(q, k, v, info.num_boxes_per_seq, pt, info.max_boxes, info.max_seqs, info.max_blocks, scale, out, lse,
-                  info.records, version, info.items_hold());
-    }
-    if (info.cache.size() >= 256) info.cache.clear();
-    info.cache[key.bytes] = L;
-  }
-  run(*L, info.records, version, q.device(), info.items_hold());
+  // (run() takes a new snapshot when the plan tables were edited in place since)
+  const std::shared_ptr<Prepared> L = it != info.cache.end() ? it->second : prepare_tree(q, k, v, tree, scale, out, lse, key);
+  run(*L, info.records, info.plan_version(), q.device(), info.items_hold());
+}
+
+// The tree form on a serving engine's tensors: query and output [tokens, heads, d], K and V the first two of the cache's leading
+// axis. The key is the one that fwd_tree makes of the views, which exist only where a launch is prepared: four views made and
+// dropped per layer were 4.4 us of a call's 10 on the host. False: not tensors of these forms; the caller makes the views.
+bool decode_attention(const at::Tensor& query, const at::Tensor& kv, PrefixTreeCPP& tree, double scale, const at::Tensor& output) {
+  if (query.dim() != 3 || output.dim() != 3 || kv.dim() != 5 || kv.size(0) < 2 || !kv.is_cuda() || !query.is_cuda() || !output.is_cuda() ||
+      query.numel() == 0 || output.numel() == 0 || kv.numel() == 0)
+    return false;
+  DeviceScope scope(query);
+  Key key;
+  auto rows = [&](const at::Tensor& t) {   // t.unsqueeze(1)
+    key.view(t.data_ptr(), t, {t.size(0), 1, t.size(1), t.size(2)}, {t.stride(0), t.size(1) * t.stride(1), t.stride(1), t.stride(2)});
+  };
+  auto half = [&](int i) {                 // kv[i]
+    key.view(static_cast<const char*>(kv.data_ptr()) + i * kv.stride(0) * (int64_t)kv.element_size(), kv,
+             {kv.size(1), kv.size(2), kv.size(3), kv.size(4)}, {kv.stride(1), kv.stride(2), kv.stride(3), kv.stride(4)});
+  };
+  rows(query); half(0); half(1); rows(output);
+  key.add(scale);
+  key.add(false);
+  KernelInfo& info = *tree.info;
+  auto it = info.cache.find(key.bytes);
+  const std::shared_ptr<Prepared> L = it != info.cache.end()
+      ? it->second
+      : prepare_tree(query.unsqueeze(1), kv.select(0, 0), kv.select(0, 1), tree, scale, output.unsqueeze(1), std::nullopt, key);
+  run(*L, info.records, info.plan_version(), query.device(), info.items_hold());
+  return true;
 }
 
 void paged_decode_baseline(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& block_table,
@@ -1199,6 +1238,10 @@ PYBIND11_MODULE(_prefix_attn, m) {
   m.def("prefix_attn_with_kvcache", &fwd_tree, py::arg("q"), py::arg("k_cache_paged"), py::arg("v_cache_paged"),
         py::arg("tree"), py::arg("softmax_scale"), py::arg("out"), py::kw_only(), py::arg("softmax_lse") = py::none(),
         "Tree form: the plan of a PrefixTreeCPP whose kernel_info is on the device.");
+  m.def("decode_attention", &decode_attention, py::arg("query"), py::arg("kv_cache"), py::arg("tree"), py::arg("softmax_scale"),
+        py::arg("output"),
+        "The tree form on query / output [tokens, heads, d] and a cache [2, blocks, page, kv_heads, d]; False (nothing launched) "
+        "where the tensors have other forms.");
   m.def("invalidate_plans", [] {
           std::lock_guard<std::mutex> lock(g_table_mutex);
           g_table_launches.clear();

@@ -34,6 +34,7 @@ import numpy as np
 import torch
 
 from ._prefix_attn import PrefixTreeCPP, prefix_attn_with_kvcache
+from ._prefix_attn import decode_attention as _decode_attention
 from .async_tree import AsyncTree
 
 __all__ = ["DecodePlan", "decode_attention"]
@@ -221,8 +222,14 @@ def decode_attention(decode_query: torch.Tensor, kv_cache: torch.Tensor, plan: D
     kv_cache: [2, num_blocks, block_size, num_kv_heads, head_size]. Writes and returns decode_output."""
     assert plan.max_decode_query_len <= 1, \
         "Speculative decoding with variable length queries is not supported yet."
-    key_cache, value_cache = kv_cache[0], kv_cache[1]
     tree = plan.tree.tree if isinstance(plan.tree, AsyncTree) else plan.tree
+    # Where a batch is small a step's layers are bound by the host, and the views below are near half of a call there (24 layers
+    # of 2 requests: 16.5 us a layer with them): plain tensors go to the extension as they are, which keys its prepared launches
+    # on the views without making them. Anything else, subclasses among it, takes the views.
+    if type(decode_query) is type(kv_cache) is type(decode_output) is torch.Tensor and \
+            _decode_attention(decode_query, kv_cache, tree, softmax_scale, decode_output):
+        return decode_output
+    key_cache, value_cache = kv_cache[0], kv_cache[1]
     prefix_attn_with_kvcache(q=decode_query.unsqueeze(1), k_cache_paged=key_cache, v_cache_paged=value_cache,
                              tree=tree, softmax_scale=softmax_scale, out=decode_output.unsqueeze(1))
     return decode_output

@@ -8,6 +8,7 @@ import torch
 
 from oracle import attn_oracle as ao
 from pat_amd import PrefixTree, workloads
+from pat_amd import prefix_attn_with_kvcache
 from pat_amd.vllm_decode import DecodePlan, decode_attention
 from conftest import plan_fields
 
@@ -381,3 +382,42 @@ def test_next_step_plan_from_the_previous_tree_equals_a_fresh_one():
         for name in ("q_tables", "num_seqs_per_CTAs", "CTA_ranks", "kv_in_CTAs", "block_tables"):
             for x, y in zip(getattr(got, name), getattr(want, name)):
                 assert torch.equal(x, y), (step, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "strided query and output", "three planes, every second page", "tuple", "subclass", "transposed planes"])
+def test_decode_attention_on_tensors_as_they_are(form):
+    # without views of its own or with them, the same launch (one entry in the plan's cache) and the same bits as the tree form
+    print(f"[case] decode on tensors as they are: {form}", flush=True)
+    dev = torch.device("cuda:0")
+    w = workloads.make("c2", seed=6)
+    q, k, v = w.tensors(dev)
+    q = q.squeeze(1)
+    scale = 1.0 / math.sqrt(w.head_dim)
+    kv_cache, query, output = torch.stack([k, v]), q.contiguous(), torch.full_like(q, float("nan")).contiguous()
+    if form == "strided query and output":
+        query = torch.cat([q, q + 1, q], dim=1)[:, :w.heads]                 # a slice of fused projections
+        output = torch.full((w.batch, w.heads + 2, w.head_dim + 8), float("nan"), dtype=q.dtype, device=dev)[:, 1:-1, :w.head_dim]
+    elif form == "three planes, every second page":
+        wide = torch.zeros(3, 2 * k.shape[0], *k.shape[1:], dtype=k.dtype, device=dev)
+        kv_cache = wide[:, ::2]
+        kv_cache[0], kv_cache[1] = k, v
+    elif form == "tuple":
+        kv_cache = (k, v)
+    elif form == "subclass":
+        kv_cache = kv_cache.as_subclass(type("Cache", (torch.Tensor,), {}))
+    elif form == "transposed planes":
+        kv_cache = torch.stack([k, v], dim=1).transpose(0, 1)                # [2, blocks, ...] over [blocks, 2, ...] in memory
+    plan = DecodePlan.from_metadata(fake_metadata(w, dev))
+    tree = plan.tree.tree
+    assert decode_attention(query, kv_cache, plan, scale, output) is output
+    views_out = output.clone()
+    output.fill_(float("nan"))
+    prefix_attn_with_kvcache(query.unsqueeze(1), kv_cache[0], kv_cache[1], tree, scale, output.unsqueeze(1))
+    torch.cuda.synchronize()
+    assert len(tree.kernel_info._launch_geometries) == 1
+    assert torch.equal(output, views_out)
+    ref, _ = ao.paged_attention_ref(q.unsqueeze(1).cpu(), k.cpu(), v.cpu(), w.rows, w.seq_lens)
+    assert (output.unsqueeze(1).float().cpu() - ref.float()).abs().max().item() <= 1.6e-2
+    with pytest.raises(RuntimeError, match="same dtype"):
+        decode_attention(query.to(torch.float16), kv_cache, plan, scale, output)
