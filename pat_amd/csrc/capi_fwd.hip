@@ -401,6 +401,21 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
         g->total_wgs -= (int64_t)a->buckets[i].num_boxes * (a->kv_heads - a->kv_heads / kWaves);
       }
     }
+    // Boxes of four steps and more that are less than a workgroup per CU go back to four waves where the launch is resident all the
+    // same: places are not short there, and the chain of a lone wave, four times as long, is what the launch ends on. us per call,
+    // a head per wave / four waves: one request of 3424..5120 tokens in 24 boxes of up to 272 and 3 of 128 at 16/8 heads 13.8 / 10.9, one box of 192
+    // tokens beside 206 of 71 at 8/8 18.7 / 15.3, one of 128 beside 33 of up to 768 at 8/8 20.8 / 17.9, two of 112 beside 17 of up to 352 at 16/8,
+    // head_dim 64, 11.0 / 9.4; 15 of 128 at 8/8, 14 of 128 at 16/16, 2 of 112 beside 10 of up to 1920 +-1 %. Not three steps (31 of 96
+    // at 32/8, head_dim 64, 21.2 / 21.7, 23 of 96 at 8/8 9.3 / 9.5), and not where four waves make the launch
+    // queue (17 of 192 beside 640 tall workgroups 77.3 / 79.5; 7 of 144 ahead of 215 of 48 17.3 / 17.8).
+    for (int i = 0; i < a->num_buckets && tune.head_per_wave_tokens < 0; ++i) {
+      const int64_t boxes = a->buckets[i].num_boxes, more = boxes * (a->kv_heads - a->kv_heads / kWaves);
+      if (g->bucket_heads_per_wg[i] == kWaves && (int64_t)a->buckets[i].max_blocks * page > 3 * kStepTokens &&
+          boxes * a->kv_heads <= kNumCUs && g->total_wgs + more <= resident) {
+        g->bucket_heads_per_wg[i] = 1;
+        g->total_wgs += more;
+      }
+    }
   }
   // Long boxes of <= 16 rows in launches far past what the device holds at once: a kv head per
   // wave there too, on chunks of kLongHeadPerWaveChunk tokens. The 4 waves of a workgroup then read

@@ -1562,3 +1562,24 @@ def test_merge_of_more_slots_than_a_workgroup_looks_at_at_once(tuning, monkeypat
     torch.cuda.synchronize()
     assert tree.kernel_info._launch_geometries[0]["num_slots"] > 512
     _assert_close("over 512 slots", out, lse, *_oracle(w, q, k, v), w.dtype)
+
+
+@pytest.mark.parametrize("boxes,tail,heads,d,dtype", [
+    (206, 192, (8, 8), 128, torch.float16),     # one long box (the request that the tall boxes leave over) beside many short ones
+    (24, 128, (16, 8), 128, torch.bfloat16),    # a few of the widest size that runs a kv head per wave in a resident launch ...
+    (24, 112, (16, 8), 64, torch.float16),      # ... a step that is half full
+    (33, 113, (32, 32), 64, torch.bfloat16),    # 32 of them would be more than a workgroup per CU
+])
+def test_few_boxes_of_several_steps(boxes, tail, heads, d, dtype, monkeypatch):
+    # (whichever of the two forms these take: a request with `tail` tokens of its own among requests with 300 or 71)
+    print(f"[case] few boxes of several steps, {boxes} x {tail}, heads {heads}, d {d}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    tails = [tail] * (boxes // 8 if boxes < 100 else 1) + [300 if boxes < 100 else 71] * boxes
+    rows, nxt = [], 20
+    for n in tails:
+        rows.append(list(range(20)) + list(range(nxt, nxt + -(-n // 16))))
+        nxt += -(-n // 16)
+    w = workloads.Workload("few", heads[0], heads[1], d, dtype, 16, [320 + n for n in tails], rows, nxt, 0, 4)
+    q, k, v = w.tensors(dev)
+    _assert_close("few", *_run_tree(w, q, k, v), *_oracle(w, q, k, v), dtype)

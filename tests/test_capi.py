@@ -411,3 +411,18 @@ def test_boxes_of_one_request_each_walked_whole_or_cut(boxes, tokens, heads, kv_
     a.max_split_per_seq = 1
     assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
     assert (g.num_slots == 1) == whole, g.num_slots
+
+
+@pytest.mark.parametrize("buckets,heads,kv_heads,d,workgroups", [
+    ([(16, 24, 1, 272, 0, 0), (16, 3, 1, 128, 0, 0)], 16, 8, 128, 600),                                  # 24 WGs on four waves each, 6 on a head per wave
+    ([(16, 24, 1, 272, 0, 0), (16, 3, 1, 96, 0, 0)], 16, 8, 128, 582),                                   # three steps: a head per wave
+    ([(64, 3, 64, 192, 0, 0), (16, 1, 1, 192, 0, 0), (16, 206, 1, 80, 0, 0)], 8, 8, 128, 444),
+    ([(64, 1, 32, 1696, 0, 0), (32, 2, 16, 480, 0, 0), (16, 23, 1, 256, 0, 0), (16, 8, 1, 128, 0, 0), (16, 2, 1, 64, 0, 0)], 16, 8, 128, 476),   # would queue
+])
+def test_few_boxes_of_several_steps_stay_on_four_waves(buckets, heads, kv_heads, d, workgroups):
+    # ... in launches that are resident all the same
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    a = _bucket_args(buckets, heads, kv_heads, d, 25, 16)
+    a.max_split_per_seq = 4
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+    assert g.num_workgroups == workgroups, (g.num_workgroups, g.tall_rows)
