@@ -334,17 +334,14 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
       if (a->buckets[i].num_boxes > 0) widest = std::max<int64_t>(widest, (int64_t)a->buckets[i].max_blocks * page);
     int64_t boxes = 0;
     for (int i = 0; i < a->num_buckets; ++i) boxes += a->buckets[i].num_boxes;
-    // With fewer boxes than one per CU and kv head, cutting them is what fills the device, and costs the second launch, its
-    // round trips and the partial rows. From 120 batches of 1..50 requests, us: a box walked whole by its workgroup's four
-    // waves, n rounds of 128 tokens, 3.5 + 1.15 n (head_dim 64: 2.2 + 0.9 n); cut 8.5 and 0.06 more per MB of K and V and 1.5
-    // per 1000 rows. (cut / whole: 24 requests of 432..638 tokens at 32/8 heads 15.3 / 11.6, 23 of 432..718 at 8/8 15.6 / 12.4,
-    // 16 of 600..800 13.6 / 11.1, 22 of 1135 at 64/8 23.4 / 17.9, 2 of 416..654 at 64/8, head_dim 64, 8.7 / 7.5, 26 of 614 at
-    // 8/8, 64, 10.0 / 7.6; past the line: 9 of 687..732 at 16/8 8.7 / 10.7, 8 of 864..1318 at 16/16 16.7 / 17.4.)
-    const double rounds = (double)ceil_div64(widest, kWaves * kStepTokens);
-    const double whole_us = a->head_dim == 64 ? 2.2 + 0.9 * rounds : 3.5 + 1.15 * rounds;
-    const double cut_us = 8.5 + 0.06e-6 * short_bytes(a) + 0.0015 * a->batch * a->heads;
+    // (with fewer boxes than one per CU and kv head, cutting them is what fills the device - unless they are so
+    // short that a workgroup's four waves walk a whole box in a few steps each: then the second launch and its
+    // round trips cost more than the cuts save; 8 requests of 288 tokens, 8 kv heads: 7.6 -> 5 us. Longer ones can be faster
+    // whole too (24 requests of 432..638 tokens at 32/8 heads 15.3 -> 11.6), but they are less exact: a probability is rounded
+    // to 16 bits against the largest score among the tokens of its wave and piece, and fewer, longer runs round worse. Against
+    // 64 bits, nine batches of 330..816 tokens were 2-5 % further off whole than cut, in both types)
     if (widest > 0 && round_unit(widest) <= std::min<int64_t>(cap, kMaxChunk) &&
-        (boxes * a->kv_heads >= kNumCUs || widest <= kSmallLaunchTokens || whole_us <= cut_us)) {
+        (boxes * a->kv_heads >= kNumCUs || widest <= kSmallLaunchTokens)) {
       chunk = std::max(chunk, widest);
       tall = std::max(tall, widest);
       single_slot = true;

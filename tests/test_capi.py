@@ -400,14 +400,18 @@ def test_static_launch_that_only_fits_box_by_box_is_not_refused():
     assert lib.pat_fwd_launch_static(C.byref(a), None) == _lib.PAT_ERR_HIP      # (got past the check: there is no GPU here)
 
 
-@pytest.mark.parametrize("boxes,tokens,heads,kv_heads,d,whole", [
-    (24, 640, 32, 8, 128, True), (27, 768, 64, 8, 128, True), (26, 624, 8, 8, 64, True), (3, 736, 16, 8, 128, False),
-    (64, 2048, 32, 8, 128, True), (8, 1344, 16, 16, 128, False), (1, 4096, 32, 8, 128, False),
+@pytest.mark.parametrize("tile,boxes,seqs,tokens,heads,kv_heads,d,even,whole", [
+    (16, 24, 1, 640, 32, 8, 128, True, False), (16, 27, 1, 768, 64, 8, 128, True, False), (16, 26, 1, 624, 8, 8, 64, True, False),
+    (16, 20, 1, 896, 16, 8, 128, False, False), (16, 30, 1, 1152, 8, 8, 128, False, False), (16, 31, 1, 896, 16, 8, 128, False, False),   # ragged: one long box, maybe
+    (64, 1, 16, 640, 32, 8, 128, True, False), (64, 30, 8, 1920, 64, 8, 128, True, False), (64, 28, 8, 1536, 64, 8, 128, True, False),   # requests with one table
+    (16, 3, 1, 736, 16, 8, 128, True, False), (16, 8, 1, 1344, 16, 16, 128, True, False), (16, 1, 1, 4096, 32, 8, 128, True, False),
+    (16, 64, 1, 2048, 32, 8, 128, True, True), (16, 8, 1, 512, 8, 8, 128, True, True), (16, 32, 1, 1152, 8, 8, 128, False, True),
 ])
-def test_boxes_of_one_request_each_walked_whole_or_cut(boxes, tokens, heads, kv_heads, d, whole):
-    # one slot a row, written by the split kernel, where that costs less than pieces and a second kernel
+def test_boxes_of_one_request_each_walked_whole_or_cut(tile, boxes, seqs, tokens, heads, kv_heads, d, even, whole):
+    # one slot a row, written by the split kernel, for short boxes and where there is one per CU and kv head; longer ones of small
+    # launches are cut, whatever their rows and whether or not the bucket is even
     lib, g = _lib.load(), _lib.FwdGeometry()
-    a = _bucket_args([(16, boxes, 1, tokens, 0, 0)], heads, kv_heads, d, boxes, 16)
+    a = _bucket_args([(tile, boxes, seqs, tokens, _lib.PAT_BUCKET_EVEN if even else 0, 0)], heads, kv_heads, d, boxes * seqs, 16)
     a.max_split_per_seq = 1
     assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
     assert (g.num_slots == 1) == whole, g.num_slots
