@@ -56,8 +56,12 @@ pat_fwd_tuning env_tuning() {
   t.chunk_tokens = 0; t.tall_chunk_tokens = 0; t.head_per_wave_tokens = -1;
   t.head_per_wave_long_wgs = -1; t.head_per_wave_long_tokens = 0; t.equalize_chunks = -1; t.direct_out = -1;
   t.tall_rows = 0; t.pairs = 0;
-  if (const char* e = std::getenv("PAT_PAIRS")) t.pairs = std::atoi(e);
-  if (const char* e = std::getenv("PAT_STREAM_V")) t.pairs |= std::atoi(e) == 1 ? PAT_STREAM_V_ALWAYS : std::atoi(e) == 2 ? PAT_STREAM_V_NEVER : 0;
+  auto one_or_two = [](const char* name) {   // (anything else: automatic)
+    const char* e = std::getenv(name);
+    const int v = e ? std::atoi(e) : 0;
+    return v == 1 || v == 2 ? v : 0;
+  };
+  t.pairs = one_or_two("PAT_PAIRS") | (one_or_two("PAT_STREAM_V") == 1 ? PAT_STREAM_V_ALWAYS : one_or_two("PAT_STREAM_V") == 2 ? PAT_STREAM_V_NEVER : 0);
   if (const char* e = std::getenv("PAT_TALL_ROWS")) t.tall_rows = std::atoi(e);
   if (const char* e = std::getenv("PAT_CHUNK_TOKENS")) t.chunk_tokens = std::atoi(e);
   if (const char* e = std::getenv("PAT_TALL_CHUNK_TOKENS")) t.tall_chunk_tokens = std::atoi(e);
@@ -76,6 +80,11 @@ pat_fwd_tuning tuning() {
   if (!g_tuning_set) { g_tuning = env_tuning(); g_tuning_set = true; }
   return g_tuning;
 }
+
+// The two switches in pat_fwd_tuning.pairs: boxes in twos (0..2), and V past the caches. Values outside the declared bits, -1 among
+// them, ask for neither.
+int pairs_switch(const pat_fwd_tuning& t) { return t.pairs >= 0 && t.pairs < 16 ? t.pairs & 3 : 0; }
+int stream_switch(const pat_fwd_tuning& t) { return t.pairs >= 0 && t.pairs < 16 ? t.pairs & (PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER) : 0; }
 
 // Widest box (tokens) of a bucket whose workgroups serve one kv head per wave (0: mode off).
 int64_t head_per_wave_tokens(const pat_fwd_tuning& t, bool oversubscribed) {
@@ -487,7 +496,8 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
   // on the same caches, find V there: 22 of 1024 (93 MB) 23.0 / 23.1, 20 18.1 / 18.8, 12 13.7 / 14.5 (but 16 layers of 16 of
   // 1024, each with its own, 412 / 394). K stays as it is: a load of its operand layout takes 64 bytes of a row, half a line,
   // and the other half would be fetched again (16 rows' halves per load; with it 837 -> 915 for 32 layers of 89 MB).
-  g->stream_v = !(tune.pairs & PAT_STREAM_V_NEVER) && ((tune.pairs & PAT_STREAM_V_ALWAYS) || short_bytes(a) >= kStreamBytes);
+  const int forced = stream_switch(tune);
+  g->stream_v = !(forced & PAT_STREAM_V_NEVER) && ((forced & PAT_STREAM_V_ALWAYS) || short_bytes(a) >= kStreamBytes);
   g->num_slots = g->chunks_per_rank * a->max_split_per_seq;
   // One slot per row (no sequence in two boxes, no box in two chunks): nothing to merge, the
   // split kernel stores the rows in `out` itself (8-byte stores: needs `out` laid out for them).
@@ -540,7 +550,7 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
     tall_box_heads += (int64_t)b.num_boxes * a->kv_heads;
     pairs = pairs || items_of(b, true) < b.num_boxes;
   }
-  pairs = pairs && (tune.pairs & 3) != 2 && ((tune.pairs & 3) == 1 || tall_box_heads >= 3 * kNumCUs / 8);
+  pairs = pairs && pairs_switch(tune) != 2 && (pairs_switch(tune) == 1 || tall_box_heads >= 3 * kNumCUs / 8);
   // (boxes of more than 64 x kMaxTall32Tokens tokens, which the bound on pieces per box makes longer pieces of, take the 16-row form)
   auto in_32 = [&]() -> int {
     if (int rc = plan_geometry_for(a, g, 32, pairs)) return rc;
@@ -979,7 +989,7 @@ int pat_fwd_launch_static(const pat_fwd_args* args, void* hip_stream) {
   if (need > kStaticScratchBytes && g.pairs && args->records == nullptr) {
     box_by_box = *args;
     tune = args->tuning != nullptr ? *args->tuning : tuning();
-    tune.pairs = (tune.pairs & ~3) | 2;
+    tune.pairs = stream_switch(tune) | 2;
     box_by_box.tuning = &tune;
     args = &box_by_box;
     g = Geometry();

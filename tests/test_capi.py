@@ -430,3 +430,40 @@ def test_few_boxes_of_several_steps_stay_on_four_waves(buckets, heads, kv_heads,
     a.max_split_per_seq = 4
     assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
     assert g.num_workgroups == workgroups, (g.num_workgroups, g.tall_rows)
+
+
+def test_switches_in_one_field_do_not_leak_into_each_other(tuning, monkeypatch):
+    # pat_fwd_tuning.pairs: 0..2, and two bits about V; other values, and other values of the environment variables, are automatic
+    lib, g, t = _lib.load(), _lib.FwdGeometry(), _lib.FwdTuning()
+    items = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS
+
+    def flags(boxes, short):
+        a = _bucket_args([(64, boxes, 8, 2048, items, boxes // 2), (16, 64, 1, short, _lib.PAT_BUCKET_EVEN, 0)], 64, 8, 128, 8 * boxes, 16)
+        a.max_split_per_seq = 2
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        return bool(g.flags & _lib.PAT_GEOMETRY_PAIRS), bool(g.flags & _lib.PAT_GEOMETRY_STREAM_V)
+
+    tuning(pairs=0)
+    large, small = flags(16, 2048), flags(4, 64)      # (pairs and V past the caches pay, neither does)
+    assert large == (True, True) and small == (False, False)
+    for value in (-1, -2, -3, 3, 16, 17, 18, 20, 1 << 30):
+        tuning(pairs=value)
+        assert (flags(16, 2048), flags(4, 64)) == (large, small), value
+    tuning(pairs=2 | _lib.PAT_STREAM_V_NEVER)
+    assert flags(16, 2048) == (False, False)
+    tuning(pairs=1 | _lib.PAT_STREAM_V_ALWAYS)
+    assert flags(4, 64) == (True, True)
+    for pairs, stream, want in (("1", "2", 1 | 8), ("4", "", 0), ("8", "1", 4), ("-1", "", 0), ("7", "3", 0), ("2", "1", 2 | 4)):
+        monkeypatch.setenv("PAT_PAIRS", pairs)
+        monkeypatch.setenv("PAT_STREAM_V", stream)
+        assert lib.pat_fwd_set_tuning(None) == 0 and lib.pat_fwd_get_tuning(C.byref(t)) == 0
+        assert t.pairs == want, (pairs, stream)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="would launch on fake addresses")
+def test_static_launch_box_by_box_with_the_switch_out_of_range(tuning):
+    # the second geometry, without boxes in twos, is asked for by a value of its own: -1 with two bits replaced would be automatic again
+    lib = _lib.load()
+    tuning(pairs=-1)
+    a = _bucket_args([(64, 8, 64, 7744, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS, 4), (16, 482, 1, 64, 0, 0)], 32, 32, 128, 482, 64)
+    assert lib.pat_fwd_launch_static(C.byref(a), None) == _lib.PAT_ERR_HIP      # (past the check of the size: there is no GPU here)
