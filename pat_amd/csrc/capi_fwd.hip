@@ -104,7 +104,8 @@ struct Geometry {
   int tall_rows = 32;        // rows per wave on boxes of 17..64 rows: 32 or 16 (the split kernel's instance)
   bool tall_apart = false;   // 32-row form: K and V tiles handed over apart
   bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
-  bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches
+  bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches ...
+  int stream_tokens = -1;    // ... where these boxes hold so many tokens (the record kernel counts)
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
   // launch records (one per workgroup): entries per record and bytes between records
   int record_max_seqs = 0, record_max_pages = 0, record_stride = 0;
@@ -489,15 +490,19 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     g->tall_apart = n_tall <= kNumCUs && longest >= kApartTokens;
   }
   // Reading V past the caches (non-temporal loads, the pieces that one box alone reads: the record kernel looks). A launch
-  // whose K and V exceed a third of the 256 MB memory-side cache finds little of them there at its next call, and V's lines,
-  // kept like K's, only push out K's, the shared pages and the partial rows. us per call, kept / past the caches: 32 requests
-  // of 4096 tokens at 64/8 heads (537 MB) 94.5 / 85.0, three levels of 128 (336 MB) 71.0 / 66.7, 1024 over 512 + 100..200 at
-  // 16/2 46.1 / 40.0, 32 of 1024 at 32/8 (134 MB) 26.0 / 22.6, 24 (101 MB) 24.4 / 23.5; below the line the same calls, repeated
-  // on the same caches, find V there: 22 of 1024 (93 MB) 23.0 / 23.1, 20 18.1 / 18.8, 12 13.7 / 14.5 (but 16 layers of 16 of
-  // 1024, each with its own, 412 / 394). K stays as it is: a load of its operand layout takes 64 bytes of a row, half a line,
-  // and the other half would be fetched again (16 rows' halves per load; with it 837 -> 915 for 32 layers of 89 MB).
+  // whose K and V exceed a third of the 256 MB memory-side cache finds little of them there when two others ran in between, as
+  // a model's layers do, each on K and V of its own, and V's lines, kept like K's, only push out K's, the shared pages and the
+  // partial rows. us per call on three caches in turn, kept / past the caches: 32 requests of 4096 tokens at 64/8 heads (537 MB)
+  // 95.1 / 85.6, 72 of 1024 at 32/8 (302 MB) 63.0 / 59.5, 40 (168 MB) 39.8 / 34.6, 28 (117 MB) 27.0 / 23.9; below the line three caches'
+  // V stays: 12 of 327..1516 at 32/32 (83 MB) 19.9 / 21.8. A program that repeats one call on one cache finds V there up to
+  // ~250 MB: 28 of 1024 22.9 / 24.3, 40 31.6 / 34.5, 56 (235 MB) 36.5 / 38.4, but 72 56.5 / 53.4.
+  // Widths decide here whether the launch is worth a look; how much there is the record kernel counts (holds_tokens): by
+  // widths alone one request of 4096 tokens among 31 of 512, 82 MB, passed for 322 and took 55.0 us in place of 46.7.
+  // K stays as it is: a load of its operand layout takes 64 bytes of a row, half a line, and the other half would be fetched
+  // again (16 rows' halves per load; with it 837 -> 915 for 32 layers of 89 MB).
   const int forced = stream_switch(tune);
   g->stream_v = !(forced & PAT_STREAM_V_NEVER) && ((forced & PAT_STREAM_V_ALWAYS) || short_bytes(a) >= kStreamBytes);
+  if (g->stream_v) g->stream_tokens = (forced & PAT_STREAM_V_ALWAYS) ? 0 : (int)std::ceil(kStreamBytes / ((double)a->kv_heads * a->head_dim * 4.));
   g->num_slots = g->chunks_per_rank * a->max_split_per_seq;
   // One slot per row (no sequence in two boxes, no box in two chunks): nothing to merge, the
   // split kernel stores the rows in `out` itself (8-byte stores: needs `out` laid out for them).
@@ -595,7 +600,7 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
   uint64_t h = 0x9e3779b97f4a7c15ull;
   auto mix = [&](uint64_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); };
   mix((uint64_t)g.tall_rows); mix((uint64_t)g.total_wgs); mix((uint64_t)g.record_stride); mix((uint64_t)g.record_max_seqs); mix((uint64_t)g.record_max_pages);
-  mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0); mix(g.stream_v ? 1 : 0);
+  mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0); mix((uint64_t)(g.stream_tokens + 1));
   mix((uint64_t)a->batch); mix((uint64_t)a->heads); mix((uint64_t)a->kv_heads); mix((uint64_t)a->page_size);
   mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq); mix(g.pairs ? 1 : 0);
   for (int i = 0; i < a->num_buckets; ++i) {
@@ -651,9 +656,45 @@ namespace pat {
 namespace {
 
 // ---- launch records ------------------------------------------------------------------------------
+// Tokens that the boxes of <= 16 rows hold between them, what a box has in common with the next one of its bucket counted once
+// (boxes over the same blocks lie next to each other): the host knows widths only, and one long box among many short ones, or
+// requests over one prefix with a box each, are many times fewer tokens than boxes x width. In common is judged by the pages at
+// 1/8, 3/8, 5/8 and 7/8 of the box; of more than kCounted boxes every second, third ... is looked at. Every workgroup counts for
+// itself: two round trips per bucket, 3 to 6 us of a kernel that runs once per plan.
+constexpr int kCounted = 256;
+__device__ bool holds_tokens(const RecordParams& p, int64_t least) {
+  __shared__ unsigned long long s_eighths[4];
+  unsigned long long eighths = 0;
+  for (int b = 0; b < p.num_buckets; ++b) {
+    const RecordBucket& bk = p.bucket[b];
+    if (bk.row_tiles != 1) continue;
+    const int step = (bk.num_boxes + kCounted - 1) / kCounted, cap = bk.max_blocks * p.page_size;
+    for (int64_t at = (int64_t)threadIdx.x * step; at < bk.num_boxes; at += 256 * (int64_t)step) {
+      const int box = (int)at, next = box + 1 < bk.num_boxes ? box + 1 : 0;
+      const int kv = min(bk.kv[box], cap), kv_next = next != box ? bk.kv[next] : 0;
+      if (kv <= 0) continue;
+      const int32_t* row = bk.block_table + (int64_t)box * bk.bt_stride;
+      const int32_t* row_next = bk.block_table + (int64_t)next * bk.bt_stride;
+      int own = 0;
+#pragma unroll
+      for (int i = 1; i < 8; i += 2) {
+        const int page = (int)((int64_t)kv * i / 8) / p.page_size;
+        own += (kv_next > page * p.page_size && row_next[page] == row[page]) ? 0 : 2;
+      }
+      eighths += (unsigned long long)kv * own * step;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) eighths += __shfl_xor(eighths, off);
+  if ((threadIdx.x & 63) == 0) s_eighths[threadIdx.x >> 6] = eighths;
+  __syncthreads();
+  return (s_eighths[0] + s_eighths[1] + s_eighths[2] + s_eighths[3]) / 8 >= (unsigned long long)least;
+}
+
 // One wave per record: decodes which (bucket, box, chunk, kv head group) the workgroup is, reads
 // the box's plan entries, checks and clamps them, and lays them out for the split kernel.
 __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
+  const bool launch_streams = p.stream_tokens >= 0 && holds_tokens(p, p.stream_tokens);   // (ahead of the returns: it has a barrier)
   const int lane = threadIdx.x & 63;
   const int wg = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (wg >= p.grid_items) return;
@@ -708,7 +749,7 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
   // a request a few shared pages at its head would keep all of it in the caches (48 requests of 805..3752 tokens, 384 of them
   // shared, 16 heads of 64: 103 us by the first page, 80 by the middle one).
   bool stream = false;
-  if (p.stream_v && bk.row_tiles == 1 && tokens > 0) {
+  if (launch_streams && bk.row_tiles == 1 && tokens > 0) {
     const int at = (t_begin + tokens / 2) / page;
     const int id = bk.block_table[(int64_t)box * bk.bt_stride + at];
     int other = box + 1 + lane;
@@ -764,7 +805,7 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   rp.record_stride = g.record_stride; rp.record_max_seqs = g.record_max_seqs; rp.record_max_pages = g.record_max_pages;
   rp.batch = args->batch; rp.kv_heads = args->kv_heads; rp.group = args->heads / args->kv_heads;
   rp.page_size = args->page_size; rp.num_pages = args->num_pages;
-  rp.chunks_per_rank = g.chunks_per_rank; rp.max_split = args->max_split_per_seq; rp.stream_v = g.stream_v ? 1 : 0;
+  rp.chunks_per_rank = g.chunks_per_rank; rp.max_split = args->max_split_per_seq; rp.stream_tokens = g.stream_tokens;
   // buckets in plan order (tall, long boxes come first in the default order)
   int nb = 0;
   int64_t items = 0;

@@ -108,7 +108,8 @@ struct RecordParams {
   int32_t batch, kv_heads, group, page_size, num_pages;
   int32_t chunks_per_rank;  // slots reserved per box ordinal
   int32_t max_split;
-  int32_t stream_v;         // V tiles of pieces that no other box reads go past the caches (kRecordModeStreamV)
+  int32_t stream_tokens;    // V tiles of pieces that no other box reads go past the caches (kRecordModeStreamV) where the boxes of
+                            // <= 16 rows hold so many tokens between them; negative: nowhere
   RecordBucket bucket[kMaxBuckets];
 };
 

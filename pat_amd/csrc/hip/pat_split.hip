@@ -841,7 +841,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       for (; st + stride < nsteps; st += stride) step(st, std::true_type{});
       step(st, std::false_type{});
     };
-    // (V past the caches: the host's choice for launches of ~100 MB and more, there 4-20 % faster. A loop of its own: inside one
+    // (V past the caches: for launches of 92 MB and more, the records say which pieces; 1-15 % faster there. A loop of its own: inside one
     // loop the two kinds of load are either merged, without the hint, or cost 3 % as a branch; and a branch known to be uniform
     // costs 28 spilled registers, like uniform loop bounds above)
     if (step0 < nsteps) {

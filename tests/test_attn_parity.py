@@ -1583,3 +1583,89 @@ def test_few_boxes_of_several_steps(boxes, tail, heads, d, dtype, monkeypatch):
     w = workloads.Workload("few", heads[0], heads[1], d, dtype, 16, [320 + n for n in tails], rows, nxt, 0, 4)
     q, k, v = w.tensors(dev)
     _assert_close("few", *_run_tree(w, q, k, v), *_oracle(w, q, k, v), dtype)
+
+
+def _stream_records(lens, rows, heads, kv_heads, d, flags=0):
+    """The launch records of one box per request over these blocks: per workgroup (box, first token, tokens, V past the caches)."""
+    import ctypes as C
+    from pat_amd import _ctypes_launch, _lib
+    dev, n, page = _device(), len(lens), 16
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)   # noqa: E731
+    table = torch.zeros(n, max(len(r) for r in rows), dtype=torch.int32)
+    for i, r in enumerate(rows):
+        table[i, :len(r)] = torch.tensor(r, dtype=torch.int32)
+    q = torch.zeros(n, 1, heads, d, dtype=torch.float16, device=dev)
+    k, v = torch.zeros(2, 1 + max(max(r) for r in rows), page, kv_heads, d, dtype=torch.float16, device=dev)
+    L = _ctypes_launch.prepare(q, k, v, i32([1] * n), [i32([[i] for i in range(n)])], [table.to(dev)], [i32([1] * n)], [i32([0] * n)],
+                               [i32(lens)], [[16, 128, 1]], 1, 1, table.shape[1], 1.0, torch.empty_like(q), None, bucket_flags=[flags])
+    g = _lib.FwdGeometry()
+    assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(g)) == 0
+    torch.cuda.synchronize()
+    words = L.keep[8].cpu().view(torch.int32)
+    size = next(s for s in range(64, 1 << 14, 64) if (g.num_workgroups * s + 255) // 256 * 256 >= words.numel() * 4)
+    words = words[:g.num_workgroups * size // 4].view(g.num_workgroups, -1)
+    groups = kv_heads // (4 if int(words[0, 2]) & 0x100 else 1)
+    chunks = g.num_workgroups // (n * groups)
+    assert chunks * n * groups == g.num_workgroups and chunks == g.num_slots
+    piece = -(-table.shape[1] * page // chunks)      # (the widest box in even pieces: sizes here divide)
+    return bool(g.flags & _lib.PAT_GEOMETRY_STREAM_V), \
+        [(w // groups % n, w // groups // n * piece, int(words[w, 0]), bool(int(words[w, 2]) & 0x200)) for w in range(g.num_workgroups)]
+
+
+def _sole_reader(lens, rows, box, first, tokens):
+    at, n = (first + tokens // 2) // 16, len(lens)
+    others = [(box + 1 + i) % n for i in range(min(64, n - 1))]
+    return not any(lens[o] > at * 16 and rows[o][at] == rows[box][at] for o in others)
+
+
+@pytest.mark.parametrize("pieces", [1, 3])
+@pytest.mark.parametrize("kind", ["private", "neighbours", "ends", "heads only"])
+@pytest.mark.parametrize("n", [1, 2, 64, 65, 66])
+def test_which_pieces_are_read_past_the_caches(n, kind, pieces, tuning):
+    # those whose middle page none of the next 64 boxes reads, round the bucket's end
+    print(f"[case] records of {n} boxes, {kind}, {pieces} pieces", flush=True)
+    from pat_amd import _lib
+    lens = [pieces * 256 - (i * 37) % 250 for i in range(n)]
+    lens[0] = pieces * 256
+    rows = [list(range(1000 * i, 1000 * i + 16 * pieces)) for i in range(n)]
+    for i in range(n):
+        if kind == "neighbours" and i % 3 == 1:
+            rows[i] = rows[i - 1]                              # two boxes over the same blocks
+        elif kind == "heads only":
+            rows[i] = rows[0][:2] + rows[i][2:]                # all begin with the same two
+    if kind == "ends":
+        rows[-1] = rows[0]                                     # the last box's next one is the first; the first sees only 64 further
+    rows = [[x % 1000 + 50 * (x // 1000) for x in r] for r in rows]
+    tuning(pairs=_lib.PAT_STREAM_V_ALWAYS, chunk_tokens=256, head_per_wave_tokens=0, head_per_wave_long_wgs=1 << 40)
+    launch, records = _stream_records(lens, rows, 8, 8, 64)
+    assert launch and len(records) == 8 * n * pieces
+    for box, first, tokens, past in records:
+        assert tokens == max(0, min(256, lens[box] - first))
+        assert past == (tokens > 0 and _sole_reader(lens, rows, box, first, tokens)), (box, first, tokens)
+    if n > 1 or kind == "private":
+        assert any(r[3] for r in records) == (kind in ("private", "heads only") or n > 2)
+
+
+@pytest.mark.parametrize("name,lens,shared,flags,launch,past", [
+    # (the line at 8 kv heads of 128: 22461 tokens)
+    ("one long box among short ones", [8192] + [64] * 63, 0, 0, True, False),
+    ("as many tokens as the line asks for", [640] * 64, 0, 0, True, True),
+    ("a few short of it, by whole pages not", [350] * 64, 0, 1, True, False),
+    ("short of it", [330] * 64, 0, 1, False, False),
+    ("a prefix with a box per request", [640] * 64, 304, 0, True, False),      # (their middle pages are their own)
+    ("a short prefix with a box per request", [640] * 64, 80, 0, True, True),
+    ("more boxes than are looked at", [32] * 1500, 0, 0, True, True),
+    ("more boxes than are looked at, nearly empty", [32] * 20 + [1] * 1980, 0, 0, True, False),
+])
+def test_v_is_read_past_the_caches_by_the_tokens_there_are(name, lens, shared, flags, launch, past, tuning):
+    # the host goes by the widest box; the records by what the boxes hold, blocks of several boxes once
+    print(f"[case] records, {name}", flush=True)
+    tuning(pairs=0)
+    rows, nxt = [], shared // 16
+    for t in lens:
+        own = max(0, -(-t // 16) - shared // 16)
+        rows.append((list(range(shared // 16)) + list(range(nxt, nxt + own)))[:-(-t // 16)])
+        nxt += own
+    got, records = _stream_records(lens, rows, 8, 8, 128, flags)
+    assert got == launch
+    assert {r[3] for r in records if r[2] > 0} == {past}
