@@ -1585,8 +1585,9 @@ def test_few_boxes_of_several_steps(boxes, tail, heads, d, dtype, monkeypatch):
     _assert_close("few", *_run_tree(w, q, k, v), *_oracle(w, q, k, v), dtype)
 
 
-def _stream_records(lens, rows, heads, kv_heads, d, flags=0):
-    """The launch records of one box per request over these blocks: per workgroup (box, first token, tokens, V past the caches)."""
+def _stream_records(lens, rows, heads, kv_heads, d, flags=0, tall=()):
+    """The launch records of one box per request over these blocks, behind boxes of 17 of the requests each over `tall` (blocks):
+    per workgroup of the former (box, first token, tokens, V past the caches)."""
     import ctypes as C
     from pat_amd import _ctypes_launch, _lib
     dev, n, page = _device(), len(lens), 16
@@ -1595,21 +1596,31 @@ def _stream_records(lens, rows, heads, kv_heads, d, flags=0):
     for i, r in enumerate(rows):
         table[i, :len(r)] = torch.tensor(r, dtype=torch.int32)
     q = torch.zeros(n, 1, heads, d, dtype=torch.float16, device=dev)
-    k, v = torch.zeros(2, 1 + max(max(r) for r in rows), page, kv_heads, d, dtype=torch.float16, device=dev)
-    L = _ctypes_launch.prepare(q, k, v, i32([1] * n), [i32([[i] for i in range(n)])], [table.to(dev)], [i32([1] * n)], [i32([0] * n)],
-                               [i32(lens)], [[16, 128, 1]], 1, 1, table.shape[1], 1.0, torch.empty_like(q), None, bucket_flags=[flags])
+    k, v = torch.zeros(2, 1 + max(max(r) for r in rows + list(tall)), page, kv_heads, d, dtype=torch.float16, device=dev)
+    q_tables, tables, seqs, ranks, kvs, tiles = [i32([[i] for i in range(n)])], [table.to(dev)], [i32([1] * n)], [i32([0] * n)], [i32(lens)], [16]
+    if tall:
+        t = len(tall)
+        wide = torch.zeros(t, max(len(r) for r in tall), dtype=torch.int32)
+        for i, r in enumerate(tall):
+            wide[i, :len(r)] = torch.tensor(r, dtype=torch.int32)
+        q_tables.insert(0, i32([[(17 * i + j) % n for j in range(17)] for i in range(t)]))
+        tables.insert(0, wide.to(dev)); seqs.insert(0, i32([17] * t)); ranks.insert(0, i32([0] * t))
+        kvs.insert(0, i32([16 * len(r) for r in tall])); tiles.insert(0, 32)
+    L = _ctypes_launch.prepare(q, k, v, i32([1] * n), q_tables, tables, seqs, ranks, kvs, [[m, 128, 1] for m in tiles], 2 if tall else 1,
+                               17 if tall else 1, max(x.shape[1] for x in tables), 1.0, torch.empty_like(q), None, bucket_flags=[flags] * len(tiles))
     g = _lib.FwdGeometry()
     assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(g)) == 0
     torch.cuda.synchronize()
     words = L.keep[8].cpu().view(torch.int32)
     size = next(s for s in range(64, 1 << 14, 64) if (g.num_workgroups * s + 255) // 256 * 256 >= words.numel() * 4)
     words = words[:g.num_workgroups * size // 4].view(g.num_workgroups, -1)
+    words = words[(words[:, 2] & 0xff) == 1]              # (boxes of <= 16 rows; the tall ones come first)
     groups = kv_heads // (4 if int(words[0, 2]) & 0x100 else 1)
-    chunks = g.num_workgroups // (n * groups)
-    assert chunks * n * groups == g.num_workgroups and chunks == g.num_slots
+    chunks = len(words) // (n * groups)
+    assert chunks * n * groups == len(words) and (tall or (chunks == g.num_slots and len(words) == g.num_workgroups))
     piece = -(-table.shape[1] * page // chunks)      # (the widest box in even pieces: sizes here divide)
     return bool(g.flags & _lib.PAT_GEOMETRY_STREAM_V), \
-        [(w // groups % n, w // groups // n * piece, int(words[w, 0]), bool(int(words[w, 2]) & 0x200)) for w in range(g.num_workgroups)]
+        [(w // groups % n, w // groups // n * piece, int(words[w, 0]), bool(int(words[w, 2]) & 0x200)) for w in range(len(words))]
 
 
 def _sole_reader(lens, rows, box, first, tokens):
@@ -1669,3 +1680,22 @@ def test_v_is_read_past_the_caches_by_the_tokens_there_are(name, lens, shared, f
     got, records = _stream_records(lens, rows, 8, 8, 128, flags)
     assert got == launch
     assert {r[3] for r in records if r[2] > 0} == {past}
+
+
+@pytest.mark.parametrize("nodes", [1, 63, 65, 130])
+def test_what_tall_boxes_leave_over_stays_in_the_caches(nodes, tuning):
+    # a box over the blocks of a tall one, anywhere in its bucket, is not read past the caches; a node's shorter copy is no match, nor
+    # are private boxes, one of them longer than any tall box
+    print(f"[case] records of what {nodes} tall boxes leave over", flush=True)
+    from pat_amd import _lib
+    tall = [list(range(16 * i, 16 * i + 16)) for i in range(nodes)]
+    tall[nodes // 2] = tall[nodes // 2][:6]
+    at = 16 * nodes
+    rows = [list(range(16 * i, 16 * i + 16)) for i in range(nodes)]
+    rows += [list(range(at + 32 * i, at + 32 * i + (32 if i == 3 else 1 + i))) for i in range(20)]
+    lens = [16 * len(r) - 3 for r in rows]
+    tuning(pairs=_lib.PAT_STREAM_V_ALWAYS, chunk_tokens=512, head_per_wave_tokens=0, head_per_wave_long_wgs=1 << 40)
+    launch, records = _stream_records(lens, rows, 8, 8, 64, 0, tall)
+    assert launch and len(records) == 8 * len(rows)
+    for box, first, tokens, past in records:
+        assert first == 0 and tokens == lens[box] and past == (box >= nodes or box == nodes // 2), box
