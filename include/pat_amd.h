@@ -452,7 +452,9 @@ typedef struct pat_fwd_geometry {
 } pat_fwd_geometry;
 #define PAT_GEOMETRY_PAIRS 1 /* the two boxes of an item are served by one workgroup */
 #define PAT_GEOMETRY_APART 2 /* 32-row form: K and V tiles handed over apart         */
-#define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows read past the caches (pieces of one reader) */
+#define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows may be read past the caches (pieces of one reader, where there is enough) */
+#define PAT_GEOMETRY_MERGE_SHIFT 8 /* (flags >> 8) & 7, the merge kernel's form: 0 no merge, 1 a wave per row, 2 a half-wave, */
+                                   /* 3 / 4 a workgroup of four / eight waves, every slot at once, 5 / 6 the filled slots only */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);
 
 /* ------------------------------------------------------------------------ *

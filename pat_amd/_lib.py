@@ -89,6 +89,7 @@ PAT_STREAM_V_NEVER = 8
 PAT_GEOMETRY_PAIRS = 1
 PAT_GEOMETRY_APART = 2
 PAT_GEOMETRY_STREAM_V = 4
+PAT_GEOMETRY_MERGE_SHIFT = 8
 
 
 class BaselineArgs(C.Structure):

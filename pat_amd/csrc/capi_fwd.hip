@@ -636,7 +636,9 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   out->num_slots = g.num_slots;
   out->num_workgroups = g.total_wgs;
   out->tall_rows = g.tall_rows;
-  out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0);
+  const int merge = g.direct ? pat::kMergeNone : pat::merge_form((int64_t)args->batch * args->heads, g.num_slots, args->head_dim);
+  out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0) |
+               merge << PAT_GEOMETRY_MERGE_SHIFT;
   return PAT_OK;
 }
 

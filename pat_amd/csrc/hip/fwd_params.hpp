@@ -11,23 +11,44 @@ constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop itera
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
 constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
-// Launches of 9 slots per row and more where a workgroup takes a row. A wave of it requests eight rows at once, as many as one of
-// the other forms. Whole calls, us (the split kernel is the same in all), a wave per row / the form taken:
+// The merge kernel's forms by slots and rows. Launches of up to 8 slots per row: a wave per row, or a half-wave from so many rows.
+// Launches of 9 slots and more: where rows are few a workgroup takes a row, a wave of which requests eight rows at once, as many as
+// one of the other forms. Whole calls, us (the split kernel is the same in all), a wave per row / the form taken:
 //  * 9..32 slots, four waves, every slot requested at once: up to so many slots over all rows. Empty slots are requested too,
 //    which has to cost less than the two round trips it saves (merges: 32 rows x 32 slots 5.1 / 3.0, 592 x 10 4.5 / 4.0, 2048 x 14
 //    5.6 / 5.0, but 4096 x 18 5.2 / 7.2).
 //  * 33..64 slots, eight waves, the same, up to so many slots of 512 bytes (head_dim 64: 256): one request of 16384 tokens in 64
 //    pieces 20.9 / 15.9, 96 rows x 41 slots 14.1 / 10.8, 512 x 48 18.6 / 16.2, 768 x 64 (head_dim 64) 16.0 / 14.1; 832 x 45
 //    25.9 / 27.2, with the LSEs first 25.7, 1024 x 64 24.4 / 24.5, 23.0.
-//  * more, and where that is too many: the LSEs first, then the filled slots only, with eight waves up to so many rows, with
-//    four up to so many (eight / four waves): 64 x 72 15.6 / 11.2 / 11.5, 528 x 138 21.1 / 14.3 / 15.1, 832 x 45 25.9 / 26.3 /
-//    25.7, 1024 x 128 36.2 / 33.3 / 33.4, 2048 x 64 35.5 / 35.8 / 35.2, 2112 x 100 42.9 / 42.1 / 40.7, 4096 x 64 70.1 / 71.5 / 69.8.
+//  * more, and where that is too many: the LSEs first, then the filled slots only, with eight waves up to so many rows (64 x 72
+//    15.6 / 11.2, 528 x 138 21.1 / 14.3), with four up to so many. A workgroup per row costs its launch also where most slots are
+//    empty, and many rows keep the chip busy either way: pieces of 32 tokens, one request in 16 of all slots and the others of four
+//    filled, head_dim 64, 1536 x 64 22.6 / 19.2, 2048 x 64 16.1 / 13.9, 3072 x 64 19.5 / 18.0, 3072 x 40 16.0 / 15.7, but 4096 x 40
+//    18.7 / 19.9, 6144 x 40 24.5 / 27.9, 8192 x 160 40.7 / 45.0, head_dim 128 8192 x 40 43.0 / 48.4; half of the requests of all
+//    slots 2048 x 40 27.1 / 25.8, 3072 x 40 36.4 / 36.3, 4096 x 40 45.5 / 46.8, 8192 x 40 88.1 / 93.1.
+constexpr int64_t kMergePairsRows = 16384;
 constexpr int kMergeWideBatch = 8;
 constexpr int kMergeWideSlots = 4 * kMergeWideBatch;
 constexpr int64_t kMergeWideMost = 32768;
 constexpr int64_t kMergeWide8Most = 28672;
 constexpr int64_t kMergeWide8Rows = 768;
-constexpr int64_t kMergeWide4Rows = 8192;
+constexpr int64_t kMergeWide4Rows = 3072;
+enum MergeForm {
+  kMergeNone = 0,       // the split kernel writes `out`
+  kMergeWave = 1,       // a wave per row
+  kMergeHalfWave = 2,
+  kMergeWide4All = 3,   // a workgroup per row, four or eight waves: every slot requested at once ...
+  kMergeWide8All = 4,
+  kMergeWide4 = 5,      // ... the filled ones only
+  kMergeWide8 = 6,
+};
+inline MergeForm merge_form(int64_t rows, int num_slots, int head_dim) {
+  const int64_t slots = rows * num_slots;
+  if (num_slots <= 8) return rows >= kMergePairsRows ? kMergeHalfWave : kMergeWave;
+  if (num_slots <= kMergeWideSlots) return slots <= kMergeWideMost ? kMergeWide4All : kMergeWave;
+  if (num_slots <= 2 * kMergeWideSlots && slots * head_dim <= kMergeWide8Most * 128) return kMergeWide8All;
+  return rows <= kMergeWide8Rows ? kMergeWide8 : rows <= kMergeWide4Rows ? kMergeWide4 : kMergeWave;
+}
 
 // One workgroup's work: a launch record, written once per plan by the record kernel
 // (capi_fwd.hip) and read by the split kernel in a single round trip. In memory:

@@ -23,10 +23,6 @@
 
 namespace pat {
 
-#ifndef PAT_MERGE_PAIRS_MIN
-#define PAT_MERGE_PAIRS_MIN 16384   // rows from which a half-wave takes a row (launches of up to 8 slots per row)
-#endif
-
 // u / d with m = ceil(2^32 / d) (0 for d = 1), any 32-bit u: the product is the quotient or one more.
 __device__ __forceinline__ unsigned divide(unsigned u, unsigned d, unsigned m) {
   if (m == 0) return u;
@@ -407,31 +403,24 @@ static MergeFn wide_instance(bool bf16, int head_dim) {
 }
 
 // Host launcher: one wave per (sequence, query head), four per workgroup; a half-wave each in large launches
-// of few slots, a workgroup each where slots are many (the lines: fwd_params.hpp).
+// of few slots, a workgroup each where slots are many and rows few (the lines: merge_form, fwd_params.hpp).
 hipError_t launch_merge(bool bf16, int head_dim, hipStream_t stream, const MergeParams& params) {
   const int64_t pairs = (int64_t)params.batch * params.heads;
   MergeFn fn;
   int per_wg = 4, threads = 256;
-  const int64_t slots = pairs * params.num_slots;
-  if (params.num_slots <= 8 && pairs >= PAT_MERGE_PAIRS_MIN) {
-    per_wg = 8;
-    if (bf16) fn = head_dim == 64 ? pat_merge_pairs_kernel<__bf16, 64> : pat_merge_pairs_kernel<__bf16, 128>;
-    else fn = head_dim == 64 ? pat_merge_pairs_kernel<_Float16, 64> : pat_merge_pairs_kernel<_Float16, 128>;
-  } else if (params.num_slots > 8 && params.num_slots <= kMergeWideSlots && slots <= kMergeWideMost) {
-    per_wg = 1;
-    fn = wide_instance<4, true>(bf16, head_dim);
-  } else if (params.num_slots > kMergeWideSlots && params.num_slots <= 2 * kMergeWideSlots && slots * head_dim <= kMergeWide8Most * 128) {
-    per_wg = 1; threads = 512;
-    fn = wide_instance<8, true>(bf16, head_dim);
-  } else if (params.num_slots > kMergeWideSlots && pairs <= kMergeWide8Rows) {
-    per_wg = 1; threads = 512;
-    fn = wide_instance<8, false>(bf16, head_dim);
-  } else if (params.num_slots > kMergeWideSlots && pairs <= kMergeWide4Rows) {
-    per_wg = 1;
-    fn = wide_instance<4, false>(bf16, head_dim);
-  } else {
-    if (bf16) fn = head_dim == 64 ? pat_merge_kernel<__bf16, 64> : pat_merge_kernel<__bf16, 128>;
-    else fn = head_dim == 64 ? pat_merge_kernel<_Float16, 64> : pat_merge_kernel<_Float16, 128>;
+  switch (merge_form(pairs, params.num_slots, head_dim)) {
+    case kMergeHalfWave:
+      per_wg = 8;
+      if (bf16) fn = head_dim == 64 ? pat_merge_pairs_kernel<__bf16, 64> : pat_merge_pairs_kernel<__bf16, 128>;
+      else fn = head_dim == 64 ? pat_merge_pairs_kernel<_Float16, 64> : pat_merge_pairs_kernel<_Float16, 128>;
+      break;
+    case kMergeWide4All: per_wg = 1; fn = wide_instance<4, true>(bf16, head_dim); break;
+    case kMergeWide8All: per_wg = 1; threads = 512; fn = wide_instance<8, true>(bf16, head_dim); break;
+    case kMergeWide4: per_wg = 1; fn = wide_instance<4, false>(bf16, head_dim); break;
+    case kMergeWide8: per_wg = 1; threads = 512; fn = wide_instance<8, false>(bf16, head_dim); break;
+    default:
+      if (bf16) fn = head_dim == 64 ? pat_merge_kernel<__bf16, 64> : pat_merge_kernel<__bf16, 128>;
+      else fn = head_dim == 64 ? pat_merge_kernel<_Float16, 64> : pat_merge_kernel<_Float16, 128>;
   }
   // (a multiple of 8 kv heads: 8 interleaved lists of pairs, one per XCD, each rounded up to whole workgroups)
   const bool xcd_lists = params.kv_heads % 8 == 0;

@@ -1196,6 +1196,7 @@ PYBIND11_MODULE(_prefix_attn, m) {
           d["num_workgroups"] = g.num_workgroups; d["tall_rows"] = g.tall_rows;
           d["pairs"] = (g.flags & PAT_GEOMETRY_PAIRS) != 0; d["apart"] = (g.flags & PAT_GEOMETRY_APART) != 0;
           d["stream_v"] = (g.flags & PAT_GEOMETRY_STREAM_V) != 0;
+          d["merge"] = (g.flags >> PAT_GEOMETRY_MERGE_SHIFT) & 7;
           out.append(d);
         }
         return out;

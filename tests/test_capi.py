@@ -467,3 +467,20 @@ def test_static_launch_box_by_box_with_the_switch_out_of_range(tuning):
     tuning(pairs=-1)
     a = _bucket_args([(64, 8, 64, 7744, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS, 4), (16, 482, 1, 64, 0, 0)], 32, 32, 128, 482, 64)
     assert lib.pat_fwd_launch_static(C.byref(a), None) == _lib.PAT_ERR_HIP      # (past the check of the size: there is no GPU here)
+
+
+@pytest.mark.parametrize("slots,rows,d,form", [
+    (8, 16383, 128, 1), (8, 16384, 128, 2), (9, 3640, 128, 3), (9, 3641, 128, 1), (32, 1024, 64, 3), (32, 1032, 64, 1),
+    (33, 868, 128, 4), (33, 872, 128, 5), (64, 896, 64, 4), (64, 904, 64, 5), (64, 448, 128, 4), (64, 456, 128, 6), (65, 8, 64, 6),
+    (65, 768, 128, 6), (65, 776, 128, 5), (320, 3072, 64, 5), (40, 3072, 128, 5), (40, 3080, 128, 1), (34, 4096, 64, 1), (320, 8192, 128, 1),
+])
+def test_the_merge_kernels_form_by_slots_and_rows(slots, rows, d, form, tuning):
+    # (rows of 8 heads each but where the line is not at a multiple of 8)
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    heads = next(h for h in (8, 4, 1) if rows % h == 0)
+    tuning(chunk_tokens=32, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    splits = next(s for s in range(1, 33) if slots % s == 0 and slots // s <= 64)
+    a = _bucket_args([(16, rows // heads, 1, 32 * (slots // splits), 0, 0)], heads, heads, d, rows // heads, 16)
+    a.max_split_per_seq = splits
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+    assert g.num_slots == slots and (g.flags >> _lib.PAT_GEOMETRY_MERGE_SHIFT) & 7 == form, (g.num_slots, g.flags >> 8)
