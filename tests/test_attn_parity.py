@@ -203,8 +203,8 @@ def test_merge_of_many_rows(spec, heads, d, dtype):
 
 def test_merge_of_more_than_256_slots(tuning):
     # five nested nodes -> every request sits in five boxes (naive_schedule: one box per node); with
-    # 32-token chunks the 2048-token root reserves 64 slots per box: 320 slots per row, so the
-    # merge kernel's loops past its 256 register-held slots run
+    # 32-token chunks the 2048-token root reserves 64 slots per box: 320 slots per row, of 128 rows: eight waves
+    # a row, in one turn (the other forms at such counts: test_every_form_of_the_merge_past_256_slots)
     print("[case] merge of 320 slots per row", flush=True)
     import ctypes as C
     from pat_amd import _ctypes_launch, _lib
@@ -1404,7 +1404,7 @@ def test_edit_of_one_box_of_a_pair(captured, tuning):
     (13, 5, (24, 3), 128, torch.bfloat16),     # one list of rows, 24 a sequence
     (14, 3, (48, 24), 64, torch.bfloat16),     # eight lists, 6 rows a sequence in each
     (32, 2, (32, 8), 128, torch.float16),      # the last slot count of it
-    (33, 2, (32, 8), 128, torch.float16),      # past it: a wave per row
+    (33, 2, (32, 8), 128, torch.float16),      # past it: eight waves a row, every slot requested at once
     (10, 409, (8, 1), 64, torch.float16),      # 32720 slots: a workgroup per row ...
     (10, 410, (8, 1), 64, torch.float16),      # ... 32800: a wave per row
 ])
@@ -1442,7 +1442,7 @@ def test_merge_of_many_slots(slots, batch, heads, d, dtype, tuning):
     (4, 3, (8, 8), 64, torch.float16),           # a wave per row, every slot requested at once
     (3, 600, (32, 8), 128, torch.bfloat16),      # a half-wave per row
     (16, 3, (32, 8), 128, torch.float16),        # a workgroup per row
-    (40, 2, (8, 8), 64, torch.bfloat16),         # a wave per row, slots by sixteens
+    (40, 2, (8, 8), 64, torch.bfloat16),         # a workgroup of eight waves per row, every slot requested at once
 ])
 def test_a_nan_in_one_piece_shows_in_the_row(slots, batch, heads, d, dtype, tuning, monkeypatch):
     # one NaN in K: the rows of its request and kv head are NaN, LSE too, however many pieces the request is cut in
@@ -1699,3 +1699,125 @@ def test_what_tall_boxes_leave_over_stays_in_the_caches(nodes, tuning):
     assert launch and len(records) == 8 * len(rows)
     for box, first, tokens, past in records:
         assert first == 0 and tokens == lens[box] and past == (box >= nodes or box == nodes // 2), box
+
+
+@pytest.mark.parametrize("slots,batch,heads,d,dtype,form", [
+    (10, 412, (8, 1), 64, torch.float16, 1),      # a wave per row, slots by sixteens
+    (64, 58, (8, 1), 128, torch.bfloat16, 6),     # eight waves a row, the filled slots only
+    (64, 113, (8, 1), 64, torch.float16, 5),      # four
+    (64, 385, (8, 1), 64, torch.bfloat16, 1),     # 3080 rows of 64 slots: a wave per row again
+])
+@pytest.mark.parametrize("piece", [0, -1])
+def test_a_nan_in_each_form_of_the_merge_past_8_slots(slots, batch, heads, d, dtype, form, piece, tuning, monkeypatch):
+    # one NaN in K of the first or the last piece of one request: its rows are NaN, LSE too, and no other
+    print(f"[case] NaN in piece {piece} of {slots}, {batch} requests, form {form}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    w = workloads.independent("nan", batch, slots * 32, heads[0], heads[1], d, dtype, 1)
+    q, k, v = w.tensors(dev)
+    k[w.rows[1][0 if piece == 0 else 2 * (slots - 1)], 3, 0, 5] = float("nan")
+    tuning(chunk_tokens=32, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    tree = PrefixTreeCPP(w.page_size)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, w.heads // w.kv_heads, w.kv_heads)
+    tree.kernel_info.to_gpu(dev)
+    out = torch.zeros_like(q)
+    lse = torch.zeros(w.batch, w.heads, dtype=torch.float32, device=dev)
+    prefix_attn_with_kvcache(q, k, v, tree, 1.0 / math.sqrt(d), out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    geo = tree.kernel_info._launch_geometries[0]
+    assert geo["num_slots"] == slots and geo["merge"] == form
+    bad = torch.zeros(batch, heads[0], dtype=torch.bool)
+    bad[1] = True
+    assert torch.isnan(out.float().cpu()[:, 0][bad]).all() and torch.isnan(lse.cpu()[bad]).all()
+    keep = [0, 2] + list(range(3, batch, max(1, batch // 24)))      # (rows are alike: two dozen of them against the oracle)
+    ref_out, ref_lse = ao.paged_attention_ref(q[keep].cpu(), k.cpu(), v.cpu(), [w.rows[i] for i in keep], [w.seq_lens[i] for i in keep])
+    assert not torch.isnan(out.float().cpu()[:, 0][~bad]).any() and not torch.isnan(lse.cpu()[~bad]).any()
+    _assert_close("the other rows", out[keep], lse[keep], ref_out, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("batch,form", [(16, 6), (100, 5), (400, 1)])
+@pytest.mark.parametrize("nan", [None, "root", "leaf"])
+def test_every_form_of_the_merge_past_256_slots(batch, form, nan, tuning):
+    # five nested nodes, one box per node, 32-token pieces of a 2048-token root: 320 slots a row. A wave per row holds 256 of
+    # them in registers and reads the others again, four waves look at them in two turns. A NaN in the root's first piece is in the first turn, one
+    # in a request's own end in the last.
+    print(f"[case] merge of over 256 slots per row, {batch} requests, NaN {nan}", flush=True)
+    import ctypes as C
+    from pat_amd import _ctypes_launch, _lib
+    dev = _device()
+    nxt = [0]
+
+    def blocks(n):
+        out = list(range(nxt[0], nxt[0] + n)); nxt[0] += n
+        return out
+
+    root = blocks(128)
+    rows, lens = [], []
+    for i in range(batch):
+        if i % 8 == 0:
+            a = blocks(4)
+        if i % 4 == 0:
+            b = blocks(4)
+        if i % 2 == 0:
+            c = blocks(2)
+        rows.append(root + a + b + c + blocks(2))
+        lens.append(len(rows[-1]) * 16 - 15)
+    w = workloads.Workload("nested", 8, 2, 64, torch.float16, 16, lens, rows, nxt[0], 0, 9)
+    q, k, v = w.tensors(dev)
+    t = PrefixTree(w.page_size)
+    t.build_radix_tree(w.seq_lens, w.rows)
+    ki = t.naive_schedule(4)
+    ki.to_tensor(device=dev)
+    tuning(chunk_tokens=32, tall_chunk_tokens=32)
+    bad = torch.zeros(batch, 8, dtype=torch.bool)
+    if nan == "root":
+        k[0, 1, 1, 7] = float("nan")
+        bad[:, 4:] = True
+    elif nan == "leaf":
+        k[rows[5][-1], 0, 1, 7] = float("nan")
+        bad[5, 4:] = True
+    out = torch.zeros_like(q)
+    lse = torch.zeros(w.batch, w.heads, dtype=torch.float32, device=dev)
+    L = _ctypes_launch.prepare(q, k, v, ki.num_split_per_seq, ki.q_tables, ki.block_tables, ki.num_seqs_per_CTAs,
+                              ki.CTA_ranks, ki.kv_in_CTAs, ki.MNWs, ki.max_split_per_seq, ki.max_seqs_in_CTA,
+                              ki.max_blocks_in_CTA, 1.0 / math.sqrt(w.head_dim), out, lse)
+    geo = _lib.FwdGeometry()
+    assert _lib.load().pat_fwd_geometry_of(C.byref(L.args), C.byref(geo)) == 0
+    assert geo.num_slots > 256 and (geo.flags >> _lib.PAT_GEOMETRY_MERGE_SHIFT) & 7 == form
+    _ctypes_launch.run(L, dev)
+    torch.cuda.synchronize()
+    assert torch.isnan(out.float().cpu()[:, 0][bad]).all() and torch.isnan(lse.cpu()[bad]).all()
+    ref_out, ref_lse = _oracle(w, q, k, v)
+    good = ~bad
+    _assert_close("over 256 slots", out.cpu()[:, 0][good], lse.cpu()[good], ref_out[:, 0][good], ref_lse[good], w.dtype)
+
+
+@pytest.mark.parametrize("block", [0, 1300, 2249])
+def test_a_nan_in_one_of_more_slots_than_a_workgroup_looks_at_at_once(block, tuning, monkeypatch):
+    # eight waves look at 512 slots a turn and carry sum and maximum on to the next: a NaN of the first turn reaches the end
+    print(f"[case] NaN in block {block} of a request of more than 512 slots", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "0")
+    dev = _device()
+    lens = [36000, 700]
+    rows = [list(range(2250)), list(range(2250, 2250 + 44))]
+    w = workloads.Workload("slots", 8, 8, 64, torch.float16, 16, lens, rows, 2294, 0, 3)
+    q, k, v = w.tensors(dev)
+    k[block, 9, 6, 11] = float("nan")
+    tuning(chunk_tokens=32, tall_chunk_tokens=32, head_per_wave_tokens=0, head_per_wave_long_wgs=1 << 40, equalize_chunks=0)
+    tree = PrefixTreeCPP(16)
+    tree.build_radix_tree(w.seq_lens, w.padded_table())
+    tree.pack_schedule(None, 1, 8)
+    tree.kernel_info.to_gpu(dev)
+    out = torch.zeros_like(q)
+    lse = torch.zeros(2, 8, dtype=torch.float32, device=dev)
+    prefix_attn_with_kvcache(q, k, v, tree, 0.125, out, softmax_lse=lse)
+    torch.cuda.synchronize()
+    geo = tree.kernel_info._launch_geometries[0]
+    assert geo["num_slots"] > 512 and geo["merge"] == 6
+    bad = torch.zeros(2, 8, dtype=torch.bool)
+    bad[0, 6] = True
+    assert torch.isnan(out.float().cpu()[:, 0][bad]).all() and torch.isnan(lse.cpu()[bad]).all()
+    ref_out, ref_lse = _oracle(w, q, k, v)
+    good = ~bad
+    _assert_close("the other rows", out.cpu()[:, 0][good], lse.cpu()[good], ref_out[:, 0][good], ref_lse[good], w.dtype)
