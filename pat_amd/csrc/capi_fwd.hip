@@ -393,6 +393,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     g->chunks_per_rank = std::max(g->chunks_per_rank, n);
     g->total_wgs += items_of(a->buckets[i], pairs) * n * (a->kv_heads / g->bucket_heads_per_wg[i]);
   }
+  int64_t back_to_four[kMaxBuckets] = {0}, all_back = 0;   // workgroups more of buckets that go back to four waves (below)
   // Buckets whose widest box is a few steps long leave most waves of a workgroup idle and pay the
   // workgroup's fixed cost once per kv head: there each wave takes a kv head of its own and walks
   // the box alone. Only when the launch has workgroups to spare (2 per CU or more): a small launch
@@ -414,22 +415,15 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     // tokens beside 206 of 71 at 8/8 18.7 / 15.3, one of 128 beside 33 of up to 768 at 8/8 20.8 / 17.9, two of 112 beside 17 of up to 352 at 16/8,
     // head_dim 64, 11.0 / 9.4; 15 of 128 at 8/8, 14 of 128 at 16/16, 2 of 112 beside 10 of up to 1920 +-1 %. Not three steps (31 of 96
     // at 32/8, head_dim 64, 21.2 / 21.7, 23 of 96 at 8/8 9.3 / 9.5), and not where four waves make the launch
-    // queue (17 of 192 beside 640 tall workgroups 77.3 / 79.5; 7 of 144 ahead of 215 of 48 17.3 / 17.8). Nor where the launch has a
-    // workgroup per CU at most and would have more: a longer box then shares its CU, and the launch ends on that one (5 of 112
-    // beside one of 1536 at 16/16, 204 workgroups for 264, 18.8 / 19.9; 5 of 128 beside 3 of 528 at 32/32 10.3 / 12.4, 13 beside 17
-    // of 256 and a tall one at 16/16 15.1 / 17.9; but 25 of 112 and 42 shorter at 8/8, head_dim 64, 6.7 / 5.2, 14 beside 2 of 144 at
-    // 16/16 8.4 / 7.5, 15 beside 16 of 192 11.1 / 10.6).
-    int64_t widest_box = 0;
-    for (int i = 0; i < a->num_buckets; ++i)
-      if (a->buckets[i].num_boxes > 0)
-        widest_box = std::max<int64_t>(widest_box, row_tiles(a->buckets[i].mnw[0]) > 1 ? INT32_MAX : (int64_t)a->buckets[i].max_blocks * page);
+    // queue (17 of 192 beside 640 tall workgroups 77.3 / 79.5; 7 of 144 ahead of 215 of 48 17.3 / 17.8).
     for (int i = 0; i < a->num_buckets && tune.head_per_wave_tokens < 0; ++i) {
       const int64_t boxes = a->buckets[i].num_boxes, more = boxes * (a->kv_heads - a->kv_heads / kWaves);
       if (g->bucket_heads_per_wg[i] == kWaves && (int64_t)a->buckets[i].max_blocks * page > 3 * kStepTokens &&
-          boxes * a->kv_heads <= kNumCUs && g->total_wgs + more <= resident &&
-          (g->total_wgs > kNumCUs || g->total_wgs + more <= kNumCUs || widest_box <= 6 * kStepTokens)) {
+          boxes * a->kv_heads <= kNumCUs && g->total_wgs + more <= resident) {
         g->bucket_heads_per_wg[i] = 1;
         g->total_wgs += more;
+        back_to_four[i] = more;
+        all_back += more;
       }
     }
   }
@@ -483,6 +477,23 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
         g->total_wgs += items_of(a->buckets[i], pairs) * g->bucket_chunks[i] * (a->kv_heads / g->bucket_heads_per_wg[i]);
       }
     }
+  }
+  // Few boxes of several steps, again: not where the launch has a workgroup per CU at most and would have more. A longer box then
+  // shares its CU, and the launch ends on that one. us per call, a head per wave / four waves: 5 of 112 beside one of 1536 at 16/16,
+  // 204 workgroups for 264, 18.8 / 19.9; 5 of 128 beside 3 of 528 at 32/32 10.3 / 12.4, 4 of 112 beside 9 of 336 14.1 / 16.2, 13
+  // beside 17 of 256 and a tall one at 16/16 15.1 / 17.9; but 25 of 112 and 42 shorter at 8/8, head_dim 64, 6.7 / 5.2, 14 beside 2
+  // of 144 at 16/16 8.4 / 7.5, 15 beside 16 of 192 11.1 / 10.6.
+  if (all_back > 0) {
+    int64_t widest_box = 0;
+    for (int i = 0; i < a->num_buckets; ++i)
+      if (a->buckets[i].num_boxes > 0)
+        widest_box = std::max<int64_t>(widest_box, row_tiles(a->buckets[i].mnw[0]) > 1 ? INT32_MAX : (int64_t)a->buckets[i].max_blocks * page);
+    for (int i = a->num_buckets - 1; i >= 0 && widest_box > 6 * kStepTokens; --i)
+      if (back_to_four[i] > 0 && g->total_wgs > kNumCUs && g->total_wgs - all_back <= kNumCUs) {
+        g->bucket_heads_per_wg[i] = kWaves;
+        g->total_wgs -= back_to_four[i];
+        all_back -= back_to_four[i];
+      }
   }
   // Where the tall workgroups do not fill the CUs twice, nothing covers a super-step's wait for memory but requests made
   // earlier: K and V tiles are handed over apart there, in flight for a step and a half instead of one (us per call,
