@@ -291,8 +291,9 @@ typedef struct pat_fwd_tuning {
   int32_t pairs;                     /* two boxes of an item served by one workgroup (32-row form): */
                                      /* 0 chosen per launch from its sizes, 1 always, 2 never;      */
                                      /* + PAT_STREAM_V_ALWAYS / _NEVER: V of boxes <= 16 rows read  */
-                                     /* past the caches where no other box reads it. Values with    */
-                                     /* other bits, negative ones too: 0                            */
+                                     /* past the caches, in pieces that no other of up to 64 boxes  */
+                                     /* of the bucket and no tall box reads. Values with other      */
+                                     /* bits, negative ones too: 0                                  */
 } pat_fwd_tuning;
 #define PAT_STREAM_V_ALWAYS 4 /* (neither: chosen per launch from its sizes) */
 #define PAT_STREAM_V_NEVER 8

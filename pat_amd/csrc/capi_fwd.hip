@@ -208,7 +208,7 @@ double short_bytes(const pat_fwd_args* a) {
 // 1.7 us alone, ~3 us beside two others on the CU.
 struct LaunchEstimate { double short_us = 0., short_rounds = 0., tall_us = 0., chain_us = 0.; };
 constexpr double kShortestLaunchUs = 5.5;
-constexpr double kMergeWideUs = 3.;  // the workgroup-per-row merge against the general one (2.1 us at 32 rows x 32 slots), and the cut's own slots
+constexpr double kMergeWideUs = 3.;  // what staying within 32 slots was put at when a merge of more had a wave per row (2.1 us at 32 rows x 32 slots, and the cut's own slots)
 constexpr double kTallEndsUs = 1.;   // a tall workgroup's record, Q and first tile, and its stores
 LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs) {
   LaunchEstimate e;
@@ -289,9 +289,12 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     const LaunchEstimate est = estimate_launch(a, tall_rows, pairs);
     const double launch_us = std::max(est.tall_us + est.short_us, kShortestLaunchUs);
     int64_t pieces = std::max<int64_t>(1, (int64_t)std::ceil((est.chain_us + kTallEndsUs) / launch_us));
-    // (not past the slots up to which the merge of few rows gives each a workgroup, where the <= 16-row boxes leave it those and
-    // the longer pieces cost less than the kMergeWideUs that this form saves: 10 requests over 4944 tokens in 17 boxes each,
-    // 336-token tall boxes in one piece 12.0 us, in two 13.7, but 33 over 8096 in three boxes each, 384 tokens 12.7, 896 16.1)
+    // (not past 32 slots, which the merge of few rows requests at once with four waves a row, where the <= 16-row boxes leave it
+    // those and the longer pieces cost less than kMergeWideUs: 10 requests over 4944 tokens in 17 boxes each, 336-token tall boxes in one
+    // piece 12.0 us, in two 13.7, but 33 over 8096 in three boxes each, 384 tokens 12.7, 896 16.1. The line and kMergeWideUs are
+    // from when a row of more slots had one wave. With a workgroup per row there too they decide 19 of 6000 drawn batches: without
+    // the bound 12 of them are 2-11 % faster (20 requests over 9872 tokens at 16/8 heads 18.0 / 16.0), 4 are 2-12 % slower
+    // (1,2,7 nodes of 4768, 400, 3-24 tokens at 64/8 12.7 / 14.2))
     if ((int64_t)a->batch * a->heads * kMergeWideSlots <= kMergeWideMost && pieces_of(chunk) * a->max_split_per_seq <= kMergeWideSlots) {
       const int64_t most = std::max<int64_t>(1, kMergeWideSlots / a->max_split_per_seq);
       if (est.chain_us / (double)most + kTallEndsUs <= launch_us + kMergeWideUs) pieces = std::min(pieces, most);
@@ -682,7 +685,8 @@ namespace {
 // (boxes over the same blocks lie next to each other): the host knows widths only, and one long box among many short ones, or
 // requests over one prefix with a box each, are many times fewer tokens than boxes x width. In common is judged by the pages at
 // 1/8, 3/8, 5/8 and 7/8 of the box; of more than kCounted boxes every second, third ... is looked at. Every workgroup counts for
-// itself: two round trips per bucket, 3 to 6 us of a kernel that runs once per plan.
+// itself: two round trips per bucket, 3 to 6 us of a kernel that runs once per plan (a wave per bucket and four boxes a lane: 1 us less
+// on most, 1 more on 1024 boxes).
 constexpr int kCounted = 256;
 __device__ bool holds_tokens(const RecordParams& p, int64_t least) {
   __shared__ unsigned long long s_eighths[4];

@@ -369,7 +369,7 @@ def test_tall_boxes_are_cut_by_what_a_workgroup_takes_ends_included():
     # in two: the chain of 352 tokens alone is shorter than the launch, with the workgroup's ends it is not
     assert plan(3, [(64, 1, 24, 352, even, 0), (16, 3, 8, 992, even, 0), (16, 24, 8, 512, 0, 0)], 16, 8, 128, 24, 16).tall_chunk_tokens == 256
     assert plan(2, [(64, 53, 8, 1440, both, 27), (16, 1, 1, 1472, even, 0), (16, 424, 1, 32, even, 0)], 64, 8, 64, 425, 32).tall_chunk_tokens == 768
-    # not in two: 34 slots a row are past what the merge gives a workgroup per row for
+    # not in two: 34 slots a row are past the 32 that the merge requests at once with four waves, and one piece is put at less than that
     assert plan(17, [(32, 16, 10, 336, even, 0), (16, 10, 8, 48, 0, 0)], 16, 8, 128, 10, 48).num_slots == 17
     # ... but in 384-token pieces where those of 32 slots would be more than twice as long
     assert plan(3, [(64, 1, 33, 8096, even, 0), (32, 1, 17, 864, even, 0), (16, 1, 16, 864, even, 0), (16, 33, 1, 32, 0, 0)], 8, 8, 64, 33, 32).tall_chunk_tokens == 384
