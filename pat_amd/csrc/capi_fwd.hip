@@ -684,52 +684,82 @@ namespace {
 // Tokens that the boxes of <= 16 rows hold between them, what a box has in common with the next one of its bucket counted once
 // (boxes over the same blocks lie next to each other): the host knows widths only, and one long box among many short ones, or
 // requests over one prefix with a box each, are many times fewer tokens than boxes x width. In common is judged by the pages at
-// 1/8, 3/8, 5/8 and 7/8 of the box; of more than kCounted boxes every second, third ... is looked at. Every workgroup counts for
-// itself: two round trips per bucket, 3 to 6 us of a kernel that runs once per plan (a wave per bucket and four boxes a lane: 1 us less
-// on most, 1 more on 1024 boxes).
-constexpr int kCounted = 256;
+// 1/8, 3/8, 5/8 and 7/8 of the box; of more than 256 boxes every second, third ... is looked at. One wave, four boxes per lane at once:
+// two round trips per bucket.
 __device__ bool holds_tokens(const RecordParams& p, int64_t least) {
-  __shared__ unsigned long long s_eighths[4];
+  constexpr int kPerLane = 4;
+  const int lane = threadIdx.x & 63;
   unsigned long long eighths = 0;
   for (int b = 0; b < p.num_buckets; ++b) {
     const RecordBucket& bk = p.bucket[b];
-    if (bk.row_tiles != 1) continue;
-    const int step = (bk.num_boxes + kCounted - 1) / kCounted, cap = bk.max_blocks * p.page_size;
-    for (int64_t at = (int64_t)threadIdx.x * step; at < bk.num_boxes; at += 256 * (int64_t)step) {
-      const int box = (int)at, next = box + 1 < bk.num_boxes ? box + 1 : 0;
-      const int kv = min(bk.kv[box], cap), kv_next = next != box ? bk.kv[next] : 0;
-      if (kv <= 0) continue;
-      const int32_t* row = bk.block_table + (int64_t)box * bk.bt_stride;
-      const int32_t* row_next = bk.block_table + (int64_t)next * bk.bt_stride;
-      int own = 0;
+    if (bk.row_tiles != 1 || bk.max_blocks <= 0) continue;
+    const int last = bk.num_boxes - 1, step = (bk.num_boxes + 64 * kPerLane - 1) / (64 * kPerLane), cap = bk.max_blocks * p.page_size;
+    int box[kPerLane], next[kPerLane], kv[kPerLane], kv_next[kPerLane], page[kPerLane][4], own[kPerLane][4], other[kPerLane][4];
 #pragma unroll
-      for (int i = 1; i < 8; i += 2) {
-        const int page = (int)((int64_t)kv * i / 8) / p.page_size;
-        own += (kv_next > page * p.page_size && row_next[page] == row[page]) ? 0 : 2;
+    for (int j = 0; j < kPerLane; ++j) {
+      const int64_t at = (int64_t)(lane + 64 * j) * step;
+      box[j] = (int)min<int64_t>(at, last);
+      next[j] = box[j] < last ? box[j] + 1 : 0;
+      kv[j] = bk.kv[box[j]];
+      kv_next[j] = next[j] != box[j] ? bk.kv[next[j]] : 0;
+      if (at > last) kv[j] = 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+      kv[j] = max(0, min(kv[j], cap));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        page[j][i] = (int)((int64_t)kv[j] * (2 * i + 1) / 8) / p.page_size;   // (below max_blocks; 0 for an empty box)
+        own[j][i] = bk.block_table[(int64_t)box[j] * bk.bt_stride + page[j][i]];
+        other[j][i] = bk.block_table[(int64_t)next[j] * bk.bt_stride + page[j][i]];
       }
-      eighths += (unsigned long long)kv * own * step;
+    }
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+      int mine = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine += (kv_next[j] > page[j][i] * p.page_size && other[j][i] == own[j][i]) ? 0 : 2;
+      eighths += (unsigned long long)kv[j] * mine * step;
     }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) eighths += __shfl_xor(eighths, off);
-  if ((threadIdx.x & 63) == 0) s_eighths[threadIdx.x >> 6] = eighths;
-  __syncthreads();
-  return (s_eighths[0] + s_eighths[1] + s_eighths[2] + s_eighths[3]) / 8 >= (unsigned long long)least;
+  return eighths / 8 >= (unsigned long long)least;
 }
 
-// One wave per record: decodes which (bucket, box, chunk, kv head group) the workgroup is, reads
-// the box's plan entries, checks and clamps them, and lays them out for the split kernel.
-__global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
-  const bool launch_streams = p.stream_tokens >= 0 && holds_tokens(p, p.stream_tokens);   // (ahead of the returns: it has a barrier)
-  const int lane = threadIdx.x & 63;
-  const int wg = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wg >= p.grid_items) return;
+// One wave per record, four a workgroup: decodes which (bucket, box, chunk, kv head group) the workgroup is, reads
+// the box's plan entries, checks and clamps them, and lays them out for the split kernel. In launches that may read V past the
+// caches a fifth wave counts meanwhile (holds_tokens), every workgroup for itself: ahead of the records by the same waves it took
+// 2-3 us longer, 8.3 for 5.6 without tall boxes or several buckets.
+struct ModeWord {
+  int32_t* word = nullptr;    // of a record written by this lane
+  int32_t mode = 0;
+  bool one_reader = false;    // of the record's piece
+};
+__device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, int lane);
+__global__ void __launch_bounds__(320) pat_record_kernel(const RecordParams p) {
+  __shared__ int s_streams;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  ModeWord m;
+  if (wave < 4) m = write_record(p, blockIdx.x * 4 + wave, lane);
+  if (p.stream_tokens < 0) return;
+  if (wave == 4) {
+    const bool holds = holds_tokens(p, p.stream_tokens);
+    if (lane == 0) s_streams = holds;
+  }
+  __syncthreads();
+  if (m.one_reader && s_streams && m.word != nullptr) *m.word = m.mode | kRecordModeStreamV;
+}
+
+__device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, int lane) {
+  ModeWord m;
+  if (wg >= p.grid_items) return m;
   if (wg >= p.total_items) {
     // padding of the grid: a workgroup with nothing to do
     char* rec = p.records + (size_t)wg * (size_t)p.record_stride;
     int32_t* words = reinterpret_cast<int32_t*>(rec);
     for (int i = lane; i < p.record_stride / 4; i += 64) words[i] = (i < 8) ? 0 : -1;
-    return;
+    return m;
   }
   int bi = 0;
   for (int i = 1; i < p.num_buckets; ++i) bi += (wg >= p.bucket[i].item_begin) ? 1 : 0;
@@ -774,24 +804,24 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
   // of a small one's are looked at). Not the first page: what requests share is how they begin, and where one work item serves
   // a request a few shared pages at its head would keep all of it in the caches (48 requests of 805..3752 tokens, 384 of them
   // shared, 16 heads of 64: 103 us by the first page, 80 by the middle one).
-  bool stream = false;
-  if (launch_streams && bk.row_tiles == 1 && tokens > 0) {
+  if (p.stream_tokens >= 0 && bk.row_tiles == 1 && tokens > 0) {
     const int at = (t_begin + tokens / 2) / page;
     const int id = bk.block_table[(int64_t)box * bk.bt_stride + at];
     int other = box + 1 + lane;
     other = other >= bk.num_boxes ? other - bk.num_boxes : other;
     const bool same = lane < bk.num_boxes - 1 && other < bk.num_boxes && bk.kv[other] > at * page &&
                       bk.block_table[(int64_t)other * bk.bt_stride + at] == id;
-    stream = __ballot(same) == 0;
+    m.one_reader = __ballot(same) == 0;
     // ... nor a tall box, which walks the same node when this one holds the few requests that its tall boxes leave over: they wait
     // for each other's V there (20 nodes of 17 requests over 2048 tokens at 32/8 heads, three caches in turn: 72.2 us past the
     // caches, 66.6 kept; 20 of 10 over 3072 at 64/8, head_dim 64, 60.5 / 56.0)
-    for (int i = 0; i < p.num_buckets && stream; ++i) {
+    for (int i = 0; i < p.num_buckets && m.one_reader; ++i) {
       const RecordBucket& tall = p.bucket[i];
       if (tall.row_tiles == 1 || at >= tall.max_blocks) continue;
-      for (int first = 0; first < tall.num_boxes && stream; first += 64) {
+      for (int first = 0; first < tall.num_boxes && m.one_reader; first += 64) {
         const int tb = min(first + lane, tall.num_boxes - 1);
-        stream = __ballot(tall.kv[tb] > at * page && tall.block_table[(int64_t)tb * tall.bt_stride + at] == id) == 0;
+        const int tall_kv = tall.kv[tb], tall_id = tall.block_table[(int64_t)tb * tall.bt_stride + at];   // (one round trip)
+        m.one_reader = __ballot(tall_kv > at * page && tall_id == id) == 0;
       }
     }
   }
@@ -801,8 +831,7 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
     RecordHead h;
     h.tokens = rows > 0 ? tokens : 0;
     h.rows = rows;
-    h.mode = (box2 >= 0 ? 2 * bk.row_tiles : bk.row_tiles) | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0) |
-             (stream ? kRecordModeStreamV : 0);
+    h.mode = (box2 >= 0 ? 2 * bk.row_tiles : bk.row_tiles) | (bk.heads_per_wg > 1 ? kRecordModeHeadPerWave : 0);
     h.head = hgroup * bk.heads_per_wg;
     // slots of this box that no workgroup fills: this one's own when it has no tokens, and the
     // ones past the bucket's last chunk (the launch reserves chunks_per_rank per box ordinal)
@@ -810,6 +839,8 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
     h.fill_end = (chunk == bk.chunks - 1) ? p.chunks_per_rank - chunk : 1;
     h.pad[0] = h.pad[1] = 0;
     *reinterpret_cast<RecordHead*>(rec) = h;
+    m.word = &reinterpret_cast<RecordHead*>(rec)->mode;
+    m.mode = h.mode;
   }
   int32_t* tab = reinterpret_cast<int32_t*>(rec + sizeof(RecordHead));
   // rows: sequence id and partial-result slot (the plan's own rank or, when the plan carries
@@ -833,6 +864,7 @@ __global__ void __launch_bounds__(256) pat_record_kernel(const RecordParams p) {
     pg = pg < 0 ? 0 : (pg >= p.num_pages ? p.num_pages - 1 : pg);
     tab[2 * p.record_max_seqs + i] = pg;
   }
+  return m;
 }
 
 int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hipStream_t stream) {
@@ -869,7 +901,7 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   rp.total_items = (int32_t)items;
   rp.grid_items = (int32_t)grid_wgs(g);
   if (items == 0) return PAT_OK;
-  hipLaunchKernelGGL(pat_record_kernel, dim3((unsigned)((rp.grid_items + 3) / 4)), dim3(256), 0, stream, rp);
+  hipLaunchKernelGGL(pat_record_kernel, dim3((unsigned)((rp.grid_items + 3) / 4)), dim3(rp.stream_tokens >= 0 ? 320 : 256), 0, stream, rp);
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) return hip_fail(e, "record kernel launch");
   return PAT_OK;
 }
