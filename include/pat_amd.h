@@ -200,7 +200,9 @@ typedef struct pat_flat_bucket {
  * more than twice as long as all others split in two (the wide head first), so that the
  * forward kernels do not reserve work for every box up to the widest one's length; the
  * second part's block_table is as wide as its widest row plus 8 spare columns (room for
- * in-place growth between decode steps). launch_order[b] is the offset of plan bucket b's
+ * in-place growth between decode steps). A bucket only some of whose boxes are tails (PAT_BUCKET_TAILS)
+ * is split as well, the tails behind the others, and where there are tails q_slot numbers a sequence's
+ * tail behind its other boxes. launch_order[b] is the offset of plan bucket b's
  * permutation: entry i = plan row of the box at launch position i. */
 typedef struct pat_flat_plan {
   int32_t num_buckets;
@@ -211,7 +213,9 @@ typedef struct pat_flat_plan {
   int64_t num_split_per_seq;   /* offset, [batch]                                        */
   int64_t num_boxes_per_seq;   /* offset, [batch]: see pat_plan_view.num_boxes_per_seq   */
   int32_t max_boxes_per_seq;
-  int32_t pad_;
+  int32_t tails;               /* 0, or (see PAT_BUCKET_TAILS) bits 0..7: the most boxes of a
+                                  sequence that are no tails; bit 8 + i: launch bucket i holds
+                                  tails; bit 20 + i: it has a tails table                */
   int64_t launch_order[PAT_MAX_FLAT_BUCKETS];
   pat_flat_bucket buckets[PAT_MAX_FLAT_BUCKETS];
   pat_flat_bucket launch[PAT_MAX_FLAT_BUCKETS];
@@ -254,7 +258,7 @@ typedef struct pat_fwd_bucket {
   int32_t max_blocks;         /* valid columns of block_table                 */
   int32_t mnw[3];
   int32_t flags;              /* PAT_BUCKET_* hints, 0 when nothing is known  */
-  int32_t num_items;          /* read only with PAT_BUCKET_ITEMS              */
+  int32_t num_items;          /* read only with PAT_BUCKET_ITEMS / _TAILS     */
 } pat_fwd_bucket;
 
 /* Hint: no box of the bucket is shorter than 3/4 of its widest box (the launcher cannot see
@@ -268,13 +272,27 @@ typedef struct pat_fwd_bucket {
  * the block_table row of the first box only, or ignore the table. The caller vouches for the items: after a write to
  * kv or block_table that may have parted two boxes of an item, launch (and build records) without this flag. */
 #define PAT_BUCKET_ITEMS 2
+/* Tails: boxes of one sequence and few tokens whose sequence also sits in a box of 17..64 rows, whose workgroup may walk them
+ * behind its own tokens; the launch then has no workgroups and no partial-result slots for them.
+ * PAT_BUCKET_TAIL: every box of the bucket is a tail (one sequence each, at most 64 tokens wide) and stands in exactly one entry of
+ * one tails table. Its sequences' ordinals (q_slot) number the tails behind all other boxes. PAT_TAIL_BOXES(flags): the most boxes of a
+ * sequence that are no tails.
+ * PAT_BUCKET_TAILS (tile labels above 16): kv and the item table (num_items rows, possibly 0, with or without PAT_BUCKET_ITEMS) are
+ * followed in memory by the tails table, int32 [num_boxes, max_seqs] - per sequence of a box its tail as bucket << 27 | row, -1 =
+ * none; `bucket` as the buckets of the launch are numbered - and, int32 [batch], the boxes of each sequence that are no tails.
+ * A launch may make use of the tails or treat those buckets like any other; it needs both flags. The caller vouches for the
+ * tables as for items: growing a tail in its own bucket keeps them right. */
+#define PAT_BUCKET_TAILS 4
+#define PAT_BUCKET_TAIL 8
+#define PAT_TAIL_BOXES_SHIFT 8
+#define PAT_TAIL_BOXES(flags) (((flags) >> PAT_TAIL_BOXES_SHIFT) & 0xff)
 
 /* Overrides of the launch geometry. pat_fwd_set_tuning sets them process-wide (a tuning and test
  * aid, not meant to change while launches are in flight on other threads); pat_fwd_args.tuning sets
  * them for one launch (what pat_fwd_autotune's result is for). 0 / -1 = automatic, as noted per field. The
  * initial values come from the environment variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS,
  * PAT_HEAD_PER_WAVE_TOKENS, PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS,
- * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, PAT_TALL_ROWS, PAT_PAIRS, PAT_STREAM_V, read once; pat_fwd_set_tuning(NULL) reads them again. */
+ * PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT, PAT_TALL_ROWS, PAT_PAIRS, PAT_STREAM_V, PAT_TAILS, read once; pat_fwd_set_tuning(NULL) reads them again. */
 typedef struct pat_fwd_tuning {
   int32_t chunk_tokens;              /* KV tokens per workgroup, boxes <= 16 rows (0: automatic)   */
   int32_t tall_chunk_tokens;         /* same for boxes of 17..64 rows (0: automatic)                */
@@ -292,11 +310,14 @@ typedef struct pat_fwd_tuning {
                                      /* 0 chosen per launch from its sizes, 1 always, 2 never;      */
                                      /* + PAT_STREAM_V_ALWAYS / _NEVER: V of boxes <= 16 rows read  */
                                      /* past the caches, in pieces that no other of up to 64 boxes  */
-                                     /* of the bucket and no tall box reads. Values with other      */
-                                     /* bits, negative ones too: 0                                  */
+                                     /* of the bucket and no tall box reads; + PAT_TAILS_ALWAYS /   */
+                                     /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS). */
+                                     /* Values with other bits, negative ones too: 0                */
 } pat_fwd_tuning;
 #define PAT_STREAM_V_ALWAYS 4 /* (neither: chosen per launch from its sizes) */
 #define PAT_STREAM_V_NEVER 8
+#define PAT_TAILS_ALWAYS 32   /* (where the launch can, neither: chosen per launch from its sizes) */
+#define PAT_TAILS_NEVER 64
 int pat_fwd_set_tuning(const pat_fwd_tuning* tuning);
 int pat_fwd_get_tuning(pat_fwd_tuning* out);
 
@@ -454,6 +475,7 @@ typedef struct pat_fwd_geometry {
 #define PAT_GEOMETRY_PAIRS 1 /* the two boxes of an item are served by one workgroup */
 #define PAT_GEOMETRY_APART 2 /* 32-row form: K and V tiles handed over apart         */
 #define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows may be read past the caches (pieces of one reader, where there is enough) */
+#define PAT_GEOMETRY_TAILS 8 /* tails are walked by the workgroups of their sequences' tall boxes */
 #define PAT_GEOMETRY_MERGE_SHIFT 8 /* (flags >> 8) & 7, the merge kernel's form: 0 no merge, 1 a wave per row, 2 a half-wave, */
                                    /* 3 / 4 a workgroup of four / eight waves, every slot at once, 5 / 6 the filled slots only */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);

@@ -69,7 +69,7 @@ class FlatPlan(C.Structure):
     _fields_ = [("num_buckets", C.c_int32), ("num_launch_buckets", C.c_int32), ("batch", C.c_int32),
                 ("max_split_per_seq", C.c_int32), ("max_seqs_in_box", C.c_int32),
                 ("max_blocks_in_box", C.c_int32), ("total", C.c_int64), ("num_split_per_seq", C.c_int64),
-                ("num_boxes_per_seq", C.c_int64), ("max_boxes_per_seq", C.c_int32), ("pad_", C.c_int32),
+                ("num_boxes_per_seq", C.c_int64), ("max_boxes_per_seq", C.c_int32), ("tails", C.c_int32),
                 ("launch_order", C.c_int64 * MAX_FLAT_BUCKETS), ("buckets", FlatBucket * MAX_FLAT_BUCKETS),
                 ("launch", FlatBucket * MAX_FLAT_BUCKETS)]
 
@@ -84,11 +84,17 @@ class FwdBucket(C.Structure):
 
 PAT_BUCKET_EVEN = 1
 PAT_BUCKET_ITEMS = 2
+PAT_BUCKET_TAILS = 4
+PAT_BUCKET_TAIL = 8
+PAT_TAIL_BOXES_SHIFT = 8
 PAT_STREAM_V_ALWAYS = 4
 PAT_STREAM_V_NEVER = 8
+PAT_TAILS_ALWAYS = 32
+PAT_TAILS_NEVER = 64
 PAT_GEOMETRY_PAIRS = 1
 PAT_GEOMETRY_APART = 2
 PAT_GEOMETRY_STREAM_V = 4
+PAT_GEOMETRY_TAILS = 8
 PAT_GEOMETRY_MERGE_SHIFT = 8
 
 

@@ -50,7 +50,7 @@ inline int row_tiles(int m_label) { return m_label <= 16 ? 1 : (m_label <= 32 ? 
 // Overrides of the launch geometry (pat_fwd_set_tuning). The defaults come from the environment
 // variables PAT_CHUNK_TOKENS, PAT_TALL_CHUNK_TOKENS, PAT_HEAD_PER_WAVE_TOKENS,
 // PAT_HEAD_PER_WAVE_LONG_WGS, PAT_HEAD_PER_WAVE_LONG_TOKENS, PAT_EQUALIZE_CHUNKS, PAT_DIRECT_OUT,
-// PAT_TALL_ROWS, PAT_PAIRS and PAT_STREAM_V, read once per process: no launch reads the environment.
+// PAT_TALL_ROWS, PAT_PAIRS, PAT_STREAM_V and PAT_TAILS, read once per process: no launch reads the environment.
 pat_fwd_tuning env_tuning() {
   pat_fwd_tuning t;
   t.chunk_tokens = 0; t.tall_chunk_tokens = 0; t.head_per_wave_tokens = -1;
@@ -61,7 +61,8 @@ pat_fwd_tuning env_tuning() {
     const int v = e ? std::atoi(e) : 0;
     return v == 1 || v == 2 ? v : 0;
   };
-  t.pairs = one_or_two("PAT_PAIRS") | (one_or_two("PAT_STREAM_V") == 1 ? PAT_STREAM_V_ALWAYS : one_or_two("PAT_STREAM_V") == 2 ? PAT_STREAM_V_NEVER : 0);
+  t.pairs = one_or_two("PAT_PAIRS") | (one_or_two("PAT_STREAM_V") == 1 ? PAT_STREAM_V_ALWAYS : one_or_two("PAT_STREAM_V") == 2 ? PAT_STREAM_V_NEVER : 0) |
+            (one_or_two("PAT_TAILS") == 1 ? PAT_TAILS_ALWAYS : one_or_two("PAT_TAILS") == 2 ? PAT_TAILS_NEVER : 0);
   if (const char* e = std::getenv("PAT_TALL_ROWS")) t.tall_rows = std::atoi(e);
   if (const char* e = std::getenv("PAT_CHUNK_TOKENS")) t.chunk_tokens = std::atoi(e);
   if (const char* e = std::getenv("PAT_TALL_CHUNK_TOKENS")) t.tall_chunk_tokens = std::atoi(e);
@@ -81,10 +82,15 @@ pat_fwd_tuning tuning() {
   return g_tuning;
 }
 
-// The two switches in pat_fwd_tuning.pairs: boxes in twos (0..2), and V past the caches. Values outside the declared bits, -1 among
-// them, ask for neither.
-int pairs_switch(const pat_fwd_tuning& t) { return t.pairs >= 0 && t.pairs < 16 ? t.pairs & 3 : 0; }
-int stream_switch(const pat_fwd_tuning& t) { return t.pairs >= 0 && t.pairs < 16 ? t.pairs & (PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER) : 0; }
+// The three switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, and tails. Values outside the declared bits,
+// -1 among them, ask for none.
+int switches(const pat_fwd_tuning& t, int bits) {
+  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER;
+  return t.pairs >= 0 && (t.pairs & ~kDeclared) == 0 ? t.pairs & bits : 0;
+}
+int pairs_switch(const pat_fwd_tuning& t) { return switches(t, 3); }
+int stream_switch(const pat_fwd_tuning& t) { return switches(t, PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER); }
+int tails_switch(const pat_fwd_tuning& t) { return switches(t, PAT_TAILS_ALWAYS | PAT_TAILS_NEVER); }
 
 // Widest box (tokens) of a bucket whose workgroups serve one kv head per wave (0: mode off).
 int64_t head_per_wave_tokens(const pat_fwd_tuning& t, bool oversubscribed) {
@@ -106,6 +112,8 @@ struct Geometry {
   bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
   bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches ...
   int stream_tokens = -1;    // ... where these boxes hold so many tokens (the record kernel counts)
+  bool tails = false;        // tails are walked by their sequences' tall workgroups (PAT_BUCKET_TAILS)
+  int tail_pages = 0;        // ... pages per tail in the records
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
   // launch records (one per workgroup): entries per record and bytes between records
   int record_max_seqs = 0, record_max_pages = 0, record_stride = 0;
@@ -115,6 +123,35 @@ struct Geometry {
 inline int64_t items_of(const pat_fwd_bucket& b, bool pairs) {
   return pairs && (b.flags & PAT_BUCKET_ITEMS) && row_tiles(b.mnw[0]) > 1 ? b.num_items : b.num_boxes;
 }
+
+// The arguments of a launch whose tails are walked by tall workgroups: without the tails' buckets, and with the other boxes' counts.
+struct WithoutTails {
+  pat_fwd_args args;
+  pat_fwd_bucket buckets[kMaxBuckets];
+  int tail_pages = 0;
+  // false: the launch has no tails, or not in this form
+  bool make(const pat_fwd_args* a) {
+    args = *a;
+    args.buckets = buckets;
+    const int32_t* counts = nullptr;
+    int most = 0;
+    for (int i = 0; i < a->num_buckets; ++i) {
+      const pat_fwd_bucket& b = buckets[i] = a->buckets[i];
+      if ((b.flags & PAT_BUCKET_TAIL) && b.num_boxes > 0) {
+        if (row_tiles(b.mnw[0]) != 1 || b.max_seqs != 1 || b.max_blocks <= 0 || (int64_t)b.max_blocks * a->page_size > kMaxTailTokens) return false;
+        tail_pages = std::max(tail_pages, (int)b.max_blocks);
+        most = std::max<int>(most, PAT_TAIL_BOXES(b.flags));
+        buckets[i].num_boxes = 0;
+      }
+      if ((b.flags & PAT_BUCKET_TAILS) && b.num_boxes > 0 && row_tiles(b.mnw[0]) > 1 && counts == nullptr)
+        counts = b.kv + b.num_boxes + 2 * (int64_t)b.num_items + (int64_t)b.num_boxes * b.max_seqs;
+    }
+    if (tail_pages == 0 || counts == nullptr || most <= 0 || most > a->max_split_per_seq) return false;
+    args.num_split_per_seq = counts;
+    args.max_split_per_seq = most;
+    return true;
+  }
+};
 
 int check_args(const pat_fwd_args* a) {
   if (a == nullptr) return fail(PAT_ERR_INVALID, "args is NULL");
@@ -541,7 +578,8 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
   }
   g->record_max_seqs = std::min(std::max(g->record_max_seqs, 1), 128);
   g->record_max_pages = std::min(std::max(g->record_max_pages, 1), kMaxChunkPages);
-  g->record_stride = (int)((sizeof(RecordHead) + (2 * g->record_max_seqs + g->record_max_pages) * sizeof(int32_t) + 63) / 64 * 64);
+  const int tail_words = g->tail_pages > 0 ? (1 + g->tail_pages) * g->record_max_seqs : 0;
+  g->record_stride = (int)((sizeof(RecordHead) + (2 * g->record_max_seqs + g->record_max_pages + tail_words) * sizeof(int32_t) + 63) / 64 * 64);
   // the kernels index partial rows with 32-bit integers
   if ((int64_t)a->batch * a->heads * g->num_slots >= ((int64_t)1 << 31))
     return fail(PAT_ERR_INVALID, "batch * heads * partial slots must stay below 2^31");
@@ -567,8 +605,9 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 // part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
 // boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice
 // as often to be as many, only add partial rows (4 boxes x 8 of 2048 tokens: 22.4 / 23.5).
-int plan_geometry(const pat_fwd_args* a, Geometry* g) {
+int plan_boxes(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
+  g->tail_pages = tail_pages;
   int64_t widest_tall = 0, tall_box_heads = 0;
   bool pairs = false;
   for (int i = 0; i < a->num_buckets; ++i) {
@@ -586,7 +625,7 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
     *g = Geometry();
     return plan_geometry_for(a, g, 16, false);
   };
-  if (tune.tall_rows == 32) return in_32();
+  if (tail_pages > 0 || tune.tall_rows == 32) return in_32();
   if (tune.tall_rows == 16) return plan_geometry_for(a, g, 16, false);
   if (widest_tall == 0) return plan_geometry_for(a, g, 16, false);   // no tall box: the form with more resident workgroups
   if (int rc = in_32()) return rc;
@@ -599,6 +638,58 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   if (outweigh) return PAT_OK;
   *g = Geometry();
   return plan_geometry_for(a, g, 16, false);
+}
+
+// Tails walked by the workgroups of their sequences' tall boxes? Only where that leaves every row one partial result, so that the
+// split kernel writes `out` and no merge follows, and where it is the cheaper one by an estimate from sizes:
+//  * there: kTailStepUs for each 32-token step of a wave's tails (a wave has one tail in flight and waits for memory once per step:
+//    2.2-2.5 us), 32 rows' tails of a pair of boxes one after the other, half of that where two waves share the rows; never less
+//    than the stream of their K and V;
+//  * by themselves: that stream, or kTailRoundUs for every further round of workgroups, as far as the tall workgroups keep the chip
+//    (on idle CUs tails run beside them), and the merge, 3 us and its partial rows at 4.5 TB/s.
+// Not where the tall workgroups, uncut for that one result, leave more than three of eight CUs idle, unless a wave has two steps at most.
+// us per call, by themselves / with the tall boxes: 1024 x (2048 + 32) tokens at 64/8 heads 118 / 100, + 64 141 / 121, + 16 116 / 94,
+// 2048 x (1024 + 32) at 32/8 114 / 92, 827 x (464 + 26) at 64/8 59.1 / 39.5, 369 x (384 + 1..4), head_dim 64, 19.9 / 14.6, but few rows per
+// sequence (many tails a wave) 1010 x (768 + 5..10) at 16/16 44.1 / 74.1, idle CUs 283 x (1504 + 58..64) at 64/8 40.0 / 49.1, 256 x
+// (544 + 32) 25.1 / 26.2, and, with a merge all the same, 512 x (1408 + 32) at 16/8 32.1 / 37.1. Of 290 drawn batches with tails the rule
+// takes 10: geometric mean 0.84, the slowest 1.01; 9 of the 41 others without a merge would be 3-27 % faster, most far slower.
+constexpr double kTailStepUs = 2.5;
+constexpr double kTailRoundUs = 4.;
+bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& without) {
+  if (with.num_slots != 1) return false;
+  const int group = a->heads / a->kv_heads;
+  double steps = 0., bytes = 0.;
+  for (int i = 0; i < a->num_buckets; ++i) {
+    const pat_fwd_bucket& b = a->buckets[i];
+    if (!(b.flags & PAT_BUCKET_TAIL) || b.num_boxes <= 0) continue;
+    const int64_t width = (int64_t)b.max_blocks * a->page_size;
+    steps = std::max(steps, (double)ceil_div64(width, kStepTokens));
+    bytes += (double)b.num_boxes * width * a->kv_heads * a->head_dim * 4.;
+  }
+  steps *= std::max(1, (with.pairs ? 32 : 16) / group);
+  if (steps > 2. && with.total_wgs < 5 * kNumCUs / 8) return false;
+  const double own_places = resident_wgs_per_cu(a->head_dim, without.tall_rows) * kNumCUs;
+  const double with_us = std::max(steps * kTailStepUs * std::max(1., (double)with.total_wgs / (resident_wgs_per_cu(a->head_dim, 32) * kNumCUs)), bytes / 6e6);
+  const double own_us = std::max(bytes / 5.8e6, kTailRoundUs * std::max(0., (double)without.total_wgs / own_places - 1.)) *
+                        std::min(1., (double)with.total_wgs / kNumCUs);
+  const double merge_us = 3. + (double)a->batch * a->heads * without.num_slots * a->head_dim * 4. / 4.5e6;
+  return with_us < own_us + merge_us;
+}
+
+int plan_geometry(const pat_fwd_args* a, Geometry* g) {
+  const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
+  const int forced = tails_switch(tune);
+  WithoutTails w;
+  if ((forced & PAT_TAILS_NEVER) || tune.tall_rows == 16 || !w.make(a)) return plan_boxes(a, g, 0);
+  Geometry with;
+  const bool can = plan_boxes(&w.args, &with, w.tail_pages) == PAT_OK && with.tall_rows == 32 && !with.stream_v;
+  if (!can || !(forced & PAT_TAILS_ALWAYS)) {
+    if (int rc = plan_boxes(a, g, 0)) return rc;
+    if (!can || !tails_pay(a, with, *g)) return PAT_OK;
+  }
+  *g = with;
+  g->tails = true;
+  return PAT_OK;
 }
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -625,7 +716,7 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
   mix((uint64_t)g.tall_rows); mix((uint64_t)g.total_wgs); mix((uint64_t)g.record_stride); mix((uint64_t)g.record_max_seqs); mix((uint64_t)g.record_max_pages);
   mix((uint64_t)g.num_slots); mix((uint64_t)g.chunks_per_rank); mix(g.direct ? 1 : 0); mix((uint64_t)(g.stream_tokens + 1));
   mix((uint64_t)a->batch); mix((uint64_t)a->heads); mix((uint64_t)a->kv_heads); mix((uint64_t)a->page_size);
-  mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq); mix(g.pairs ? 1 : 0);
+  mix((uint64_t)a->num_pages); mix((uint64_t)a->max_split_per_seq); mix(g.pairs ? 1 : 0); mix((uint64_t)(g.tails ? 1 + g.tail_pages : 0));
   for (int i = 0; i < a->num_buckets; ++i) {
     const pat_fwd_bucket& b = a->buckets[i];
     mix((uint64_t)g.bucket_chunk[i]); mix((uint64_t)g.bucket_chunks[i]); mix((uint64_t)g.bucket_heads_per_wg[i]);
@@ -633,6 +724,7 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
     mix((uint64_t)reinterpret_cast<uintptr_t>(b.q_table)); mix((uint64_t)reinterpret_cast<uintptr_t>(b.block_table));
     mix((uint64_t)reinterpret_cast<uintptr_t>(b.kv)); mix((uint64_t)reinterpret_cast<uintptr_t>(b.q_slot));
     if (g.pairs) mix((uint64_t)items_of(b, true));
+    if (g.tails) { mix((uint64_t)b.flags); mix((uint64_t)b.num_items); }
   }
   return h ? h : 1;
 }
@@ -661,6 +753,7 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   out->tall_rows = g.tall_rows;
   const int merge = g.direct ? pat::kMergeNone : pat::merge_form((int64_t)args->batch * args->heads, g.num_slots, args->head_dim);
   out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0) |
+               (g.tails ? PAT_GEOMETRY_TAILS : 0) |
                merge << PAT_GEOMETRY_MERGE_SHIFT;
   return PAT_OK;
 }
@@ -692,7 +785,7 @@ __device__ bool holds_tokens(const RecordParams& p, int64_t least) {
   unsigned long long eighths = 0;
   for (int b = 0; b < p.num_buckets; ++b) {
     const RecordBucket& bk = p.bucket[b];
-    if (bk.row_tiles != 1 || bk.max_blocks <= 0) continue;
+    if (bk.row_tiles != 1 || bk.max_blocks <= 0 || bk.num_items == 0) continue;
     const int last = bk.num_boxes - 1, step = (bk.num_boxes + 64 * kPerLane - 1) / (64 * kPerLane), cap = bk.max_blocks * p.page_size;
     int box[kPerLane], next[kPerLane], kv[kPerLane], kv_next[kPerLane], page[kPerLane][4], own[kPerLane][4], other[kPerLane][4];
 #pragma unroll
@@ -736,12 +829,15 @@ struct ModeWord {
   int32_t mode = 0;
   bool one_reader = false;    // of the record's piece
 };
+template <bool TAILS>
 __device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, int lane);
+// (an instance of its own for launches with tails)
+template <bool TAILS>
 __global__ void __launch_bounds__(320) pat_record_kernel(const RecordParams p) {
   __shared__ int s_streams;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   ModeWord m;
-  if (wave < 4) m = write_record(p, blockIdx.x * 4 + wave, lane);
+  if (wave < 4) m = write_record<TAILS>(p, blockIdx.x * 4 + wave, lane);
   if (p.stream_tokens < 0) return;
   if (wave == 4) {
     const bool holds = holds_tokens(p, p.stream_tokens);
@@ -751,6 +847,7 @@ __global__ void __launch_bounds__(320) pat_record_kernel(const RecordParams p) {
   if (m.one_reader && s_streams && m.word != nullptr) *m.word = m.mode | kRecordModeStreamV;
 }
 
+template <bool TAILS>
 __device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, int lane) {
   ModeWord m;
   if (wg >= p.grid_items) return m;
@@ -864,6 +961,33 @@ __device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, 
     pg = pg < 0 ? 0 : (pg >= p.num_pages ? p.num_pages - 1 : pg);
     tab[2 * p.record_max_seqs + i] = pg;
   }
+  if constexpr (TAILS) {
+    // tails: the pieces that a box is cut into take its sequences' in turn
+    int32_t* tail = tab + 2 * p.record_max_seqs + p.record_max_pages;
+    const int pieces = max(1, (kv + bk.chunk_tokens - 1) / bk.chunk_tokens);
+    for (int j = lane; j < p.record_max_seqs; j += 64) {
+      int entry = -1, seq = -1;
+      if (bk.tails != nullptr && j < nseq && j % pieces == chunk) {
+        const int b = j < nseq0 ? box : box2, at = j < nseq0 ? j : j - nseq0;
+        entry = bk.tails[(int64_t)b * bk.max_seqs + at];
+        seq = tab[j];
+      }
+      tail[j] = 0;
+      for (int i = 0; i < p.tail_pages; ++i) tail[p.record_max_seqs + j * p.tail_pages + i] = 0;
+      for (int i = 0; i < p.num_buckets; ++i) {   // (not by the entry's bucket: an index that differs over the lanes copies all of `p`)
+        const RecordBucket& tb = p.bucket[i];
+        const int row = entry & ((1 << 27) - 1);
+        if (tb.tail_id < 0 || entry < 0 || entry >> 27 != tb.tail_id || row >= tb.num_boxes) continue;
+        // (a tail of another sequence, from a malformed table, is no tail)
+        if (seq < 0 || tb.q_table[(int64_t)row * tb.q_stride] != seq) continue;
+        tail[j] = max(0, min(tb.kv[row], min(tb.max_blocks, p.tail_pages) * page));
+        for (int c = 0; c < min(tb.max_blocks, p.tail_pages); ++c) {
+          const int pg = tb.block_table[(int64_t)row * tb.bt_stride + c];
+          tail[p.record_max_seqs + j * p.tail_pages + c] = pg < 0 ? 0 : (pg >= p.num_pages ? p.num_pages - 1 : pg);
+        }
+      }
+    }
+  }
   return m;
 }
 
@@ -874,13 +998,18 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   rp.record_stride = g.record_stride; rp.record_max_seqs = g.record_max_seqs; rp.record_max_pages = g.record_max_pages;
   rp.batch = args->batch; rp.kv_heads = args->kv_heads; rp.group = args->heads / args->kv_heads;
   rp.page_size = args->page_size; rp.num_pages = args->num_pages;
-  rp.chunks_per_rank = g.chunks_per_rank; rp.max_split = args->max_split_per_seq; rp.stream_tokens = g.stream_tokens;
+  rp.chunks_per_rank = g.chunks_per_rank; rp.stream_tokens = g.stream_tokens;
+  WithoutTails w;
+  if (g.tails && !w.make(args)) return fail(PAT_ERR_INVALID, "internal: a launch with tails has none");
+  rp.max_split = g.tails ? w.args.max_split_per_seq : args->max_split_per_seq;
+  rp.tail_pages = g.tail_pages;
   // buckets in plan order (tall, long boxes come first in the default order)
   int nb = 0;
   int64_t items = 0;
   for (int i = 0; i < args->num_buckets; ++i) {
     const pat_fwd_bucket& b = args->buckets[i];
     if (b.num_boxes == 0) continue;
+    const bool tail = g.tails && (b.flags & PAT_BUCKET_TAIL) != 0;   // (in no workgroup of its own)
     RecordBucket& d = rp.bucket[nb];
     d.q_table = b.q_table; d.block_table = b.block_table; d.num_seqs = b.num_seqs;
     d.rank = b.rank; d.kv = b.kv; d.q_slot = b.q_slot;
@@ -891,8 +1020,10 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
     d.row_tiles = row_tiles(b.mnw[0]);
     d.heads_per_wg = g.bucket_heads_per_wg[i];
     d.item_begin = (int32_t)items;
-    d.num_items = (int32_t)items_of(b, g.pairs);
-    d.items = d.num_items < b.num_boxes ? b.kv + b.num_boxes : nullptr;
+    d.num_items = tail ? 0 : (int32_t)items_of(b, g.pairs);
+    d.items = !tail && d.num_items < b.num_boxes ? b.kv + b.num_boxes : nullptr;
+    d.tail_id = tail ? i : -1;
+    d.tails = g.tails && (b.flags & PAT_BUCKET_TAILS) && d.row_tiles > 1 ? b.kv + b.num_boxes + 2 * (int64_t)b.num_items : nullptr;
     ++nb;
     items += (int64_t)d.num_items * d.chunks * (args->kv_heads / d.heads_per_wg);
   }
@@ -901,7 +1032,7 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   rp.total_items = (int32_t)items;
   rp.grid_items = (int32_t)grid_wgs(g);
   if (items == 0) return PAT_OK;
-  hipLaunchKernelGGL(pat_record_kernel, dim3((unsigned)((rp.grid_items + 3) / 4)), dim3(rp.stream_tokens >= 0 ? 320 : 256), 0, stream, rp);
+  hipLaunchKernelGGL(g.tails ? pat_record_kernel<true> : pat_record_kernel<false>, dim3((unsigned)((rp.grid_items + 3) / 4)), dim3(rp.stream_tokens >= 0 ? 320 : 256), 0, stream, rp);
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) return hip_fail(e, "record kernel launch");
   return PAT_OK;
 }
@@ -936,6 +1067,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   sp.tall_rows = g.tall_rows;
   sp.stream_v = g.stream_v ? 1 : 0;
   sp.tall_apart = g.tall_apart ? 1 : 0;
+  sp.tail_pages = g.tail_pages;
   if (g.direct) {
     sp.out = args->out; sp.lse_out = args->lse_out;
     sp.o_stride_b = args->o_stride[0]; sp.o_stride_h = args->o_stride[2];
@@ -965,13 +1097,16 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
 
   if (g.direct) return PAT_OK;   // the rows are in `out` already
 
+  WithoutTails w;
+  if (g.tails && !w.make(args)) return fail(PAT_ERR_INVALID, "internal: a launch with tails has none");
+  const pat_fwd_args& counts = g.tails ? w.args : *args;
   MergeParams mp;
   std::memset(&mp, 0, sizeof(mp));
-  mp.o_part = o_part; mp.lse_part = lse_part; mp.num_split_per_seq = args->num_split_per_seq;
+  mp.o_part = o_part; mp.lse_part = lse_part; mp.num_split_per_seq = counts.num_split_per_seq;
   mp.out = args->out; mp.lse_out = args->lse_out;
   mp.o_stride_b = args->o_stride[0]; mp.o_stride_h = args->o_stride[2];
   mp.batch = args->batch; mp.heads = args->heads; mp.head_dim = args->head_dim; mp.kv_heads = args->kv_heads;
-  mp.chunks_per_rank = g.chunks_per_rank; mp.num_slots = g.num_slots; mp.max_split = args->max_split_per_seq;
+  mp.chunks_per_rank = g.chunks_per_rank; mp.num_slots = g.num_slots; mp.max_split = counts.max_split_per_seq;
   const hipError_t e = launch_merge(args->dtype == PAT_DTYPE_BF16, args->head_dim, stream, mp);
   if (e != hipSuccess) return hip_fail(e, "merge kernel launch");
   return PAT_OK;
@@ -1093,13 +1228,13 @@ int pat_fwd_launch_static(const pat_fwd_args* args, void* hip_stream) {
   Geometry g;
   if (int rc = plan_geometry(args, &g)) return rc;
   size_t need = workspace_need(args, g);
-  // The records of boxes served in twos are longer: a launch that only fits box by box is made box by box.
+  // The records of boxes served in twos, and of tails, are longer: a launch that only fits box by box is made box by box.
   pat_fwd_args box_by_box;
   pat_fwd_tuning tune;
-  if (need > kStaticScratchBytes && g.pairs && args->records == nullptr) {
+  if (need > kStaticScratchBytes && (g.pairs || g.tails) && args->records == nullptr) {
     box_by_box = *args;
     tune = args->tuning != nullptr ? *args->tuning : tuning();
-    tune.pairs = stream_switch(tune) | 2;
+    tune.pairs = stream_switch(tune) | PAT_TAILS_NEVER | 2;
     box_by_box.tuning = &tune;
     args = &box_by_box;
     g = Geometry();

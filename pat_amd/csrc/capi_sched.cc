@@ -164,6 +164,7 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   if (nb > PAT_MAX_FLAT_BUCKETS)
     return pat::fail(PAT_ERR_INVALID, "the flat plan holds at most 12 buckets");
   constexpr int kGrowthBlocks = 8;
+  const int page = tree->block_size;
   std::memset(layout, 0, sizeof(*layout));
   layout->num_buckets = nb;
   layout->batch = (int32_t)p.num_split_per_seq.size();
@@ -177,6 +178,43 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   std::vector<std::vector<int32_t>> order((size_t)nb);
   std::vector<Part> parts;
   int spare = PAT_MAX_FLAT_BUCKETS - nb;
+
+  // Tails: boxes of one sequence, up to kMaxTailTokens wide, whose sequence also sits in a box of more than 16 rows. A launch may
+  // have that box's workgroup walk them too (PAT_BUCKET_TAILS). Of several such boxes the shortest takes the tail.
+  constexpr int kMaxTailTokens = 64;
+  struct Claim { int bucket = -1, box = -1, j = 0; };
+  std::vector<Claim> claim((size_t)layout->batch);   // per sequence: where its tail may go
+  std::vector<std::vector<char>> is_tail((size_t)nb);
+  bool any_tail = false;
+  auto may_hold_tails = [&](const pat::Bucket& bk) {
+    return bk.mnw[0] <= 16 && bk.max_seqs == 1 && (int64_t)bk.max_blocks * page <= kMaxTailTokens;
+  };
+  const bool look = std::any_of(p.buckets.begin(), p.buckets.end(), may_hold_tails);
+  for (int b = 0; b < nb && look; ++b) {
+    const pat::Bucket& bk = p.buckets[(size_t)b];
+    if (bk.mnw[0] <= 16) continue;
+    for (size_t box = 0; box < bk.kv.size(); ++box)
+      for (int j = 0; j < bk.q_len[box]; ++j) {
+        const int32_t s = bk.q_table[box * (size_t)bk.max_seqs + (size_t)j];
+        if (s < 0 || s >= layout->batch) continue;
+        Claim& c = claim[(size_t)s];
+        if (c.bucket < 0 || bk.kv[box] <= p.buckets[(size_t)c.bucket].kv[(size_t)c.box]) c = {b, (int)box, j};
+      }
+  }
+  {
+    std::vector<char> taken((size_t)layout->batch, 0);
+    for (int b = 0; b < nb; ++b) {
+      const pat::Bucket& bk = p.buckets[(size_t)b];
+      is_tail[(size_t)b].assign(bk.kv.size(), 0);
+      if (!may_hold_tails(bk)) continue;
+      for (size_t box = 0; box < bk.kv.size(); ++box) {
+        const int32_t s = bk.q_table[box];
+        if (bk.q_len[box] != 1 || s < 0 || s >= layout->batch || claim[(size_t)s].bucket < 0 || taken[(size_t)s]) continue;
+        taken[(size_t)s] = is_tail[(size_t)b][box] = 1;
+      }
+    }
+  }
+
   for (int b = 0; b < nb; ++b) {
     const pat::Bucket& bk = p.buckets[(size_t)b];
     const int n = (int)bk.kv.size();
@@ -191,7 +229,15 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
       while (k < n && bk.kv[(size_t)ord[(size_t)k]] > widest / 2) ++k;
       if (k > 0 && k <= n / 4) { cut = k; --spare; }
     }
-    if (cut == 0) {
+    // a bucket of which only some boxes are tails: those in a launch bucket of their own, behind the others
+    const auto& tail = is_tail[(size_t)b];
+    const int n_tail = (int)std::count(tail.begin(), tail.end(), 1);
+    if (n_tail > 0 && n_tail < n && cut == 0 && spare > 0) {
+      std::stable_partition(ord.begin(), ord.end(), [&](int32_t x) { return !tail[(size_t)x]; });
+      --spare;
+      parts.push_back({b, 0, n - n_tail, bk.max_blocks});
+      parts.push_back({b, n - n_tail, n, bk.max_blocks});
+    } else if (cut == 0) {
       parts.push_back({b, 0, n, bk.max_blocks});
     } else {
       parts.push_back({b, 0, cut, bk.max_blocks});
@@ -238,6 +284,62 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
     if (!any) items[i].clear();
   }
 
+  // The launch buckets that hold nothing but tails, and per box of more than 16 rows the tails of its sequences there: launch
+  // bucket << 27 | row, -1 = none.
+  std::vector<char> tail_part(parts.size(), 0);
+  std::vector<std::vector<int32_t>> tails(parts.size());
+  std::vector<std::vector<int32_t>> slot((size_t)nb);   // launch copies of q_slot, and the boxes per sequence that are no tails
+  std::vector<int32_t> without((size_t)layout->batch, 0);
+  {
+    std::vector<std::vector<std::array<int32_t, 2>>> place((size_t)nb);   // plan box -> (launch bucket, row)
+    for (int b = 0; b < nb; ++b) place[(size_t)b].resize(p.buckets[(size_t)b].kv.size());
+    for (size_t i = 0; i < parts.size(); ++i) {
+      const Part& pt = parts[i];
+      const auto& ord = order[(size_t)pt.parent];
+      bool all = pt.hi > pt.lo;
+      for (int at = pt.lo; at < pt.hi; ++at) {
+        place[(size_t)pt.parent][(size_t)ord[(size_t)at]] = {(int32_t)i, at - pt.lo};
+        all = all && is_tail[(size_t)pt.parent][(size_t)ord[(size_t)at]];
+      }
+      tail_part[i] = all;
+      any_tail = any_tail || all;
+    }
+    if (any_tail) {
+      for (size_t i = 0; i < parts.size(); ++i) {
+        if (!tail_part[i]) continue;
+        const Part& pt = parts[i];
+        const pat::Bucket& bk = p.buckets[(size_t)pt.parent];
+        for (int at = pt.lo; at < pt.hi; ++at) {
+          const Claim& c = claim[(size_t)bk.q_table[(size_t)order[(size_t)pt.parent][(size_t)at]]];
+          const auto& where = place[(size_t)c.bucket][(size_t)c.box];
+          const pat::Bucket& tall = p.buckets[(size_t)c.bucket];
+          auto& t = tails[(size_t)where[0]];
+          if (t.empty()) t.assign((size_t)(parts[(size_t)where[0]].hi - parts[(size_t)where[0]].lo) * (size_t)tall.max_seqs, -1);
+          t[(size_t)where[1] * (size_t)tall.max_seqs + (size_t)c.j] = (int32_t)i << 27 | (at - pt.lo);
+        }
+      }
+      // ordinals of a sequence's boxes with the tails behind all others: a launch that has no slots for tails leaves the last ones out
+      std::vector<int32_t> seen((size_t)layout->batch, 0);
+      for (int b = 0; b < nb; ++b) slot[(size_t)b].assign(p.buckets[(size_t)b].q_slot.size(), 0);
+      for (int pass = 0; pass < 2; ++pass) {
+        for (int b = 0; b < nb; ++b) {
+          const pat::Bucket& bk = p.buckets[(size_t)b];
+          for (size_t box = 0; box < bk.kv.size(); ++box) {
+            if ((int)tail_part[(size_t)place[(size_t)b][box][0]] != pass) continue;
+            for (int j = 0; j < bk.q_len[box]; ++j) {
+              const size_t e = box * (size_t)bk.max_seqs + (size_t)j;
+              slot[(size_t)b][e] = seen.at((size_t)bk.q_table[e])++;
+            }
+          }
+        }
+        if (pass == 0) without = seen;
+      }
+      uint32_t word = (uint32_t)*std::max_element(without.begin(), without.end());
+      for (size_t i = 0; i < parts.size(); ++i) word |= (tail_part[i] ? 1u << (8 + i) : 0u) | (!tails[i].empty() ? 1u << (20 + i) : 0u);
+      layout->tails = (int32_t)word;
+    }
+  }
+
   // offsets
   int64_t at = 0;
   auto take = [&](int64_t n) { const int64_t o = at; at += n; return o; };
@@ -262,6 +364,7 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
     place(layout->launch[i], p.buckets[(size_t)pt.parent], pt.hi - pt.lo, pt.width, pt.parent, pt.lo);
     layout->launch[i].num_items = (int32_t)(items[i].size() / 2);
     take((int64_t)items[i].size());   // (right behind kv, the last table of the bucket)
+    if (!tails[i].empty()) take((int64_t)tails[i].size() + layout->batch);
   }
   // hints: a bucket is even when no box is shorter than 3/4 of its widest one
   auto even = [&](const pat::Bucket& bk, const int32_t* ord, int lo, int hi) {
@@ -293,9 +396,9 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   auto vec_to = [&](int32_t* out, const std::vector<int32_t>& v, const int32_t* ord, int lo, int hi) {
     for (int i = lo; i < hi; ++i) out[i - lo] = v[(size_t)(ord ? ord[i] : i)];
   };
-  auto fill = [&](const pat_flat_bucket& f, const pat::Bucket& bk, const int32_t* ord, int lo, int hi) {
+  auto fill = [&](const pat_flat_bucket& f, const pat::Bucket& bk, const std::vector<int32_t>& q_slot, const int32_t* ord, int lo, int hi) {
     rows_to(dst + f.q_table, bk.q_table, bk.max_seqs, bk.max_seqs, ord, lo, hi);
-    rows_to(dst + f.q_slot, bk.q_slot, bk.max_seqs, bk.max_seqs, ord, lo, hi);
+    rows_to(dst + f.q_slot, q_slot, bk.max_seqs, bk.max_seqs, ord, lo, hi);
     rows_to(dst + f.block_table, bk.block_table, bk.max_blocks, f.max_blocks, ord, lo, hi);
     vec_to(dst + f.num_seqs, bk.num_seqs, ord, lo, hi);
     vec_to(dst + f.rank, bk.rank, ord, lo, hi);
@@ -303,13 +406,15 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   };
   for (int b = 0; b < nb; ++b) {
     const pat::Bucket& bk = p.buckets[(size_t)b];
-    fill(layout->buckets[b], bk, nullptr, 0, (int)bk.kv.size());
+    fill(layout->buckets[b], bk, bk.q_slot, nullptr, 0, (int)bk.kv.size());
     std::copy(order[(size_t)b].begin(), order[(size_t)b].end(), dst + layout->launch_order[b]);
   }
   for (size_t i = 0; i < parts.size(); ++i) {
     const Part& pt = parts[i];
-    fill(layout->launch[i], p.buckets[(size_t)pt.parent], order[(size_t)pt.parent].data(), pt.lo, pt.hi);
-    std::copy(items[i].begin(), items[i].end(), dst + layout->launch[i].kv + layout->launch[i].num_boxes);
+    const pat::Bucket& bk = p.buckets[(size_t)pt.parent];
+    fill(layout->launch[i], bk, any_tail ? slot[(size_t)pt.parent] : bk.q_slot, order[(size_t)pt.parent].data(), pt.lo, pt.hi);
+    int32_t* behind = std::copy(items[i].begin(), items[i].end(), dst + layout->launch[i].kv + layout->launch[i].num_boxes);
+    if (!tails[i].empty()) std::copy(without.begin(), without.end(), std::copy(tails[i].begin(), tails[i].end(), behind));
   }
   return PAT_OK;
 }

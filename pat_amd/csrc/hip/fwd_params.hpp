@@ -11,6 +11,7 @@ constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop itera
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
 constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
+constexpr int kMaxTailTokens = 64;  // tokens of a tail: two steps, at most four pages, so that those of a wave's 32 rows are two per lane
 // The merge kernel's forms by slots and rows. Launches of up to 8 slots per row: a wave per row, or a half-wave from so many rows.
 // Launches of 9 slots and more: where rows are few a workgroup takes a row, a wave of which requests eight rows at once, as many as
 // one of the other forms. Whole calls, us (the split kernel is the same in all), a wave per row / the form taken:
@@ -53,14 +54,16 @@ inline MergeForm merge_form(int64_t rows, int num_slots, int head_dim) {
 // One workgroup's work: a launch record, written once per plan by the record kernel
 // (capi_fwd.hip) and read by the split kernel in a single round trip. In memory:
 //   RecordHead | int32 seq[max_seqs] | int32 slot[max_seqs] | int32 page[max_pages]
+//   (tails: | int32 tail_tokens[max_seqs] | int32 tail_page[max_seqs][tail_pages])
 // seq[j] / slot[j]: batch index of the box's j-th sequence and the partial-result slot its rows
 // of this piece go to (-1 / -1: no such row); page[i]: physical KV block of the piece's i-th page,
-// already clamped to the cache. Records are record_stride bytes apart (a multiple of 64).
+// already clamped to the cache. tail_tokens[j]: tokens of the j-th sequence's tail that this workgroup walks (0: none), on pages
+// tail_page[j][..]. Records are record_stride bytes apart (a multiple of 64).
 struct RecordHead {
   int32_t tokens;      // KV tokens of this piece; 0: nothing to compute (the workgroup only marks slots empty)
   int32_t rows;        // rows of the box, or of the two boxes of an item (sequences x heads per kv head), <= 16 x tiles
   int32_t mode;        // bits 0-7: 16-row tiles (1 = KV steps split over waves on wave-private tiles,
-                       // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave; bit 9: V read past the caches
+                       // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave; bit 9: V read past the caches;
   int32_t head;        // first kv head this workgroup serves
   int32_t fill_begin;  // slots slot[j] + fill_begin .. slot[j] + fill_end - 1 of every row stay empty:
   int32_t fill_end;    // this workgroup marks them (-inf)
@@ -97,6 +100,7 @@ struct SplitParams {
   int32_t direct;    // 1: such a launch
   int32_t tall_apart;  // 32-row form: K and V tiles of a super-step handed over apart (see the kernel)
   int32_t stream_v;  // records may ask for V past the caches (host side: picks the kernel instance)
+  int32_t tail_pages; // tails: pages per tail in the records, 0: the launch has none
   int32_t tall_rows; // rows per wave on boxes of 17..64 rows: 32 (32x32x16 tiles) or 16 (host side: picks the kernel instance)
 };
 
@@ -120,6 +124,8 @@ struct RecordBucket {
   const int32_t* items;  // [num_items, 2]: boxes served together (-1: no second one), or null: every box by itself
   int32_t num_items;     // work items along the box axis: rows of `items`, or num_boxes
   int32_t heads_per_wg;  // 1, or kWaves: wave w serves kv head h0 + w alone
+  const int32_t* tails;  // [num_boxes, max_seqs]: launch bucket << 27 | row of each sequence's tail, or null
+  int32_t tail_id;       // a bucket of tails: its place among the launch's buckets, as `tails` numbers them; else -1
 };
 
 struct RecordParams {
@@ -129,6 +135,7 @@ struct RecordParams {
   int32_t batch, kv_heads, group, page_size, num_pages;
   int32_t chunks_per_rank;  // slots reserved per box ordinal
   int32_t max_split;
+  int32_t tail_pages;       // pages per tail in a record; 0: no tails. Buckets of tails have no items, only tables.
   int32_t stream_tokens;    // V tiles of pieces that no other box reads go past the caches (kRecordModeStreamV) where the boxes of
                             // <= 16 rows hold so many tokens between them; negative: nowhere
   RecordBucket bucket[kMaxBuckets];

@@ -107,7 +107,8 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
 // DIRECT instances serve launches in which every row has one partial slot: they store `out`. STREAM instances serve launches
 // whose records may ask for V past the caches (kRecordModeStreamV): a second loop over short boxes, whose mere presence cost
 // the smallest launches 0.14 us of 5.5.
-template <typename T, int D, bool DIRECT, int TALLK, bool STREAM>
+// TAILS instances (32-row form): tall workgroups also walk the tails of their rows' sequences.
+template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS>
 __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
                                                                              const int record_max_seqs, const int record_max_pages, const SplitParams p) {
   using E = Elem<T>;
@@ -122,7 +123,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   constexpr int OROW = D + 4;            // padded row of the combine buffer, floats
   constexpr int WSTAGE = VSTAGE;                       // one wave's private staging (V only)
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  extern __shared__ __attribute__((aligned(256))) char smem[];
   __shared__ float s_m[kWaves * 16];
   __shared__ float s_l[kWaves * 16];
 
@@ -308,7 +309,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   // K operand of half a / k-step kk; vtile is a row-major V tile in LDS with row stride RSV.
   // after_scores() runs once the K operands have been consumed: the caller refills their
   // registers there, so the next step's K is in flight during the softmax and the PV product.
-  auto attend = [&](auto k_op, const PAT_LDS char* vtile, int t0, auto after_scores) {
+  auto attend = [&](auto k_op, const PAT_LDS char* vtile, int t0, int t_end, float& m_run, float& l_run, auto after_scores) {
     f32x4 sc[2];
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -438,7 +439,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
         __syncthreads();
         if (has_rows)
           attend([&](int a, int kk) { return *(const PAT_LDS vec8*)(stage + (a * 16 + n) * RSK + (kk * 32 + g * 8) * 2); },
-                 stage + kStepTokens * RSK, t_begin + st * kStepTokens, []() {});
+                 stage + kStepTokens * RSK, t_begin + st * kStepTokens, t_end, m_run, l_run, []() {});
       }
     }
     l_run = sum_xor32(sum_xor16(l_run));
@@ -513,6 +514,141 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       for (int i = 0; i < 16; ++i) acc2[db][i] = 0.f;
 
     // this lane's place in its wave's half: row RPI*i + r_in of load i, and the piece it fetches there
+    // ---- tails: the few tokens that each sequence of the box has behind it, alone ----------------------
+    // Behind the piece, whose registers are free again. A wave takes those of its own 32 rows one after the other (of two waves on the same rows every second one): rows of one
+    // sequence on 16x16x32 tiles, as the boxes of <= 16 rows are walked, K straight into operand registers, V through a region of
+    // LDS of this wave's own, the next step's tiles in flight. Each tail is a softmax of its own, added to its rows' state in fp32: a
+    // tile that several sequences shared, masked, would carry one's infinite or NaN V into the others' sums.
+    const int* __restrict__ tail_tab = pages_tab + record_max_pages;   // tokens by sequence, then pages
+    const int per_tile = 32 >> gshift, tail_pages = TAILS ? p.tail_pages : 0;
+    int tok_mine = 0, tp0 = 0, tp1 = 0;   // lane i: tokens of the tail of the tile's sequence i; pages i and 64 + i of the tile's tails
+    uint64_t tails_mine = 0;              // bit i: this wave walks the tail of the tile's sequence i
+    if constexpr (TAILS) {
+      const int j0 = rt * per_tile, entries = record_max_seqs * (1 + tail_pages);
+      if (lane < per_tile && j0 + lane < record_max_seqs) tok_mine = tail_tab[j0 + lane];
+      const int first = record_max_seqs + j0 * tail_pages;
+      tp0 = tail_tab[min(first + lane, entries - 1)];
+      tp1 = tail_tab[min(first + 64 + lane, entries - 1)];
+      tails_mine = __builtin_amdgcn_ballot_w64(tok_mine > 0);
+      if (!one_tile_per_wave) {
+        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(tails_mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)tails_mine, 0u));
+        tails_mine = __builtin_amdgcn_ballot_w64(tok_mine > 0 && (rank & 1) == ph);
+      }
+    }
+    auto walk_tails = [&]() {
+      constexpr int REGION = split_smem_bytes(D, 32) / kWaves;
+      static_assert(VSTAGE + 8 * OROW * 4 <= REGION, "a wave's V tile and the result of a sequence's rows fit its part of LDS");
+      uint64_t live = tails_mine;
+      if (live == 0) return;
+      PAT_LDS char* vtile = (PAT_LDS char*)smem + wave * REGION;
+      PAT_LDS float* result = (PAT_LDS float*)(vtile + VSTAGE);   // [row of the sequence][OROW]
+      u32x4 kd[2][KK], vd[NV];
+      // half a of the step at token t0 of tail j (`tok` tokens): base address; `lim`: its last row that exists (rows past the end
+      // re-read the last token, as everywhere)
+      auto tail_half = [&](const char* base, int64_t sp, int64_t ss, int j, int tok, int t, int& lim) -> const char* {
+        const int left = tok - 1 - t;
+        lim = left < 0 ? (tok - 1) & 15 : (left > 15 ? 15 : left);
+        const int h = left < 0 ? (tok - 1) >> 4 : t >> 4;
+        int pidx, s16;
+        if (hshift >= 0) { pidx = h >> hshift; s16 = h & (hpp - 1); }
+        else { pidx = (int)__umulhi((unsigned)h, p.hpp_magic); s16 = h - pidx * hpp; }
+        const int e = j * tail_pages + pidx;
+        const int pg = __builtin_amdgcn_readlane(e < 64 ? tp0 : tp1, e & 63);
+        return base + (int64_t)pg * sp + (int64_t)(s16 * 16) * ss;
+      };
+      auto tail_v = [&](int j, int tok, int t0) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          int lim;
+          const char* vb = tail_half(vbase, vsp, vss, j, tok, t0 + a * 16, lim);
+#pragma unroll
+          for (int i = 0; i < NV / 2; ++i) {
+            const unsigned vo = (unsigned)min(i * TPL + lane / CPR, lim) * (unsigned)vss + (lane % CPR) * 16;
+            vd[a * (NV / 2) + i] = *(const u32x4*)(vb + vo);
+          }
+        }
+      };
+      auto tail_k = [&](int j, int tok, int t0) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          int lim;
+          const char* kb = tail_half(kbase, ksp, kss, j, tok, t0 + a * 16, lim);
+          const unsigned ko = (unsigned)min(n, lim) * (unsigned)kss + g * 16;
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) kd[a][kk] = *(const u32x4*)(kb + ko + kk * 64);
+        }
+      };
+      auto tail_q = [&](int j) {   // (columns past the sequence's rows hold one of them again: they go nowhere)
+        const int seq = __builtin_amdgcn_readlane(my_seq, j << gshift);
+        const T* qrow = (const T*)p.q + ((int64_t)seq * p.q_stride_b + (int64_t)(head * G + (n & (G - 1))) * p.q_stride_h);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) qreg[kk] = __builtin_bit_cast(vec8, *(const u32x4*)(qrow + kk * 32 + g * 8));
+      };
+      int j = (int)__builtin_ctzll(live), t0 = 0, tok = __builtin_amdgcn_readlane(tok_mine, j);
+      float m_t = neg_inf(), l_t = 0.f;
+      tail_v(j, tok, t0);
+      tail_k(j, tok, t0);
+      tail_q(j);
+      // One step. Every request is made in every step but the last, which stands apart, so that a wait counts exactly the loads
+      // behind the one it is for; with requests that may not be made each step waited for all of them, a full trip to memory
+      // per tail.
+      auto step = [&](auto more_c) {
+        constexpr bool more = decltype(more_c)::value;
+        // the step behind this one: of this tail, or the next one's first
+        const bool ends = !more || t0 + kStepTokens >= tok;
+        int next_j = j, next_t0 = t0 + kStepTokens, next_tok = tok;
+        if (more && ends) {
+          live &= live - 1;
+          next_j = (int)__builtin_ctzll(live);
+          next_t0 = 0;
+          next_tok = __builtin_amdgcn_readlane(tok_mine, next_j);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          *(PAT_LDS u32x4*)(vtile + (i * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vd[i];
+        if (more) tail_v(next_j, next_tok, next_t0);
+        attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kd[a][kk]); }, vtile, t0, tok, m_t, l_t, [&]() {
+          if (more) {
+            tail_k(next_j, next_tok, next_t0);
+            tail_q(next_j);
+          }
+        });
+        if (ends) {
+          // into the state of the sequence's rows: from lane (g, n), row n, columns 16 db + 4 g .. to lane (n32, h2)
+          l_t = sum_xor32(sum_xor16(l_t));
+          if (n < G) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) *(PAT_LDS f32x4*)(result + n * OROW + db * 16 + g * 4) = acc_o[db];
+          }
+          const int row = n32 & (G - 1);
+          const float mt = __shfl(m_t, row), lt = __shfl(l_t, row);
+          asm volatile("" ::: "memory");   // (the wave reads what its own lanes wrote: in order, no barrier)
+          if ((n32 >> gshift) == j) {
+            const float m_new = fmaxf(m_run, mt);
+            const float wa = m_run == m_new ? 1.f : fast_exp2(m_run - m_new), wb = fast_exp2(mt - m_new);
+            m_run = m_new;
+            l_run = l_run * wa + (h2 == 0 ? lt * wb : 0.f);   // (the two lanes of a row hold parts of its sum)
+#pragma unroll
+            for (int db = 0; db < DB2; ++db)
+#pragma unroll
+              for (int b = 0; b < 4; ++b) {
+                const f32x4 x = *(const PAT_LDS f32x4*)(result + row * OROW + db * 32 + b * 8 + h2 * 4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc2[db][4 * b + r] = __builtin_fmaf(x[r], wb, acc2[db][4 * b + r] * wa);
+              }
+          }
+          m_t = neg_inf();
+          l_t = 0.f;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) acc_o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        j = next_j;
+        t0 = next_t0;
+        tok = next_tok;
+      };
+      while ((live & (live - 1)) != 0 || t0 + kStepTokens < tok) step(std::true_type{});
+      step(std::false_type{});
+    };
     const int r_in = lane / CPR, c_in = lane % CPR;
     auto k_piece = [&](int i) { return (unsigned)(D == 128 ? c_in ^ ((RPI * i + r_in) & 15) : c_in ^ (((RPI * i + r_in) >> 1) & 7)) * 16u; };
     const unsigned v_piece = (unsigned)(D == 128 ? c_in ^ ((r_in & 3) << 2) : c_in ^ (((r_in >> 1) & 1) << 2)) * 16u;
@@ -575,14 +711,11 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       }
     };
 
-    // LDS offsets of this lane's operand reads inside a stage (token 0 of the stage; + 32 ROWB for tokens 32..)
-    unsigned k_rd[KK2], v_rd[DB2];
-#pragma unroll
-    for (int kk = 0; kk < KK2; ++kk)
-      k_rd[kk] = (unsigned)(n32 * ROWB + ((2 * kk + h2) ^ (D == 128 ? n32 & 15 : (n32 >> 1) & 7)) * 16);
-#pragma unroll
-    for (int db = 0; db < DB2; ++db)
-      v_rd[db] = (unsigned)(KTILE + (h2 * 4 + (n >> 2)) * ROWB + (db ^ (D == 128 ? n >> 2 : (n >> 3) & 1)) * 64 + (g & 1) * 32 + (n & 3) * 8);
+    // LDS offsets of this lane's operand reads inside a stage (token 0 of the stage; + 32 ROWB for tokens 32..), those of kk = 0 and
+    // db = 0: the others differ in the place inside the row alone, which is an exclusive or with 32 kk and 64 db (the stages
+    // start at multiples of a row). Kept one by one they were 10 more registers.
+    const unsigned k_rd = (unsigned)(n32 * ROWB + (h2 ^ (D == 128 ? n32 & 15 : (n32 >> 1) & 7)) * 16);
+    const unsigned v_rd = (unsigned)(KTILE + (h2 * 4 + (n >> 2)) * ROWB + (D == 128 ? n >> 2 : (n >> 3) & 1) * 64 + (g & 1) * 32 + (n & 3) * 8);
 
     // HALVES x 32 tokens of online-softmax attention for this wave's 32 rows; `stage` points at the first of them
     // (its K rows; the V rows KTILE further), t0 is that token's place in the piece. First the scores and probabilities ...
@@ -595,7 +728,8 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       for (int a = 0; a < HALVES; ++a) {
         vec8 kop[KK2];
 #pragma unroll
-        for (int kk = 0; kk < KK2; ++kk) kop[kk] = *(const PAT_LDS vec8*)(stage + k_rd[kk] + a * 32 * ROWB);
+        for (int kk = 0; kk < KK2; ++kk)
+          kop[kk] = *(const PAT_LDS vec8*)((const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + k_rd) ^ (kk * 32u)) + a * 32 * ROWB);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[a][i] = 0.f;
@@ -648,7 +782,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       auto read_v = [&](int t, s16x8 (&v)[DB2]) {
 #pragma unroll
         for (int db = 0; db < DB2; ++db) {
-          const PAT_LDS char* src = stage + v_rd[db] + t * 16 * ROWB;
+          const PAT_LDS char* src = (const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + v_rd) ^ (db * 64u)) + t * 16 * ROWB;
           s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)src);
           s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)(src + 8 * ROWB));
           v[db] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -716,6 +850,10 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     } else {
       if (apart) walk(std::integral_constant<int, 1>{}, std::true_type{});
       else walk(std::integral_constant<int, 1>{}, std::false_type{});
+    }
+    if constexpr (TAILS) {
+      __syncthreads();   // (every wave is done with the stages)
+      walk_tails();
     }
     l_run = sum_xor32(l_run);
     if (one_tile_per_wave) {
@@ -835,7 +973,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
         }
         // the K registers are refilled as soon as the score MFMAs have read them
         attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kd[a][kk]); }, vstage,
-               t_begin + st * kStepTokens, [&]() { if (more) fetch_k(st + stride, kd); });
+               t_begin + st * kStepTokens, t_end, m_run, l_run, [&]() { if (more) fetch_k(st + stride, kd); });
       };
       int st = step0;
       for (; st + stride < nsteps; st += stride) step(st, std::true_type{});
@@ -910,12 +1048,12 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   }
 }
 
-// Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path, V past the caches).
+// Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path, V past the caches, tails).
 typedef void (*SplitFn)(const char*, int, int, int, const SplitParams);
-template <bool DIRECT, int TALLK, bool STREAM>
+template <bool DIRECT, int TALLK, bool STREAM, bool TAILS = false>
 static SplitFn split_instance(bool bf16, int head_dim) {
-  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM>;
-  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM>;
+  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM, TAILS> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM, TAILS>;
+  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM, TAILS> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM, TAILS>;
 }
 template <bool STREAM>
 static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
@@ -925,16 +1063,17 @@ static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
 
 hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const SplitParams& params) {
   const bool t32 = params.tall_rows != 16;
-  const bool past = params.stream_v != 0;
-  SplitFn fn = past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
+  const bool past = params.stream_v != 0, tails = params.tail_pages > 0;   // (never both, and tails in the 32-row form only)
+  SplitFn fn = tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
+             : past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
   const unsigned lds = (unsigned)split_smem_bytes(head_dim, t32 ? 32 : 16);
   // more dynamic LDS than the default limit of a kernel: raised once per instance and device
   {
     static std::mutex mutex;
-    static bool raised[64][32] = {{false}};
+    static bool raised[64][64] = {{false}};
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const int inst = (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
+    const int inst = (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
     std::lock_guard<std::mutex> lock(mutex);
     if (dev >= 0 && dev < 64 && !raised[dev][inst]) {
       if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -82,19 +82,22 @@ struct Prepared {
   size_t need_inline = 0;   // workspace bytes when the launch builds its records itself (args.records NULL)
   bool derive_slots = false;   // the plan came without slot tables: ordinals derived on the device
   std::vector<size_t> item_buckets;   // buckets with an item table (see use_items)
+  std::vector<std::pair<size_t, int>> tail_buckets;   // buckets with the flags that their tails, or tables of them, go by
   bool items_on = false;    // ... and whether `buckets` hands them to the launch
   bool records_items = false;   // the same when `records` were built
   pat_fwd_tuning tuning;    // the measured geometry of this plan shape (args.tuning points here when set)
   Prepared() { std::memset(&args, 0, sizeof(args)); std::memset(&tuning, 0, sizeof(tuning)); }
 };
 
-// Hands the plan's item tables (boxes that one workgroup may serve together) to the launch, or keeps them back. An item
+// Hands the plan's item tables (boxes that one workgroup may serve together) and its tails (PAT_BUCKET_TAILS: which short box
+// belongs to which sequence of a tall one) to the launch, or keeps them back. An item
 // is a statement about the tables' contents - its boxes have the same length and blocks, and the launch reads those of the
 // first box only - so it goes with a snapshot of tables nobody has written to since the planner made them
 // (KernelInfo::items_hold); wherever the tables are read as they are at the time, every box stands alone.
 void use_items(Prepared& L, bool on) {
   if (L.items_on == on) return;
   for (size_t i : L.item_buckets) L.buckets[i].flags ^= PAT_BUCKET_ITEMS;
+  for (const auto& t : L.tail_buckets) L.buckets[t.first].flags ^= t.second;
   L.items_on = on;
 }
 
@@ -260,6 +263,7 @@ struct PlanTables {
   const std::vector<std::vector<int>>* mnw;
   const std::vector<int>* flags;                 // may be null
   const TensorList* items = nullptr;             // per bucket [items, 2] (PAT_BUCKET_ITEMS) or empty; may be null
+  int32_t tails = 0;                             // pat_flat_plan.tails of these buckets
 };
 
 // Checks that need tensor metadata follow csrc/api.h:131-181, :256-277 of the reference.
@@ -335,6 +339,11 @@ std::shared_ptr<Prepared> prepare(const at::Tensor& q, const at::Tensor& k, cons
       fb.num_items = (int32_t)(*pt.items)[i].size(0);
       L->item_buckets.push_back(i);
       L->keep.push_back((*pt.items)[i]);
+    }
+    if (const uint32_t word = (uint32_t)pt.tails; word != 0 && i < PAT_MAX_FLAT_BUCKETS) {
+      const int flags = ((word >> (8 + i)) & 1 ? PAT_BUCKET_TAIL | (int)(word & 0xff) << PAT_TAIL_BOXES_SHIFT : 0) |
+                        ((word >> (20 + i)) & 1 ? PAT_BUCKET_TAILS : 0);
+      if (flags != 0) L->tail_buckets.emplace_back(i, flags);
     }
   }
   L->keep.push_back(num_split);
@@ -1025,7 +1034,7 @@ std::shared_ptr<Prepared> prepare_tree(const at::Tensor& q, const at::Tensor& k,
   PlanTables pt{l ? &info.l_q_tables : &info.q_tables, l ? &info.l_block_tables : &info.block_tables,
                 l ? &info.l_num_seqs : &info.num_seqs, l ? &info.l_ranks : &info.ranks, l ? &info.l_kvs : &info.kvs,
                 l ? &info.l_slot_tables : &info.slot_tables, l ? &info.l_mnws : &info.mnws,
-                l ? &info.l_flags : &no_flags, l ? &info.l_items : nullptr};
+                l ? &info.l_flags : &no_flags, l ? &info.l_items : nullptr, l ? info.layout.tails : 0};
   require(!pt.mnw->empty(), "the tree has no plan: call pack_schedule and kernel_info.to_gpu first");
   if (info.whole_seqs && !info.ws_q_table.empty()) {
     // a small batch of short requests: one work item per request, one kernel (see KernelInfo::whole_seqs)
@@ -1196,6 +1205,7 @@ PYBIND11_MODULE(_prefix_attn, m) {
           d["num_workgroups"] = g.num_workgroups; d["tall_rows"] = g.tall_rows;
           d["pairs"] = (g.flags & PAT_GEOMETRY_PAIRS) != 0; d["apart"] = (g.flags & PAT_GEOMETRY_APART) != 0;
           d["stream_v"] = (g.flags & PAT_GEOMETRY_STREAM_V) != 0;
+          d["tails"] = (g.flags & PAT_GEOMETRY_TAILS) != 0;
           d["merge"] = (g.flags >> PAT_GEOMETRY_MERGE_SHIFT) & 7;
           out.append(d);
         }
