@@ -311,13 +311,17 @@ typedef struct pat_fwd_tuning {
                                      /* + PAT_STREAM_V_ALWAYS / _NEVER: V of boxes <= 16 rows read  */
                                      /* past the caches, in pieces that no other of up to 64 boxes  */
                                      /* of the bucket and no tall box reads; + PAT_TAILS_ALWAYS /   */
-                                     /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS). */
+                                     /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS); */
+                                     /* + PAT_WAVES_8 / _4: waves per workgroup of single-slot      */
+                                     /* launches without tall boxes.                                */
                                      /* Values with other bits, negative ones too: 0                */
 } pat_fwd_tuning;
 #define PAT_STREAM_V_ALWAYS 4 /* (neither: chosen per launch from its sizes) */
 #define PAT_STREAM_V_NEVER 8
 #define PAT_TAILS_ALWAYS 32   /* (where the launch can, neither: chosen per launch from its sizes) */
 #define PAT_TAILS_NEVER 64
+#define PAT_WAVES_8 128       /* (where the launch can, neither: chosen per launch from its sizes) */
+#define PAT_WAVES_4 256
 int pat_fwd_set_tuning(const pat_fwd_tuning* tuning);
 int pat_fwd_get_tuning(pat_fwd_tuning* out);
 
@@ -476,6 +480,7 @@ typedef struct pat_fwd_geometry {
 #define PAT_GEOMETRY_APART 2 /* 32-row form: K and V tiles handed over apart         */
 #define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows may be read past the caches (pieces of one reader, where there is enough) */
 #define PAT_GEOMETRY_TAILS 8 /* tails are walked by the workgroups of their sequences' tall boxes */
+#define PAT_GEOMETRY_WAVES_8 16 /* eight waves per workgroup */
 #define PAT_GEOMETRY_MERGE_SHIFT 8 /* (flags >> 8) & 7, the merge kernel's form: 0 no merge, 1 a wave per row, 2 a half-wave, */
                                    /* 3 / 4 a workgroup of four / eight waves, every slot at once, 5 / 6 the filled slots only */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);

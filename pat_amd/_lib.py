@@ -91,10 +91,13 @@ PAT_STREAM_V_ALWAYS = 4
 PAT_STREAM_V_NEVER = 8
 PAT_TAILS_ALWAYS = 32
 PAT_TAILS_NEVER = 64
+PAT_WAVES_8 = 128
+PAT_WAVES_4 = 256
 PAT_GEOMETRY_PAIRS = 1
 PAT_GEOMETRY_APART = 2
 PAT_GEOMETRY_STREAM_V = 4
 PAT_GEOMETRY_TAILS = 8
+PAT_GEOMETRY_WAVES_8 = 16
 PAT_GEOMETRY_MERGE_SHIFT = 8
 
 

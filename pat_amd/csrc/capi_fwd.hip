@@ -82,12 +82,13 @@ pat_fwd_tuning tuning() {
   return g_tuning;
 }
 
-// The three switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, and tails. Values outside the declared bits,
+// The switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, tails, and waves per workgroup. Values outside the declared bits,
 // -1 among them, ask for none.
 int switches(const pat_fwd_tuning& t, int bits) {
-  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER;
+  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER | PAT_WAVES_8 | PAT_WAVES_4;
   return t.pairs >= 0 && (t.pairs & ~kDeclared) == 0 ? t.pairs & bits : 0;
 }
+int waves_switch(const pat_fwd_tuning& t) { return switches(t, PAT_WAVES_8 | PAT_WAVES_4); }
 int pairs_switch(const pat_fwd_tuning& t) { return switches(t, 3); }
 int stream_switch(const pat_fwd_tuning& t) { return switches(t, PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER); }
 int tails_switch(const pat_fwd_tuning& t) { return switches(t, PAT_TAILS_ALWAYS | PAT_TAILS_NEVER); }
@@ -112,6 +113,7 @@ struct Geometry {
   bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
   bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches ...
   int stream_tokens = -1;    // ... where these boxes hold so many tokens (the record kernel counts)
+  int waves = kWaves;        // waves per workgroup of the split kernel
   bool tails = false;        // tails are walked by their sequences' tall workgroups (PAT_BUCKET_TAILS)
   int tail_pages = 0;        // ... pages per tail in the records
   bool direct = false;       // one slot per row: the split kernel writes `out`, no workspace, no merge kernel
@@ -569,6 +571,24 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
   // pat_fwd_tuning.direct_out = 0 keeps the two-kernel route (tests).
   g->direct = g->num_slots == 1 && reinterpret_cast<uintptr_t>(a->out) % 8 == 0 && a->o_stride[0] % 4 == 0 &&
               a->o_stride[2] % 4 == 0 && tune.direct_out != 0;
+  // Eight waves per workgroup: single-slot launches of few workgroups, boxes of more than eight 32-token steps. A wave of four has three
+  // steps and more then, each a trip to memory behind the last; eight halve them, and softmaxes over fewer tokens each are rounded no
+  // worse. us per call, four / eight waves: head_dim 64, 2 requests of 306..459 at 64/8 heads (16 workgroups) 6.5 / 5.3, 20 of 370 (160) 5.9 / 5.1,
+  // 9 of 282 at 16/16 (144) 5.6 / 4.9, but 28 of 240..350 at 8/8 (224) 5.95 / 6.05 and, of up to eight steps, 28 of 106 at 16/8 (224) 4.5 / 4.8;
+  // head_dim 128, where a CU takes in a longer box no faster than four waves ask for it, 17 of 188..282 at 8/8 (136) 6.8 / 6.3, 1 of
+  // 336..512 at 32/32 (32) 8.1 / 7.5, but 8 of 300..512 at 8/8 (64) 8.24 / 8.27, 16 at 32/8 (128) 8.7 / 9.1.
+  if (g->direct && !g->stream_v) {
+    int64_t widest = 0;
+    bool plain = true;
+    for (int i = 0; i < a->num_buckets; ++i) {
+      if (a->buckets[i].num_boxes == 0) continue;
+      widest = std::max<int64_t>(widest, (int64_t)a->buckets[i].max_blocks * page);
+      plain = plain && row_tiles(a->buckets[i].mnw[0]) == 1 && g->bucket_heads_per_wg[i] == 1;
+    }
+    const int forced = waves_switch(tune);
+    const bool few = g->total_wgs <= kNumCUs / 4 || (g->total_wgs <= 5 * kNumCUs / 8 && (a->head_dim == 64 || widest <= 12 * kStepTokens));
+    if (plain && !(forced & PAT_WAVES_4) && ((forced & PAT_WAVES_8) || (few && widest > 8 * kStepTokens))) g->waves = 8;
+  }
   if (g->total_wgs > (int64_t)kGridX * 65535 || g->total_wgs >= INT32_MAX)
     return fail(PAT_ERR_INVALID, "too many workgroups for one launch");
   for (int i = 0; i < a->num_buckets; ++i) {
@@ -753,7 +773,7 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   out->tall_rows = g.tall_rows;
   const int merge = g.direct ? pat::kMergeNone : pat::merge_form((int64_t)args->batch * args->heads, g.num_slots, args->head_dim);
   out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0) |
-               (g.tails ? PAT_GEOMETRY_TAILS : 0) |
+               (g.tails ? PAT_GEOMETRY_TAILS : 0) | (g.waves == 8 ? PAT_GEOMETRY_WAVES_8 : 0) |
                merge << PAT_GEOMETRY_MERGE_SHIFT;
   return PAT_OK;
 }
@@ -1068,6 +1088,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   sp.stream_v = g.stream_v ? 1 : 0;
   sp.tall_apart = g.tall_apart ? 1 : 0;
   sp.tail_pages = g.tail_pages;
+  sp.waves = g.waves;
   if (g.direct) {
     sp.out = args->out; sp.lse_out = args->lse_out;
     sp.o_stride_b = args->o_stride[0]; sp.o_stride_h = args->o_stride[2];

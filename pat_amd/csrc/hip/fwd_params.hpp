@@ -100,6 +100,7 @@ struct SplitParams {
   int32_t direct;    // 1: such a launch
   int32_t tall_apart;  // 32-row form: K and V tiles of a super-step handed over apart (see the kernel)
   int32_t stream_v;  // records may ask for V past the caches (host side: picks the kernel instance)
+  int32_t waves;     // waves per workgroup (host side: picks the kernel instance)
   int32_t tail_pages; // tails: pages per tail in the records, 0: the launch has none
   int32_t tall_rows; // rows per wave on boxes of 17..64 rows: 32 (32x32x16 tiles) or 16 (host side: picks the kernel instance)
 };

@@ -89,10 +89,10 @@ __host__ __device__ constexpr int split_occupancy(int head_dim, int tallk) {
 }
 
 // LDS bytes of one workgroup (dynamic: more than the 64 KB a static allocation may have).
-__host__ __device__ constexpr int split_smem_bytes(int D, int tallk) {
-  const int wave_private = kWaves * kStepTokens * (D * 2 + 32);     // 4 private V tiles
-  const int combine = kWaves * 16 * (D + 4) * 4;                     // short boxes: the waves' states
-  const int tall = tallk == 32 ? 2 * (2 * kStepTokens) * 2 * (D * 2)                     // two stages of 64 K rows + 64 V rows
+__host__ __device__ constexpr int split_smem_bytes(int D, int tallk, int waves = kWaves) {
+  const int wave_private = waves * kStepTokens * (D * 2 + 32);      // private V tiles
+  const int combine = waves * 16 * (D + 4) * 4;                      // short boxes: the waves' states
+  const int tall = tallk == 0 ? 0 : tallk == 32 ? 2 * (2 * kStepTokens) * 2 * (D * 2)                     // two stages of 64 K rows + 64 V rows
                                : 2 * kStepTokens * ((D * 2 + 16) + (D * 2 + 32));        // two stages of 32 K rows + 32 V rows
   int m = wave_private > combine ? wave_private : combine;
   return m > tall ? m : tall;
@@ -107,9 +107,12 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
 // DIRECT instances serve launches in which every row has one partial slot: they store `out`. STREAM instances serve launches
 // whose records may ask for V past the caches (kRecordModeStreamV): a second loop over short boxes, whose mere presence cost
 // the smallest launches 0.14 us of 5.5.
+// WAVES: 4, or 8 in instances without a tall path (TALLK 0) for single launches of few workgroups whose boxes are more than eight steps
+// long: a wave has half the steps, each a trip to memory behind the last (us per call: 8 requests of 288 tokens, 8 kv heads of 64, 64 workgroups, 5.47 / 4.66;
+// 2 of 306..459 at 64/8, head_dim 64, 6.5 / 5.3; 17 of 188..282 at 8/8, head_dim 128, 6.8 / 6.3).
 // TAILS instances (32-row form): tall workgroups also walk the tails of their rows' sequences.
-template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS>
-__global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
+template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS, int WAVES>
+__global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
                                                                              const int record_max_seqs, const int record_max_pages, const SplitParams p) {
   using E = Elem<T>;
   using vec8 = typename E::vec8;
@@ -124,8 +127,8 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   constexpr int WSTAGE = VSTAGE;                       // one wave's private staging (V only)
 
   extern __shared__ __attribute__((aligned(256))) char smem[];
-  __shared__ float s_m[kWaves * 16];
-  __shared__ float s_l[kWaves * 16];
+  __shared__ float s_m[WAVES * 16];
+  __shared__ float s_l[WAVES * 16];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -174,7 +177,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
   // with a kv head per wave, each wave walks all steps of its own head).
   // Taller boxes: tiles shared through LDS; the 32-row form gives a wave rows 32w.. and every token, or, up to
   // 64 rows, rows 32(w&1).. and tokens 32(w>>1).. of every 64-token super-step.
-  const bool tall = (mode & 0xff) > 1;
+  const bool tall = TALLK != 0 && (mode & 0xff) > 1;
   // (both uniform, and known to be: branches on them are scalar branches)
   const bool one_tile_per_wave = R > 64;   // tall boxes, 32-row tiles: four row tiles, a wave each
   const int rt = __builtin_amdgcn_readfirstlane(one_tile_per_wave ? wave : wave & 1);   // this wave's 32-row tile
@@ -452,7 +455,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       for (int db = 0; db < DB; ++db) put4(dst + db * 16, o + db * 16, acc_o[db] * inv);
       if (g == 0) put_lse(prow, (m_run + __builtin_amdgcn_logf(l_run)) * 0.6931471805599453f);
     }
-    } else {
+    } else if constexpr (TALLK == 32) {
     // ====================== tall box: 32-row tiles, K/V shared through LDS ======================
     // The piece is walked in super-steps of 64 tokens, whose K and V rows go from memory straight into one of
     // two LDS stages (global_load_lds, 16 bytes per lane): the next super-step is in flight while the waves work
@@ -945,7 +948,7 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     };
     // steps of this wave: every kWaves-th one of the chunk, or, with a kv head per wave, all of them
     const int step0 = head_per_wave ? 0 : wave;
-    const int stride = head_per_wave ? 1 : kWaves;
+    const int stride = head_per_wave ? 1 : WAVES;
     auto walk = [&](auto stream_c) {
       u32x4 kd[2][KK], vd[NV];
       fetch_v(step0, vd, stream_c);
@@ -1008,8 +1011,9 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     } else {
     // combine the 4 waves' states through LDS and write the partial
     float* cbuf = (float*)smem;
-    const int crow = tid >> 4;                 // row this thread finalises
-    const int ccol = (tid & 15) * (D / 16);    // its first column
+    constexpr int COLS = 16 * D / (WAVES * 64) > 4 ? 16 * D / (WAVES * 64) : 4;   // columns a thread finalises
+    const int crow = tid / (D / COLS);          // row this thread finalises (past 16: none)
+    const int ccol = (tid % (D / COLS)) * COLS; // its first column
     __syncthreads();  // every wave is done with its staging region
     if (g == 0) { s_m[wave * 16 + n] = m_run; s_l[wave * 16 + n] = l_run; }
 #pragma unroll
@@ -1018,14 +1022,14 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
     __syncthreads();
 
     // the slot of row crow sits in lane crow of every wave
-    const int cslot0 = __shfl(my_slot0, crow);
-    if (cslot0 >= 0) {
-      float mw[kWaves], mmax = neg_inf();
+    const int cslot0 = __shfl(my_slot0, crow & 15);
+    if (cslot0 >= 0 && crow < 16) {
+      float mw[WAVES], mmax = neg_inf();
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) { mw[w] = s_m[w * 16 + crow]; mmax = fmaxf(mmax, mw[w]); }
-      float wsum = 0.f, wgt[kWaves];
+      for (int w = 0; w < WAVES; ++w) { mw[w] = s_m[w * 16 + crow]; mmax = fmaxf(mmax, mw[w]); }
+      float wsum = 0.f, wgt[WAVES];
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
+      for (int w = 0; w < WAVES; ++w) {
         wgt[w] = fast_exp2(mw[w] - mmax);   // a wave without steps has m = -inf -> weight 0
         wsum += wgt[w] * s_l[w * 16 + crow];
       }
@@ -1034,14 +1038,14 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
       float* dst = p.o_part + prow * D + ccol;
       T* od = direct ? row_out(cslot0) + ccol : nullptr;
 #pragma unroll
-      for (int c = 0; c < D / 16; c += 4) {
+      for (int c = 0; c < COLS; c += 4) {
         f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w)
+        for (int w = 0; w < WAVES; ++w)
           o += *(const f32x4*)(cbuf + (w * 16 + crow) * OROW + ccol + c) * wgt[w];
         put4(dst + c, od + c, o * inv);
       }
-      if ((tid & 15) == 0)
+      if (ccol == 0)
         put_lse(prow, (mmax + __builtin_amdgcn_logf(wsum)) * 0.6931471805599453f);
     }
     }   // combine
@@ -1050,10 +1054,10 @@ __global__ void __launch_bounds__(kThreads, split_occupancy(D, TALLK)) pat_split
 
 // Host launcher: picks the instance for (element type, head_dim, single-slot launch, form of the tall path, V past the caches, tails).
 typedef void (*SplitFn)(const char*, int, int, int, const SplitParams);
-template <bool DIRECT, int TALLK, bool STREAM, bool TAILS = false>
+template <bool DIRECT, int TALLK, bool STREAM, bool TAILS = false, int WAVES = kWaves>
 static SplitFn split_instance(bool bf16, int head_dim) {
-  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM, TAILS> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM, TAILS>;
-  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM, TAILS> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM, TAILS>;
+  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES>;
+  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES>;
 }
 template <bool STREAM>
 static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
@@ -1064,16 +1068,18 @@ static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
 hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const SplitParams& params) {
   const bool t32 = params.tall_rows != 16;
   const bool past = params.stream_v != 0, tails = params.tail_pages > 0;   // (never both, and tails in the 32-row form only)
-  SplitFn fn = tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
+  const int waves = params.waves;   // (eight: single-slot launches without tall boxes)
+  SplitFn fn = waves == 8 ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
+             : tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
              : past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
-  const unsigned lds = (unsigned)split_smem_bytes(head_dim, t32 ? 32 : 16);
+  const unsigned lds = (unsigned)split_smem_bytes(head_dim, waves != kWaves ? 0 : t32 ? 32 : 16, waves);
   // more dynamic LDS than the default limit of a kernel: raised once per instance and device
   {
     static std::mutex mutex;
-    static bool raised[64][64] = {{false}};
+    static bool raised[64][128] = {{false}};
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const int inst = (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
+    const int inst = (waves == 8 ? 64 : 0) + (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
     std::lock_guard<std::mutex> lock(mutex);
     if (dev >= 0 && dev < 64 && !raised[dev][inst]) {
       if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1084,7 +1090,7 @@ hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const Split
   }
   const unsigned wgs = (unsigned)params.total_items;
   const dim3 grid(wgs < (unsigned)kGridX ? wgs : (unsigned)kGridX, (wgs + kGridX - 1) / kGridX);
-  hipLaunchKernelGGL(fn, grid, dim3(kThreads), lds, stream, params.records, params.record_stride, params.record_max_seqs,
+  hipLaunchKernelGGL(fn, grid, dim3((unsigned)waves * 64u), lds, stream, params.records, params.record_stride, params.record_max_seqs,
                      params.record_max_pages, params);
   return hipGetLastError();
 }

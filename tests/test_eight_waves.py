@@ -1,0 +1,75 @@
+"""Single-slot launches of few workgroups run eight waves per workgroup: when they do, and the results at the edges of the waves' steps."""
+import ctypes as C
+import math
+
+import pytest
+import torch
+
+from oracle import attn_oracle as ao
+from pat_amd import PrefixTreeCPP, _lib, prefix_attn_with_kvcache, workloads
+
+
+def _args(requests, tokens, heads, kv_heads, d, page=16):
+    b = (_lib.FwdBucket * 1)()
+    b[0].q_table = b[0].block_table = b[0].num_seqs = b[0].rank = b[0].kv = 0x10000
+    b[0].mnw[:] = [16, 128, 1]
+    b[0].num_boxes, b[0].max_seqs, b[0].max_blocks = requests, 1, tokens // page
+    b[0].q_table_stride, b[0].block_table_stride = 1, tokens // page
+    a = _lib.FwdArgs()
+    a.dtype, a.batch, a.seqlen_q, a.heads, a.kv_heads = _lib.PAT_DTYPE_F16, requests, 1, heads, kv_heads
+    a.head_dim, a.page_size, a.num_pages = d, page, 1 << 16
+    a.q = a.k = a.v = a.out = a.num_split_per_seq = 0x10000
+    a.q_stride = a.o_stride = (C.c_int64 * 3)(heads * d, heads * d, d)
+    a.k_stride = a.v_stride = (C.c_int64 * 3)(page * kv_heads * d, kv_heads * d, d)
+    a.max_split_per_seq, a.max_seqs_in_box, a.max_blocks_in_box, a.softmax_scale = 1, 1, tokens // page, 0.1
+    a.num_buckets, a.buckets = 1, C.cast(b, C.POINTER(_lib.FwdBucket))
+    a._keep = b
+    return a
+
+
+@pytest.mark.parametrize("requests,tokens,heads,d,eight", [
+    (8, 288, (8, 8), 64, True), (8, 256, (8, 8), 64, False),          # more than eight steps
+    (20, 384, (8, 8), 64, True), (21, 384, (8, 8), 64, False),        # 160 workgroups at most ...
+    (20, 384, (8, 8), 128, True), (20, 400, (8, 8), 128, False),      # ... at head_dim 128 for boxes of up to twelve steps,
+    (8, 512, (8, 8), 128, True), (9, 512, (8, 8), 128, False),        # 64 for longer ones
+    (8, 528, (8, 8), 64, False),                                      # cut into pieces: a merge follows
+])
+def test_launch_rule(requests, tokens, heads, d, eight, tuning):
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    for switch, want in ((0, eight), (_lib.PAT_WAVES_4, False), (_lib.PAT_WAVES_8, tokens <= 512)):
+        tuning(pairs=switch)
+        assert lib.pat_fwd_geometry_of(C.byref(_args(requests, tokens, *heads, d)), C.byref(g)) == 0, _lib.last_error()
+        assert bool(g.flags & _lib.PAT_GEOMETRY_WAVES_8) == want, switch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,d,dtype,page", [((8, 8), 64, torch.float16, 16), ((16, 2), 128, torch.bfloat16, 48),
+                                                ((32, 8), 128, torch.float16, 32), ((16, 8), 64, torch.bfloat16, 64)])
+def test_against_the_oracle(heads, d, dtype, page, tuning, monkeypatch):
+    print(f"[case] eight waves, heads {heads}, d {d}, {dtype}, page {page}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "1")
+    dev = torch.device("cuda:0")
+    # waves without a step, a last step of one token, one and two steps per wave and one token more
+    lens = [n for n in (1, 31, 33, 224, 255, 256, 257, 288, 480, 511, 512) if -(-n // page) * page <= 512]
+    rows, nxt = [], 0
+    for n in lens:
+        rows.append(list(range(nxt, nxt + -(-n // page))))
+        nxt += -(-n // page)
+    w = workloads.Workload("eight", heads[0], heads[1], d, dtype, page, lens, rows, nxt, 0, 2)
+    q, k, v = w.tensors(dev)
+    ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, lens)
+    for switch in (_lib.PAT_WAVES_8, _lib.PAT_WAVES_4):
+        tuning(pairs=switch)
+        tree = PrefixTreeCPP(page)
+        tree.build_radix_tree(lens, w.padded_table())
+        tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+        tree.kernel_info.to_gpu(dev)
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((w.batch, w.heads), float("nan"), dtype=torch.float32, device=dev)
+        prefix_attn_with_kvcache(q, k, v, tree, 1.0 / math.sqrt(d), out, softmax_lse=lse)
+        torch.cuda.synchronize()
+        assert [g["waves"] for g in tree.kernel_info._launch_geometries] == [8 if switch == _lib.PAT_WAVES_8 else 4]
+        err = (out.float().cpu() - ref_out.float()).abs().max().item()
+        lerr = ((lse.cpu() - ref_lse).abs() / ref_lse.abs().clamp_min(1.0)).max().item()
+        print(f"[parity] {err:.3e} {lerr:.3e}", flush=True)
+        assert err <= (2e-3 if dtype == torch.float16 else 1.6e-2) and lerr <= 1e-4
