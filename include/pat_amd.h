@@ -313,7 +313,9 @@ typedef struct pat_fwd_tuning {
                                      /* of the bucket and no tall box reads; + PAT_TAILS_ALWAYS /   */
                                      /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS); */
                                      /* + PAT_WAVES_8 / _4: waves per workgroup of single-slot      */
-                                     /* launches without tall boxes.                                */
+                                     /* launches without tall boxes; + PAT_LISTS_ALWAYS / _NEVER:   */
+                                     /* short private boxes several per workgroup (32-row form,     */
+                                     /* head_dim 128).                                              */
                                      /* Values with other bits, negative ones too: 0                */
 } pat_fwd_tuning;
 #define PAT_STREAM_V_ALWAYS 4 /* (neither: chosen per launch from its sizes) */
@@ -322,6 +324,8 @@ typedef struct pat_fwd_tuning {
 #define PAT_TAILS_NEVER 64
 #define PAT_WAVES_8 128       /* (where the launch can, neither: chosen per launch from its sizes) */
 #define PAT_WAVES_4 256
+#define PAT_LISTS_ALWAYS 512  /* (the same) */
+#define PAT_LISTS_NEVER 1024
 int pat_fwd_set_tuning(const pat_fwd_tuning* tuning);
 int pat_fwd_get_tuning(pat_fwd_tuning* out);
 
@@ -481,6 +485,7 @@ typedef struct pat_fwd_geometry {
 #define PAT_GEOMETRY_STREAM_V 4 /* V of boxes <= 16 rows may be read past the caches (pieces of one reader, where there is enough) */
 #define PAT_GEOMETRY_TAILS 8 /* tails are walked by the workgroups of their sequences' tall boxes */
 #define PAT_GEOMETRY_WAVES_8 16 /* eight waves per workgroup */
+#define PAT_GEOMETRY_LISTS 32 /* workgroups that walk several short private boxes */
 #define PAT_GEOMETRY_MERGE_SHIFT 8 /* (flags >> 8) & 7, the merge kernel's form: 0 no merge, 1 a wave per row, 2 a half-wave, */
                                    /* 3 / 4 a workgroup of four / eight waves, every slot at once, 5 / 6 the filled slots only */
 int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out);

@@ -93,11 +93,14 @@ PAT_TAILS_ALWAYS = 32
 PAT_TAILS_NEVER = 64
 PAT_WAVES_8 = 128
 PAT_WAVES_4 = 256
+PAT_LISTS_ALWAYS = 512
+PAT_LISTS_NEVER = 1024
 PAT_GEOMETRY_PAIRS = 1
 PAT_GEOMETRY_APART = 2
 PAT_GEOMETRY_STREAM_V = 4
 PAT_GEOMETRY_TAILS = 8
 PAT_GEOMETRY_WAVES_8 = 16
+PAT_GEOMETRY_LISTS = 32
 PAT_GEOMETRY_MERGE_SHIFT = 8
 
 

@@ -82,10 +82,11 @@ pat_fwd_tuning tuning() {
   return g_tuning;
 }
 
-// The switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, tails, and waves per workgroup. Values outside the declared bits,
+// The switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, tails, waves per workgroup, and lists. Values outside the declared bits,
 // -1 among them, ask for none.
 int switches(const pat_fwd_tuning& t, int bits) {
-  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER | PAT_WAVES_8 | PAT_WAVES_4;
+  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER | PAT_WAVES_8 | PAT_WAVES_4 | PAT_LISTS_ALWAYS |
+                            PAT_LISTS_NEVER;
   return t.pairs >= 0 && (t.pairs & ~kDeclared) == 0 ? t.pairs & bits : 0;
 }
 int waves_switch(const pat_fwd_tuning& t) { return switches(t, PAT_WAVES_8 | PAT_WAVES_4); }
@@ -113,6 +114,8 @@ struct Geometry {
   bool pairs = false;        // the two boxes of an item (PAT_BUCKET_ITEMS) are served by one workgroup
   bool stream_v = false;     // V tiles of boxes of <= 16 rows that nobody shares are read past the caches ...
   int stream_tokens = -1;    // ... where these boxes hold so many tokens (the record kernel counts)
+  int bucket_lists[kMaxBuckets] = {0};          // boxes that a workgroup serves one after the other, 0: one
+  int list_boxes = 0, list_pages = 0;           // the most of them, and of their pages per box
   int waves = kWaves;        // waves per workgroup of the split kernel
   bool tails = false;        // tails are walked by their sequences' tall workgroups (PAT_BUCKET_TAILS)
   int tail_pages = 0;        // ... pages per tail in the records
@@ -267,6 +270,13 @@ LaunchEstimate estimate_launch(const pat_fwd_args* a, int tall_rows, bool pairs)
     }
   }
   return e;
+}
+
+void size_records(Geometry* g) {
+  g->record_max_seqs = std::min(std::max({g->record_max_seqs, 1, g->list_boxes}), 128);
+  g->record_max_pages = std::min(std::max({g->record_max_pages, 1, g->list_boxes * (1 + g->list_pages)}), kMaxChunkPages);
+  const int tail_words = g->tail_pages > 0 ? (1 + g->tail_pages) * g->record_max_seqs : 0;
+  g->record_stride = (int)((sizeof(RecordHead) + (2 * g->record_max_seqs + g->record_max_pages + tail_words) * sizeof(int32_t) + 63) / 64 * 64);
 }
 
 // Launch geometry. A workgroup streams one chunk of one box's KV for one kv head; a bucket
@@ -596,10 +606,7 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
     g->record_max_seqs = std::max(g->record_max_seqs, (int)a->buckets[i].max_seqs * (items_of(a->buckets[i], pairs) < a->buckets[i].num_boxes ? 2 : 1));
     g->record_max_pages = std::max(g->record_max_pages, (int)ceil_div64(g->bucket_chunk[i], page));
   }
-  g->record_max_seqs = std::min(std::max(g->record_max_seqs, 1), 128);
-  g->record_max_pages = std::min(std::max(g->record_max_pages, 1), kMaxChunkPages);
-  const int tail_words = g->tail_pages > 0 ? (1 + g->tail_pages) * g->record_max_seqs : 0;
-  g->record_stride = (int)((sizeof(RecordHead) + (2 * g->record_max_seqs + g->record_max_pages + tail_words) * sizeof(int32_t) + 63) / 64 * 64);
+  size_records(g);
   // the kernels index partial rows with 32-bit integers
   if ((int64_t)a->batch * a->heads * g->num_slots >= ((int64_t)1 << 31))
     return fail(PAT_ERR_INVALID, "batch * heads * partial slots must stay below 2^31");
@@ -625,7 +632,48 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
 // part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
 // boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice
 // as often to be as many, only add partial rows (4 boxes x 8 of 2048 tokens: 22.4 / 23.5).
-int plan_boxes(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
+// Lists: workgroups that walk several private boxes of one step each, one after the other (32-row form at head_dim 128, whose
+// two places per CU such boxes queue for). A workgroup of one of them is 4-5 us of launch, record, page ids, first tiles and
+// stores for half a microsecond of work; in a list a further box costs 2-2.5 us. Taken where the launch holds 1.75 times what
+// fits at once and all of it fits with the boxes in lists, so that nothing starts late any more. us per call, a box a workgroup /
+// lists: 512 x (1408 + 32) tokens at 16/8 heads (1280 workgroups, 512 with lists of four) 32.0 / 28.7, 245 x (1696 + 352 + 3..6)
+// at 16/16 (1236, 504) 23.9 / 21.0, 240 x (1968 + 4..16) at 32/32 34.7 / 31.6, 945 x (1376 + 1..4) at 8/8 30.7 / 27.9. Of 250
+// drawn batches of short ends the rule takes 24: geometric mean 0.978, the slowest 1.02. Outside of it: some still wait, 499 x
+// (864 + 4..8) at 32/8 31.3 / 34.4; fewer workgroups, 339 x (384 + 96 + 8..16) at 64/8 (878) 27.2 / 32.1, 310 x (1104 + 144 +
+// 7..28) at 8/8 (852) 17.1 / 17.9; two steps and more, 175 x (1248 + 320 + 11..44) at 16/16 22.8 / 24.6; head_dim 64 (three
+// places per CU): 100 batches 0.99, fourteen of them 2-13 % slower.
+void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) {
+  const int forced = switches(tune, PAT_LISTS_ALWAYS | PAT_LISTS_NEVER);
+  if (g->tall_rows != 32 || a->head_dim != 128 || g->direct || g->stream_v || g->tail_pages > 0 || a->kv_heads % kWaves != 0 || (forced & PAT_LISTS_NEVER)) return;
+  auto fits = [&](int i) {
+    const pat_fwd_bucket& b = a->buckets[i];
+    return b.num_boxes > 0 && row_tiles(b.mnw[0]) == 1 && b.max_seqs == 1 && g->bucket_chunks[i] == 1 &&
+           (int64_t)b.max_blocks * a->page_size <= kStepTokens && g->bucket_heads_per_wg[i] == kWaves;
+  };
+  int64_t others = 0, single = 0;
+  int pages = 0;
+  for (int i = 0; i < a->num_buckets; ++i) {
+    if (a->buckets[i].num_boxes == 0) continue;
+    const int64_t wgs = items_of(a->buckets[i], g->pairs) * g->bucket_chunks[i] * (a->kv_heads / g->bucket_heads_per_wg[i]);
+    (fits(i) ? single : others) += wgs;
+    if (fits(i)) pages = std::max(pages, (int)a->buckets[i].max_blocks);
+  }
+  if (single == 0) return;
+  const int64_t resident = (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs;
+  if (!(forced & PAT_LISTS_ALWAYS) && (others >= resident || 4 * (others + single) < 7 * resident)) return;
+  const int64_t per = std::max<int64_t>(2, std::min<int64_t>(kMaxListBoxes, ceil_div64(single, std::max<int64_t>(1, resident - others))));
+  auto saved = [&](int i) { return ((int64_t)a->buckets[i].num_boxes - ceil_div64(a->buckets[i].num_boxes, per)) * (a->kv_heads / kWaves); };
+  int64_t total = others + single;
+  for (int i = 0; i < a->num_buckets; ++i) total -= fits(i) ? saved(i) : 0;
+  if (!(forced & PAT_LISTS_ALWAYS) && total > resident) return;
+  for (int i = 0; i < a->num_buckets; ++i) g->bucket_lists[i] = fits(i) ? (int)per : 0;
+  g->total_wgs = total;
+  g->list_boxes = (int)per;
+  g->list_pages = pages;
+  size_records(g);
+}
+
+int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
   g->tail_pages = tail_pages;
   int64_t widest_tall = 0, tall_box_heads = 0;
@@ -700,15 +748,17 @@ int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
   const int forced = tails_switch(tune);
   WithoutTails w;
-  if ((forced & PAT_TAILS_NEVER) || tune.tall_rows == 16 || !w.make(a)) return plan_boxes(a, g, 0);
-  Geometry with;
-  const bool can = plan_boxes(&w.args, &with, w.tail_pages) == PAT_OK && with.tall_rows == 32 && !with.stream_v;
-  if (!can || !(forced & PAT_TAILS_ALWAYS)) {
-    if (int rc = plan_boxes(a, g, 0)) return rc;
-    if (!can || !tails_pay(a, with, *g)) return PAT_OK;
+  if (!(forced & PAT_TAILS_NEVER) && tune.tall_rows != 16 && w.make(a)) {
+    Geometry with, without;
+    if (plan_form(&w.args, &with, w.tail_pages) == PAT_OK && with.tall_rows == 32 && !with.stream_v &&
+        ((forced & PAT_TAILS_ALWAYS) || (plan_form(a, &without, 0) == PAT_OK && tails_pay(a, with, without)))) {
+      *g = with;
+      g->tails = true;
+      return PAT_OK;
+    }
   }
-  *g = with;
-  g->tails = true;
+  if (int rc = plan_form(a, g, 0)) return rc;
+  make_lists(a, tune, g);
   return PAT_OK;
 }
 
@@ -745,6 +795,7 @@ uint64_t records_tag(const pat_fwd_args* a, const Geometry& g) {
     mix((uint64_t)reinterpret_cast<uintptr_t>(b.kv)); mix((uint64_t)reinterpret_cast<uintptr_t>(b.q_slot));
     if (g.pairs) mix((uint64_t)items_of(b, true));
     if (g.tails) { mix((uint64_t)b.flags); mix((uint64_t)b.num_items); }
+    mix((uint64_t)g.bucket_lists[i]);
   }
   return h ? h : 1;
 }
@@ -774,6 +825,7 @@ int pat_fwd_geometry_of(const pat_fwd_args* args, pat_fwd_geometry* out) {
   const int merge = g.direct ? pat::kMergeNone : pat::merge_form((int64_t)args->batch * args->heads, g.num_slots, args->head_dim);
   out->flags = (g.pairs ? PAT_GEOMETRY_PAIRS : 0) | (g.tall_apart && g.tall_rows == 32 ? PAT_GEOMETRY_APART : 0) | (g.stream_v ? PAT_GEOMETRY_STREAM_V : 0) |
                (g.tails ? PAT_GEOMETRY_TAILS : 0) | (g.waves == 8 ? PAT_GEOMETRY_WAVES_8 : 0) |
+               (g.list_boxes > 0 ? PAT_GEOMETRY_LISTS : 0) |
                merge << PAT_GEOMETRY_MERGE_SHIFT;
   return PAT_OK;
 }
@@ -892,6 +944,45 @@ __device__ __forceinline__ ModeWord write_record(const RecordParams& p, int wg, 
   // chunks, land on the same engines every time and leave the others idle.
   const int chunk = local / bk.num_items;
   const int item = local - chunk * bk.num_items;
+  if (bk.list_boxes > 0) {
+    // several boxes of one sequence each: what they are, a lane each, then their pages
+    const int first = item * bk.list_boxes, count = min(bk.list_boxes, bk.num_boxes - first);
+    char* rec = p.records + (size_t)wg * (size_t)p.record_stride;
+    int32_t* tab = reinterpret_cast<int32_t*>(rec + sizeof(RecordHead));
+    if (lane == 0) {
+      RecordHead h;
+      h.tokens = count; h.rows = 0; h.mode = 1 | kRecordModeHeadPerWave | kRecordModeList; h.head = hgroup * bk.heads_per_wg;
+      h.fill_begin = 0; h.fill_end = p.chunks_per_rank;
+      h.pad[0] = h.pad[1] = 0;
+      *reinterpret_cast<RecordHead*>(rec) = h;
+    }
+    for (int j = lane; j < p.record_max_seqs; j += 64) {
+      int seq = -1, slot = -1;
+      if (j < count && bk.num_seqs[first + j] > 0) {
+        const int64_t at = (int64_t)(first + j) * bk.q_stride;
+        if ((unsigned)bk.q_table[at] < (unsigned)p.batch) seq = bk.q_table[at];
+        const int ord = bk.q_slot ? bk.q_slot[at] : bk.rank[first + j];
+        if ((unsigned)ord < (unsigned)p.max_split) slot = ord * p.chunks_per_rank;
+      }
+      tab[j] = seq;
+      tab[p.record_max_seqs + j] = slot;
+    }
+    for (int i = lane; i < p.record_max_pages; i += 64) {
+      int v = 0;
+      const int e = i - p.list_boxes, j = i < p.list_boxes ? i : e / p.list_pages, c = e - j * p.list_pages;
+      if (j < count) {
+        const int box = first + j;
+        if (i < p.list_boxes) {
+          v = max(0, min(bk.kv[box], min(bk.max_blocks, p.list_pages) * p.page_size));
+        } else {
+          v = c < bk.max_blocks ? bk.block_table[(int64_t)box * bk.bt_stride + c] : 0;
+          v = v < 0 ? 0 : (v >= p.num_pages ? p.num_pages - 1 : v);
+        }
+      }
+      tab[2 * p.record_max_seqs + i] = v;
+    }
+    return m;
+  }
   // the item's boxes (indices clamped: a malformed table gives wrong numbers, not a fault)
   int box = item, box2 = -1;
   if (bk.items != nullptr) {
@@ -1023,6 +1114,7 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
   if (g.tails && !w.make(args)) return fail(PAT_ERR_INVALID, "internal: a launch with tails has none");
   rp.max_split = g.tails ? w.args.max_split_per_seq : args->max_split_per_seq;
   rp.tail_pages = g.tail_pages;
+  rp.list_boxes = g.list_boxes; rp.list_pages = g.list_pages;
   // buckets in plan order (tall, long boxes come first in the default order)
   int nb = 0;
   int64_t items = 0;
@@ -1040,8 +1132,9 @@ int build_records(const pat_fwd_args* args, const Geometry& g, void* buffer, hip
     d.row_tiles = row_tiles(b.mnw[0]);
     d.heads_per_wg = g.bucket_heads_per_wg[i];
     d.item_begin = (int32_t)items;
-    d.num_items = tail ? 0 : (int32_t)items_of(b, g.pairs);
-    d.items = !tail && d.num_items < b.num_boxes ? b.kv + b.num_boxes : nullptr;
+    d.list_boxes = g.bucket_lists[i];
+    d.num_items = tail ? 0 : d.list_boxes > 0 ? (int32_t)ceil_div64(b.num_boxes, d.list_boxes) : (int32_t)items_of(b, g.pairs);
+    d.items = !tail && d.list_boxes == 0 && d.num_items < b.num_boxes ? b.kv + b.num_boxes : nullptr;
     d.tail_id = tail ? i : -1;
     d.tails = g.tails && (b.flags & PAT_BUCKET_TAILS) && d.row_tiles > 1 ? b.kv + b.num_boxes + 2 * (int64_t)b.num_items : nullptr;
     ++nb;
@@ -1088,6 +1181,7 @@ int launch_core(const pat_fwd_args* args, const Geometry& g, void* workspace, vo
   sp.stream_v = g.stream_v ? 1 : 0;
   sp.tall_apart = g.tall_apart ? 1 : 0;
   sp.tail_pages = g.tail_pages;
+  sp.list_boxes = g.list_boxes; sp.list_pages = g.list_pages;
   sp.waves = g.waves;
   if (g.direct) {
     sp.out = args->out; sp.lse_out = args->lse_out;

@@ -64,6 +64,8 @@ struct RecordHead {
   int32_t rows;        // rows of the box, or of the two boxes of an item (sequences x heads per kv head), <= 16 x tiles
   int32_t mode;        // bits 0-7: 16-row tiles (1 = KV steps split over waves on wave-private tiles,
                        // 2/4/8 = tiles shared through LDS); bit 8: a kv head per wave; bit 9: V read past the caches;
+                       // bit 10: a list of `tokens` boxes of one sequence each, seq[i] / slot[i] of box i; page[] holds the boxes' tokens
+                       // (list_boxes entries), then their pages (list_pages each)
   int32_t head;        // first kv head this workgroup serves
   int32_t fill_begin;  // slots slot[j] + fill_begin .. slot[j] + fill_end - 1 of every row stay empty:
   int32_t fill_end;    // this workgroup marks them (-inf)
@@ -72,6 +74,8 @@ struct RecordHead {
 static_assert(sizeof(RecordHead) == 32, "RecordHead is read as two 16-byte pieces");
 constexpr int kRecordModeHeadPerWave = 0x100;
 constexpr int kRecordModeStreamV = 0x200;
+constexpr int kRecordModeList = 0x400;      // several boxes of one sequence each: see RecordHead
+constexpr int kMaxListBoxes = 8;            // (their tokens and pages, two at most for 32 tokens, fit the 64 page entries of a record's first trip)
 
 struct SplitParams {
   const char* records;      // one per workgroup, in launch order
@@ -101,6 +105,8 @@ struct SplitParams {
   int32_t tall_apart;  // 32-row form: K and V tiles of a super-step handed over apart (see the kernel)
   int32_t stream_v;  // records may ask for V past the caches (host side: picks the kernel instance)
   int32_t waves;     // waves per workgroup (host side: picks the kernel instance)
+  int32_t list_boxes; // most boxes of a list workgroup (kRecordModeList), 0: the launch has none
+  int32_t list_pages; // ... and pages per box in its record
   int32_t tail_pages; // tails: pages per tail in the records, 0: the launch has none
   int32_t tall_rows; // rows per wave on boxes of 17..64 rows: 32 (32x32x16 tiles) or 16 (host side: picks the kernel instance)
 };
@@ -125,6 +131,7 @@ struct RecordBucket {
   const int32_t* items;  // [num_items, 2]: boxes served together (-1: no second one), or null: every box by itself
   int32_t num_items;     // work items along the box axis: rows of `items`, or num_boxes
   int32_t heads_per_wg;  // 1, or kWaves: wave w serves kv head h0 + w alone
+  int32_t list_boxes;    // 0, or: a workgroup serves so many boxes one after the other (num_items counts such lists)
   const int32_t* tails;  // [num_boxes, max_seqs]: launch bucket << 27 | row of each sequence's tail, or null
   int32_t tail_id;       // a bucket of tails: its place among the launch's buckets, as `tails` numbers them; else -1
 };
@@ -136,6 +143,7 @@ struct RecordParams {
   int32_t batch, kv_heads, group, page_size, num_pages;
   int32_t chunks_per_rank;  // slots reserved per box ordinal
   int32_t max_split;
+  int32_t list_boxes, list_pages;   // as in SplitParams
   int32_t tail_pages;       // pages per tail in a record; 0: no tails. Buckets of tails have no items, only tables.
   int32_t stream_tokens;    // V tiles of pieces that no other box reads go past the caches (kRecordModeStreamV) where the boxes of
                             // <= 16 rows hold so many tokens between them; negative: nowhere

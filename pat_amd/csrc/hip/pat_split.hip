@@ -111,7 +111,8 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
 // long: a wave has half the steps, each a trip to memory behind the last (us per call: 8 requests of 288 tokens, 8 kv heads of 64, 64 workgroups, 5.47 / 4.66;
 // 2 of 306..459 at 64/8, head_dim 64, 6.5 / 5.3; 17 of 188..282 at 8/8, head_dim 128, 6.8 / 6.3).
 // TAILS instances (32-row form): tall workgroups also walk the tails of their rows' sequences.
-template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS, int WAVES>
+// LISTS instances: workgroups of short buckets may serve several boxes of one sequence each (kRecordModeList).
+template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS, int WAVES, bool LISTS>
 __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occupancy(D, TALLK)) pat_split_kernel(const char* __restrict__ records, const int record_stride,
                                                                              const int record_max_seqs, const int record_max_pages, const SplitParams p) {
   using E = Elem<T>;
@@ -366,6 +367,93 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
     }
   };
 
+  // Short boxes of one sequence each, one after the other by one wave (`live`: which of up to 64): rows of a sequence on 16x16x32
+  // tiles, K straight into operand registers, V through the wave's own LDS tile, the next step's tiles in flight. finish(j, max, sum)
+  // takes box j's sums out of acc_o.
+  auto walk_list = [&](uint64_t live, auto tokens_of, auto page_of, auto seq_of, PAT_LDS char* vtile, auto finish) {
+    u32x4 kd[2][KK], vd[NV];
+    // half of a step at token t of box j (`tok` tokens): base address; `lim`: its last row that exists (rows past the end
+    // re-read the last token, as everywhere)
+    auto half_at = [&](const char* base, int64_t sp, int64_t ss, int j, int tok, int t, int& lim) -> const char* {
+      const int left = tok - 1 - t;
+      lim = left < 0 ? (tok - 1) & 15 : (left > 15 ? 15 : left);
+      const int h = left < 0 ? (tok - 1) >> 4 : t >> 4;
+      int pidx, s16;
+      if (hshift >= 0) { pidx = h >> hshift; s16 = h & (hpp - 1); }
+      else { pidx = (int)__umulhi((unsigned)h, p.hpp_magic); s16 = h - pidx * hpp; }
+      return base + (int64_t)page_of(j, pidx) * sp + (int64_t)(s16 * 16) * ss;
+    };
+    auto get_v = [&](int j, int tok, int t0) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        int lim;
+        const char* vb = half_at(vbase, vsp, vss, j, tok, t0 + a * 16, lim);
+#pragma unroll
+        for (int i = 0; i < NV / 2; ++i) {
+          const unsigned vo = (unsigned)min(i * TPL + lane / CPR, lim) * (unsigned)vss + (lane % CPR) * 16;
+          vd[a * (NV / 2) + i] = *(const u32x4*)(vb + vo);
+        }
+      }
+    };
+    auto get_k = [&](int j, int tok, int t0) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        int lim;
+        const char* kb = half_at(kbase, ksp, kss, j, tok, t0 + a * 16, lim);
+        const unsigned ko = (unsigned)min(n, lim) * (unsigned)kss + g * 16;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) kd[a][kk] = *(const u32x4*)(kb + ko + kk * 64);
+      }
+    };
+    auto get_q = [&](int j) {   // (columns past the sequence's rows hold one of them again: they go nowhere)
+      const T* qrow = (const T*)p.q + ((int64_t)seq_of(j) * p.q_stride_b + (int64_t)(head * G + (n & (G - 1))) * p.q_stride_h);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) qreg[kk] = __builtin_bit_cast(vec8, *(const u32x4*)(qrow + kk * 32 + g * 8));
+    };
+    int j = (int)__builtin_ctzll(live), t0 = 0, tok = tokens_of(j);
+    float m_t = neg_inf(), l_t = 0.f;
+    get_v(j, tok, t0);
+    get_k(j, tok, t0);
+    get_q(j);
+    // One step. Every request is made in every step but the last, which stands apart, so that a wait counts exactly the loads
+    // behind the one it is for; with requests that may not be made each step waited for all of them, a full trip to memory
+    // per box.
+    auto step = [&](auto more_c) {
+      constexpr bool more = decltype(more_c)::value;
+      // the step behind this one: of this box, or the next one's first
+      const bool ends = !more || t0 + kStepTokens >= tok;
+      int next_j = j, next_t0 = t0 + kStepTokens, next_tok = tok;
+      if (more && ends) {
+        live &= live - 1;
+        next_j = (int)__builtin_ctzll(live);
+        next_t0 = 0;
+        next_tok = tokens_of(next_j);
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        *(PAT_LDS u32x4*)(vtile + (i * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vd[i];
+      if (more) get_v(next_j, next_tok, next_t0);
+      attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kd[a][kk]); }, vtile, t0, tok, m_t, l_t, [&]() {
+        if (more) {
+          get_k(next_j, next_tok, next_t0);
+          get_q(next_j);
+        }
+      });
+      if (ends) {
+        finish(j, m_t, sum_xor32(sum_xor16(l_t)));
+        m_t = neg_inf();
+        l_t = 0.f;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc_o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      j = next_j;
+      t0 = next_t0;
+      tok = next_tok;
+    };
+    while ((live & (live - 1)) != 0 || t0 + kStepTokens < tok) step(std::true_type{});
+    step(std::false_type{});
+  };
+
   if (tall) {
     if constexpr (TALLK == 16) {
     constexpr int NP = D / 64;             // 16-byte K (and V) loads per thread per step
@@ -545,112 +633,35 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
       if (live == 0) return;
       PAT_LDS char* vtile = (PAT_LDS char*)smem + wave * REGION;
       PAT_LDS float* result = (PAT_LDS float*)(vtile + VSTAGE);   // [row of the sequence][OROW]
-      u32x4 kd[2][KK], vd[NV];
-      // half a of the step at token t0 of tail j (`tok` tokens): base address; `lim`: its last row that exists (rows past the end
-      // re-read the last token, as everywhere)
-      auto tail_half = [&](const char* base, int64_t sp, int64_t ss, int j, int tok, int t, int& lim) -> const char* {
-        const int left = tok - 1 - t;
-        lim = left < 0 ? (tok - 1) & 15 : (left > 15 ? 15 : left);
-        const int h = left < 0 ? (tok - 1) >> 4 : t >> 4;
-        int pidx, s16;
-        if (hshift >= 0) { pidx = h >> hshift; s16 = h & (hpp - 1); }
-        else { pidx = (int)__umulhi((unsigned)h, p.hpp_magic); s16 = h - pidx * hpp; }
-        const int e = j * tail_pages + pidx;
-        const int pg = __builtin_amdgcn_readlane(e < 64 ? tp0 : tp1, e & 63);
-        return base + (int64_t)pg * sp + (int64_t)(s16 * 16) * ss;
-      };
-      auto tail_v = [&](int j, int tok, int t0) {
+      walk_list(live, [&](int j) { return __builtin_amdgcn_readlane(tok_mine, j); },
+                [&](int j, int page) {
+                  const int e = j * tail_pages + page;
+                  return __builtin_amdgcn_readlane(e < 64 ? tp0 : tp1, e & 63);
+                },
+                [&](int j) { return __builtin_amdgcn_readlane(my_seq, j << gshift); }, vtile, [&](int j, float m_t, float l_t) {
+        // into the state of the sequence's rows: from lane (g, n), row n, columns 16 db + 4 g .. to lane (n32, h2)
+        if (n < G) {
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          int lim;
-          const char* vb = tail_half(vbase, vsp, vss, j, tok, t0 + a * 16, lim);
-#pragma unroll
-          for (int i = 0; i < NV / 2; ++i) {
-            const unsigned vo = (unsigned)min(i * TPL + lane / CPR, lim) * (unsigned)vss + (lane % CPR) * 16;
-            vd[a * (NV / 2) + i] = *(const u32x4*)(vb + vo);
-          }
+          for (int db = 0; db < DB; ++db) *(PAT_LDS f32x4*)(result + n * OROW + db * 16 + g * 4) = acc_o[db];
         }
-      };
-      auto tail_k = [&](int j, int tok, int t0) {
+        const int row = n32 & (G - 1);
+        const float mt = __shfl(m_t, row), lt = __shfl(l_t, row);
+        asm volatile("" ::: "memory");   // (the wave reads what its own lanes wrote: in order, no barrier)
+        if ((n32 >> gshift) == j) {
+          const float m_new = fmaxf(m_run, mt);
+          const float wa = m_run == m_new ? 1.f : fast_exp2(m_run - m_new), wb = fast_exp2(mt - m_new);
+          m_run = m_new;
+          l_run = l_run * wa + (h2 == 0 ? lt * wb : 0.f);   // (the two lanes of a row hold parts of its sum)
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          int lim;
-          const char* kb = tail_half(kbase, ksp, kss, j, tok, t0 + a * 16, lim);
-          const unsigned ko = (unsigned)min(n, lim) * (unsigned)kss + g * 16;
+          for (int db = 0; db < DB2; ++db)
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) kd[a][kk] = *(const u32x4*)(kb + ko + kk * 64);
+            for (int b = 0; b < 4; ++b) {
+              const f32x4 x = *(const PAT_LDS f32x4*)(result + row * OROW + db * 32 + b * 8 + h2 * 4);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc2[db][4 * b + r] = __builtin_fmaf(x[r], wb, acc2[db][4 * b + r] * wa);
+            }
         }
-      };
-      auto tail_q = [&](int j) {   // (columns past the sequence's rows hold one of them again: they go nowhere)
-        const int seq = __builtin_amdgcn_readlane(my_seq, j << gshift);
-        const T* qrow = (const T*)p.q + ((int64_t)seq * p.q_stride_b + (int64_t)(head * G + (n & (G - 1))) * p.q_stride_h);
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) qreg[kk] = __builtin_bit_cast(vec8, *(const u32x4*)(qrow + kk * 32 + g * 8));
-      };
-      int j = (int)__builtin_ctzll(live), t0 = 0, tok = __builtin_amdgcn_readlane(tok_mine, j);
-      float m_t = neg_inf(), l_t = 0.f;
-      tail_v(j, tok, t0);
-      tail_k(j, tok, t0);
-      tail_q(j);
-      // One step. Every request is made in every step but the last, which stands apart, so that a wait counts exactly the loads
-      // behind the one it is for; with requests that may not be made each step waited for all of them, a full trip to memory
-      // per tail.
-      auto step = [&](auto more_c) {
-        constexpr bool more = decltype(more_c)::value;
-        // the step behind this one: of this tail, or the next one's first
-        const bool ends = !more || t0 + kStepTokens >= tok;
-        int next_j = j, next_t0 = t0 + kStepTokens, next_tok = tok;
-        if (more && ends) {
-          live &= live - 1;
-          next_j = (int)__builtin_ctzll(live);
-          next_t0 = 0;
-          next_tok = __builtin_amdgcn_readlane(tok_mine, next_j);
-        }
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-          *(PAT_LDS u32x4*)(vtile + (i * TPL + lane / CPR) * RSV + (lane % CPR) * 16) = vd[i];
-        if (more) tail_v(next_j, next_tok, next_t0);
-        attend([&](int a, int kk) { return __builtin_bit_cast(vec8, kd[a][kk]); }, vtile, t0, tok, m_t, l_t, [&]() {
-          if (more) {
-            tail_k(next_j, next_tok, next_t0);
-            tail_q(next_j);
-          }
-        });
-        if (ends) {
-          // into the state of the sequence's rows: from lane (g, n), row n, columns 16 db + 4 g .. to lane (n32, h2)
-          l_t = sum_xor32(sum_xor16(l_t));
-          if (n < G) {
-#pragma unroll
-            for (int db = 0; db < DB; ++db) *(PAT_LDS f32x4*)(result + n * OROW + db * 16 + g * 4) = acc_o[db];
-          }
-          const int row = n32 & (G - 1);
-          const float mt = __shfl(m_t, row), lt = __shfl(l_t, row);
-          asm volatile("" ::: "memory");   // (the wave reads what its own lanes wrote: in order, no barrier)
-          if ((n32 >> gshift) == j) {
-            const float m_new = fmaxf(m_run, mt);
-            const float wa = m_run == m_new ? 1.f : fast_exp2(m_run - m_new), wb = fast_exp2(mt - m_new);
-            m_run = m_new;
-            l_run = l_run * wa + (h2 == 0 ? lt * wb : 0.f);   // (the two lanes of a row hold parts of its sum)
-#pragma unroll
-            for (int db = 0; db < DB2; ++db)
-#pragma unroll
-              for (int b = 0; b < 4; ++b) {
-                const f32x4 x = *(const PAT_LDS f32x4*)(result + row * OROW + db * 32 + b * 8 + h2 * 4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc2[db][4 * b + r] = __builtin_fmaf(x[r], wb, acc2[db][4 * b + r] * wa);
-              }
-          }
-          m_t = neg_inf();
-          l_t = 0.f;
-#pragma unroll
-          for (int db = 0; db < DB; ++db) acc_o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        j = next_j;
-        t0 = next_t0;
-        tok = next_tok;
-      };
-      while ((live & (live - 1)) != 0 || t0 + kStepTokens < tok) step(std::true_type{});
-      step(std::false_type{});
+      });
     };
     const int r_in = lane / CPR, c_in = lane % CPR;
     auto k_piece = [&](int i) { return (unsigned)(D == 128 ? c_in ^ ((RPI * i + r_in) & 15) : c_in ^ (((RPI * i + r_in) >> 1) & 7)) * 16u; };
@@ -908,6 +919,39 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
       if (h2 == 0) put_lse(prow, (mm + __builtin_amdgcn_logf(lsum)) * 0.6931471805599453f);
     }
     }   // TALLK
+  } else if (LISTS && (mode & kRecordModeList)) {
+    // ====================== several short boxes: each wave walks them all for its kv head ======================
+    // Launches of more short private boxes than places (a step of K and V each, the requests' own ends): a workgroup of one of
+    // them is 4-5 us of launch, record, page ids and first tiles for 0.5 us of work, and the boxes beyond the places wait for as
+    // long again. Here that is paid once per list, and a further box costs 2-2.5 us, a trip to memory of which its neighbour's
+    // arithmetic covers part (512 requests of 1408 + 32 tokens at 16/8 heads: 32.0 us per call, 28.7 in lists of four).
+    const int count = ntok_u, pages = p.list_pages, most = p.list_boxes;
+    const int seq_l = lane < count ? rows_tab[min(lane, record_max_seqs - 1)] : -1;
+    const int slot_l = lane < count ? rows_tab[record_max_seqs + min(lane, record_max_seqs - 1)] : -1;
+    // (the record's page entries: the boxes' tokens, then their pages)
+    const uint64_t live = __builtin_amdgcn_ballot_w64(lane < count && pg0 > 0 && seq_l >= 0);
+    auto slot_of = [&](int j) {   // the first partial slot of box j's row n
+      const int seq = __builtin_amdgcn_readlane(seq_l, j), sl = __builtin_amdgcn_readlane(slot_l, j);
+      return seq >= 0 && sl >= 0 && n < G ? (int64_t)(seq * p.heads + head * G + n) * p.num_slots + sl : (int64_t)-1;
+    };
+    for (int j = 0; j < count; ++j) {   // slots that stay empty
+      const int64_t at = slot_of(j);
+      if (g == 0 && at >= 0)
+        for (int c = __builtin_amdgcn_readlane(pg0, j) > 0 ? 1 : 0; c < fill_end; ++c) p.lse_part[at + c] = neg_inf();
+    }
+    if (live != 0)
+      walk_list(live, [&](int j) { return __builtin_amdgcn_readlane(pg0, j); },
+                [&](int j, int page) { return __builtin_amdgcn_readlane(pg0, most + j * pages + page); },
+                [&](int j) { return __builtin_amdgcn_readlane(seq_l, j); }, (PAT_LDS char*)smem + wave * WSTAGE, [&](int j, float m_t, float l_t) {
+        const int64_t at = slot_of(j);
+        if (at >= 0) {
+          const float inv = 1.f / l_t;
+          float* dst = p.o_part + at * D + g * 4;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) *(f32x4*)(dst + db * 16) = acc_o[db] * inv;
+          if (g == 0) p.lse_part[at] = (m_t + __builtin_amdgcn_logf(l_t)) * 0.6931471805599453f;
+        }
+      });
   } else {
     // ====================== short box: KV steps split over the 4 waves ========================
     // Each wave holds one step's K and V in registers and refills either as soon as it has been consumed: V when it has gone to
@@ -1056,8 +1100,8 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
 typedef void (*SplitFn)(const char*, int, int, int, const SplitParams);
 template <bool DIRECT, int TALLK, bool STREAM, bool TAILS = false, int WAVES = kWaves>
 static SplitFn split_instance(bool bf16, int head_dim) {
-  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES>;
-  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES>;
+  if (bf16) return head_dim == 64 ? pat_split_kernel<__bf16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES, false> : pat_split_kernel<__bf16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES, false>;
+  return head_dim == 64 ? pat_split_kernel<_Float16, 64, DIRECT, TALLK, STREAM, TAILS, WAVES, false> : pat_split_kernel<_Float16, 128, DIRECT, TALLK, STREAM, TAILS, WAVES, false>;
 }
 template <bool STREAM>
 static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
@@ -1070,16 +1114,17 @@ hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const Split
   const bool past = params.stream_v != 0, tails = params.tail_pages > 0;   // (never both, and tails in the 32-row form only)
   const int waves = params.waves;   // (eight: single-slot launches without tall boxes)
   SplitFn fn = waves == 8 ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
+             : params.list_boxes > 0 ? (bf16 ? pat_split_kernel<__bf16, 128, false, 32, false, false, kWaves, true> : pat_split_kernel<_Float16, 128, false, 32, false, false, kWaves, true>)
              : tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
              : past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
   const unsigned lds = (unsigned)split_smem_bytes(head_dim, waves != kWaves ? 0 : t32 ? 32 : 16, waves);
   // more dynamic LDS than the default limit of a kernel: raised once per instance and device
   {
     static std::mutex mutex;
-    static bool raised[64][128] = {{false}};
+    static bool raised[64][256] = {{false}};
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const int inst = (waves == 8 ? 64 : 0) + (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
+    const int inst = (params.list_boxes > 0 ? 128 : 0) + (waves == 8 ? 64 : 0) + (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
     std::lock_guard<std::mutex> lock(mutex);
     if (dev >= 0 && dev < 64 && !raised[dev][inst]) {
       if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

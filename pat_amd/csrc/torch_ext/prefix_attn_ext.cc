@@ -1206,6 +1206,7 @@ PYBIND11_MODULE(_prefix_attn, m) {
           d["pairs"] = (g.flags & PAT_GEOMETRY_PAIRS) != 0; d["apart"] = (g.flags & PAT_GEOMETRY_APART) != 0;
           d["stream_v"] = (g.flags & PAT_GEOMETRY_STREAM_V) != 0;
           d["tails"] = (g.flags & PAT_GEOMETRY_TAILS) != 0;
+          d["lists"] = (g.flags & PAT_GEOMETRY_LISTS) != 0;
           d["waves"] = (g.flags & PAT_GEOMETRY_WAVES_8) != 0 ? 8 : 4;
           d["merge"] = (g.flags >> PAT_GEOMETRY_MERGE_SHIFT) & 7;
           out.append(d);
