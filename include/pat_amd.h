@@ -313,7 +313,8 @@ typedef struct pat_fwd_tuning {
                                      /* of the bucket and no tall box reads; + PAT_TAILS_ALWAYS /   */
                                      /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS); */
                                      /* + PAT_WAVES_8 / _4: waves per workgroup of single-slot      */
-                                     /* launches without tall boxes; + PAT_LISTS_ALWAYS / _NEVER:   */
+                                     /* launches without tall boxes (_4 also where pieces of double */
+                                     /* length would have eight); + PAT_LISTS_ALWAYS / _NEVER:      */
                                      /* short private boxes several per workgroup (32-row form,     */
                                      /* head_dim 128).                                              */
                                      /* Values with other bits, negative ones too: 0                */

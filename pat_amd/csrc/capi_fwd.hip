@@ -673,6 +673,32 @@ void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) 
   size_records(g);
 }
 
+// Pieces twice as long, eight waves per workgroup: launches without tall boxes whose pieces put two workgroups on some CUs and one on
+// the others, so that the two set the time while the others idle. In pieces of double length every workgroup has a CU of its own; a wave
+// has the steps it had (its softmax covers as many tokens: results are as exact), there are half the partial rows and, where one piece is
+// left, no merge. At head_dim 128 from 289 to 400 workgroups that become 256 at most. 694 drawn batches there: geometric mean 0.943, eight
+// 2-5 % slower (8 of 693..1039 tokens at 32/8 heads, five pieces that become three, 10.7 / 11.3), errors against 64 bits 0.998 of four waves'.
+// us per call, four waves / eight: 8 of 782 at 64/8 10.8 / 10.0, 4 of 2033..2541 at 16/8 13.3 / 12.3, 8 of 2239 at 64/8 18.1 / 16.9, 12 of
+// 552..690 at 16/16, whole with eight, 16.0 / 13.3. Outside: 257..288 workgroups 0.965, but eight of 69 3-8 % slower (4 of 1453..1598 at
+// 64/8, 288, 10.3 / 10.9: CUs left without work); 401..512, where nearly every CU had two, 0.99, fourteen of 202 2-9 % slower; more than
+// 256 left 1.13; head_dim 64 0.98 where one piece of several is left, 0.99 else.
+int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) {
+  if (a->head_dim != 128 || g->direct || g->stream_v || g->waves != kWaves || tune.chunk_tokens > 0 || (waves_switch(tune) & PAT_WAVES_4) ||
+      8 * g->total_wgs <= 9 * kNumCUs || 16 * g->total_wgs > 25 * kNumCUs) return PAT_OK;
+  pat_fwd_tuning twice = tune;
+  twice.chunk_tokens = 2 * g->chunk;
+  pat_fwd_args b = *a;
+  b.tuning = &twice;
+  Geometry wide;
+  if (int rc = plan_geometry_for(&b, &wide, 16, false)) return rc;
+  bool plain = wide.total_wgs <= kNumCUs && wide.num_slots < g->num_slots;
+  for (int i = 0; i < a->num_buckets; ++i) plain = plain && (a->buckets[i].num_boxes == 0 || (g->bucket_heads_per_wg[i] == 1 && wide.bucket_heads_per_wg[i] == 1));
+  if (!plain) return PAT_OK;
+  *g = wide;
+  g->waves = 8;
+  return PAT_OK;
+}
+
 int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
   g->tail_pages = tail_pages;
@@ -695,7 +721,10 @@ int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
   };
   if (tail_pages > 0 || tune.tall_rows == 32) return in_32();
   if (tune.tall_rows == 16) return plan_geometry_for(a, g, 16, false);
-  if (widest_tall == 0) return plan_geometry_for(a, g, 16, false);   // no tall box: the form with more resident workgroups
+  if (widest_tall == 0) {   // no tall box: the form with more resident workgroups
+    if (int rc = plan_geometry_for(a, g, 16, false)) return rc;
+    return double_pieces(a, tune, g);
+  }
   if (int rc = in_32()) return rc;
   if (g->tall_rows == 16) return PAT_OK;
   if (g->total_wgs <= (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs) return PAT_OK;

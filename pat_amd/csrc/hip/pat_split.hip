@@ -109,7 +109,8 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
 // the smallest launches 0.14 us of 5.5.
 // WAVES: 4, or 8 in instances without a tall path (TALLK 0) for single launches of few workgroups whose boxes are more than eight steps
 // long: a wave has half the steps, each a trip to memory behind the last (us per call: 8 requests of 288 tokens, 8 kv heads of 64, 64 workgroups, 5.47 / 4.66;
-// 2 of 306..459 at 64/8, head_dim 64, 6.5 / 5.3; 17 of 188..282 at 8/8, head_dim 128, 6.8 / 6.3).
+// 2 of 306..459 at 64/8, head_dim 64, 6.5 / 5.3; 17 of 188..282 at 8/8, head_dim 128, 6.8 / 6.3); and for launches of such boxes in pieces of
+// double length, a workgroup per CU (8 of 2239 at 64/8, head_dim 128, 384 workgroups of four / 192 of eight, 18.1 / 16.9).
 // TAILS instances (32-row form): tall workgroups also walk the tails of their rows' sequences.
 // LISTS instances: workgroups of short buckets may serve several boxes of one sequence each (kRecordModeList).
 template <typename T, int D, bool DIRECT, int TALLK, bool STREAM, bool TAILS, int WAVES, bool LISTS>
@@ -1112,8 +1113,9 @@ static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
 hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const SplitParams& params) {
   const bool t32 = params.tall_rows != 16;
   const bool past = params.stream_v != 0, tails = params.tail_pages > 0;   // (never both, and tails in the 32-row form only)
-  const int waves = params.waves;   // (eight: single-slot launches without tall boxes)
-  SplitFn fn = waves == 8 ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
+  const int waves = params.waves;   // (eight: launches without tall boxes)
+  SplitFn fn = waves == 8 ? (params.direct ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
+                           : bf16 ? pat_split_kernel<__bf16, 128, false, 0, false, false, 8, false> : pat_split_kernel<_Float16, 128, false, 0, false, false, 8, false>)
              : params.list_boxes > 0 ? (bf16 ? pat_split_kernel<__bf16, 128, false, 32, false, false, kWaves, true> : pat_split_kernel<_Float16, 128, false, 32, false, false, kWaves, true>)
              : tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
              : past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);

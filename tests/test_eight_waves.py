@@ -73,3 +73,57 @@ def test_against_the_oracle(heads, d, dtype, page, tuning, monkeypatch):
         lerr = ((lse.cpu() - ref_lse).abs() / ref_lse.abs().clamp_min(1.0)).max().item()
         print(f"[parity] {err:.3e} {lerr:.3e}", flush=True)
         assert err <= (2e-3 if dtype == torch.float16 else 1.6e-2) and lerr <= 1e-4
+
+
+@pytest.mark.parametrize("requests,tokens,heads,d,want", [
+    (8, 2240, (64, 8), 128, (8, 192, 3)),     # 384 workgroups of 384 tokens: 192 of 768
+    (16, 512, (16, 16), 128, None),           # (whole: nothing to merge)
+    (12, 768, (16, 16), 128, (8, 192, 1)),    # two pieces become one
+    (4, 1152, (8, 8), 128, None), (4, 1280, (8, 8), 128, (8, 160, 5)),    # 288 workgroups are too few, 320 not
+    (5, 1280, (8, 8), 128, (8, 200, 5)), (8, 832, (8, 8), 128, None),     # 400 still, 448 not
+    (12, 2048, (64, 8), 128, None),           # 288 would be left
+    (8, 2240, (64, 8), 64, None),             # head_dim 64
+])
+def test_double_pieces_rule(requests, tokens, heads, d, want, tuning):
+    lib, g, a = _lib.load(), _lib.FwdGeometry(), _args(requests, tokens, *heads, d)
+    tuning(pairs=_lib.PAT_WAVES_4)
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0 and not g.flags & _lib.PAT_GEOMETRY_WAVES_8
+    four = (4, g.num_workgroups, g.num_slots)
+    tuning()
+    assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+    assert (8 if g.flags & _lib.PAT_GEOMETRY_WAVES_8 else 4, g.num_workgroups, g.num_slots) == (want or four)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,heads,dtype,page,direct", [
+    ([2239, 1, 767, 768, 769, 2240, 1537, 800], (64, 8), torch.float16, 16, False),        # pieces unfilled, of one token and full
+    ([1280, 1249, 33, 1025], (8, 8), torch.bfloat16, 16, False),
+    ([1000, 1279, 257, 31, 256], (16, 8), torch.float16, 32, False),
+    ([767, 768, 1, 33, 736, 500, 255, 256, 384, 385, 640, 700], (16, 16), torch.bfloat16, 48, True),    # one piece: straight to `out`
+])
+def test_double_pieces_against_the_oracle(lens, heads, dtype, page, direct, tuning, monkeypatch):
+    print(f"[case] double pieces, {lens}, heads {heads}, {dtype}, page {page}", flush=True)
+    monkeypatch.setenv("PAT_WHOLE_SEQUENCES", "1")
+    rows, nxt = [], 0
+    for n in lens:
+        rows.append(list(range(nxt, nxt + -(-n // page))))
+        nxt += -(-n // page)
+    w = workloads.Workload("double", heads[0], heads[1], 128, dtype, page, lens, rows, nxt, 0, 4)
+    q, k, v = w.tensors(torch.device("cuda:0"))
+    ref_out, ref_lse = ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), rows, lens)
+    for switch in (0, _lib.PAT_WAVES_4):
+        tuning(pairs=switch)
+        tree = PrefixTreeCPP(page)
+        tree.build_radix_tree(lens, w.padded_table())
+        tree.pack_schedule(None, heads[0] // heads[1], heads[1])
+        tree.kernel_info.to_gpu(q.device)
+        out = torch.full_like(q, float("nan"))
+        lse = torch.full((w.batch, w.heads), float("nan"), dtype=torch.float32, device=q.device)
+        for _ in range(2):    # (the second call finds the first one's partial rows in the workspace)
+            prefix_attn_with_kvcache(q, k, v, tree, 1.0 / math.sqrt(128), out, softmax_lse=lse)
+        torch.cuda.synchronize()
+        assert [(g["waves"], g["num_slots"] == 1) for g in tree.kernel_info._launch_geometries] == [(8, direct) if switch == 0 else (4, False)]
+        err = (out.float().cpu() - ref_out.float()).abs().max().item()
+        lerr = ((lse.cpu() - ref_lse).abs() / ref_lse.abs().clamp_min(1.0)).max().item()
+        print(f"[parity] {err:.3e} {lerr:.3e}", flush=True)
+        assert err <= (2e-3 if dtype == torch.float16 else 1.6e-2) and lerr <= 1e-4
