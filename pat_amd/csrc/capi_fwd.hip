@@ -681,9 +681,9 @@ void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) 
 // us per call, four waves / eight: 8 of 782 at 64/8 10.8 / 10.0, 4 of 2033..2541 at 16/8 13.3 / 12.3, 8 of 2239 at 64/8 18.1 / 16.9, 12 of
 // 552..690 at 16/16, whole with eight, 16.0 / 13.3. Outside: 257..288 workgroups 0.965, but eight of 69 3-8 % slower (4 of 1453..1598 at
 // 64/8, 288, 10.3 / 10.9: CUs left without work); 401..512, where nearly every CU had two, 0.99, fourteen of 202 2-9 % slower; more than
-// 256 left 1.13; head_dim 64 0.98 where one piece of several is left, 0.99 else.
+// 256 left 1.13; head_dim 64 0.98 to 0.99. (Not where V past the caches is forced on or off: that switch changes no launch's pieces.)
 int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) {
-  if (a->head_dim != 128 || g->direct || g->stream_v || g->waves != kWaves || tune.chunk_tokens > 0 || (waves_switch(tune) & PAT_WAVES_4) ||
+  if (a->head_dim != 128 || g->direct || g->stream_v || g->waves != kWaves || tune.chunk_tokens > 0 || (waves_switch(tune) & PAT_WAVES_4) || stream_switch(tune) != 0 ||
       8 * g->total_wgs <= 9 * kNumCUs || 16 * g->total_wgs > 25 * kNumCUs) return PAT_OK;
   pat_fwd_tuning twice = tune;
   twice.chunk_tokens = 2 * g->chunk;
