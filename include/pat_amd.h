@@ -286,6 +286,9 @@ typedef struct pat_fwd_bucket {
 #define PAT_BUCKET_TAIL 8
 #define PAT_TAIL_BOXES_SHIFT 8
 #define PAT_TAIL_BOXES(flags) (((flags) >> PAT_TAIL_BOXES_SHIFT) & 0xff)
+/* Some sequence of the batch sits in no box of the launch (a request without tokens). Its rows are the merge kernel's to write, so
+ * the launch has one even where every row has a single partial slot. The planner sets it for all launch buckets; one is enough. */
+#define PAT_BUCKET_UNBOXED 16
 
 /* Overrides of the launch geometry. pat_fwd_set_tuning sets them process-wide (a tuning and test
  * aid, not meant to change while launches are in flight on other threads); pat_fwd_args.tuning sets
@@ -380,9 +383,10 @@ int pat_fwd_validate(const pat_fwd_args* args);
  * partial LSE (the reference allocates the equivalent per call at csrc/api.h:217-229) and,
  * when args->records is NULL, the launch records of this call. Depends only on sizes,
  * pointers' alignment and strides, never on device data. With prebuilt records it is 0 when
- * every row has a single partial slot (max_split_per_seq 1 and no box longer than a chunk):
- * the launch then writes `out` from its first kernel, as the reference does for
- * max_split_per_seq 1 (csrc/api.h:230-238), and `workspace` may be NULL. */
+ * every row has a single partial slot (max_split_per_seq 1 and no box longer than a chunk) and no
+ * sequence is known to sit in no box (see pat_fwd_launch): the launch then writes `out` from its
+ * first kernel, as the reference does for max_split_per_seq 1 (csrc/api.h:230-238), and `workspace`
+ * may be NULL. */
 int pat_fwd_workspace_bytes(const pat_fwd_args* args, size_t* bytes);
 
 /* Launch records: one small record per workgroup of the launch (which rows, which partial
@@ -410,9 +414,11 @@ int pat_fwd_build_records(const pat_fwd_args* args, void* buffer, size_t buffer_
  * Enqueues the split-KV kernel and (unless the workspace size is 0, see above) the merge
  * kernel on `hip_stream` (a hipStream_t; NULL = the null stream) of the current device and
  * returns without synchronising. Rows of `out` (and `lse_out`) whose sequence sits in no box of
- * the plan: the merge kernel writes 0 (LSE -inf) there; a single-slot launch, which has no merge
- * kernel, leaves them as they were (the scheduler's plans put every sequence in a box; only a
- * hand-made plan can leave one out). */
+ * the plan, as the scheduler leaves a request without tokens: the merge kernel writes 0 (LSE -inf)
+ * there. A launch is known to have such rows by PAT_BUCKET_UNBOXED, or where its boxes have fewer
+ * places (num_boxes x max_seqs) than the batch has sequences, and gets a merge kernel for them. Only
+ * a plan that shows neither and whose rows have a single slot each - boxes of several sequences whose
+ * q_table is not full, without the flag - leaves them as they were. */
 int pat_fwd_launch(const pat_fwd_args* args, void* hip_stream);
 
 /* pat_fwd_launch for callers that cannot allocate device memory (code under HIP graph capture,

@@ -87,6 +87,7 @@ PAT_BUCKET_ITEMS = 2
 PAT_BUCKET_TAILS = 4
 PAT_BUCKET_TAIL = 8
 PAT_TAIL_BOXES_SHIFT = 8
+PAT_BUCKET_UNBOXED = 16
 PAT_STREAM_V_ALWAYS = 4
 PAT_STREAM_V_NEVER = 8
 PAT_TAILS_ALWAYS = 32

@@ -231,6 +231,18 @@ int check_args(const pat_fwd_args* a) {
   return PAT_OK;
 }
 
+// Is a sequence of the batch known to sit in no box (a request without tokens)? Said by the plan, or by sizes: fewer places in the
+// boxes than sequences. Nobody but the merge kernel writes its rows.
+bool leaves_rows_out(const pat_fwd_args* a) {
+  int64_t places = 0;
+  int flags = 0;
+  for (int i = 0; i < a->num_buckets; ++i) {
+    places += (int64_t)a->buckets[i].num_boxes * a->buckets[i].max_seqs;
+    flags |= a->buckets[i].flags;
+  }
+  return (flags & PAT_BUCKET_UNBOXED) != 0 || places < a->batch;
+}
+
 // K and V bytes that a launch's boxes of <= 16 rows stream, from sizes: ragged buckets, without the PAT_BUCKET_EVEN hint, hold
 // ~0.6 of their widest box on average.
 double short_bytes(const pat_fwd_args* a) {
@@ -577,9 +589,9 @@ int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pa
   if (g->stream_v) g->stream_tokens = (forced & PAT_STREAM_V_ALWAYS) ? 0 : (int)std::ceil(kStreamBytes / ((double)a->kv_heads * a->head_dim * 4.));
   g->num_slots = g->chunks_per_rank * a->max_split_per_seq;
   // One slot per row (no sequence in two boxes, no box in two chunks): nothing to merge, the
-  // split kernel stores the rows in `out` itself (8-byte stores: needs `out` laid out for them).
+  // split kernel stores the rows in `out` itself (8-byte stores: needs `out` laid out for them, and every sequence in a box).
   // pat_fwd_tuning.direct_out = 0 keeps the two-kernel route (tests).
-  g->direct = g->num_slots == 1 && reinterpret_cast<uintptr_t>(a->out) % 8 == 0 && a->o_stride[0] % 4 == 0 &&
+  g->direct = g->num_slots == 1 && !leaves_rows_out(a) && reinterpret_cast<uintptr_t>(a->out) % 8 == 0 && a->o_stride[0] % 4 == 0 &&
               a->o_stride[2] % 4 == 0 && tune.direct_out != 0;
   // Eight waves per workgroup: single-slot launches of few workgroups, boxes of more than eight 32-token steps. A wave of four has three
   // steps and more then, each a trip to memory behind the last; eight halve them, and softmaxes over fewer tokens each are rounded no

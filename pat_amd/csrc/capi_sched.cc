@@ -375,10 +375,11 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
     }
     return hi > lo && (int64_t)shortest * 4 >= (int64_t)widest * 3 ? PAT_BUCKET_EVEN : 0;
   };
+  const int unboxed = std::find(p.num_boxes_per_seq.begin(), p.num_boxes_per_seq.end(), 0) != p.num_boxes_per_seq.end() ? PAT_BUCKET_UNBOXED : 0;
   for (int b = 0; b < nb; ++b)
     layout->buckets[b].flags = even(p.buckets[(size_t)b], nullptr, 0, (int)p.buckets[(size_t)b].kv.size());
   for (size_t i = 0; i < parts.size(); ++i)
-    layout->launch[i].flags = even(p.buckets[(size_t)parts[i].parent], order[(size_t)parts[i].parent].data(), parts[i].lo, parts[i].hi);
+    layout->launch[i].flags = even(p.buckets[(size_t)parts[i].parent], order[(size_t)parts[i].parent].data(), parts[i].lo, parts[i].hi) | unboxed;
   layout->total = at;
   if (dst == nullptr) return PAT_OK;
   if (capacity < at) return pat::fail(PAT_ERR_INVALID, "flat plan: buffer too small");
