@@ -14,10 +14,27 @@
 #include "pat_amd.h"
 #include "sched/radix_plan.hpp"
 
+namespace {
+// A flat plan as far as it is laid out before its contents are written: the layout, the boxes' launch order, the launch buckets they
+// fall into, and the tables that exist in the launch copies only.
+struct FlatPlan {
+  struct Part { int parent, lo, hi, width; };   // boxes lo..hi of a bucket's launch order
+  pat_flat_plan layout;
+  std::vector<std::vector<int32_t>> order;      // per bucket
+  std::vector<Part> parts;                      // the launch buckets
+  std::vector<std::vector<int32_t>> items;      // per launch bucket: boxes of one node in twos
+  std::vector<std::vector<int32_t>> tails;      // per launch bucket, where a bucket holds tails: PAT_BUCKET_TAILS
+  std::vector<std::vector<int32_t>> slot;       // per bucket, there too: q_slot with the tails behind all other boxes
+  std::vector<int32_t> without;                 // ... and the boxes per sequence that are no tails
+};
+}  // namespace
+
 struct pat_tree {
   int block_size;
   std::unique_ptr<pat::RadixPlanner> planner;
   std::vector<int32_t> child_scratch;
+  // Between the call that asks how large the flat plan is and the one that writes it (half of the two was laying it out again).
+  mutable std::unique_ptr<FlatPlan> flat;
 };
 
 namespace pat {
@@ -43,6 +60,12 @@ int guarded(F&& f) {
   }
 }
 }  // namespace
+
+// The planner, for calls that change the tree or its plan.
+static pat::RadixPlanner& edit(pat_tree* tree) {
+  tree->flat.reset();
+  return *tree->planner;
+}
 
 extern "C" {
 
@@ -76,7 +99,7 @@ int pat_tree_build_rows(pat_tree* tree, const int32_t* seq_lens, const int32_t* 
   return guarded([&] {
     // A tree is built once per batch; building again starts from an empty tree.
     tree->planner.reset(new pat::RadixPlanner(tree->block_size));
-    tree->planner->build(seq_lens, flat_blocks, row_offsets, num_seqs);
+    edit(tree).build(seq_lens, flat_blocks, row_offsets, num_seqs);
   });
 }
 
@@ -108,18 +131,18 @@ int pat_tree_append(pat_tree* tree, int32_t seq_len, const int32_t* blocks, int3
   if (tree == nullptr) return pat::fail(PAT_ERR_INVALID, "tree is NULL");
   if (seq_len < 0 || num_blocks < 0) return pat::fail(PAT_ERR_INVALID, "seq_len / num_blocks must be >= 0");
   if (num_blocks > 0 && blocks == nullptr) return pat::fail(PAT_ERR_INVALID, "blocks is NULL");
-  return guarded([&] { tree->planner->append(seq_len, blocks, num_blocks); });
+  return guarded([&] { edit(tree).append(seq_len, blocks, num_blocks); });
 }
 
 int pat_tree_remove(pat_tree* tree, int32_t seq) {
   if (tree == nullptr) return pat::fail(PAT_ERR_INVALID, "tree is NULL");
-  return guarded([&] { tree->planner->remove(seq); });
+  return guarded([&] { edit(tree).remove(seq); });
 }
 
 int pat_tree_grow(pat_tree* tree, int32_t seq, int32_t new_len, const int32_t* more_blocks, int32_t num_more) {
   if (tree == nullptr) return pat::fail(PAT_ERR_INVALID, "tree is NULL");
   if (num_more > 0 && more_blocks == nullptr) return pat::fail(PAT_ERR_INVALID, "more_blocks is NULL");
-  return guarded([&] { tree->planner->grow(seq, new_len, more_blocks, num_more); });
+  return guarded([&] { edit(tree).grow(seq, new_len, more_blocks, num_more); });
 }
 
 int pat_tree_num_seqs(const pat_tree* tree) {
@@ -132,12 +155,12 @@ int pat_tree_pack(pat_tree* tree, const int32_t* mnws, int32_t n_mnws, int32_t h
   if (tree == nullptr) return pat::fail(PAT_ERR_INVALID, "tree is NULL");
   if (n_mnws > 0 && mnws == nullptr) return pat::fail(PAT_ERR_INVALID, "mnws is NULL");
   return guarded(
-      [&] { tree->planner->pack(mnws, n_mnws, hratio, kv_heads, use_compute_model != 0, opts); });
+      [&] { edit(tree).pack(mnws, n_mnws, hratio, kv_heads, use_compute_model != 0, opts); });
 }
 
 int pat_tree_naive_schedule(pat_tree* tree, int32_t hratio) {
   if (tree == nullptr) return pat::fail(PAT_ERR_INVALID, "tree is NULL");
-  return guarded([&] { tree->planner->naive(hratio); });
+  return guarded([&] { edit(tree).naive(hratio); });
 }
 
 int pat_tree_plan(const pat_tree* tree, pat_plan_view* out) {
@@ -156,15 +179,13 @@ int pat_tree_plan(const pat_tree* tree, pat_plan_view* out) {
   return PAT_OK;
 }
 
-static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* dst, int64_t capacity) {
-  if (tree == nullptr || layout == nullptr) return pat::fail(PAT_ERR_INVALID, "tree / layout is NULL");
-  const pat::Plan& p = tree->planner->plan();
-  if (!p.valid) return pat::fail(PAT_ERR_INVALID, "no plan: call pat_tree_pack first");
+// Lays out the flat form of a plan.
+static int lay_out(const pat::Plan& p, int page, FlatPlan& f) {
   const int nb = (int)p.buckets.size();
   if (nb > PAT_MAX_FLAT_BUCKETS)
     return pat::fail(PAT_ERR_INVALID, "the flat plan holds at most 12 buckets");
   constexpr int kGrowthBlocks = 8;
-  const int page = tree->block_size;
+  pat_flat_plan* layout = &f.layout;
   std::memset(layout, 0, sizeof(*layout));
   layout->num_buckets = nb;
   layout->batch = (int32_t)p.num_split_per_seq.size();
@@ -174,9 +195,10 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   layout->max_blocks_in_box = p.max_blocks_in_box;
 
   // launch order and parts of every bucket
-  struct Part { int parent, lo, hi, width; };
-  std::vector<std::vector<int32_t>> order((size_t)nb);
-  std::vector<Part> parts;
+  using Part = FlatPlan::Part;
+  auto& order = f.order;
+  auto& parts = f.parts;
+  order.resize((size_t)nb);
   int spare = PAT_MAX_FLAT_BUCKETS - nb;
 
   // Tails: boxes of one sequence, up to kMaxTailTokens wide, whose sequence also sits in a box of more than 16 rows. A launch may
@@ -211,6 +233,7 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
         const int32_t s = bk.q_table[box];
         if (bk.q_len[box] != 1 || s < 0 || s >= layout->batch || claim[(size_t)s].bucket < 0 || taken[(size_t)s]) continue;
         taken[(size_t)s] = is_tail[(size_t)b][box] = 1;
+        any_tail = true;
       }
     }
   }
@@ -251,7 +274,8 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   // Boxes of one node (same blocks, different sequences) in twos, for launches that serve two of them with one
   // workgroup. Only buckets of more than 16 rows, and only boxes of several sequences: a box of one sequence may be
   // grown in place between decode steps.
-  std::vector<std::vector<int32_t>> items(parts.size());
+  auto& items = f.items;
+  items.resize(parts.size());
   for (size_t i = 0; i < parts.size(); ++i) {
     const Part& pt = parts[i];
     const pat::Bucket& bk = p.buckets[(size_t)pt.parent];
@@ -286,11 +310,13 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
 
   // The launch buckets that hold nothing but tails, and per box of more than 16 rows the tails of its sequences there: launch
   // bucket << 27 | row, -1 = none.
-  std::vector<char> tail_part(parts.size(), 0);
-  std::vector<std::vector<int32_t>> tails(parts.size());
-  std::vector<std::vector<int32_t>> slot((size_t)nb);   // launch copies of q_slot, and the boxes per sequence that are no tails
-  std::vector<int32_t> without((size_t)layout->batch, 0);
-  {
+  auto& tails = f.tails;
+  tails.resize(parts.size());
+  if (any_tail) {
+    std::vector<char> tail_part(parts.size(), 0);
+    auto& slot = f.slot;
+    auto& without = f.without;
+    any_tail = false;
     std::vector<std::vector<std::array<int32_t, 2>>> place((size_t)nb);   // plan box -> (launch bucket, row)
     for (int b = 0; b < nb; ++b) place[(size_t)b].resize(p.buckets[(size_t)b].kv.size());
     for (size_t i = 0; i < parts.size(); ++i) {
@@ -320,6 +346,7 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
       }
       // ordinals of a sequence's boxes with the tails behind all others: a launch that has no slots for tails leaves the last ones out
       std::vector<int32_t> seen((size_t)layout->batch, 0);
+      slot.resize((size_t)nb);
       for (int b = 0; b < nb; ++b) slot[(size_t)b].assign(p.buckets[(size_t)b].q_slot.size(), 0);
       for (int pass = 0; pass < 2; ++pass) {
         for (int b = 0; b < nb; ++b) {
@@ -381,8 +408,23 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   for (size_t i = 0; i < parts.size(); ++i)
     layout->launch[i].flags = even(p.buckets[(size_t)parts[i].parent], order[(size_t)parts[i].parent].data(), parts[i].lo, parts[i].hi) | unboxed;
   layout->total = at;
+  return PAT_OK;
+}
+
+static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* dst, int64_t capacity) {
+  if (tree == nullptr || layout == nullptr) return pat::fail(PAT_ERR_INVALID, "tree / layout is NULL");
+  const pat::Plan& p = tree->planner->plan();
+  if (!p.valid) return pat::fail(PAT_ERR_INVALID, "no plan: call pat_tree_pack first");
+  if (!tree->flat) {
+    auto fresh = std::make_unique<FlatPlan>();
+    if (int rc = lay_out(p, tree->block_size, *fresh)) return rc;
+    tree->flat = std::move(fresh);
+  }
+  *layout = tree->flat->layout;
   if (dst == nullptr) return PAT_OK;
-  if (capacity < at) return pat::fail(PAT_ERR_INVALID, "flat plan: buffer too small");
+  if (capacity < layout->total) return pat::fail(PAT_ERR_INVALID, "flat plan: buffer too small");
+  const std::unique_ptr<FlatPlan> f = std::move(tree->flat);   // (given back once it is written)
+  const auto& order = f->order;
 
   // contents
   std::copy(p.num_split_per_seq.begin(), p.num_split_per_seq.end(), dst + layout->num_split_per_seq);
@@ -397,25 +439,26 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   auto vec_to = [&](int32_t* out, const std::vector<int32_t>& v, const int32_t* ord, int lo, int hi) {
     for (int i = lo; i < hi; ++i) out[i - lo] = v[(size_t)(ord ? ord[i] : i)];
   };
-  auto fill = [&](const pat_flat_bucket& f, const pat::Bucket& bk, const std::vector<int32_t>& q_slot, const int32_t* ord, int lo, int hi) {
-    rows_to(dst + f.q_table, bk.q_table, bk.max_seqs, bk.max_seqs, ord, lo, hi);
-    rows_to(dst + f.q_slot, q_slot, bk.max_seqs, bk.max_seqs, ord, lo, hi);
-    rows_to(dst + f.block_table, bk.block_table, bk.max_blocks, f.max_blocks, ord, lo, hi);
-    vec_to(dst + f.num_seqs, bk.num_seqs, ord, lo, hi);
-    vec_to(dst + f.rank, bk.rank, ord, lo, hi);
-    vec_to(dst + f.kv, bk.kv, ord, lo, hi);
+  auto fill = [&](const pat_flat_bucket& to, const pat::Bucket& bk, const std::vector<int32_t>& q_slot, const int32_t* ord, int lo, int hi) {
+    rows_to(dst + to.q_table, bk.q_table, bk.max_seqs, bk.max_seqs, ord, lo, hi);
+    rows_to(dst + to.q_slot, q_slot, bk.max_seqs, bk.max_seqs, ord, lo, hi);
+    rows_to(dst + to.block_table, bk.block_table, bk.max_blocks, to.max_blocks, ord, lo, hi);
+    vec_to(dst + to.num_seqs, bk.num_seqs, ord, lo, hi);
+    vec_to(dst + to.rank, bk.rank, ord, lo, hi);
+    vec_to(dst + to.kv, bk.kv, ord, lo, hi);
   };
-  for (int b = 0; b < nb; ++b) {
+  for (int b = 0; b < layout->num_buckets; ++b) {
     const pat::Bucket& bk = p.buckets[(size_t)b];
     fill(layout->buckets[b], bk, bk.q_slot, nullptr, 0, (int)bk.kv.size());
     std::copy(order[(size_t)b].begin(), order[(size_t)b].end(), dst + layout->launch_order[b]);
   }
-  for (size_t i = 0; i < parts.size(); ++i) {
-    const Part& pt = parts[i];
+  for (size_t i = 0; i < f->parts.size(); ++i) {
+    const FlatPlan::Part& pt = f->parts[i];
     const pat::Bucket& bk = p.buckets[(size_t)pt.parent];
-    fill(layout->launch[i], bk, any_tail ? slot[(size_t)pt.parent] : bk.q_slot, order[(size_t)pt.parent].data(), pt.lo, pt.hi);
-    int32_t* behind = std::copy(items[i].begin(), items[i].end(), dst + layout->launch[i].kv + layout->launch[i].num_boxes);
-    if (!tails[i].empty()) std::copy(without.begin(), without.end(), std::copy(tails[i].begin(), tails[i].end(), behind));
+    fill(layout->launch[i], bk, layout->tails != 0 ? f->slot[(size_t)pt.parent] : bk.q_slot, order[(size_t)pt.parent].data(), pt.lo, pt.hi);
+    int32_t* behind = std::copy(f->items[i].begin(), f->items[i].end(), dst + layout->launch[i].kv + layout->launch[i].num_boxes);
+    if (!f->tails[i].empty())
+      std::copy(f->without.begin(), f->without.end(), std::copy(f->tails[i].begin(), f->tails[i].end(), behind));
   }
   return PAT_OK;
 }

@@ -1,5 +1,6 @@
 """The C++ scheduler of libpat_amd (through `PrefixTree` / `PrefixTreeCPP`) against the golden
 plans of the reference scheduler and against the plan oracle on fresh random batches."""
+import ctypes as C
 import random
 
 import pytest
@@ -7,7 +8,7 @@ import torch
 
 from conftest import plan_fields, run_plan_case
 from oracle.plan_oracle import PlanOracle, pad_rows
-from pat_amd import PrefixTree, PrefixTreeCPP
+from pat_amd import PrefixTree, PrefixTreeCPP, _lib
 from pat_amd import workloads
 
 
@@ -280,3 +281,67 @@ def test_item_tables_pair_boxes_of_one_node(name):
                 pairs += 1
                 assert kv[a] == kv[b] and torch.equal(bt[a], bt[b])
     assert pairs == {"c2": 2, "c3": 0, "c5a": 12}[name]
+
+
+@pytest.mark.parametrize("edit", ["grow", "append", "remove", "build", "pack", "naive"])
+def test_a_flat_plan_is_that_of_the_plan_as_it_is(edit):
+    # what the first of the two calls lays out serves the second one only while the tree and its plan are the same
+    lib = _lib.load()
+    rows = [list(range(20)) + [20 + i] for i in range(40)]
+    lens = [16 * 20 + 5] * 40
+
+    def tree():
+        h = C.c_void_p()
+        assert lib.pat_tree_create(16, C.byref(h)) == 0
+        return h
+
+    def build(h, lens, rows):
+        offsets = [0]
+        for r in rows:
+            offsets.append(offsets[-1] + len(r))
+        flat = [x for r in rows for x in r]
+        assert lib.pat_tree_build_rows(h, (C.c_int32 * len(lens))(*lens), (C.c_int32 * len(flat))(*flat), (C.c_int64 * len(offsets))(*offsets), len(lens)) == 0
+
+    def pack(h, ratio=8):
+        assert lib.pat_tree_pack(h, None, 0, ratio, 8, 0, None) == 0
+
+    def change(h):
+        block = (C.c_int32 * 1)(99)
+        if edit == "grow":
+            assert lib.pat_tree_grow(h, 3, 16 * 21 + 2, block, 1) == 0
+        elif edit == "append":
+            assert lib.pat_tree_append(h, 9, block, 1) == 0
+        elif edit == "remove":
+            assert lib.pat_tree_remove(h, 7) == 0
+        elif edit == "build":
+            build(h, lens[:30], rows[:30])
+        if edit == "naive":
+            assert lib.pat_tree_naive_schedule(h, 8) == 0
+        else:
+            pack(h, 4 if edit == "pack" else 8)
+
+    def flat(h, layout_first):
+        f = _lib.FlatPlan()
+        if layout_first:
+            assert lib.pat_tree_flat_plan(h, C.byref(f), None, 0) == 0
+        buf = torch.full((1 << 15,), -99, dtype=torch.int32)
+        assert lib.pat_tree_flat_plan(h, C.byref(f), buf.data_ptr(), f.total - 1 if layout_first else 3) != 0      # too small: nothing written
+        assert bool((buf == -99).all())
+        assert lib.pat_tree_flat_plan(h, C.byref(f), buf.data_ptr(), buf.numel()) == 0
+        return bytes(f), buf
+
+    asked, fresh = tree(), tree()
+    for h in (asked, fresh):
+        build(h, lens, rows)
+        pack(h)
+    before = _lib.FlatPlan()
+    assert lib.pat_tree_flat_plan(asked, C.byref(before), None, 0) == 0     # laid out, then the tree changes
+    for h in (asked, fresh):
+        change(h)
+    got, want = flat(asked, False), flat(fresh, True)
+    assert got[0] == want[0] and torch.equal(got[1], want[1])
+    assert bytes(before) != got[0]
+    again = flat(asked, True)                                               # and once more, laid out anew
+    assert again[0] == got[0] and torch.equal(again[1], got[1])
+    for h in (asked, fresh):
+        lib.pat_tree_destroy(h)
