@@ -208,25 +208,25 @@ int check_args(const pat_fwd_args* a) {
     return fail(PAT_ERR_INVALID, "MNW must list between 1 and 12 tile buckets");
   for (int i = 0; i < a->num_buckets; ++i) {
     const pat_fwd_bucket& b = a->buckets[i];
-    const std::string at = " (bucket " + std::to_string(i) + ")";
+    auto at = [i](const char* message) { return std::string(message) + " (bucket " + std::to_string(i) + ")"; };
     if (b.mnw[0] != 16 && b.mnw[0] != 32 && b.mnw[0] != 64)
-      return fail(PAT_ERR_INVALID, "MNW tile_q must be 16, 32 or 64" + at);
+      return fail(PAT_ERR_INVALID, at("MNW tile_q must be 16, 32 or 64"));
     if (b.num_boxes < 0 || b.max_seqs < 0 || b.max_blocks < 0)
-      return fail(PAT_ERR_INVALID, "plan table sizes must be non-negative" + at);
+      return fail(PAT_ERR_INVALID, at("plan table sizes must be non-negative"));
     if (b.num_boxes > 0 && (b.q_table == nullptr || b.block_table == nullptr || b.num_seqs == nullptr ||
                             b.rank == nullptr || b.kv == nullptr))
-      return fail(PAT_ERR_INVALID, "plan tables must be device int32 tensors" + at);
+      return fail(PAT_ERR_INVALID, at("plan tables must be device int32 tensors"));
     if (b.q_table_stride < b.max_seqs || b.block_table_stride < b.max_blocks)
-      return fail(PAT_ERR_INVALID, "plan table row stride smaller than its width" + at);
+      return fail(PAT_ERR_INVALID, at("plan table row stride smaller than its width"));
     if ((b.flags & PAT_BUCKET_ITEMS) && (b.num_items > b.num_boxes || b.num_items < (b.num_boxes + 1) / 2))
-      return fail(PAT_ERR_INVALID, "a bucket's items hold one or two of its boxes each" + at);
+      return fail(PAT_ERR_INVALID, at("a bucket's items hold one or two of its boxes each"));
     if (b.q_table_stride > INT32_MAX || b.block_table_stride > INT32_MAX)
-      return fail(PAT_ERR_INVALID, "plan table row stride too large" + at);
+      return fail(PAT_ERR_INVALID, at("plan table row stride too large"));
     if ((int64_t)b.max_seqs * ratio > 64)
-      return fail(PAT_ERR_INVALID, "a box may pack at most 64 rows (sequences x heads per kv head)" + at);
+      return fail(PAT_ERR_INVALID, at("a box may pack at most 64 rows (sequences x heads per kv head)"));
     // the tile label is the bucket's row class: a box with more rows than its label would lose them
     if ((int64_t)b.max_seqs * ratio > 16 * row_tiles(b.mnw[0]))
-      return fail(PAT_ERR_INVALID, "a box packs more rows (sequences x heads per kv head) than its bucket's tile_q" + at);
+      return fail(PAT_ERR_INVALID, at("a box packs more rows (sequences x heads per kv head) than its bucket's tile_q"));
   }
   return PAT_OK;
 }
@@ -302,8 +302,7 @@ void size_records(Geometry* g) {
 //    estimated time of the launch allows (see below).
 // pat_fwd_tuning.chunk_tokens / tall_chunk_tokens override the two sizes (tuning aid).
 // (tall_rows: the form of the tall path the geometry is made for, 16 or 32; pairs: items of two boxes as one workgroup)
-int plan_geometry_for(const pat_fwd_args* a, Geometry* g, int tall_rows, bool pairs) {
-  const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
+int plan_geometry_for(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, int tall_rows, bool pairs) {
   const int page = a->page_size;
   const int64_t unit = (int64_t)page * kStepTokens / gcd64(page, kStepTokens);  // lcm(page, 32)
   auto round_unit = [&](int64_t c) { return std::max<int64_t>(unit, ceil_div64(c, unit) * unit); };
@@ -699,10 +698,8 @@ int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g
       8 * g->total_wgs <= 9 * kNumCUs || 16 * g->total_wgs > 25 * kNumCUs) return PAT_OK;
   pat_fwd_tuning twice = tune;
   twice.chunk_tokens = 2 * g->chunk;
-  pat_fwd_args b = *a;
-  b.tuning = &twice;
   Geometry wide;
-  if (int rc = plan_geometry_for(&b, &wide, 16, false)) return rc;
+  if (int rc = plan_geometry_for(a, twice, &wide, 16, false)) return rc;
   bool plain = wide.total_wgs <= kNumCUs && wide.num_slots < g->num_slots;
   for (int i = 0; i < a->num_buckets; ++i) plain = plain && (a->buckets[i].num_boxes == 0 || (g->bucket_heads_per_wg[i] == 1 && wide.bucket_heads_per_wg[i] == 1));
   if (!plain) return PAT_OK;
@@ -711,8 +708,7 @@ int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g
   return PAT_OK;
 }
 
-int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
-  const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
+int plan_form(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, const int tail_pages) {
   g->tail_pages = tail_pages;
   int64_t widest_tall = 0, tall_box_heads = 0;
   bool pairs = false;
@@ -726,15 +722,16 @@ int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
   pairs = pairs && pairs_switch(tune) != 2 && (pairs_switch(tune) == 1 || tall_box_heads >= 3 * kNumCUs / 8);
   // (boxes of more than 64 x kMaxTall32Tokens tokens, which the bound on pieces per box makes longer pieces of, take the 16-row form)
   auto in_32 = [&]() -> int {
-    if (int rc = plan_geometry_for(a, g, 32, pairs)) return rc;
+    if (int rc = plan_geometry_for(a, tune, g, 32, pairs)) return rc;
     if (g->tall_rows == 32) return PAT_OK;
     *g = Geometry();
-    return plan_geometry_for(a, g, 16, false);
+    return plan_geometry_for(a, tune, g, 16, false);
   };
-  if (tail_pages > 0 || tune.tall_rows == 32) return in_32();
-  if (tune.tall_rows == 16) return plan_geometry_for(a, g, 16, false);
+  if (tail_pages > 0) return plan_geometry_for(a, tune, g, 32, pairs);   // (that form or none: see plan_geometry)
+  if (tune.tall_rows == 32) return in_32();
+  if (tune.tall_rows == 16) return plan_geometry_for(a, tune, g, 16, false);
   if (widest_tall == 0) {   // no tall box: the form with more resident workgroups
-    if (int rc = plan_geometry_for(a, g, 16, false)) return rc;
+    if (int rc = plan_geometry_for(a, tune, g, 16, false)) return rc;
     return double_pieces(a, tune, g);
   }
   if (int rc = in_32()) return rc;
@@ -746,7 +743,7 @@ int plan_form(const pat_fwd_args* a, Geometry* g, const int tail_pages) {
                                           : widest_tall >= 1024 && est.tall_us >= est.short_us;
   if (outweigh) return PAT_OK;
   *g = Geometry();
-  return plan_geometry_for(a, g, 16, false);
+  return plan_geometry_for(a, tune, g, 16, false);
 }
 
 // Tails walked by the workgroups of their sequences' tall boxes? Only where that leaves every row one partial result, so that the
@@ -785,20 +782,33 @@ bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& with
   return with_us < own_us + merge_us;
 }
 
+// (Every launch comes through here, and small ones wait for the host: the overrides are read once, and arguments without tails are made only
+// where there are tails. 0.16-0.2 us for one to three buckets, 0.33 where a form with tails is planned beside the other.)
 int plan_geometry(const pat_fwd_args* a, Geometry* g) {
   const pat_fwd_tuning tune = a->tuning != nullptr ? *a->tuning : tuning();
   const int forced = tails_switch(tune);
-  WithoutTails w;
-  if (!(forced & PAT_TAILS_NEVER) && tune.tall_rows != 16 && w.make(a)) {
-    Geometry with, without;
-    if (plan_form(&w.args, &with, w.tail_pages) == PAT_OK && with.tall_rows == 32 && !with.stream_v &&
-        ((forced & PAT_TAILS_ALWAYS) || (plan_form(a, &without, 0) == PAT_OK && tails_pay(a, with, without)))) {
-      *g = with;
-      g->tails = true;
-      return PAT_OK;
+  int flags = 0;
+  for (int i = 0; i < a->num_buckets; ++i) flags |= a->buckets[i].flags;
+  bool planned = false;   // `g`, as the launch is without tails
+  if ((flags & PAT_BUCKET_TAIL) && (flags & PAT_BUCKET_TAILS) && !(forced & PAT_TAILS_NEVER) && tune.tall_rows != 16) {
+    WithoutTails w;
+    Geometry with;
+    if (w.make(a) && plan_form(&w.args, tune, &with, w.tail_pages) == PAT_OK && with.tall_rows == 32 && !with.stream_v) {
+      bool take = (forced & PAT_TAILS_ALWAYS) != 0;
+      if (!take) {
+        if (int rc = plan_form(a, tune, g, 0)) return rc;
+        planned = true;
+        take = tails_pay(a, with, *g);
+      }
+      if (take) {
+        *g = with;
+        g->tails = true;
+        return PAT_OK;
+      }
     }
   }
-  if (int rc = plan_form(a, g, 0)) return rc;
+  if (!planned)
+    if (int rc = plan_form(a, tune, g, 0)) return rc;
   make_lists(a, tune, g);
   return PAT_OK;
 }
