@@ -762,7 +762,7 @@ int plan_form(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, co
 constexpr double kTailStepUs = 2.5;
 constexpr double kTailRoundUs = 4.;
 bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& without) {
-  if (with.num_slots != 1) return false;
+  if (!with.direct) return false;
   const int group = a->heads / a->kv_heads;
   double steps = 0., bytes = 0.;
   for (int i = 0; i < a->num_buckets; ++i) {

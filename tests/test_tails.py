@@ -281,3 +281,25 @@ def test_growing_in_place_and_capture(tuning, monkeypatch):
     assert [g["tails"] for g in info._launch_geometries] == [False]
     _close("after a write of somebody else", out, lse,
            ao.paged_attention_ref(q.cpu(), k.cpu(), v.cpu(), w.rows, [n - 1 for n in lens], 0.09), w.dtype)
+
+
+def test_not_taken_where_a_merge_follows_all_the_same(tuning):
+    # the rule counts a merge that tails save: not an `out` that the split kernel may not store to, nor one kept from it
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    leaf = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAIL | 1 << _lib.PAT_TAIL_BOXES_SHIFT
+
+    def tails(**other):
+        a = _tail_args((64, 128, 8, 2048, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS | _lib.PAT_BUCKET_TAILS, 64), (16, 1024, 1, 32, leaf, 0),
+                       64, 8, 128, 1024, 32)
+        for name, value in other.items():
+            setattr(a, name, value)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        return bool(g.flags & _lib.PAT_GEOMETRY_TAILS)
+
+    assert tails() is True
+    assert tails(out=0x10004) is False
+    assert tails(o_stride=(C.c_int64 * 3)(64 * 130, 64 * 130, 130)) is False
+    tuning(direct_out=0)
+    assert tails() is False
+    tuning(pairs=_lib.PAT_TAILS_ALWAYS)      # (asked for, they are walked by the tall workgroups and merged)
+    assert tails(out=0x10004) is True
