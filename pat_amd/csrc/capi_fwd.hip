@@ -84,11 +84,9 @@ pat_fwd_tuning tuning() {
 
 // The switches in pat_fwd_tuning.pairs: boxes in twos (0..2), V past the caches, tails, waves per workgroup, and lists. Values outside the declared bits,
 // -1 among them, ask for none.
-int switches(const pat_fwd_tuning& t, int bits) {
-  constexpr int kDeclared = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER | PAT_WAVES_8 | PAT_WAVES_4 | PAT_LISTS_ALWAYS |
-                            PAT_LISTS_NEVER;
-  return t.pairs >= 0 && (t.pairs & ~kDeclared) == 0 ? t.pairs & bits : 0;
-}
+constexpr int kSwitches = 3 | PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER | PAT_TAILS_ALWAYS | PAT_TAILS_NEVER | PAT_WAVES_8 | PAT_WAVES_4 | PAT_LISTS_ALWAYS |
+                          PAT_LISTS_NEVER;
+int switches(const pat_fwd_tuning& t, int bits) { return t.pairs >= 0 && (t.pairs & ~kSwitches) == 0 ? t.pairs & bits : 0; }
 int waves_switch(const pat_fwd_tuning& t) { return switches(t, PAT_WAVES_8 | PAT_WAVES_4); }
 int pairs_switch(const pat_fwd_tuning& t) { return switches(t, 3); }
 int stream_switch(const pat_fwd_tuning& t) { return switches(t, PAT_STREAM_V_ALWAYS | PAT_STREAM_V_NEVER); }
@@ -1400,7 +1398,7 @@ int pat_fwd_launch_static(const pat_fwd_args* args, void* hip_stream) {
   if (need > kStaticScratchBytes && (g.pairs || g.tails) && args->records == nullptr) {
     box_by_box = *args;
     tune = args->tuning != nullptr ? *args->tuning : tuning();
-    tune.pairs = stream_switch(tune) | PAT_TAILS_NEVER | 2;
+    tune.pairs = (switches(tune, kSwitches) & ~(3 | PAT_TAILS_ALWAYS)) | PAT_TAILS_NEVER | 2;
     box_by_box.tuning = &tune;
     args = &box_by_box;
     g = Geometry();

@@ -102,3 +102,22 @@ def test_against_the_oracle(seqs, prefix, ends, heads, dtype, page, chunk, tunin
     prefix_attn_with_kvcache(q, k, v, tree, 0.09, got)
     others = [s for s in range(seqs) if s != victim]
     assert torch.equal(got[others], out[others]) and not bool(torch.isfinite(got[victim]).any())
+
+
+def test_static_launch_box_by_box_keeps_the_switches(tuning):
+    # a launch with boxes in twos that its scratch does not hold is made box by box, and is otherwise the launch that was asked for. This one
+    # is too large either way, and the error names the bytes: records of lists are fewer
+    lib = _lib.load()
+    a = _args((64, 128, 32, 1408, EVEN | _lib.PAT_BUCKET_ITEMS), (16, 4096, 1, 32, EVEN), 64, 32, 4096, 32)
+    a._keep[0].num_items = 64
+    sizes = []
+    for lists in (_lib.PAT_LISTS_ALWAYS, _lib.PAT_LISTS_NEVER):
+        switch = lists | _lib.PAT_STREAM_V_NEVER
+        need = C.c_size_t()
+        tuning(tall_rows=32, pairs=switch | _lib.PAT_TAILS_NEVER | 2)
+        assert lib.pat_fwd_workspace_bytes(C.byref(a), C.byref(need)) == 0 and need.value > lib.pat_fwd_static_scratch_bytes()
+        tuning(tall_rows=32, pairs=switch | 1)
+        assert lib.pat_fwd_launch_static(C.byref(a), None) == -6, _lib.last_error()
+        assert f"needs {need.value} bytes" in _lib.last_error()
+        sizes.append(need.value)
+    assert sizes[0] < sizes[1]
