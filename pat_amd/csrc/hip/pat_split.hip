@@ -1111,14 +1111,19 @@ static SplitFn split_instance(bool bf16, int head_dim, bool direct, bool t32) {
 }
 
 hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const SplitParams& params) {
-  const bool t32 = params.tall_rows != 16;
-  const bool past = params.stream_v != 0, tails = params.tail_pages > 0;   // (never both, and tails in the 32-row form only)
-  const int waves = params.waves;   // (eight: launches without tall boxes)
-  SplitFn fn = waves == 8 ? (params.direct ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
+  const bool t32 = params.tall_rows != 16, direct = params.direct != 0;
+  const bool past = params.stream_v != 0, tails = params.tail_pages > 0, lists = params.list_boxes > 0;
+  const int waves = params.waves;
+  // Eight waves: launches without tall boxes, at head_dim 64 those that write `out`. Lists: the 32-row form at head_dim 128, partial rows.
+  // Tails: the 32-row form. None of them with another or with V past the caches: there is no such instance.
+  if ((waves != kWaves && waves != 8) || (waves == 8 && (past || tails || lists || (!direct && head_dim != 128))) ||
+      (lists && (past || tails || direct || !t32 || head_dim != 128)) || (tails && (past || !t32)))
+    return hipErrorInvalidValue;
+  SplitFn fn = waves == 8 ? (direct ? split_instance<true, 0, false, false, 8>(bf16, head_dim)
                            : bf16 ? pat_split_kernel<__bf16, 128, false, 0, false, false, 8, false> : pat_split_kernel<_Float16, 128, false, 0, false, false, 8, false>)
-             : params.list_boxes > 0 ? (bf16 ? pat_split_kernel<__bf16, 128, false, 32, false, false, kWaves, true> : pat_split_kernel<_Float16, 128, false, 32, false, false, kWaves, true>)
-             : tails ? (params.direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
-             : past ? split_instance<true>(bf16, head_dim, params.direct != 0, t32) : split_instance<false>(bf16, head_dim, params.direct != 0, t32);
+             : lists ? (bf16 ? pat_split_kernel<__bf16, 128, false, 32, false, false, kWaves, true> : pat_split_kernel<_Float16, 128, false, 32, false, false, kWaves, true>)
+             : tails ? (direct ? split_instance<true, 32, false, true>(bf16, head_dim) : split_instance<false, 32, false, true>(bf16, head_dim))
+             : past ? split_instance<true>(bf16, head_dim, direct, t32) : split_instance<false>(bf16, head_dim, direct, t32);
   const unsigned lds = (unsigned)split_smem_bytes(head_dim, waves != kWaves ? 0 : t32 ? 32 : 16, waves);
   // more dynamic LDS than the default limit of a kernel: raised once per instance and device
   {
@@ -1126,7 +1131,7 @@ hipError_t launch_split(bool bf16, int head_dim, hipStream_t stream, const Split
     static bool raised[64][256] = {{false}};
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    const int inst = (params.list_boxes > 0 ? 128 : 0) + (waves == 8 ? 64 : 0) + (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (params.direct ? 1 : 0);
+    const int inst = (lists ? 128 : 0) + (waves == 8 ? 64 : 0) + (tails ? 32 : 0) + (past ? 16 : 0) + (t32 ? 8 : 0) + (bf16 ? 4 : 0) + (head_dim == 128 ? 2 : 0) + (direct ? 1 : 0);
     std::lock_guard<std::mutex> lock(mutex);
     if (dev >= 0 && dev < 64 && !raised[dev][inst]) {
       if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -127,3 +127,34 @@ def test_double_pieces_against_the_oracle(lens, heads, dtype, page, direct, tuni
         lerr = ((lse.cpu() - ref_lse).abs() / ref_lse.abs().clamp_min(1.0)).max().item()
         print(f"[parity] {err:.3e} {lerr:.3e}", flush=True)
         assert err <= (2e-3 if dtype == torch.float16 else 1.6e-2) and lerr <= 1e-4
+
+
+def test_the_launcher_refuses_what_it_has_no_instance_for(tmp_path):
+    # asked of the launcher itself, which answers before anything touches a GPU: combinations that no launch rule makes
+    import os
+    import shutil
+    import subprocess
+    _lib.load()
+    here = os.path.dirname(os.path.abspath(_lib.__file__))
+    src, so = tmp_path / "probe.cc", tmp_path / "probe.so"
+    src.write_text("""
+#include "hip/fwd_params.hpp"
+#include <cstring>
+struct ihipStream_t;
+namespace pat { int launch_split(bool bf16, int head_dim, ihipStream_t* stream, const SplitParams& params); }
+extern "C" int probe(int head_dim, int direct, int waves, int rows, int lists, int tail_pages, int stream_v) {
+  pat::SplitParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.direct = direct; p.waves = waves; p.tall_rows = rows; p.list_boxes = lists; p.tail_pages = tail_pages; p.stream_v = stream_v;
+  return pat::launch_split(false, head_dim, nullptr, p);
+}
+""")
+    subprocess.run([shutil.which("g++") or "c++", "-std=c++17", "-shared", "-fPIC", f"-I{here}/csrc", f"-I{os.path.dirname(here)}/include", str(src), "-o", str(so),
+                    f"-L{here}", "-lpat_amd", f"-Wl,-rpath,{here}", "-Wl,--allow-shlib-undefined"], check=True)
+    probe = C.CDLL(str(so)).probe
+    for case in [(64, 0, 8, 16, 0, 0, 0),                                                                  # eight waves and partial rows at head_dim 64
+                 (128, 1, 8, 16, 0, 0, 1), (128, 0, 8, 32, 0, 2, 0), (128, 0, 8, 32, 4, 0, 0), (128, 1, 5, 16, 0, 0, 0),
+                 (64, 0, 4, 32, 4, 0, 0), (128, 0, 4, 16, 4, 0, 0), (128, 1, 4, 32, 4, 0, 0),              # lists: head_dim 128, 32-row form, partial rows
+                 (128, 0, 4, 32, 4, 2, 0), (128, 0, 4, 32, 4, 0, 1),
+                 (128, 1, 4, 16, 0, 2, 0), (128, 1, 4, 32, 0, 2, 1)]:                                      # tails: 32-row form, V through the caches
+        assert probe(*case) == 1, case                                                                     # hipErrorInvalidValue
