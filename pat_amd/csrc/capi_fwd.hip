@@ -218,6 +218,8 @@ int check_args(const pat_fwd_args* a) {
       return fail(PAT_ERR_INVALID, at("plan table row stride smaller than its width"));
     if ((b.flags & PAT_BUCKET_ITEMS) && (b.num_items > b.num_boxes || b.num_items < (b.num_boxes + 1) / 2))
       return fail(PAT_ERR_INVALID, at("a bucket's items hold one or two of its boxes each"));
+    if ((b.flags & PAT_BUCKET_TAILS) && (b.num_items < 0 || b.num_items > b.num_boxes))   // (where its tails table stands)
+      return fail(PAT_ERR_INVALID, at("a bucket with tails has no item table, or items that hold one or two of its boxes each"));
     if (b.q_table_stride > INT32_MAX || b.block_table_stride > INT32_MAX)
       return fail(PAT_ERR_INVALID, at("plan table row stride too large"));
     if ((int64_t)b.max_seqs * ratio > 64)

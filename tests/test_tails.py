@@ -303,3 +303,12 @@ def test_not_taken_where_a_merge_follows_all_the_same(tuning):
     assert tails() is False
     tuning(pairs=_lib.PAT_TAILS_ALWAYS)      # (asked for, they are walked by the tall workgroups and merged)
     assert tails(out=0x10004) is True
+
+
+def test_an_item_count_that_is_none_is_refused():
+    # the tails table is found behind so many items, with or without their own flag
+    lib = _lib.load()
+    leaf = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAIL | 1 << _lib.PAT_TAIL_BOXES_SHIFT
+    for items, ok in ((0, True), (64, True), (128, True), (-1, False), (129, False)):
+        a = _tail_args((64, 128, 8, 2048, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAILS, items), (16, 1024, 1, 32, leaf, 0), 64, 8, 128, 1024, 32)
+        assert (lib.pat_fwd_validate(C.byref(a)) == 0) is ok, items
