@@ -274,7 +274,7 @@ typedef struct pat_fwd_bucket {
 #define PAT_BUCKET_ITEMS 2
 /* Tails: boxes of one sequence and few tokens whose sequence also sits in a box of 17..64 rows, whose workgroup may walk them
  * behind its own tokens; the launch then has no workgroups and no partial-result slots for them.
- * PAT_BUCKET_TAIL: every box of the bucket is a tail (one sequence each, at most 64 tokens wide) and stands in exactly one entry of
+ * PAT_BUCKET_TAIL: every box of the bucket is a tail (one sequence each, at most PAT_MAX_TAIL_TOKENS wide) and stands in exactly one entry of
  * one tails table. Its sequences' ordinals (q_slot) number the tails behind all other boxes. PAT_TAIL_BOXES(flags): the most boxes of a
  * sequence that are no tails.
  * PAT_BUCKET_TAILS (tile labels above 16): kv and the item table (num_items rows, possibly 0, with or without PAT_BUCKET_ITEMS) are
@@ -282,6 +282,7 @@ typedef struct pat_fwd_bucket {
  * none; `bucket` as the buckets of the launch are numbered - and, int32 [batch], the boxes of each sequence that are no tails.
  * A launch may make use of the tails or treat those buckets like any other; it needs both flags. The caller vouches for the
  * tables as for items: growing a tail in its own bucket keeps them right. */
+#define PAT_MAX_TAIL_TOKENS 64
 #define PAT_BUCKET_TAILS 4
 #define PAT_BUCKET_TAIL 8
 #define PAT_TAIL_BOXES_SHIFT 8

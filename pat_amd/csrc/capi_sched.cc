@@ -201,15 +201,14 @@ static int lay_out(const pat::Plan& p, int page, FlatPlan& f) {
   order.resize((size_t)nb);
   int spare = PAT_MAX_FLAT_BUCKETS - nb;
 
-  // Tails: boxes of one sequence, up to kMaxTailTokens wide, whose sequence also sits in a box of more than 16 rows. A launch may
+  // Tails: boxes of one sequence, up to PAT_MAX_TAIL_TOKENS wide, whose sequence also sits in a box of more than 16 rows. A launch may
   // have that box's workgroup walk them too (PAT_BUCKET_TAILS). Of several such boxes the shortest takes the tail.
-  constexpr int kMaxTailTokens = 64;
   struct Claim { int bucket = -1, box = -1, j = 0; };
   std::vector<Claim> claim((size_t)layout->batch);   // per sequence: where its tail may go
   std::vector<std::vector<char>> is_tail((size_t)nb);
   bool any_tail = false;
   auto may_hold_tails = [&](const pat::Bucket& bk) {
-    return bk.mnw[0] <= 16 && bk.max_seqs == 1 && (int64_t)bk.max_blocks * page <= kMaxTailTokens;
+    return bk.mnw[0] <= 16 && bk.max_seqs == 1 && (int64_t)bk.max_blocks * page <= PAT_MAX_TAIL_TOKENS;
   };
   const bool look = std::any_of(p.buckets.begin(), p.buckets.end(), may_hold_tails);
   for (int b = 0; b < nb && look; ++b) {

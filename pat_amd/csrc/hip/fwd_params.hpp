@@ -2,6 +2,8 @@
 #pragma once
 #include <cstdint>
 
+#include "pat_amd.h"
+
 namespace pat {
 
 constexpr int kMaxBuckets = 12;    // the reference dispatches 12 tile shapes (static_switch.h:3-66)
@@ -11,7 +13,8 @@ constexpr int kStepTokens = 32;    // KV tokens one wave consumes per loop itera
 constexpr int kGridX = 1 << 20;     // workgroups per grid.x slice (grid.y counts slices)
 constexpr int kMaxTall32Tokens = 64 * 64; // tokens of a tall piece in the 32-row form (an address per lane and 64-token super-step)
 constexpr int kMaxChunkPages = 128; // page ids of a chunk: two per lane of a wave
-constexpr int kMaxTailTokens = 64;  // tokens of a tail: two steps, at most four pages, so that those of a wave's 32 rows are two per lane
+constexpr int kMaxTailTokens = PAT_MAX_TAIL_TOKENS;  // tokens of a tail (the planner's bound)
+static_assert(32 * (kMaxTailTokens / 16) <= 2 * 64, "the pages, of 16 tokens and more, of the tails of a wave's 32 rows are two per lane");
 // The merge kernel's forms by slots and rows. Launches of up to 8 slots per row: a wave per row, or a half-wave from so many rows.
 // Launches of 9 slots and more: where rows are few a workgroup takes a row, a wave of which requests eight rows at once, as many as
 // one of the other forms. Whole calls, us (the split kernel is the same in all), a wave per row / the form taken:
