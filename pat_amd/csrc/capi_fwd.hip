@@ -658,7 +658,7 @@ void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) 
   if (g->tall_rows != 32 || a->head_dim != 128 || g->direct || g->stream_v || g->tail_pages > 0 || a->kv_heads % kWaves != 0 || (forced & PAT_LISTS_NEVER)) return;
   auto fits = [&](int i) {
     const pat_fwd_bucket& b = a->buckets[i];
-    return b.num_boxes > 0 && row_tiles(b.mnw[0]) == 1 && b.max_seqs == 1 && g->bucket_chunks[i] == 1 &&
+    return b.num_boxes > 0 && row_tiles(b.mnw[0]) == 1 && b.max_seqs == 1 && b.max_blocks > 0 && g->bucket_chunks[i] == 1 &&
            (int64_t)b.max_blocks * a->page_size <= kStepTokens && g->bucket_heads_per_wg[i] == kWaves;
   };
   int64_t others = 0, single = 0;

@@ -121,3 +121,12 @@ def test_static_launch_box_by_box_keeps_the_switches(tuning):
         assert f"needs {need.value} bytes" in _lib.last_error()
         sizes.append(need.value)
     assert sizes[0] < sizes[1]
+
+
+def test_boxes_without_blocks_are_no_lists(tuning):
+    # (the record kernel divides by a list's pages per box)
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    tuning(pairs=_lib.PAT_LISTS_ALWAYS)
+    for end, lists in ((0, False), (32, True)):
+        assert lib.pat_fwd_geometry_of(C.byref(_args((64, 16, 32, 1408, EVEN), (16, 512, 1, end, EVEN), 16, 8, 512, 32)), C.byref(g)) == 0
+        assert bool(g.flags & _lib.PAT_GEOMETRY_LISTS) is lists
