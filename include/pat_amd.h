@@ -314,7 +314,8 @@ typedef struct pat_fwd_tuning {
                                      /* 0 chosen per launch from its sizes, 1 always, 2 never;      */
                                      /* + PAT_STREAM_V_ALWAYS / _NEVER: V of boxes <= 16 rows read  */
                                      /* past the caches, in pieces that no other of up to 64 boxes  */
-                                     /* of the bucket and no tall box reads; + PAT_TAILS_ALWAYS /   */
+                                     /* of the bucket and no tall box reads (with either the launch  */
+                                     /* keeps its pieces, none of double length); + PAT_TAILS_ALWAYS / */
                                      /* _NEVER: tails walked by tall workgroups (PAT_BUCKET_TAILS); */
                                      /* + PAT_WAVES_8 / _4: waves per workgroup of single-slot      */
                                      /* launches without tall boxes (_4 also where pieces of double */

@@ -624,25 +624,6 @@ int plan_geometry_for(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometr
   return PAT_OK;
 }
 
-// Which form of the tall path (boxes of 17..64 rows)? 32-row tiles walk a tall box faster and cost a
-// resident workgroup per CU at head_dim 128. They are taken when that costs nothing - the whole launch
-// is resident anyway - or when its tall boxes outweigh that, estimated from sizes (tall_us against short_us and
-// short_rounds of estimate_launch). The lines were checked on 420 batches drawn over 1..1024 requests, 2..32 kv heads and both
-// head sizes whose launch is not resident in the 32-row form, both forms timed in their own cuts:
-//  * with items of two boxes (119 at head_dim 128): tall boxes longer than the shortest piece (shorter ones are mostly
-//    prologue and epilogue in either form) that take 0.6 of the others' streaming time and 3 us for every round of their
-//    workgroups, each of which waits longer for a place (us per call, 16 / 32 rows: 691 x (368 + 6..48) tokens at 16/2 heads
-//    23.7 / 25.2, 777 x (400 + 9..72) 26.1 / 27.6, but 198 x (512 + 1..2) at 64/8 21.8 / 19.8, `1,1024_2048,32` 153 / 117,
-//    `1,4,256_32,256,32` 25.8 / 21.4). More than 3 % behind the other form: 8.
-//  * without items (213 at head_dim 128): from 1024 tokens and an equal share (128 x (4096 + 64..512) at 32/8 heads,
-//    boxes not in twos: 52.5 / 57.3). More than 3 % behind: 54, nearly all left to the 16-row form.
-//  * at head_dim 64 (88) the 32-row form costs no place: from 640 tokens, 0.3 of the streaming time and 2 us a round
-//    (102 x (4848 + 580..1160) at 32/8 heads, six nodes: 69.6 / 62.3). More than 3 % behind: 7; the lines above: 11.
-// Two boxes of a node are served by one workgroup (32-row form, PAT_BUCKET_ITEMS) where the tall boxes fill the
-// device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
-// part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
-// boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice
-// as often to be as many, only add partial rows (4 boxes x 8 of 2048 tokens: 22.4 / 23.5).
 // Lists: workgroups that walk several private boxes of one step each, one after the other (32-row form at head_dim 128, whose
 // two places per CU such boxes queue for). A workgroup of one of them is 4-5 us of launch, record, page ids, first tiles and
 // stores for half a microsecond of work; in a list a further box costs 2-2.5 us. Taken where the launch holds 1.75 times what
@@ -708,6 +689,25 @@ int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g
   return PAT_OK;
 }
 
+// Which form of the tall path (boxes of 17..64 rows)? 32-row tiles walk a tall box faster and cost a
+// resident workgroup per CU at head_dim 128. They are taken when that costs nothing - the whole launch
+// is resident anyway - or when its tall boxes outweigh that, estimated from sizes (tall_us against short_us and
+// short_rounds of estimate_launch). The lines were checked on 420 batches drawn over 1..1024 requests, 2..32 kv heads and both
+// head sizes whose launch is not resident in the 32-row form, both forms timed in their own cuts:
+//  * with items of two boxes (119 at head_dim 128): tall boxes longer than the shortest piece (shorter ones are mostly
+//    prologue and epilogue in either form) that take 0.6 of the others' streaming time and 3 us for every round of their
+//    workgroups, each of which waits longer for a place (us per call, 16 / 32 rows: 691 x (368 + 6..48) tokens at 16/2 heads
+//    23.7 / 25.2, 777 x (400 + 9..72) 26.1 / 27.6, but 198 x (512 + 1..2) at 64/8 21.8 / 19.8, `1,1024_2048,32` 153 / 117,
+//    `1,4,256_32,256,32` 25.8 / 21.4). More than 3 % behind the other form: 8.
+//  * without items (213 at head_dim 128): from 1024 tokens and an equal share (128 x (4096 + 64..512) at 32/8 heads,
+//    boxes not in twos: 52.5 / 57.3). More than 3 % behind: 54, nearly all left to the 16-row form.
+//  * at head_dim 64 (88) the 32-row form costs no place: from 640 tokens, 0.3 of the streaming time and 2 us a round
+//    (102 x (4848 + 580..1160) at 32/8 heads, six nodes: 69.6 / 62.3). More than 3 % behind: 7; the lines above: 11.
+// Two boxes of a node are served by one workgroup (32-row form, PAT_BUCKET_ITEMS) where the tall boxes fill the
+// device without being cut along KV: three workgroups per eight CUs. The pair takes as long as one box, so the tall
+// part of such a launch halves (us per call, boxes / pairs: 24 boxes x 8 kv heads of 2736 tokens 69.4 / 60.0, 128
+// boxes x 8 of 2048 tokens 141.8 / 127.7). With fewer boxes the other workgroups are idle CUs anyway and pairs, cut twice
+// as often to be as many, only add partial rows (4 boxes x 8 of 2048 tokens: 22.4 / 23.5).
 int plan_form(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, const int tail_pages) {
   g->tail_pages = tail_pages;
   int64_t widest_tall = 0, tall_box_heads = 0;
@@ -908,7 +908,7 @@ __device__ bool holds_tokens(const RecordParams& p, int64_t least) {
   unsigned long long eighths = 0;
   for (int b = 0; b < p.num_buckets; ++b) {
     const RecordBucket& bk = p.bucket[b];
-    if (bk.row_tiles != 1 || bk.max_blocks <= 0 || bk.num_items == 0) continue;
+    if (bk.row_tiles != 1 || bk.max_blocks <= 0) continue;
     const int last = bk.num_boxes - 1, step = (bk.num_boxes + 64 * kPerLane - 1) / (64 * kPerLane), cap = bk.max_blocks * p.page_size;
     int box[kPerLane], next[kPerLane], kv[kPerLane], kv_next[kPerLane], page[kPerLane][4], own[kPerLane][4], other[kPerLane][4];
 #pragma unroll

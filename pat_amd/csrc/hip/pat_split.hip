@@ -605,10 +605,9 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc2[db][i] = 0.f;
 
-    // this lane's place in its wave's half: row RPI*i + r_in of load i, and the piece it fetches there
     // ---- tails: the few tokens that each sequence of the box has behind it, alone ----------------------
-    // Behind the piece, whose registers are free again. A wave takes those of its own 32 rows one after the other (of two waves on the same rows every second one): rows of one
-    // sequence on 16x16x32 tiles, as the boxes of <= 16 rows are walked, K straight into operand registers, V through a region of
+    // Behind the piece, whose registers are free again. A wave takes those of its own 32 rows one after the other (of two waves on the
+    // same rows every second one): rows of one sequence on 16x16x32 tiles, as the boxes of <= 16 rows are walked, K straight into operand registers, V through a region of
     // LDS of this wave's own, the next step's tiles in flight. Each tail is a softmax of its own, added to its rows' state in fp32: a
     // tile that several sequences shared, masked, would carry one's infinite or NaN V into the others' sums.
     const int* __restrict__ tail_tab = pages_tab + record_max_pages;   // tokens by sequence, then pages
@@ -664,6 +663,7 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
         }
       });
     };
+    // this lane's place in its wave's half: row RPI*i + r_in of load i, and the piece it fetches there
     const int r_in = lane / CPR, c_in = lane % CPR;
     auto k_piece = [&](int i) { return (unsigned)(D == 128 ? c_in ^ ((RPI * i + r_in) & 15) : c_in ^ (((RPI * i + r_in) >> 1) & 7)) * 16u; };
     const unsigned v_piece = (unsigned)(D == 128 ? c_in ^ ((r_in & 3) << 2) : c_in ^ (((r_in >> 1) & 1) << 2)) * 16u;
