@@ -68,6 +68,7 @@ def _merge_form(a):
 
 @pytest.mark.parametrize("shared,lens,heads", [
     (2048, [32] * 1023, (64, 8)),       # tails by the rule
+    (384, [1, 2, 3, 4] * 92, (64, 8)),  # the same, short
     (0, [320] * 40, (32, 8)),           # nothing shared, whole boxes
     (0, [690] * 5 + [600], (32, 32)),   # pieces of double length that leave one
 ])
@@ -93,11 +94,11 @@ def test_a_merge_follows(shared, lens, heads, at, tuning):
 @pytest.mark.parametrize("name,shared,lens,heads,d,dtype,page,switch,tails", [
     ("tails, forced", 640, (64, 5, 40), (32, 8), 128, torch.float16, 16, _lib.PAT_TAILS_ALWAYS, True),
     ("tails, forced, pieces", 1680, (48, 1, 60), (16, 8), 128, torch.bfloat16, 16, _lib.PAT_TAILS_ALWAYS, True),
-    ("tails or not by the rule", 384, (369, 1, 4), (64, 8), 64, torch.float16, 16, 0, None),
+    ("tails but for them", 384, (369, 1, 4), (64, 8), 64, torch.float16, 16, 0, False),
     ("unshared", 0, (40, 300, 320), (32, 8), 128, torch.bfloat16, 16, 0, False),
     ("unshared, head_dim 64", 0, (64, 100, 200), (8, 8), 64, torch.float16, 32, 0, False),
     ("pieces of double length", 0, (6, 600, 690), (32, 32), 128, torch.float16, 16, 0, False),
-    ("eight waves", 0, (8, 288, 288), (8, 8), 128, torch.float16, 16, _lib.PAT_WAVES_8, False),
+    ("eight waves asked for", 0, (8, 288, 288), (8, 8), 128, torch.float16, 16, _lib.PAT_WAVES_8, False),
 ])
 @pytest.mark.parametrize("form", ["tree", "table"])
 def test_rows_of_empty_requests(name, shared, lens, heads, d, dtype, page, switch, tails, form, tuning, monkeypatch):
@@ -129,7 +130,7 @@ def test_rows_of_empty_requests(name, shared, lens, heads, d, dtype, page, switc
             prefix_attn_with_kvcache(q, k, v, i.num_split_per_seq, i.q_tables, i.block_tables, i.num_seqs_per_CTAs, i.CTA_ranks, i.kv_in_CTAs,
                                      i.MNWs, i.max_split_per_seq, i.max_seqs_in_CTA, i.max_blocks_in_CTA, 0.09, out, None, softmax_lse=lse)
         torch.cuda.synchronize()
-        if form == "tree" and tails is not None:
+        if form == "tree":
             assert [g["tails"] for g in i._launch_geometries] == [tails]
         assert bool((out[empty] == 0).all()) and bool((lse[empty] == float("-inf")).all())
         err = (out[full].float().cpu() - ref_out.float()).abs().max().item()

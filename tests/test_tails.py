@@ -62,7 +62,8 @@ def _flat_layout(w):
     (38, 640, (20, 32), (32, 8), 16),       # six requests over: a box of 24 rows of another label
     (67, 512, (9, 16), (16, 8), 16),        # three over: a box of 6 rows, whose tails are nobody's
     (130, [256, 512], (1, 60), (8, 8), 64),
-    (40, 640, (60, 120), (32, 8), 16),      # too long
+    (40, 640, (60, 120), (32, 8), 16),      # some too long: the others in a launch bucket of their own
+    (40, 640, (65, 120), (32, 8), 16),      # all too long
 ])
 def test_planner_tables(seqs, prefix, tails, heads, page):
     w = _batch(seqs, prefix, tails, heads, 128, torch.float16, page)
