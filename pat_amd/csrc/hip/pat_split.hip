@@ -726,11 +726,29 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
       }
     };
 
-    // LDS offsets of this lane's operand reads inside a stage (token 0 of the stage; + 32 ROWB for tokens 32..), those of kk = 0 and
-    // db = 0: the others differ in the place inside the row alone, which is an exclusive or with 32 kk and 64 db (the stages
-    // start at multiples of a row). Kept one by one they were 10 more registers.
-    const unsigned k_rd = (unsigned)(n32 * ROWB + (h2 ^ (D == 128 ? n32 & 15 : (n32 >> 1) & 7)) * 16);
-    const unsigned v_rd = (unsigned)(KTILE + (h2 * 4 + (n >> 2)) * ROWB + (D == 128 ? n >> 2 : (n >> 3) & 1) * 64 + (g & 1) * 32 + (n & 3) * 8);
+    // LDS offsets of this lane's operand reads inside a stage (token 0 of the stage; + 32 ROWB for tokens 32..). Those of kk and db differ from
+    // those of 0 in the place inside the row alone, which is an exclusive or with 32 kk and 64 db (the stages start at multiples of a
+    // row). Two offsets instead of twelve, 10 registers less, where those count: with tails or lists, and at head_dim 64, where 128 registers
+    // are a fourth workgroup per CU (102 requests over 4848 tokens, 580..1160 of their own, at 32/8 heads 49.0 us, with twelve 54.3). Elsewhere
+    // the sum ahead of the exclusive or is one more wait for each read (34 tall boxes in 170 workgroups 15.39 / 15.33, 64 requests behind one prefix
+    // 21.81 / 21.71).
+    constexpr bool TWO_OFFSETS = TAILS || LISTS || D == 64;
+    constexpr int KRD = TWO_OFFSETS ? 1 : KK2, VRD = TWO_OFFSETS ? 1 : DB2;
+    unsigned k_rd[KRD], v_rd[VRD];
+#pragma unroll
+    for (int kk = 0; kk < KRD; ++kk)
+      k_rd[kk] = (unsigned)(n32 * ROWB + ((2 * kk + h2) ^ (D == 128 ? n32 & 15 : (n32 >> 1) & 7)) * 16);
+#pragma unroll
+    for (int db = 0; db < VRD; ++db)
+      v_rd[db] = (unsigned)(KTILE + (h2 * 4 + (n >> 2)) * ROWB + (db ^ (D == 128 ? n >> 2 : (n >> 3) & 1)) * 64 + (g & 1) * 32 + (n & 3) * 8);
+    auto k_row = [&](const PAT_LDS char* stage, int kk) -> const PAT_LDS char* {
+      if constexpr (TWO_OFFSETS) return (const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + k_rd[0]) ^ (kk * 32u));
+      else return stage + k_rd[kk];
+    };
+    auto v_row = [&](const PAT_LDS char* stage, int db) -> const PAT_LDS char* {
+      if constexpr (TWO_OFFSETS) return (const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + v_rd[0]) ^ (db * 64u));
+      else return stage + v_rd[db];
+    };
 
     // HALVES x 32 tokens of online-softmax attention for this wave's 32 rows; `stage` points at the first of them
     // (its K rows; the V rows KTILE further), t0 is that token's place in the piece. First the scores and probabilities ...
@@ -744,7 +762,7 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
         vec8 kop[KK2];
 #pragma unroll
         for (int kk = 0; kk < KK2; ++kk)
-          kop[kk] = *(const PAT_LDS vec8*)((const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + k_rd) ^ (kk * 32u)) + a * 32 * ROWB);
+          kop[kk] = *(const PAT_LDS vec8*)(k_row(stage, kk) + a * 32 * ROWB);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[a][i] = 0.f;
@@ -797,7 +815,7 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
       auto read_v = [&](int t, s16x8 (&v)[DB2]) {
 #pragma unroll
         for (int db = 0; db < DB2; ++db) {
-          const PAT_LDS char* src = (const PAT_LDS char*)(size_t)(((unsigned)(size_t)stage + v_rd) ^ (db * 64u)) + t * 16 * ROWB;
+          const PAT_LDS char* src = v_row(stage, db) + t * 16 * ROWB;
           s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)src);
           s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PAT_LDS s16x4*)(src + 8 * ROWB));
           v[db] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -1057,8 +1075,9 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
     // combine the 4 waves' states through LDS and write the partial
     float* cbuf = (float*)smem;
     constexpr int COLS = 16 * D / (WAVES * 64) > 4 ? 16 * D / (WAVES * 64) : 4;   // columns a thread finalises
-    const int crow = tid / (D / COLS);          // row this thread finalises (past 16: none)
-    const int ccol = (tid % (D / COLS)) * COLS; // its first column
+    constexpr int TPR = D / COLS;               // threads a row
+    const int crow = (int)((unsigned)tid / TPR);          // row this thread finalises (past 16: none)
+    const int ccol = (int)((unsigned)tid % TPR) * COLS;   // its first column
     __syncthreads();  // every wave is done with its staging region
     if (g == 0) { s_m[wave * 16 + n] = m_run; s_l[wave * 16 + n] = l_run; }
 #pragma unroll
@@ -1067,8 +1086,8 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
     __syncthreads();
 
     // the slot of row crow sits in lane crow of every wave
-    const int cslot0 = __shfl(my_slot0, crow & 15);
-    if (cslot0 >= 0 && crow < 16) {
+    const int cslot0 = __shfl(my_slot0, WAVES * 64 > 16 * TPR ? crow & 15 : crow);
+    if (cslot0 >= 0 && (WAVES * 64 == 16 * TPR || crow < 16)) {
       float mw[WAVES], mmax = neg_inf();
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) { mw[w] = s_m[w * 16 + crow]; mmax = fmaxf(mmax, mw[w]); }
