@@ -668,15 +668,17 @@ void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) 
 // Pieces twice as long, eight waves per workgroup: launches without tall boxes whose pieces put two workgroups on some CUs and one on
 // the others, so that the two set the time while the others idle. In pieces of double length every workgroup has a CU of its own; a wave
 // has the steps it had (its softmax covers as many tokens: results are as exact), there are half the partial rows and, where one piece is
-// left, no merge. At head_dim 128 from 289 to 400 workgroups that become 256 at most. 694 drawn batches there: geometric mean 0.943, eight
-// 2-5 % slower (8 of 693..1039 tokens at 32/8 heads, five pieces that become three, 10.7 / 11.3), errors against 64 bits 0.998 of four waves'.
-// us per call, four waves / eight: 8 of 782 at 64/8 10.8 / 10.0, 4 of 2033..2541 at 16/8 13.3 / 12.3, 8 of 2239 at 64/8 18.1 / 16.9, 12 of
-// 552..690 at 16/16, whole with eight, 16.0 / 13.3. Outside: 257..288 workgroups 0.965, but eight of 69 3-8 % slower (4 of 1453..1598 at
+// left, no merge. At head_dim 128 from 289 to 400 workgroups that become 256 at most, of requests that sit in one box each. 5458 drawn batches
+// there: geometric mean 0.943, one piece left 0.81; 53 more than 2 % slower, twelve of them 5-20 % (mostly five pieces of a few steps that become three: 8
+// of 782 tokens, pages of 48, at 64/8 heads 10.0 / 10.3); errors against 64 bits 0.9986 of four waves'. us per call, four waves / eight: 4 of
+// 2033..2541 at 16/8 13.3 / 12.4, 8 of 2239 at 64/8 18.1 / 16.8, 12 of 552..690 at 16/16, whole with eight, 15.9 / 13.3. Outside: requests in several
+// boxes 1.010 over 209, 62 of them 2-31 % slower (4 over 3792, 992 and 12..48 tokens at 16/8 10.6 / 12.1: what one piece saves elsewhere, the
+// merge, stays); 257..288 workgroups 0.965, but eight of 69 3-8 % slower (4 of 1453..1598 at
 // 64/8, 288, 10.3 / 10.9: CUs left without work); 401..512, where nearly every CU had two, 0.99, fourteen of 202 2-9 % slower; more than
 // 256 left 1.13; head_dim 64 0.98 to 0.99. (Not where V past the caches is forced on or off: that switch changes no launch's pieces.)
 int double_pieces(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) {
-  if (a->head_dim != 128 || g->direct || g->stream_v || g->waves != kWaves || tune.chunk_tokens > 0 || (waves_switch(tune) & PAT_WAVES_4) || stream_switch(tune) != 0 ||
-      8 * g->total_wgs <= 9 * kNumCUs || 16 * g->total_wgs > 25 * kNumCUs) return PAT_OK;
+  if (a->head_dim != 128 || a->max_split_per_seq != 1 || g->direct || g->stream_v || g->waves != kWaves || tune.chunk_tokens > 0 ||
+      (waves_switch(tune) & PAT_WAVES_4) || stream_switch(tune) != 0 || 8 * g->total_wgs <= 9 * kNumCUs || 16 * g->total_wgs > 25 * kNumCUs) return PAT_OK;
   pat_fwd_tuning twice = tune;
   twice.chunk_tokens = 2 * g->chunk;
   Geometry wide;

@@ -158,3 +158,18 @@ extern "C" int probe(int head_dim, int direct, int waves, int rows, int lists, i
                  (128, 0, 4, 32, 4, 2, 0), (128, 0, 4, 32, 4, 0, 1),
                  (128, 1, 4, 16, 0, 2, 0), (128, 1, 4, 32, 0, 2, 1)]:                                      # tails: 32-row form, V through the caches
         assert probe(*case) == 1, case                                                                     # hipErrorInvalidValue
+
+
+def test_double_pieces_are_for_requests_of_one_box(tuning):
+    # requests that sit in several boxes are merged all the same, and longer pieces lose there
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    for most, eight in ((1, True), (2, False), (3, False)):
+        a = _args(8, 2240, 64, 8, 128)
+        a.max_split_per_seq = most
+        tuning()
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        assert bool(g.flags & _lib.PAT_GEOMETRY_WAVES_8) is eight
+        got = (g.num_workgroups, g.num_slots)
+        tuning(pairs=_lib.PAT_WAVES_4)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0
+        assert (got == (g.num_workgroups, g.num_slots)) is not eight
