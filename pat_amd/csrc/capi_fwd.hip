@@ -626,13 +626,13 @@ int plan_geometry_for(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometr
 
 // Lists: workgroups that walk several private boxes of one step each, one after the other (32-row form at head_dim 128, whose
 // two places per CU such boxes queue for). A workgroup of one of them is 4-5 us of launch, record, page ids, first tiles and
-// stores for half a microsecond of work; in a list a further box costs 2-2.5 us. Taken where the launch holds 1.75 times what
-// fits at once and all of it fits with the boxes in lists, so that nothing starts late any more. us per call, a box a workgroup /
-// lists: 512 x (1408 + 32) tokens at 16/8 heads (1280 workgroups, 512 with lists of four) 32.0 / 28.7, 245 x (1696 + 352 + 3..6)
-// at 16/16 (1236, 504) 23.9 / 21.0, 240 x (1968 + 4..16) at 32/32 34.7 / 31.6, 945 x (1376 + 1..4) at 8/8 30.7 / 27.9. Of 250
-// drawn batches of short ends the rule takes 24: geometric mean 0.978, the slowest 1.02. Outside of it: some still wait, 499 x
-// (864 + 4..8) at 32/8 31.3 / 34.4; fewer workgroups, 339 x (384 + 96 + 8..16) at 64/8 (878) 27.2 / 32.1, 310 x (1104 + 144 +
-// 7..28) at 8/8 (852) 17.1 / 17.9; two steps and more, 175 x (1248 + 320 + 11..44) at 16/16 22.8 / 24.6; head_dim 64 (three
+// stores for half a microsecond of work; in a list a further box costs 2-2.5 us. Taken where the launch holds 2.25 times what
+// fits at once, its other workgroups leave half the places, and all of it fits with the boxes in lists, so that nothing starts late any more. us per call, a
+// box a workgroup / lists: 512 ends of 32 tokens behind 16 paths of 1408 at 16/8 heads (1280 workgroups, 512 with lists of four) 31.2 / 27.6, 240 x (1968 +
+// 4..16) at 32/32 35.1 / 31.0, 945 x (1376 + 1..4) at 8/8 29.4 / 26.3. Of 1988 drawn batches of short ends that hold 1.75 times what fits, the rule takes
+// 716: geometric mean 0.968, 43 more than 2 % slower, two of them 7-10 % (217 x (1136 + 480 + 13..26) at 32/32 42.5 / 46.7). Outside of it: fewer workgroups,
+// 1.75 to 2.25 times, 0.997, 75 of 394 slower; less than half the places left, 1.006, 216 of 868, up to 23 %; some still wait, 499 x
+// (864 + 4..8) at 32/8 31.3 / 34.4; two steps and more, 175 x (1248 + 320 + 11..44) at 16/16 22.8 / 24.6; head_dim 64 (three
 // places per CU): 100 batches 0.99, fourteen of them 2-13 % slower.
 void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) {
   const int forced = switches(tune, PAT_LISTS_ALWAYS | PAT_LISTS_NEVER);
@@ -652,7 +652,7 @@ void make_lists(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g) 
   }
   if (single == 0) return;
   const int64_t resident = (int64_t)resident_wgs_per_cu(a->head_dim, 32) * kNumCUs;
-  if (!(forced & PAT_LISTS_ALWAYS) && (others >= resident || 4 * (others + single) < 7 * resident)) return;
+  if (!(forced & PAT_LISTS_ALWAYS) && (2 * others > resident || 4 * (others + single) < 9 * resident)) return;
   const int64_t per = std::max<int64_t>(2, std::min<int64_t>(kMaxListBoxes, ceil_div64(single, std::max<int64_t>(1, resident - others))));
   auto saved = [&](int i) { return ((int64_t)a->buckets[i].num_boxes - ceil_div64(a->buckets[i].num_boxes, per)) * (a->kv_heads / kWaves); };
   int64_t total = others + single;
@@ -755,12 +755,14 @@ int plan_form(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, co
 //    than the stream of their K and V;
 //  * by themselves: that stream, or kTailRoundUs for every further round of workgroups, as far as the tall workgroups keep the chip
 //    (on idle CUs tails run beside them), and the merge, 3 us and its partial rows at 4.5 TB/s.
-// Not where the tall workgroups, uncut for that one result, leave more than three of eight CUs idle, unless a wave has two steps at most.
-// us per call, by themselves / with the tall boxes: 1024 x (2048 + 32) tokens at 64/8 heads 118 / 100, + 64 141 / 121, + 16 116 / 94,
-// 2048 x (1024 + 32) at 32/8 114 / 92, 827 x (464 + 26) at 64/8 59.1 / 39.5, 369 x (384 + 1..4), head_dim 64, 19.9 / 14.6, but few rows per
-// sequence (many tails a wave) 1010 x (768 + 5..10) at 16/16 44.1 / 74.1, idle CUs 283 x (1504 + 58..64) at 64/8 40.0 / 49.1, 256 x
-// (544 + 32) 25.1 / 26.2, and, with a merge all the same, 512 x (1408 + 32) at 16/8 32.1 / 37.1. Of 290 drawn batches with tails the rule
-// takes 10: geometric mean 0.84, the slowest 1.01; 9 of the 41 others without a merge would be 3-27 % faster, most far slower.
+// Not where the tall workgroups, uncut for that one result, leave more than three of eight CUs idle, unless a wave has two steps at most, nor,
+// with more than four steps, where their last round on the CUs is less than three quarters full (264 of them end on the eight CUs with two), and only
+// where the estimate is a fifth lower.
+// us per call, by themselves / with the tall boxes: 1024 x (2048 + 32) tokens at 64/8 heads 117.7 / 99.4, + 64 140.3 / 121.0, + 16 112.9 / 90.9,
+// 2048 x (1024 + 32) at 32/8 112.2 / 90.9, 827 x (464 + 26) at 64/8 59.4 / 43.8, 369 x (384 + 1..4), head_dim 64, 18.5 / 14.1, but few rows per
+// sequence (many tails a wave) 1010 x (768 + 5..10) at 16/16 44.1 / 74.1, idle CUs 283 x (1504 + 58..64) at 64/8 40.0 / 49.1, 264 workgroups 528 x
+// (1248 + 54) at 64/8 61.6 / 75.5, and, with a merge all the same, the 512 ends behind 16 paths of 1408 at 16/8 32.1 / 37.1. Of 1487 drawn batches that the
+// estimate alone would take (0.832, 133 more than 2 % slower, up to 38 %) the rule takes 910: 0.791, 19 more than 2 % slower, up to 14 %.
 constexpr double kTailStepUs = 2.5;
 constexpr double kTailRoundUs = 4.;
 bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& without) {
@@ -776,12 +778,13 @@ bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& with
   }
   steps *= std::max(1, (with.pairs ? 32 : 16) / group);
   if (steps > 2. && with.total_wgs < 5 * kNumCUs / 8) return false;
+  if (steps > 4. && 4 * with.total_wgs < 3 * kNumCUs * ceil_div64(with.total_wgs, kNumCUs)) return false;
   const double own_places = resident_wgs_per_cu(a->head_dim, without.tall_rows) * kNumCUs;
   const double with_us = std::max(steps * kTailStepUs * std::max(1., (double)with.total_wgs / (resident_wgs_per_cu(a->head_dim, 32) * kNumCUs)), bytes / 6e6);
   const double own_us = std::max(bytes / 5.8e6, kTailRoundUs * std::max(0., (double)without.total_wgs / own_places - 1.)) *
                         std::min(1., (double)with.total_wgs / kNumCUs);
   const double merge_us = 3. + (double)a->batch * a->heads * without.num_slots * a->head_dim * 4. / 4.5e6;
-  return with_us < own_us + merge_us;
+  return with_us < 0.8 * (own_us + merge_us);
 }
 
 // (Every launch comes through here, and small ones wait for the host: the overrides are read once, and arguments without tails are made only

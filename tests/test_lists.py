@@ -130,3 +130,19 @@ def test_boxes_without_blocks_are_no_lists(tuning):
     for end, lists in ((0, False), (32, True)):
         assert lib.pat_fwd_geometry_of(C.byref(_args((64, 16, 32, 1408, EVEN), (16, 512, 1, end, EVEN), 16, 8, 512, 32)), C.byref(g)) == 0
         assert bool(g.flags & _lib.PAT_GEOMETRY_LISTS) is lists
+
+
+def test_lists_only_where_they_leave_nothing_waiting(tuning):
+    # the lines of the rule: half the places left by the others, 2.25 times what fits at once
+    lib, g = _lib.load(), _lib.FwdGeometry()
+
+    def lists(boxes, requests):       # tall boxes in two pieces each, 8 kv heads: 16 workgroups a box; ends: two workgroups a request
+        a = _args((64, boxes, 32, 1408, EVEN), (16, requests, 1, 32, EVEN), 16, 8, requests, 32)
+        tuning(pairs=_lib.PAT_LISTS_NEVER, tall_rows=32)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0 and g.num_workgroups == 16 * boxes + 2 * requests
+        tuning(tall_rows=32)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        return bool(g.flags & _lib.PAT_GEOMETRY_LISTS)
+
+    assert lists(16, 448) and not lists(16, 447)        # 1152 workgroups
+    assert lists(16, 600) and not lists(17, 600)        # 256 others

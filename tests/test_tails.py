@@ -313,3 +313,19 @@ def test_an_item_count_that_is_none_is_refused():
     for items, ok in ((0, True), (64, True), (128, True), (-1, False), (129, False)):
         a = _tail_args((64, 128, 8, 2048, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAILS, items), (16, 1024, 1, 32, leaf, 0), 64, 8, 128, 1024, 32)
         assert (lib.pat_fwd_validate(C.byref(a)) == 0) is ok, items
+
+
+def test_not_taken_where_the_last_round_of_workgroups_is_thin(tuning):
+    # a wave of more than four steps of tails: the tall workgroups fill the CUs three quarters of every round, or the launch ends on a few
+    lib, g = _lib.load(), _lib.FwdGeometry()
+    leaf = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAIL | 1 << _lib.PAT_TAIL_BOXES_SHIFT
+
+    def tails(boxes, tokens):         # 8 requests a box, in twos: four a wave; 8 kv heads
+        a = _tail_args((64, 2 * boxes, 8, 1248, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS | _lib.PAT_BUCKET_TAILS, boxes), (16, 16 * boxes, 1, tokens, leaf, 0),
+                       64, 8, 128, 16 * boxes, 16)
+        assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
+        return bool(g.flags & _lib.PAT_GEOMETRY_TAILS)
+
+    tuning()
+    assert [tails(n, 64) for n in (32, 33, 47, 48, 64)] == [True, False, False, True, True]    # 256, 264, 376, 384 and 512 workgroups
+    assert tails(33, 32) is True                                                                # four steps
