@@ -628,7 +628,7 @@ int plan_geometry_for(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometr
 // two places per CU such boxes queue for). A workgroup of one of them is 4-5 us of launch, record, page ids, first tiles and
 // stores for half a microsecond of work; in a list a further box costs 2-2.5 us. Taken where the launch holds 2.25 times what
 // fits at once, its other workgroups leave half the places, and all of it fits with the boxes in lists, so that nothing starts late any more. us per call, a
-// box a workgroup / lists: 512 ends of 32 tokens behind 16 paths of 1408 at 16/8 heads (1280 workgroups, 512 with lists of four) 31.2 / 27.6, 240 x (1968 +
+// box a workgroup / lists: 512 ends of 32 tokens behind 16 paths of 1408 at 16/8 heads (1280 workgroups, 512 with lists of four) 30.6 / 27.3, 240 x (1968 +
 // 4..16) at 32/32 35.1 / 31.0, 945 x (1376 + 1..4) at 8/8 29.4 / 26.3. Of 1988 drawn batches of short ends that hold 1.75 times what fits, the rule takes
 // 716: geometric mean 0.968, 43 more than 2 % slower, two of them 7-10 % (217 x (1136 + 480 + 13..26) at 32/32 42.5 / 46.7). Outside of it: fewer workgroups,
 // 1.75 to 2.25 times, 0.997, 75 of 394 slower; less than half the places left, 1.006, 216 of 868, up to 23 %; some still wait, 499 x
@@ -749,42 +749,60 @@ int plan_form(const pat_fwd_args* a, const pat_fwd_tuning& tune, Geometry* g, co
 }
 
 // Tails walked by the workgroups of their sequences' tall boxes? Only where that leaves every row one partial result, so that the
-// split kernel writes `out` and no merge follows, and where it is the cheaper one by an estimate from sizes:
-//  * there: kTailStepUs for each 32-token step of a wave's tails (a wave has one tail in flight and waits for memory once per step:
-//    2.2-2.5 us), 32 rows' tails of a pair of boxes one after the other, half of that where two waves share the rows; never less
-//    than the stream of their K and V;
-//  * by themselves: that stream, or kTailRoundUs for every further round of workgroups, as far as the tall workgroups keep the chip
-//    (on idle CUs tails run beside them), and the merge, 3 us and its partial rows at 4.5 TB/s.
-// Not where the tall workgroups, uncut for that one result, leave more than three of eight CUs idle, unless a wave has two steps at most, nor,
-// with more than four steps, where their last round on the CUs is less than three quarters full (264 of them end on the eight CUs with two), and only
-// where the estimate is a fifth lower.
-// us per call, by themselves / with the tall boxes: 1024 x (2048 + 32) tokens at 64/8 heads 117.7 / 99.4, + 64 140.3 / 121.0, + 16 112.9 / 90.9,
-// 2048 x (1024 + 32) at 32/8 112.2 / 90.9, 827 x (464 + 26) at 64/8 59.4 / 43.8, 369 x (384 + 1..4), head_dim 64, 18.5 / 14.1, but few rows per
-// sequence (many tails a wave) 1010 x (768 + 5..10) at 16/16 44.1 / 74.1, idle CUs 283 x (1504 + 58..64) at 64/8 40.0 / 49.1, 264 workgroups 528 x
-// (1248 + 54) at 64/8 61.6 / 75.5, and, with a merge all the same, the 512 ends behind 16 paths of 1408 at 16/8 32.1 / 37.1. Of 1487 drawn batches that the
-// estimate alone would take (0.832, 133 more than 2 % slower, up to 38 %) the rule takes 910: 0.791, 19 more than 2 % slower, up to 14 %.
+// split kernel writes `out` and no merge follows, and where what it costs is a tenth below what it saves, estimated from sizes:
+//  * it costs kTailStepUs for each 32-token step of a wave's tails (a wave has one tail in flight and waits for memory once per step:
+//    2.2-2.5 us), 32 rows' tails of a pair of boxes one after the other, half of that where two waves share the rows, in every round of
+//    workgroups, and never less than the stream of their K and V; and, where the tall boxes, uncut for that one result, leave CUs idle,
+//    the share of the widest one's walk that those CUs would have had;
+//  * it saves that stream, or kTailRoundUs for every further round of workgroups, as far as the tall workgroups keep the chip (on idle
+//    CUs tails run beside them); the launch, records and pages of the tails' workgroups and the merge; its partial rows; and, where
+//    the launch without it would be in the 16-row form, what a super-step is slower there.
+// Not, with more than four steps a wave, where up to an eighth of the CUs would have two workgroups and the others one: the launch ends on those.
+// Where the tall boxes would be walked in the same way without it, results are as exact (1.0000 of the distance from 64 bits, 622 batches). Where they
+// would be in the 16-row form, whose probabilities are rounded against the largest score so far, they are 4 % (in pieces, each with a largest of its
+// own, 7 %) further from 64 bits, and 1 % where they would be in pieces of the 32-row form: only where what is saved without counting that form's
+// slower walk pays by itself, a merge at 3 us and its partial rows at 4.5 TB/s.
+// The constants are fitted to both times of 5030 drawn batches whose tails leave no merge; of 6772 others the rule takes 4246: geometric mean 0.800, 163
+// more than 2 % slower, up to 23 %. Of the ones it leaves 470 would be more than 10 % slower, 1197 5 % and more faster (most would change their form).
+// us per call, by themselves / with the tall boxes: 1024 x (2048 + 32) tokens at 64/8 heads 117.8 / 98.6, + 64 139 / 121, + 16 112 / 87, 2048 x (1024 +
+// 32) at 32/8 111 / 91, 827 x (464 + 26) at 64/8 57.0 / 36.5, 369 x (384 + 1..4), head_dim 64, 18.4 / 14.0, but few rows per sequence (many tails a
+// wave) 1010 x (768 + 5..10) at 16/16 49.0 / 73.1, idle CUs 283 x (1504 + 58..64) at 64/8 37.9 / 48.4, 264 workgroups 528 x (1248 + 54) at 64/8 56.2 /
+// 69.3, and, with a merge all the same, the 512 ends behind 16 paths of 1408 at 16/8 1.15 times as long.
 constexpr double kTailStepUs = 2.5;
-constexpr double kTailRoundUs = 4.;
+constexpr double kTailRoundUs = 3.3;
 bool tails_pay(const pat_fwd_args* a, const Geometry& with, const Geometry& without) {
   if (!with.direct) return false;
   const int group = a->heads / a->kv_heads;
-  double steps = 0., bytes = 0.;
+  double steps = 0., bytes = 0., super_steps = 0.;
   for (int i = 0; i < a->num_buckets; ++i) {
     const pat_fwd_bucket& b = a->buckets[i];
-    if (!(b.flags & PAT_BUCKET_TAIL) || b.num_boxes <= 0) continue;
+    if (b.num_boxes <= 0) continue;
     const int64_t width = (int64_t)b.max_blocks * a->page_size;
-    steps = std::max(steps, (double)ceil_div64(width, kStepTokens));
-    bytes += (double)b.num_boxes * width * a->kv_heads * a->head_dim * 4.;
+    if (b.flags & PAT_BUCKET_TAIL) {
+      steps = std::max(steps, (double)ceil_div64(width, kStepTokens));
+      bytes += (double)b.num_boxes * width * a->kv_heads * a->head_dim * 4.;
+    } else if (row_tiles(b.mnw[0]) > 1) {
+      super_steps = std::max(super_steps, (double)width / (2 * kStepTokens));
+    }
   }
   steps *= std::max(1, (with.pairs ? 32 : 16) / group);
-  if (steps > 2. && with.total_wgs < 5 * kNumCUs / 8) return false;
-  if (steps > 4. && 4 * with.total_wgs < 3 * kNumCUs * ceil_div64(with.total_wgs, kNumCUs)) return false;
-  const double own_places = resident_wgs_per_cu(a->head_dim, without.tall_rows) * kNumCUs;
-  const double with_us = std::max(steps * kTailStepUs * std::max(1., (double)with.total_wgs / (resident_wgs_per_cu(a->head_dim, 32) * kNumCUs)), bytes / 6e6);
-  const double own_us = std::max(bytes / 5.8e6, kTailRoundUs * std::max(0., (double)without.total_wgs / own_places - 1.)) *
-                        std::min(1., (double)with.total_wgs / kNumCUs);
-  const double merge_us = 3. + (double)a->batch * a->heads * without.num_slots * a->head_dim * 4. / 4.5e6;
-  return with_us < 0.8 * (own_us + merge_us);
+  if (steps > 4. && with.total_wgs > kNumCUs && 8 * with.total_wgs <= 9 * kNumCUs) return false;
+  const double per_cu = (double)with.total_wgs / kNumCUs;
+  const double rounds = std::ceil(per_cu / resident_wgs_per_cu(a->head_dim, 32));
+  const double stream_us = bytes / 6e6;
+  const double costs_us = std::max(steps * kTailStepUs * rounds, stream_us) + 3. * super_steps * std::max(0., 1. - per_cu);
+  const double more_rounds = std::max(0., (double)without.total_wgs / (resident_wgs_per_cu(a->head_dim, without.tall_rows) * kNumCUs) - 1.);
+  const double kept = std::min(1., per_cu), partial_bytes = (double)a->batch * a->heads * without.num_slots * a->head_dim * 4.;
+  const double saves_us = std::max(bytes / 8.3e6, kTailRoundUs * more_rounds) * kept + 10. + partial_bytes / 2.8e6 +
+                          (without.tall_rows == 16 ? 0.7 * super_steps * std::max(1., per_cu) : 0.);
+  if (costs_us >= 0.9 * saves_us) return false;
+  bool same_walk = without.tall_rows == 32;
+  for (int i = 0; i < a->num_buckets; ++i)
+    same_walk = same_walk && (a->buckets[i].num_boxes <= 0 || row_tiles(a->buckets[i].mnw[0]) == 1 || without.bucket_chunks[i] == 1);
+  if (same_walk) return true;
+  return (steps <= 2. || 8 * with.total_wgs >= 5 * kNumCUs) &&
+         std::max(steps * kTailStepUs * std::max(1., per_cu / resident_wgs_per_cu(a->head_dim, 32)), stream_us) <
+             std::max(bytes / 5.8e6, 4. * more_rounds) * kept + 3. + partial_bytes / 4.5e6;
 }
 
 // (Every launch comes through here, and small ones wait for the host: the overrides are read once, and arguments without tails are made only

@@ -108,7 +108,7 @@ __device__ __forceinline__ void load_to_lds(const char* base, unsigned lane_offs
 // whose records may ask for V past the caches (kRecordModeStreamV): a second loop over short boxes, whose mere presence cost
 // the smallest launches 0.14 us of 5.5.
 // WAVES: 4, or 8 in instances without a tall path (TALLK 0) for single launches of few workgroups whose boxes are more than eight steps
-// long: a wave has half the steps, each a trip to memory behind the last (us per call: 8 requests of 288 tokens, 8 kv heads of 64, 64 workgroups, 5.47 / 4.66;
+// long: a wave has half the steps, each a trip to memory behind the last (us per call: 8 requests of 288 tokens, 8 kv heads of 64, 64 workgroups, 5.5 / 4.7;
 // 2 of 306..459 at 64/8, head_dim 64, 6.5 / 5.3; 17 of 188..282 at 8/8, head_dim 128, 6.8 / 6.3); and for launches of such boxes in pieces of
 // double length, a workgroup per CU (8 of 2239 at 64/8, head_dim 128, 384 workgroups of four / 192 of eight, 18.1 / 16.9).
 // TAILS instances (32-row form): tall workgroups also walk the tails of their rows' sequences.
@@ -943,7 +943,7 @@ __global__ void __launch_bounds__(WAVES * 64, TALLK == 0 ? WAVES / 4 : split_occ
     // Launches of more short private boxes than places (a step of K and V each, the requests' own ends): a workgroup of one of
     // them is 4-5 us of launch, record, page ids and first tiles for 0.5 us of work, and the boxes beyond the places wait for as
     // long again. Here that is paid once per list, and a further box costs 2-2.5 us, a trip to memory of which its neighbour's
-    // arithmetic covers part (512 requests of 1408 + 32 tokens at 16/8 heads: 32.0 us per call, 28.7 in lists of four).
+    // arithmetic covers part (512 requests of 1408 + 32 tokens at 16/8 heads: 30.6 us per call, 27.3 in lists of four).
     const int count = ntok_u, pages = p.list_pages, most = p.list_boxes;
     const int seq_l = lane < count ? rows_tab[min(lane, record_max_seqs - 1)] : -1;
     const int slot_l = lane < count ? rows_tab[record_max_seqs + min(lane, record_max_seqs - 1)] : -1;

@@ -315,17 +315,28 @@ def test_an_item_count_that_is_none_is_refused():
         assert (lib.pat_fwd_validate(C.byref(a)) == 0) is ok, items
 
 
-def test_not_taken_where_the_last_round_of_workgroups_is_thin(tuning):
-    # a wave of more than four steps of tails: the tall workgroups fill the CUs three quarters of every round, or the launch ends on a few
+def test_lines_of_the_rule(tuning):
     lib, g = _lib.load(), _lib.FwdGeometry()
     leaf = _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_TAIL | 1 << _lib.PAT_TAIL_BOXES_SHIFT
 
-    def tails(boxes, tokens):         # 8 requests a box, in twos: four a wave; 8 kv heads
-        a = _tail_args((64, 2 * boxes, 8, 1248, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS | _lib.PAT_BUCKET_TAILS, boxes), (16, 16 * boxes, 1, tokens, leaf, 0),
-                       64, 8, 128, 16 * boxes, 16)
+    def tails(items, tokens, shared=1248, d=128, heads=(64, 8), page=16):         # boxes of 64 rows in twos, and an end a request
+        seqs = 64 * heads[1] // heads[0]
+        a = _tail_args((64, 2 * items, seqs, shared, _lib.PAT_BUCKET_EVEN | _lib.PAT_BUCKET_ITEMS | _lib.PAT_BUCKET_TAILS, items),
+                       (16, 2 * items * seqs, 1, tokens, leaf, 0), *heads, d, 2 * items * seqs, page)
         assert lib.pat_fwd_geometry_of(C.byref(a), C.byref(g)) == 0, _lib.last_error()
         return bool(g.flags & _lib.PAT_GEOMETRY_TAILS)
 
     tuning()
-    assert [tails(n, 64) for n in (32, 33, 47, 48, 64)] == [True, False, False, True, True]    # 256, 264, 376, 384 and 512 workgroups
+    # more than four steps a wave: not where up to an eighth of the CUs have two workgroups (256, 264, 288, 296 and 512 workgroups)
+    assert [tails(n, 64) for n in (32, 33, 36, 37, 64)] == [True, False, False, True, True]
     assert tails(33, 32) is True                                                                # four steps
+    # tall boxes that leave CUs idle and would be cut: not where they are long
+    assert tails(23, 16, shared=384) and not tails(18, 64, shared=1504) and not tails(16, 32, shared=4096)
+    # many ends a wave
+    assert not tails(8, 16, shared=768, heads=(16, 16))
+    # a launch that would be in the 16-row form, which rounds less: where the ends and the merge alone pay, not for the form's sake
+    for shared, taken in ((384, True), (64, False)):
+        tuning(pairs=_lib.PAT_TAILS_NEVER)
+        assert tails(23, 16, shared=shared, d=64) is False and g.tall_rows == 16
+        tuning()
+        assert tails(23, 16, shared=shared, d=64) is taken
