@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -34,7 +35,9 @@ struct pat_tree {
   std::unique_ptr<pat::RadixPlanner> planner;
   std::vector<int32_t> child_scratch;
   // Between the call that asks how large the flat plan is and the one that writes it (half of the two was laying it out again).
+  // Both are const calls: whoever uses it takes it away, and a call that finds nothing lays it out itself.
   mutable std::unique_ptr<FlatPlan> flat;
+  mutable std::mutex flat_mutex;
 };
 
 namespace pat {
@@ -414,15 +417,21 @@ static int flat_plan_impl(const pat_tree* tree, pat_flat_plan* layout, int32_t* 
   if (tree == nullptr || layout == nullptr) return pat::fail(PAT_ERR_INVALID, "tree / layout is NULL");
   const pat::Plan& p = tree->planner->plan();
   if (!p.valid) return pat::fail(PAT_ERR_INVALID, "no plan: call pat_tree_pack first");
-  if (!tree->flat) {
-    auto fresh = std::make_unique<FlatPlan>();
-    if (int rc = lay_out(p, tree->block_size, *fresh)) return rc;
-    tree->flat = std::move(fresh);
+  std::unique_ptr<FlatPlan> f;
+  {
+    const std::lock_guard<std::mutex> lock(tree->flat_mutex);
+    f = std::move(tree->flat);
   }
-  *layout = tree->flat->layout;
-  if (dst == nullptr) return PAT_OK;
-  if (capacity < layout->total) return pat::fail(PAT_ERR_INVALID, "flat plan: buffer too small");
-  const std::unique_ptr<FlatPlan> f = std::move(tree->flat);   // (given back once it is written)
+  if (!f) {
+    f = std::make_unique<FlatPlan>();
+    if (int rc = lay_out(p, tree->block_size, *f)) return rc;
+  }
+  *layout = f->layout;
+  if (dst == nullptr || capacity < layout->total) {
+    const std::lock_guard<std::mutex> lock(tree->flat_mutex);
+    tree->flat = std::move(f);
+    return dst == nullptr ? PAT_OK : pat::fail(PAT_ERR_INVALID, "flat plan: buffer too small");
+  }
   const auto& order = f->order;
 
   // contents

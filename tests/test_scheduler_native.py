@@ -345,3 +345,34 @@ def test_a_flat_plan_is_that_of_the_plan_as_it_is(edit):
     assert again[0] == got[0] and torch.equal(again[1], got[1])
     for h in (asked, fresh):
         lib.pat_tree_destroy(h)
+
+
+def test_a_flat_plan_may_be_asked_for_by_several_threads():
+    # a const call: what it keeps between asking for the size and writing is handed on whole, or laid out again
+    import threading
+    lib, h = _lib.load(), C.c_void_p()
+    rows = [list(range(20)) + [20 + i] for i in range(2000)]
+    table = torch.tensor(rows, dtype=torch.int32)
+    assert lib.pat_tree_create(16, C.byref(h)) == 0
+    assert lib.pat_tree_build(h, (C.c_int32 * 2000)(*[16 * 20 + 5] * 2000), C.cast(table.data_ptr(), _lib.i32p), 2000, 21) == 0
+    assert lib.pat_tree_pack(h, None, 0, 8, 8, 0, None) == 0
+    want, first = torch.full((1 << 17,), -99, dtype=torch.int32), _lib.FlatPlan()
+    assert lib.pat_tree_flat_plan(h, C.byref(first), want.data_ptr(), want.numel()) == 0
+    wrong = []
+
+    def ask():
+        f, buf = _lib.FlatPlan(), torch.full((1 << 17,), -99, dtype=torch.int32)
+        for _ in range(150):
+            if lib.pat_tree_flat_plan(h, C.byref(f), None, 0) != 0 or bytes(f) != bytes(first):
+                wrong.append("layout")
+            if lib.pat_tree_flat_plan(h, C.byref(f), buf.data_ptr(), buf.numel()) != 0 or bytes(f) != bytes(first) or not torch.equal(buf, want):
+                wrong.append("contents")
+            buf.fill_(-99)
+
+    threads = [threading.Thread(target=ask) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    lib.pat_tree_destroy(h)
