@@ -526,8 +526,11 @@ struct KernelInfo {
   void bind(const at::Tensor& buf) {
     clear_tables();
     const pat_flat_plan& lay = layout;
-    auto vec = [&](int64_t off, int64_t n) { return buf.narrow(0, off, n); };
-    auto mat = [&](int64_t off, int64_t n, int64_t w) { return buf.narrow(0, off, n * w).view({n, w}); };
+    // (one view operation per table: a decode step makes them twice, on the host buffer and on its copy; with narrow and view a bucket
+    // more, as tails often are, was 10 us each time)
+    const int64_t at0 = buf.storage_offset();
+    auto vec = [&](int64_t off, int64_t n) { return buf.as_strided({n}, {1}, at0 + off); };
+    auto mat = [&](int64_t off, int64_t n, int64_t w) { return buf.as_strided({n, w}, {std::max<int64_t>(w, 1), 1}, at0 + off); };
     num_split_per_seq = vec(lay.num_split_per_seq, lay.batch);
     num_boxes_per_seq = vec(lay.num_boxes_per_seq, lay.batch);
     for (int b = 0; b < lay.num_buckets; ++b) {

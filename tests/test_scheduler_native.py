@@ -376,3 +376,27 @@ def test_a_flat_plan_may_be_asked_for_by_several_threads():
         t.join()
     assert not wrong
     lib.pat_tree_destroy(h)
+
+
+@pytest.mark.parametrize("seqs,own", [(35, 9), (64, 200), (1, 40)])
+def test_plan_tensors_are_views_of_one_buffer(seqs, own):
+    # contiguous, in bounds, and with one version counter: an edit of any of them is seen by whoever watches another
+    rows = [list(range(20)) + [20 + 16 * i + j for j in range(-(-own // 16))] for i in range(seqs)]
+    tree = PrefixTreeCPP(16)
+    tree.build_radix_tree([16 * 20 + own] * seqs, torch.tensor(rows, dtype=torch.int32))
+    tree.pack_schedule(None, 4, 8)
+    info = tree.kernel_info
+    launch = info.launch_tables()
+    tables = [info.num_split_per_seq, info.num_boxes_per_seq]
+    for l in (info.q_tables, info.slot_tables, info.block_tables, info.num_seqs_per_CTAs, info.CTA_ranks, info.kv_in_CTAs, launch["q_tables"],
+              launch["slot_tables"], launch["block_tables"], launch["num_seqs_per_CTAs"], launch["CTA_ranks"], launch["kv_in_CTAs"], launch["items"]):
+        tables += list(l)
+    storage = tables[0].untyped_storage()
+    for t in tables:
+        assert t.is_contiguous() and t.stride(-1) == 1 and t.untyped_storage().data_ptr() == storage.data_ptr()
+        assert 4 * (t.storage_offset() + t.numel()) <= storage.nbytes()
+    before = [t._version for t in tables]
+    info.kv_in_CTAs[-1].add_(0)
+    assert len(set(before)) == 1 and [t._version for t in tables] == [v + 1 for v in before]
+    for b, q in enumerate(info.q_tables):
+        assert q.shape == info.slot_tables[b].shape and q.shape[0] == info.block_tables[b].shape[0] == info.kv_in_CTAs[b].shape[0]
